@@ -97,7 +97,7 @@ struct larql_hip_ctx {
     std::mutex mu;
     std::string name, info, last_error;
     std::vector<Region> regions;
-    DevBuf w[kHostMats], aux[kHostMats], x, out, tables[kTableSlots], misc, scores, q8, q8s, parts;
+    DevBuf w[kHostMats], aux[kHostMats], x, out, tables[kTableSlots], misc, scores, q8, q8s, parts, topk;
     // pinned staging for job tables: the upload is asynchronous, the event says when a slot may be rewritten
     void *table_host[kTableSlots] = {};
     size_t table_host_cap[kTableSlots] = {};
@@ -484,6 +484,15 @@ int enqueue_jobs(larql_hip_ctx *c, std::vector<GemvJob> &jobs_in) {
     return LARQL_OK;
 }
 
+// top-K over rows of device scores, with the workspace that long rows are selected through
+int run_topk(larql_hip_ctx *c, const float *scores, uint32_t batch, uint32_t n, uint32_t k, bool by_abs, uint32_t *idx, float *val,
+             uint32_t *count, int *nan_flag) {
+    const size_t ws = topk_workspace_bytes(batch, n, k);
+    if (ws) { int rc = ensure(c, c->topk, ws); if (rc) return rc; }
+    HIPCHECK(c, topk_launch(c->stream, scores, batch, n, k, by_abs, idx, val, count, nan_flag, c->topk.p, ws));
+    return LARQL_OK;
+}
+
 GemvJob make_job(int kind, const void *w, const void *aux, const void *x, float *out, uint64_t rows, uint64_t k) {
     GemvJob j;
     memset(&j, 0, sizeof j);
@@ -556,7 +565,7 @@ void larql_hip_destroy(larql_hip_ctx *c) {
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     for (Region &r : c->regions) (void)hipFree(r.dev);
-    DevBuf *bufs[] = {&c->x, &c->out, &c->misc, &c->scores, &c->q8, &c->q8s, &c->parts};
+    DevBuf *bufs[] = {&c->x, &c->out, &c->misc, &c->scores, &c->q8, &c->q8s, &c->parts, &c->topk};
     for (DevBuf &t : c->tables) if (t.p) (void)hipFree(t.p);
     for (DevBuf *b : bufs) if (b->p) (void)hipFree(b->p);
     for (size_t i = 0; i < kHostMats; i++) {
@@ -1017,8 +1026,9 @@ static int host_matvec_topk(larql_hip_ctx *c, int kind, const uint8_t *w, size_t
     Submission sub(c);
     rc = enqueue_jobs(c, jobs);
     if (rc) { (void)wait_stream(c); return rc; }
-    HIPCHECK(c, topk_launch(c->stream, (const float *)c->scores.p, 1, (uint32_t)num_rows, (uint32_t)top_k, false, hits.idx, hits.val,
-                            hits.cnt, c->nan_flag + 1, nullptr, 0));
+    rc = run_topk(c, (const float *)c->scores.p, 1, (uint32_t)num_rows, (uint32_t)top_k, false, hits.idx, hits.val,
+                  hits.cnt, c->nan_flag + 1);
+    if (rc) return rc;
     rc = topk_queue_flag(c, hits);
     if (rc) return rc;
     rc = sub.finish();
@@ -1358,8 +1368,9 @@ int larql_hip_gate_knn(larql_hip_ctx *c, int format, const uint8_t *gate, size_t
     Submission sub(c);
     rc = dev_gate_scores(c, kind, dg, (const float *)c->x.p, batch, n, hidden, (float *)c->scores.p);
     if (rc) { (void)wait_stream(c); return rc; }
-    HIPCHECK(c, topk_launch(c->stream, (const float *)c->scores.p, (uint32_t)batch, (uint32_t)n, (uint32_t)top_k, true, hits.idx,
-                            hits.val, hits.cnt, c->nan_flag + 1, nullptr, 0));
+    rc = run_topk(c, (const float *)c->scores.p, (uint32_t)batch, (uint32_t)n, (uint32_t)top_k, true, hits.idx,
+                  hits.val, hits.cnt, c->nan_flag + 1);
+    if (rc) return rc;
     rc = topk_queue_flag(c, hits); if (rc) return rc;
     rc = sub.finish();
     if (rc) return rc;
@@ -1630,8 +1641,9 @@ int larql_hip_dev_gate_knn(larql_hip_ctx *c, int format, const void *gate, const
     if (!count_out) { rc = ensure(c, c->misc, batch * 4 + 64); if (rc) return rc; count_out = (uint32_t *)c->misc.p; }
     rc = dev_gate_scores(c, kind, gate, x, batch, n, hidden, scores_scratch);
     if (rc) return rc;
-    HIPCHECK(c, topk_launch(c->stream, scores_scratch, (uint32_t)batch, (uint32_t)n, (uint32_t)top_k, true, idx_out, score_out,
-                            count_out, c->nan_flag, nullptr, 0));
+    rc = run_topk(c, scores_scratch, (uint32_t)batch, (uint32_t)n, (uint32_t)top_k, true, idx_out, score_out,
+                  count_out, c->nan_flag);
+    if (rc) return rc;
     return LARQL_OK;
 }
 
@@ -1707,8 +1719,9 @@ int larql_hip_dev_gate_knn_static(larql_hip_ctx *c, int format, const void *gate
         if (rc) return rc;
         HIPCHECK(c, gemv_launch(c->stream, P.kind, P.L, P.threads, P.grid, P.lds));
     }
+    // (the matvecs have read the Q8 codes by the time the selection writes there; a row it does not suffice for is streamed)
     HIPCHECK(c, topk_launch(c->stream, scores, (uint32_t)batch, (uint32_t)n, (uint32_t)top_k, true, idx_out, score_out,
-                            count_out ? count_out : counts, c->nan_flag, nullptr, 0));
+                            count_out ? count_out : counts, c->nan_flag, q8, kStaticQ8Bytes));
     return LARQL_OK;
 }
 
@@ -2402,8 +2415,9 @@ int larql_hip_dev_gate_walk(larql_hip_ctx *c, int format, const void *const *gat
         push_gate_jobs(jobs, kind, gates[l], x + l * x_layer_stride, batch, n, hidden, scores_scratch + l * batch * n);
     rc = enqueue_jobs(c, jobs);
     if (rc) return rc;
-    HIPCHECK(c, topk_launch(c->stream, scores_scratch, (uint32_t)(n_layers * batch), (uint32_t)n, (uint32_t)top_k, true, idx_out,
-                            score_out, count_out, c->nan_flag, nullptr, 0));
+    rc = run_topk(c, scores_scratch, (uint32_t)(n_layers * batch), (uint32_t)n, (uint32_t)top_k, true, idx_out,
+                  score_out, count_out, c->nan_flag);
+    if (rc) return rc;
     return LARQL_OK;
 }
 

@@ -23,11 +23,17 @@
 // its up to 16 ordered scores in registers, and a bound with at least 64 scores
 // at or above it (the smallest maximum of 64 slices of the row) usually leaves
 // a few hundred candidates, which are ranked directly; the radix passes remain
-// for rows with more than 1024 candidates and for longer rows (a vocabulary),
-// which are streamed.
+// for rows with more than 1024 candidates.
+// Longer rows (a vocabulary) are selected in two launches: every chunk of a row
+// leaves its own K best keys, sorted, in a workspace, and one workgroup per row
+// selects among those.  One workgroup cannot keep enough loads in flight for a
+// 262144-score row (405 us on one CU, six passes over 1 MB); 64 chunks of 4096
+// plus the merge of their 64 x 64 keys take 18 us together (the lm_head call over
+// 262144 x 2560: 562 -> 174 us).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <atomic>
 
 #include "kernels.h"
@@ -95,52 +101,97 @@ __device__ __forceinline__ uint64_t make_key(float s, uint32_t idx, int *nan_fla
 constexpr int kTopkCached = 16;  // rounds of 64 scores per wavefront held in registers
 constexpr int kTopkCandidates = kTopkThreads;  // candidates of the short way: one per thread
 
+// What a workgroup selects from: `n` scores of a row, cut into chunks of `chunk` (chunk == n: the whole row), or — KEYS_IN —
+// the row's `n` keys that the chunks' workgroups left.  A chunk's workgroup leaves keys (KEYS_OUT): its K best, best
+// first, zeros behind them where it has fewer.
+struct TopkArgs {
+    const float *scores;       // [batch, scores_n]
+    const uint64_t *keys_in;   // KEYS_IN: [batch, n]
+    uint64_t *keys_out;        // KEYS_OUT: [batch, chunks, k]
+    uint32_t *idx_out;
+    float *val_out;
+    uint32_t *count_out;
+    int *nan_flag;
+    uint32_t scores_n, n, chunk, k, cap;
+};
+
+// ROUNDS: scores per thread held in registers (0: streamed on every pass).
 // LARGE (K above 64, up to kTopkMaxK): the selection is the same radix select; the winners are gathered into a
 // power-of-two array in dynamic LDS (`cap` keys, zero-padded) and ordered by a bitonic sort of the whole workgroup.
+// KEYS_IN: equal scores stand in index order in the workspace (chunks in index order, a chunk's keys best first, the
+// lower index before the higher), so the ranking of ties by position serves there too.
 // (80 scalar registers: with the 96 the compiler would take, a second 16-wavefront workgroup was not placed on a CU
 // until half of the first one's wavefronts had left — more rows than CUs then ran in two rounds)
-template <bool BY_ABS, bool CACHED, bool LARGE>
-__global__ void __launch_bounds__(kTopkThreads) __attribute__((amdgpu_num_sgpr(80))) topk_kernel(const float *__restrict__ scores, uint32_t n, uint32_t k,
-                                                            uint32_t *__restrict__ idx_out, float *__restrict__ val_out,
-                                                            uint32_t *__restrict__ count_out, int *nan_flag, uint32_t cap) {
-    static_assert(!(LARGE && CACHED), "the candidate short cut bounds 64 winners only");
+template <bool BY_ABS, int ROUNDS, bool LARGE, bool KEYS_IN, bool KEYS_OUT>
+__global__ void __launch_bounds__(kTopkThreads) __attribute__((amdgpu_num_sgpr(80))) topk_kernel(const TopkArgs A) {
+    constexpr bool CACHED = ROUNDS > 0, SHORT_WAY = CACHED && !LARGE;  // (the candidate short cut bounds 64 winners only)
     extern __shared__ __attribute__((aligned(16))) uint64_t big[];  // LARGE: cap keys
     __shared__ uint32_t hist[256];
     __shared__ uint32_t wave_ties[kTopkWaves];
     __shared__ uint64_t winners[64];
     __shared__ uint32_t sh_prefix, sh_need, sh_nwin, sh_ncand;
     __shared__ uint32_t group_max[64];
-    __shared__ __attribute__((aligned(16))) uint64_t cand[CACHED ? kTopkCandidates + 4 : 1];
-    __shared__ uint32_t rank_sh[CACHED ? kTopkCandidates : 1];  // ranks counted in shares (short way)
-    const uint32_t row = blockIdx.x, tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    const float *s = scores + (size_t)row * n;
+    __shared__ __attribute__((aligned(16))) uint64_t cand[SHORT_WAY ? kTopkCandidates + 4 : 1];
+    __shared__ uint32_t rank_sh[SHORT_WAY ? kTopkCandidates : 1];  // ranks counted in shares (short way)
+    const uint32_t row = blockIdx.y, tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const uint32_t k = A.k, cap = A.cap, first = blockIdx.x * A.chunk, n = min(A.chunk, A.n - first);
+    int *const nan_flag = A.nan_flag;
+    const float *const srow = A.scores + (size_t)row * A.scores_n;
+    const float *const s = srow + first;
+    const uint64_t *const keys = KEYS_IN ? A.keys_in + (size_t)row * A.n + first : nullptr;
+    uint64_t *const kout = KEYS_OUT ? A.keys_out + ((size_t)row * gridDim.x + blockIdx.x) * k : nullptr;
     // wavefront w owns the contiguous indices [w0, w1), 64 at a time (lane = index within the 64)
     const uint32_t perw = ((n + kTopkWaves * 64 - 1) / (kTopkWaves * 64)) * 64;
     const uint32_t w0 = min(n, wave * perw), w1 = min(n, w0 + perw);
 
-    // the ordered score of index i (0: nothing there), from the register copy or from memory
-    uint32_t cache[CACHED ? kTopkCached : 1];
-    if (CACHED) {
+    // winner number `rank` of the row (or of the chunk)
+    auto emit = [&](uint32_t rank, uint64_t key) {
+        if (KEYS_OUT) {
+            kout[rank] = key;
+        } else {
+            const uint32_t idx = ~(uint32_t)key;
+            A.idx_out[(size_t)row * k + rank] = idx;
+            A.val_out[(size_t)row * k + rank] = srow[idx];
+        }
+    };
+    // index i as a key: its ordered score (0: nothing there) and the low word, from the register copy or from memory
+    uint32_t cache[CACHED ? ROUNDS : 1], low[KEYS_IN && CACHED ? ROUNDS : 1];
+    if (CACHED && KEYS_IN) {
+        uint64_t raw[CACHED ? ROUNDS : 1];
+#pragma unroll
+        for (int it = 0; it < ROUNDS; it++) raw[it] = keys[min(w0 + it * 64 + lane, n - 1)];
+#pragma unroll
+        for (int it = 0; it < ROUNDS; it++) {
+            cache[it] = w0 + it * 64 + lane < w1 ? (uint32_t)(raw[it] >> 32) : 0u;
+            low[it] = (uint32_t)raw[it];
+        }
+    } else if (CACHED) {
         // every load leaves before the first score is looked at (a load inside a condition is waited for where it
         // stands: sixteen round trips instead of one); an index past the wavefront's range reads the row's last score
-        float raw[kTopkCached];
+        float raw[CACHED ? ROUNDS : 1];
 #pragma unroll
-        for (int it = 0; it < kTopkCached; it++) raw[it] = s[min(w0 + it * 64 + lane, n - 1)];
+        for (int it = 0; it < ROUNDS; it++) raw[it] = s[min(w0 + it * 64 + lane, n - 1)];
 #pragma unroll
-        for (int it = 0; it < kTopkCached; it++) {
+        for (int it = 0; it < ROUNDS; it++) {
             const uint32_t i = w0 + it * 64 + lane;
             cache[it] = i < w1 ? (uint32_t)(make_key<BY_ABS>(raw[it], i, nan_flag) >> 32) : 0u;
         }
     }
-    // f(ord, i) for every index of this wavefront, 64 at a time, all lanes taking part in every round
+    auto low_word = [&](int it) -> uint32_t { return KEYS_IN ? low[KEYS_IN && CACHED ? it : 0] : ~(first + w0 + it * 64 + lane); };
+    // f(ord, low) for every index of this wavefront, 64 at a time, all lanes taking part in every round
     auto for_each = [&](auto &&f, int *flag) {
         if (CACHED) {
 #pragma unroll
-            for (int it = 0; it < kTopkCached; it++) f(cache[it], w0 + it * 64 + lane);
+            for (int it = 0; it < ROUNDS; it++) f(cache[it], low_word(it));
         } else {
             for (uint32_t base = w0; base < w1; base += 64) {
                 const uint32_t i = base + lane;
-                f(i < w1 ? (uint32_t)(make_key<BY_ABS>(s[i], i, flag) >> 32) : 0u, i);
+                if (KEYS_IN) {
+                    const uint64_t key = i < w1 ? keys[i] : 0ull;
+                    f((uint32_t)(key >> 32), (uint32_t)key);
+                } else {
+                    f(i < w1 ? (uint32_t)(make_key<BY_ABS>(s[i], i, flag) >> 32) : 0u, ~(first + i));
+                }
             }
         }
     };
@@ -149,7 +200,7 @@ __global__ void __launch_bounds__(kTopkThreads) __attribute__((amdgpu_num_sgpr(8
     if (LARGE)
         for (uint32_t i = tid; i < cap; i += kTopkThreads) big[i] = 0;
     if (tid == 0) { sh_prefix = 0; sh_need = k; sh_nwin = 0; sh_ncand = 0; }
-    if (CACHED) {
+    if (SHORT_WAY) {
         // ---- short way for a row held in registers.  The 64 groups of 16 lanes each own a slice of the row; the
         //      smallest of the 64 group maxima, L, has at least 64 scores at or above it (one per group), so the
         //      winners are among the scores >= L: a few hundred of a typical row.  Those are collected and each one
@@ -157,13 +208,21 @@ __global__ void __launch_bounds__(kTopkThreads) __attribute__((amdgpu_num_sgpr(8
         //      candidates do not fit (sorted input, a group without valid scores) takes the radix passes below. ----
         uint32_t gmax = 0;
 #pragma unroll
-        for (int it = 0; it < kTopkCached; it++) gmax = max(gmax, cache[it]);
-        // (reductions by DPP row operations: a few cycles each, where a cross-lane shuffle costs an LDS round trip)
-        gmax = max(gmax, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)gmax, 0xB1, 0xF, 0xF, true));   // quad_perm [1,0,3,2]
-        gmax = max(gmax, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)gmax, 0x4E, 0xF, 0xF, true));   // quad_perm [2,3,0,1]
-        gmax = max(gmax, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)gmax, 0x141, 0xF, 0xF, true));  // row_half_mirror
-        gmax = max(gmax, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)gmax, 0x140, 0xF, 0xF, true));  // row_mirror
-        if ((lane & 15u) == 0) group_max[wave * 4 + (lane >> 4)] = gmax;
+        for (int it = 0; it < ROUNDS; it++) gmax = max(gmax, cache[it]);
+        if (KEYS_IN) {
+            // a chunk's keys stand best first: slices of every fourth lane each hold one of the four best of every chunk
+            // (slices of 16 neighbours would leave the worst of a chunk to themselves and bound nothing)
+#pragma unroll
+            for (int o = 4; o < 64; o <<= 1) gmax = max(gmax, (uint32_t)__shfl_xor((int)gmax, o, 64));
+            if (lane < 4u) group_max[wave * 4 + lane] = gmax;
+        } else {
+            // (reductions by DPP row operations: a few cycles each, where a cross-lane shuffle costs an LDS round trip)
+            gmax = max(gmax, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)gmax, 0xB1, 0xF, 0xF, true));   // quad_perm [1,0,3,2]
+            gmax = max(gmax, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)gmax, 0x4E, 0xF, 0xF, true));   // quad_perm [2,3,0,1]
+            gmax = max(gmax, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)gmax, 0x141, 0xF, 0xF, true));  // row_half_mirror
+            gmax = max(gmax, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)gmax, 0x140, 0xF, 0xF, true));  // row_mirror
+            if ((lane & 15u) == 0) group_max[wave * 4 + (lane >> 4)] = gmax;
+        }
         __syncthreads();
         uint32_t L = group_max[lane];
         L = min(L, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)L, 0xB1, 0xF, 0xF, false));
@@ -177,16 +236,16 @@ __global__ void __launch_bounds__(kTopkThreads) __attribute__((amdgpu_num_sgpr(8
             // a wavefront reserves room for all its candidates at once, then places them round by round
             uint32_t mine = 0;
 #pragma unroll
-            for (int it = 0; it < kTopkCached; it++) mine += (uint32_t)__popcll(__ballot(cache[it] >= L));
+            for (int it = 0; it < ROUNDS; it++) mine += (uint32_t)__popcll(__ballot(cache[it] >= L));
             uint32_t base = 0;
             if (lane == 0 && mine) base = atomicAdd(&sh_ncand, mine);
             base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
 #pragma unroll
-            for (int it = 0; it < kTopkCached; it++) {
+            for (int it = 0; it < ROUNDS; it++) {
                 const bool c = cache[it] >= L;
                 const uint64_t m = __ballot(c);
                 const uint32_t pos = base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-                if (c && pos < (uint32_t)kTopkCandidates) cand[pos] = ((uint64_t)cache[it] << 32) | (uint32_t)(~(w0 + it * 64 + lane));
+                if (c && pos < (uint32_t)kTopkCandidates) cand[pos] = ((uint64_t)cache[it] << 32) | low_word(it);
                 base += (uint32_t)__popcll(m);
             }
             __syncthreads();
@@ -221,12 +280,8 @@ __global__ void __launch_bounds__(kTopkThreads) __attribute__((amdgpu_num_sgpr(8
                     __syncthreads();
                     if (tid < nc) rank = rank_sh[tid];
                 }
-                if (tid < nc && rank < k) {  // (tid < nc: ci == tid, the key is this thread's candidate)
-                    const uint32_t idx = ~(uint32_t)key;
-                    idx_out[(size_t)row * k + rank] = idx;
-                    val_out[(size_t)row * k + rank] = s[idx];
-                }
-                if (tid == 0) count_out[row] = min(k, nc);
+                if (tid < nc && rank < k) emit(rank, key);  // (tid < nc: ci == tid, the key is this thread's candidate)
+                if (!KEYS_OUT && tid == 0) A.count_out[row] = min(k, nc);  // (a chunk's nc is at least 64)
                 return;
             }
         }
@@ -287,8 +342,8 @@ __global__ void __launch_bounds__(kTopkThreads) __attribute__((amdgpu_num_sgpr(8
     uint32_t tie_rank = 0;  // ties at lower indices than this wavefront's current 64
     for (uint32_t w = 0; w < wave; w++) tie_rank += wave_ties[w];
     // ---- gather the winners ----
-    for_each([&](uint32_t ord, uint32_t i) {
-        const uint64_t key = ((uint64_t)ord << 32) | (uint32_t)(~i);
+    for_each([&](uint32_t ord, uint32_t lo) {
+        const uint64_t key = ((uint64_t)ord << 32) | lo;
         bool in = ord != 0 && ord > T;
         if (!take_all) {
             const bool tie = ord != 0 && ord == T;
@@ -319,56 +374,97 @@ __global__ void __launch_bounds__(kTopkThreads) __attribute__((amdgpu_num_sgpr(8
             }
         }
         const uint32_t nw = min(min(sh_nwin, cap), k);
-        for (uint32_t i = tid; i < nw; i += kTopkThreads) {
-            const uint32_t idx = ~(uint32_t)big[i];
-            idx_out[(size_t)row * k + i] = idx;
-            val_out[(size_t)row * k + i] = s[idx];
-        }
-        if (tid == 0) count_out[row] = nw;
+        for (uint32_t i = tid; i < nw; i += kTopkThreads) emit(i, big[i]);
+        if (KEYS_OUT) for (uint32_t i = nw + tid; i < k; i += kTopkThreads) kout[i] = 0ull;
+        else if (tid == 0) A.count_out[row] = nw;
         return;
     }
     if (wave == 0) {
         const uint64_t top = sort_desc(winners[lane], lane);
         const bool valid = top != 0 && lane < k;
-        if (valid) {
-            const uint32_t idx = ~(uint32_t)top;
-            idx_out[(size_t)row * k + lane] = idx;
-            val_out[(size_t)row * k + lane] = s[idx];
-        }
+        if (KEYS_OUT ? lane < k : valid) emit(lane, top);
         const uint64_t mask = __ballot(valid);
-        if (lane == 0) count_out[row] = (uint32_t)__popcll(mask);
+        if (!KEYS_OUT && lane == 0) A.count_out[row] = (uint32_t)__popcll(mask);
     }
 }
 
-size_t topk_workspace_bytes(uint32_t, uint32_t, uint32_t) { return 0; }
+// How a row is cut.  A row that one workgroup can hold in registers is not: two launches cost 4 us more than one.  Above
+// that, K <= 64 takes chunks of 4096 (four scores a thread; 16 times as many where the chunks' winners would not fit the
+// merging workgroup's registers), a larger K chunks of 16384 while they shrink the row to a quarter at least.
+static uint32_t topk_chunk(uint32_t n, uint32_t k) {
+    constexpr uint32_t held = kTopkThreads * kTopkCached, small = held / 4;
+    if (n <= held) return n;
+    if (k <= 64) {
+        for (uint32_t chunk : {small, held})
+            if ((uint64_t)((n + chunk - 1) / chunk) * k <= held) return chunk;
+        return n;
+    }
+    return k <= held / 4 && n <= 0x7FFFFFFFu ? held : n;
+}
+
+size_t topk_workspace_bytes(uint32_t batch, uint32_t n, uint32_t k) {
+    const uint32_t chunk = n ? topk_chunk(n, k) : n;
+    return chunk == n ? 0 : (size_t)batch * ((n + chunk - 1) / chunk) * k * sizeof(uint64_t);
+}
+
+// one launch over `batch` rows of `chunks` chunks each
+template <bool BY_ABS, int ROUNDS, bool LARGE, bool KEYS_IN, bool KEYS_OUT>
+static hipError_t topk_stage(hipStream_t stream, TopkArgs A, uint32_t chunks, uint32_t batch) {
+    size_t lds = 0;
+    if (LARGE) {
+        // more than 64 winners: ordered in LDS (room for the next power of two above min(k, n) keys)
+        A.cap = 128;
+        while (A.cap < A.k && A.cap < A.n) A.cap <<= 1;
+        lds = (size_t)A.cap * sizeof(uint64_t);
+        static std::atomic<bool> allowed{false};
+        if (!allowed) {  // dynamic LDS above 64 KB has to be allowed once per process
+            hipError_t e = hipFuncSetAttribute((const void *)topk_kernel<BY_ABS, ROUNDS, LARGE, KEYS_IN, KEYS_OUT>,
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kTopkMaxK * sizeof(uint64_t)));
+            if (e != hipSuccess) return e;
+            allowed = true;
+        }
+    }
+    hipLaunchKernelGGL((topk_kernel<BY_ABS, ROUNDS, LARGE, KEYS_IN, KEYS_OUT>), dim3(chunks, batch), dim3(kTopkThreads), lds, stream, A);
+    return hipGetLastError();
+}
+
+template <bool BY_ABS>
+static hipError_t topk_rows(hipStream_t stream, TopkArgs A, uint32_t batch, void *workspace, size_t workspace_bytes) {
+    const bool large = A.k > 64 && A.n > 64;
+    const size_t need = topk_workspace_bytes(batch, A.n, A.k);
+    A.chunk = A.n;
+    if (need && workspace && workspace_bytes >= need) {
+        const uint32_t chunk = topk_chunk(A.n, A.k), chunks = (A.n + chunk - 1) / chunk;
+        A.chunk = chunk;
+        A.keys_out = (uint64_t *)workspace;
+        hipError_t e = large ? topk_stage<BY_ABS, kTopkCached, true, false, true>(stream, A, chunks, batch)
+                       : chunk <= kTopkThreads * kTopkCached / 4 ? topk_stage<BY_ABS, kTopkCached / 4, false, false, true>(stream, A, chunks, batch)
+                                                                 : topk_stage<BY_ABS, kTopkCached, false, false, true>(stream, A, chunks, batch);
+        if (e != hipSuccess) return e;
+        A.keys_in = A.keys_out;
+        A.n = A.chunk = chunks * A.k;
+        if (A.n > kTopkThreads * kTopkCached) return topk_stage<false, 0, true, true, false>(stream, A, 1, batch);
+        return large ? topk_stage<false, kTopkCached, true, true, false>(stream, A, 1, batch)
+                     : topk_stage<false, kTopkCached, false, true, false>(stream, A, 1, batch);
+    }
+    const bool cached = A.n <= (uint32_t)(kTopkThreads * kTopkCached);
+    if (large) return cached ? topk_stage<BY_ABS, kTopkCached, true, false, false>(stream, A, 1, batch) : topk_stage<BY_ABS, 0, true, false, false>(stream, A, 1, batch);
+    return cached ? topk_stage<BY_ABS, kTopkCached, false, false, false>(stream, A, 1, batch) : topk_stage<BY_ABS, 0, false, false, false>(stream, A, 1, batch);
+}
 
 hipError_t topk_launch(hipStream_t stream, const float *scores, uint32_t batch, uint32_t n, uint32_t k, bool by_abs,
-                       uint32_t *idx_out, float *val_out, uint32_t *count_out, int *nan_flag, void *, size_t) {
-    if (batch == 0) return hipSuccess;
+                       uint32_t *idx_out, float *val_out, uint32_t *count_out, int *nan_flag, void *workspace, size_t workspace_bytes) {
     if (k > kTopkMaxK) return hipErrorInvalidValue;
-    if (k > 64 && n > 64) {
-        // more than 64 winners: ordered in LDS (room for the next power of two above min(k, n) keys)
-        uint32_t cap = 128;
-        while (cap < k && cap < n) cap <<= 1;
-        const size_t lds = (size_t)cap * sizeof(uint64_t);
-        static std::atomic<bool> attr_abs{false}, attr_val{false};
-        std::atomic<bool> &flag = by_abs ? attr_abs : attr_val;
-        if (!flag) {  // dynamic LDS above 64 KB has to be allowed once per process
-            const void *fn = by_abs ? (const void *)topk_kernel<true, false, true> : (const void *)topk_kernel<false, false, true>;
-            hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kTopkMaxK * sizeof(uint64_t)));
-            if (e != hipSuccess) return e;
-            flag = true;
-        }
-        if (by_abs) hipLaunchKernelGGL((topk_kernel<true, false, true>), dim3(batch), dim3(kTopkThreads), lds, stream, scores, n, k, idx_out, val_out, count_out, nan_flag, cap);
-        else hipLaunchKernelGGL((topk_kernel<false, false, true>), dim3(batch), dim3(kTopkThreads), lds, stream, scores, n, k, idx_out, val_out, count_out, nan_flag, cap);
-        return hipGetLastError();
+    TopkArgs A = {};
+    A.scores_n = A.n = n; A.k = k; A.nan_flag = nan_flag;
+    for (uint32_t b0 = 0; b0 < batch; b0 += 65535) {  // (rows are the grid's y)
+        A.scores = scores + (size_t)b0 * n;
+        A.idx_out = idx_out + (size_t)b0 * k; A.val_out = val_out + (size_t)b0 * k; A.count_out = count_out + b0;
+        const hipError_t e = by_abs ? topk_rows<true>(stream, A, std::min(65535u, batch - b0), workspace, workspace_bytes)
+                                    : topk_rows<false>(stream, A, std::min(65535u, batch - b0), workspace, workspace_bytes);
+        if (e != hipSuccess) return e;
     }
-    const bool cached = n <= (uint32_t)(kTopkWaves * 64 * kTopkCached);
-#define LARQL_TOPK(ABS, C) hipLaunchKernelGGL((topk_kernel<ABS, C, false>), dim3(batch), dim3(kTopkThreads), 0, stream, scores, n, k, idx_out, val_out, count_out, nan_flag, 0u)
-    if (by_abs) { if (cached) LARQL_TOPK(true, true); else LARQL_TOPK(true, false); }
-    else { if (cached) LARQL_TOPK(false, true); else LARQL_TOPK(false, false); }
-#undef LARQL_TOPK
-    return hipGetLastError();
+    return hipSuccess;
 }
 
 }  // namespace larql

@@ -1846,6 +1846,38 @@ def test_top_k_above_64(be, fmt, n, k):
         assert sorted(idx.tolist()) == list(range(n))
 
 
+@pytest.mark.parametrize("n,k,case", [(16385, 64, "normal"), (20480, 1, "normal"), (65537, 40, "ties"), (262144, 64, "ties"), (262145, 64, "sorted"),
+                                      (300001, 16, "constant"), (1100000, 64, "normal"), (16385, 65, "normal"), (98305, 200, "ties"),
+                                      (65536, 4096, "ties"), (40000, 5000, "normal"), (70000, 300, "few")])
+def test_top_k_of_rows_cut_into_chunks(be, fmt, n, k, case):
+    """Rows longer than a workgroup holds (above 16384 scores): selected chunk by chunk, then among the chunks' winners.  Row
+    lengths around the cut and the chunk sizes, K on both sides of 64; equal scores in several chunks go to the lower index."""
+    rng = np.random.default_rng(n + k)
+    sc = {"normal": lambda: rng.standard_normal(n), "ties": lambda: np.round(rng.standard_normal(n) * 8) / 8, "constant": lambda: np.full(n, 0.5),
+          "sorted": lambda: np.linspace(-2.0, 3.0, n), "few": lambda: np.where(rng.random(n) < 0.002, rng.standard_normal(n), np.inf)}[case]().astype(F)
+    order = np.lexsort((np.arange(n), -np.abs(sc)))[:k]
+    if case != "few":
+        gate = np.zeros((n, 32), F)
+        gate[:, 0] = sc
+        x = np.zeros(32, F)
+        x[0] = 1.0
+        hits = be.gate_knn(fmt.FMT_F32, gate, x, n, 32, k)
+        assert [i for i, _ in hits] == order.tolist()
+        assert [v for _, v in hits] == sc[order].tolist()
+    # by value through the lm_head call, on the scores the device itself computes: infinite ones are skipped (a row with
+    # fewer finite scores than K gives what there is)
+    blocks = np.zeros((n, 34), np.uint8)
+    blocks[:, :2] = np.where(np.isfinite(sc), sc, np.inf).astype(np.float16).view(np.uint8).reshape(n, 2)
+    blocks[:, 2] = 1
+    x = np.zeros(32, F)
+    x[0] = 1.0
+    got = be.q8_0_gemv_topk(blocks, x, n, 32, k)
+    s16 = np.where(np.isfinite(sc), sc, np.inf).astype(np.float16).astype(F)
+    valid = np.flatnonzero(np.isfinite(s16))
+    want = valid[np.lexsort((valid, -s16[valid]))[:k]]
+    assert [i for i, _ in got] == want.tolist()
+
+
 def test_top_k_above_64_limits_and_by_value(be, fmt):
     rng = np.random.default_rng(3)
     rows, hidden = 5000, 512
