@@ -1907,69 +1907,50 @@ static int moe_mxfp4_block(larql_hip_ctx *c, const larql_hip_mxfp4_experts *bank
     }
     const bool route_in_launch = route_logits && tokens == 1 &&
         gemv_effective_kind(make_job(KIND_MXFP4, bank->gate_packed, bank->gate_scales, x, g, gu_rows, hidden)) == KIND_MXFP4_MFMA;
-    // (the selection kernel, unless the planner below does the selecting itself)
-    bool router_pending = route_logits && !route_in_launch;
-    // Several tokens: slots that chose the same expert share its weights up to four at a time.  The job lists are built on
-    // the device from the router's choice (moe_plan_kernel) into the workspace's spare activation area.
-    {
-        GemvJob tg = make_job(KIND_MXFP4, bank->gate_packed, bank->gate_scales, x, g, gu_rows, hidden);
-        set_gate_up_bias(tg, 0);
-        GemvJob tu = fused ? tg : make_job(KIND_MXFP4, bank->up_packed, bank->up_scales, x, u, inter, hidden);
-        if (!fused) set_gate_up_bias(tu, 1);
-        GemvJob td = make_job(KIND_MXFP4, bank->down_packed, bank->down_scales, g, d, hidden, inter);
-        td.x_glu = fused ? g : u; td.glu_limit = bank->limit; td.glu_alpha = bank->alpha;
-        set_down_bias(td);
-        constexpr uint32_t kFirstMax = 1024;  // workgroups per launch whose first jobs the planner looks up
-        const size_t table_bytes = slots * 3 * sizeof(GemvJob) + 64 + 2 * kFirstMax * sizeof(uint32_t);
-        const bool mfma = gemv_effective_kind(tg) == KIND_MXFP4_MFMA && gemv_effective_kind(td) == KIND_MXFP4_MFMA;
-        if (mfma && tokens > 1 && slots <= 4096 && bank->n_experts <= 1024 && slots * inter * sizeof(float) >= table_bytes) {
-            tg.kind = tu.kind = td.kind = KIND_MXFP4_MFMA;
-            uint32_t *hdr = (uint32_t *)h;  // {gate/up count, passes, down count, passes}
-            GemvJob *gu_table = (GemvJob *)((uint8_t *)h + 64), *dn_table = gu_table + 2 * slots;
-            PreparedLaunch Pg, Pd;
-            // four tokens per job where the launches' LDS has room for their partial sums, else two
-            uint32_t group = 4;
-            for (int which = 0; which < 2 && group > 2; which++) {
-                GemvJob tj = which == 0 ? tg : td;
-                const uint32_t th = gemv_pick_threads(&tj, 1);
-                tj.batch = group;
-                if (th == 0 || !gemv_job_geometry(tj, th) || gemv_lds_bytes(&tj, 1, th) > 160 * 1024) group = 2;
-            }
-            for (int which = 0; which < 2; which++) {
-                GemvJob &tj = which == 0 ? tg : td;
-                PreparedLaunch &P = which == 0 ? Pg : Pd;
-                P.kind = KIND_MXFP4_MFMA;
-                P.threads = gemv_pick_threads(&tj, 1);
-                if (P.threads == 0 || !gemv_job_geometry(tj, P.threads)) return fail(c, LARQL_UNSUPPORTED, "moe_mxfp4: unsupported geometry");
-                const uint64_t max_jobs = which == 0 && !fused ? 2 * slots : slots;
-                // (the planner's cost per job: at most 1060 units a tile and under 11 more tiles' worth of start-up)
-                if (max_jobs * (((uint64_t)tj.rows + 15) / 16 + 11) * 1060 > 0x7FFFFFFFull) return fail(c, LARQL_UNSUPPORTED, "moe_mxfp4: launch too large");
-                memset(&P.L, 0, sizeof P.L);
-                P.L.table = which == 0 ? gu_table : dn_table;
-                P.L.dyn = hdr + 2 * which;
-                P.L.pad = gemv_launch_param(&tj, 1);
-                tj.batch = group;  // (sizes the partial sums; the planner sets every job's own count)
-                P.lds = gemv_lds_bytes(&tj, 1, P.threads);
-                P.grid = (uint32_t)((uint64_t)c->cu_count * gemv_wgs_per_cu(P.kind, P.threads, P.lds, (uint32_t)c->wgs_per_cu));
-            }
-            if (!gemv_job_geometry(tu, Pg.threads)) return fail(c, LARQL_UNSUPPORTED, "moe_mxfp4: unsupported geometry");
-            uint32_t *gu_first = nullptr, *dn_first = nullptr;
-            if (Pg.grid <= kFirstMax && Pd.grid <= kFirstMax) {
-                gu_first = (uint32_t *)(dn_table + slots);
-                dn_first = gu_first + kFirstMax;
-                Pg.L.wg_first = gu_first;
-                Pd.L.wg_first = dn_first;
-            }
-            HIPCHECK(c, moe_plan_launch(c->stream, router_pending ? route_logits : nullptr, bank->router_bias, route_policy, weights, experts,
-                                        (uint32_t)slots, (uint32_t)k, (uint32_t)bank->n_experts, tg, tu, td, gu_w_stride,
-                                        gu_s_stride, dn_w_stride, dn_s_stride, (uint32_t)hidden, (uint32_t)inter, fused, group, Pg.grid, Pd.grid, gu_table,
-                                        hdr, dn_table, hdr + 2, gu_first, dn_first));
-            HIPCHECK(c, gemv_launch(c->stream, Pg.kind, Pg.L, Pg.threads, Pg.grid, Pg.lds));
-            HIPCHECK(c, gemv_launch(c->stream, Pd.kind, Pd.L, Pd.threads, Pd.grid, Pd.lds));
-            HIPCHECK(c, weighted_sum_launch(c->stream, d, weights, experts, (uint32_t)bank->n_experts, out, (uint32_t)tokens, (uint32_t)k,
-                                            (uint32_t)hidden));
-            return LARQL_OK;
+    const bool router_pending = route_logits && !route_in_launch;
+    // Several tokens: the tokens that chose the same expert share its weights, up to sixteen at a time.  Four launches: the
+    // selection and the activations' terms, gate/up (gated on the way out, as terms), down, the weighted sum.
+    if (tokens > 1 && k <= kMoeGroupMaxSlots && bank->n_experts <= kMoeGroupMaxExperts && hidden < (1u << 22) && inter < (1u << 20) &&
+        moe_group_serves((uint32_t)(2 * inter), (uint32_t)hidden) && moe_group_serves((uint32_t)hidden, (uint32_t)inter)) {
+        const size_t most = kMoeGroupMaxSlots / k;  // tokens a launch takes
+        // the terms of the gated activations, then those of the tokens, in the workspace's gate / up / h areas (12 bytes per slot
+        // and element) where they fit (k > 1 in practice)
+        const size_t act_bytes = 6 * slots * moe_terms_pad(inter), x_bytes = 6 * std::min(tokens, most) * moe_terms_pad(hidden);
+        uint16_t *act_terms = (uint16_t *)g, *x_terms = (uint16_t *)((uint8_t *)g + act_bytes);
+        if (act_bytes + x_bytes > 12 * slots * inter) {
+            int rc = ensure(c, c->misc, x_bytes);
+            if (rc) return rc;
+            x_terms = (uint16_t *)c->misc.p;
         }
+        for (size_t t0 = 0; t0 < tokens; t0 += most) {
+            const size_t nt = std::min(most, tokens - t0), s0 = t0 * k;
+            HIPCHECK(c, moe_route_terms_launch(c->stream, route_logits ? route_logits + t0 * bank->n_experts : nullptr, bank->router_bias, (uint32_t)nt,
+                                               (uint32_t)bank->n_experts, (uint32_t)k, route_policy, experts + s0, weights + s0, x + t0 * hidden,
+                                               (uint32_t)hidden, x_terms));
+            MoeGroupArgs a = {};
+            a.experts = experts + s0; a.slots = (uint32_t)(nt * k); a.k = (uint32_t)k; a.n_experts = (uint32_t)bank->n_experts;
+            MoeGroupArgs b = a;
+            a.split = !fused;
+            a.w[0] = (const uint8_t *)bank->gate_packed; a.aux[0] = (const uint8_t *)bank->gate_scales;
+            a.w[1] = (const uint8_t *)bank->up_packed; a.aux[1] = (const uint8_t *)bank->up_scales;
+            a.w_stride = gu_w_stride; a.aux_stride = gu_s_stride;
+            a.bias = bank->gate_up_bias;
+            a.rows = (uint32_t)(2 * inter); a.kdim = (uint32_t)hidden;
+            a.terms_in = x_terms; a.in_rows = (uint32_t)nt;
+            a.glu_limit = bank->limit; a.glu_alpha = bank->alpha;
+            a.terms_out = act_terms;
+            b.w[0] = (const uint8_t *)bank->down_packed; b.aux[0] = (const uint8_t *)bank->down_scales;
+            b.w_stride = dn_w_stride; b.aux_stride = dn_s_stride;
+            b.bias = bank->down_bias;
+            b.rows = (uint32_t)hidden; b.kdim = (uint32_t)inter;
+            b.terms_in = act_terms; b.in_rows = a.slots;
+            b.out = d;
+            HIPCHECK(c, moe_group_launch(c->stream, a, false, (uint32_t)c->cu_count));
+            HIPCHECK(c, moe_group_launch(c->stream, b, true, (uint32_t)c->cu_count));
+            HIPCHECK(c, weighted_sum_launch(c->stream, d, weights + s0, experts + s0, (uint32_t)bank->n_experts, out + t0 * hidden, (uint32_t)nt,
+                                            (uint32_t)k, (uint32_t)hidden));
+        }
+        return LARQL_OK;
     }
     if (router_pending)
         HIPCHECK(c, router_select_launch(c->stream, route_logits, bank->router_bias, (uint32_t)tokens, (uint32_t)bank->n_experts, (uint32_t)k,

@@ -28,21 +28,10 @@
 #include <algorithm>
 
 #include "kernels.h"
+#include "mx4.h"
 #include "router.h"
 
 namespace larql {
-
-// Pointers that arrive inside a job record are generic; telling the compiler
-// they are global memory turns flat_load into global_load.
-#define GLOBAL_AS __attribute__((address_space(1)))
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef const GLOBAL_AS uint8_t *g_u8p;
-typedef const GLOBAL_AS uint32_t *g_u32p;
-typedef const GLOBAL_AS u32x4 *g_u4p;
-typedef const GLOBAL_AS f32x4 *g_f4p;
-typedef const GLOBAL_AS float *g_f32p;
-typedef GLOBAL_AS float *g_f32wp;
 
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef float float2_t __attribute__((ext_vector_type(2)));
@@ -583,8 +572,6 @@ __device__ __forceinline__ void run_q4k(const GemvJob &j, uint32_t p0, uint32_t 
 // ---------------------------------------------------------------------------
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) void *lds_vp;
-typedef const GLOBAL_AS void *g_vp;
 union Q4kOp { i32x4 v; uint32_t u[4]; };  // one MFMA operand: 16 int8 k-slots of a lane
 
 constexpr int kQ4kStages = 4;      // wave-tiles in flight per wavefront (ring slots of 2304 B)
@@ -593,9 +580,6 @@ constexpr int kQ4kMaxColPasses = 4;
 constexpr int kQ4kMaxWaves = 10;  // with the ring, the partials and 4 prepared columns per wavefront this fills the 160 KB of LDS
 constexpr uint32_t kQ4kTileBytes = 16 * 144;
 constexpr uint32_t kQ4kColBytes = 1024 + 64;  // a column's activation limbs for 64 lanes, then {k, -, -, -, sums of 8 sub-blocks}
-
-// s_waitcnt vmcnt(n), n < 64, leaving the other counters alone (gfx9 encoding)
-#define LARQL_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | (0x7 << 4) | (0xF << 8))
 
 struct Q4kCol {
     uint32_t xq[4];        // this lane's 8 activations as int8 limbs: {limb i: 2 dwords, limb 2+i: 2 dwords}, i = lane & 1
@@ -1233,17 +1217,14 @@ __device__ __forceinline__ void run_q4k_q8k(const GemvJob &j, uint32_t tile_a, u
 // rows need at least 4 blocks).
 //
 // The activations ride in bf16 as well: x = hi + mid + lo, each term the next 8 significant bits of x (exact, so the
-// three terms reproduce the f32 value), and A row 4t + i holds term i of token t (row 4t + 3 is zero): up to four
-// tokens share one read of the weights.  MFMA m of a step takes from lane (row, kg) the elements 32kg + 8m .. + 7 of
+// three terms reproduce the f32 value), and A row i holds term i (a job folded over up to four experts: row 4q + i term i
+// of expert q's activation).  MFMA m of a step takes from lane (row, kg) the elements 32kg + 8m .. + 7 of
 // the step on both sides (dword m of the lane's block), so neither operand is shuffled.  After the wavefront's steps
-// lane (j, rq) holds the three term sums of token rq for weight row j and adds them up.  Products are exact in f32
+// lane (j, 0) holds the three term sums for weight row j and adds them up.  Products are exact in f32
 // (8 x 8 significant bits) and accumulate in f32.
 // e8m0 0 means 0.0 in the reference and 255 NaN: the scale handed to the conversion is (byte << 23) as an f32, i.e.
 // 2^(byte-127) for 1..254 and 0.0 for 0, and a NaN for 255.
 // ---------------------------------------------------------------------------
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-union BfOp { bf16x8_t v; uint32_t u[4]; };
 constexpr int kMx4Stages = 3;
 constexpr int kMx4BatchTiles = 4;
 constexpr int kMx4FoldTiles = 4;   // row tiles per batch of a job folded over experts
@@ -1256,10 +1237,10 @@ constexpr uint32_t kMx4TermBytes = 768;       // per step: three planes of 128 b
 // A operands of a wavefront's K-range: [step][MFMA of the step]
 struct Mx4Ops { BfOp a[kMx4MaxSteps][4]; };
 
-// The two activations of lane `lane` in step `step`, for every token of the job (the gate and up values of a gated
+// The two activations of lane `lane` in step `step`, for every activation of the job (the gate and up values of a gated
 // job): loaded apart from their conversion so that all steps' loads fly together (a load's first use waits for
 // everything in flight, the weight tiles included, so loads issued one step at a time cost a round trip each).
-constexpr int kMx4MaxTokens = 4;    // tokens that share one job's weights: four A rows each
+constexpr int kMx4MaxTokens = 4;    // activations of a job folded over experts: four A rows each
 // (As loaded: `a` and `b` are the two 8-byte reads of a lane — plain: a = x0 x1 (b repeats it); gate and up apart: a = g0 g1,
 // b = u0 u1; interleaved g0 u0 g1 u1: a = g0 u0, b = g1 u1 — taken apart when the operands are made, so that no move of
 // loaded data sits between the loads: the compiler waits for a load where its result is first touched.)
@@ -1276,7 +1257,6 @@ struct Mx4Sel {
 
 __device__ __forceinline__ uint32_t mx4_tokens(const GemvJob &j) { return j.batch > 1 ? min(j.batch, (uint32_t)kMx4MaxTokens) : 1u; }
 __device__ __forceinline__ int64_t mx4_x_off(const GemvJob &j, int q) { return q == 0 ? 0 : q == 1 ? (int64_t)j.x_stride : q == 2 ? j.x_off[0] : j.x_off[1]; }
-__device__ __forceinline__ int64_t mx4_out_off(const GemvJob &j, uint32_t q) { return q == 0 ? 0 : q == 1 ? (int64_t)j.out_stride : q == 2 ? j.out_off[0] : j.out_off[1]; }
 
 __device__ __forceinline__ Mx4In mx4_load_step(const GemvJob &j, uint32_t step, uint32_t lane) {
     const uint32_t k = (uint32_t)j.k, i0 = step * 128 + 2 * lane;
@@ -1305,31 +1285,6 @@ __device__ __forceinline__ void mx4_pair(const GemvJob &j, const Mx4In &in, int 
     v.x = in.a[q].x; v.y = il ? in.b[q].x : in.a[q].y;
     u.x = il ? in.a[q].y : in.b[q].x; u.y = in.b[q].y;
     if (!in.inside) { v = (float2_t){0.f, 0.f}; u = (float2_t){0.f, 0.f}; }
-}
-
-// MoeGateRule::ClampedGlu (larql-compute/src/pipeline/moe.rs:88-92): g = min(g, L); u = clamp(u, -L, L);
-// (u + 1) * (g * sigmoid(alpha * g))
-__device__ __forceinline__ float clamped_glu(float g, float u, float L, float al) {
-    const float gc = fminf(g, L);
-    const float uc = u < -L ? -L : (u > L ? L : u);
-    return (uc + 1.0f) * (gc * (1.0f / (1.0f + expf(-(gc * al)))));
-}
-
-// The three bf16 terms of two activations, packed pairwise (a in the low half): x = t0 + t1 + t2 exactly.  An infinite
-// or NaN activation stays in the first term alone (its residual would be a NaN of its own making).
-__device__ __forceinline__ void mx4_terms(float a, float b, uint32_t (&t)[3]) {
-    const uint32_t ab = __builtin_bit_cast(uint32_t, a), bb = __builtin_bit_cast(uint32_t, b);
-    uint32_t a0 = ab & 0xFFFF0000u, b0 = bb & 0xFFFF0000u;
-    float ra = a - __builtin_bit_cast(float, a0), rb = b - __builtin_bit_cast(float, b0);  // exact
-    if ((ab & 0x7F800000u) == 0x7F800000u) { ra = 0.f; a0 = (ab & 0x007FFFFFu) ? (a0 | 0x00400000u) : a0; }
-    if ((bb & 0x7F800000u) == 0x7F800000u) { rb = 0.f; b0 = (bb & 0x007FFFFFu) ? (b0 | 0x00400000u) : b0; }
-    const uint32_t a1 = __builtin_bit_cast(uint32_t, ra) & 0xFFFF0000u, b1 = __builtin_bit_cast(uint32_t, rb) & 0xFFFF0000u;
-    ra -= __builtin_bit_cast(float, a1);
-    rb -= __builtin_bit_cast(float, b1);
-    const uint32_t a2 = __builtin_bit_cast(uint32_t, ra) & 0xFFFF0000u, b2 = __builtin_bit_cast(uint32_t, rb) & 0xFFFF0000u;
-    t[0] = (a0 >> 16) | b0;
-    t[1] = (a1 >> 16) | b1;
-    t[2] = (a2 >> 16) | b2;
 }
 
 // One token's operands of all `cw` steps of a wavefront: every lane splits its two activations of a step into terms
@@ -1379,18 +1334,6 @@ __device__ __forceinline__ void mx4_clear_ops(Mx4Ops &ops) {
         for (int m = 0; m < 4; m++) ops.a[s][m].u[0] = ops.a[s][m].u[1] = ops.a[s][m].u[2] = ops.a[s][m].u[3] = 0u;
 }
 
-// The operands of every token of a job: token q's terms are A rows 4q .. 4q+2, so its sums come out in D rows of
-// their own (lanes with rq = q).
-__device__ __forceinline__ void mx4_setup_ops(const GemvJob &j, const Mx4In (&in)[kMx4MaxSteps], Mx4Ops &ops, uint32_t cw,
-                                              uint32_t lane, uint8_t *scratch) {
-    const uint32_t ntok = mx4_tokens(j);
-    mx4_clear_ops(ops);
-    mx4_setup_token<0>(j, false, 1.0f, in, ops, 0, cw, lane, scratch);
-    if (ntok > 1) mx4_setup_token<1>(j, false, 1.0f, in, ops, 1, cw, lane, scratch);
-    if (ntok > 2) mx4_setup_token<2>(j, false, 1.0f, in, ops, 2, cw, lane, scratch);
-    if (ntok > 3) mx4_setup_token<3>(j, false, 1.0f, in, ops, 3, cw, lane, scratch);
-}
-
 // One step of a wave-tile from its LDS slot: the lane's block (16 bytes of nibbles, scale byte `sc`) against the four
 // operands of the step.  `live` is false for a block past the row end or of an expert outside the bank.
 __device__ __forceinline__ f32x4 mx4_step_mfma(const BfOp (&a)[4], const u32x4 q, uint32_t sc, bool live, f32x4 D) {
@@ -1415,15 +1358,12 @@ __device__ __forceinline__ f32x4 mx4_step_mfma(const BfOp (&a)[4], const u32x4 q
 
 // tiles [tile_a, tile_b) of one job
 __device__ __forceinline__ void run_mxfp4_mfma(const GemvJob &j, const Mx4Sel &sel, uint32_t tile_a, uint32_t tile_b, uint8_t *lds,
-                                               uint32_t slot_bytes, uint32_t &parity, bool fresh) {
+                                               uint32_t slot_bytes, uint32_t &parity) {
     constexpr int NS = kMx4Stages, R = kMx4BatchTiles;
     const uint32_t lane = threadIdx.x & 63u, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t nw_launch = blockDim.x >> 6;
     const uint32_t jr = lane & 15u, kg = lane >> 4;
-    // up to four tokens share the weights: token q rides in A rows 4q .. 4q+2, its sums leave in D rows 4q .. 4q+2 (lanes rq = q)
-    const uint32_t ntok = mx4_tokens(j);
-    const uint32_t hw_sh = ntok == 1 ? 0u : (ntok == 2 ? 1u : 2u), hw = 1u << hw_sh;  // partial sums per weight row and wavefront
-    const uint32_t nwj = j.rpp, steps = j.cpr, cw = (uint32_t)j.pad, PW = nwj * hw;
+    const uint32_t nwj = j.rpp, steps = j.cpr, cw = (uint32_t)j.pad, PW = nwj;
     const uint32_t rows = (uint32_t)j.rows, k = (uint32_t)j.k, nb = k / 32, row_bytes = (uint32_t)j.row_bytes;
     uint8_t *ring = lds + wv * (NS * slot_bytes);
     float *part = reinterpret_cast<float *>(lds + nw_launch * (NS * slot_bytes));
@@ -1482,15 +1422,14 @@ __device__ __forceinline__ void run_mxfp4_mfma(const GemvJob &j, const Mx4Sel &s
     if (working)
         for (int s = 0; s < NS - 1; s++) issue();
     Mx4Ops ops;
-    if (working) mx4_setup_ops(j, xin, ops, cw, lane, ring + (NS - 1) * slot_bytes);  // (768 bytes per step fit the 1024 of a slot's step)
+    if (working) {
+        mx4_clear_ops(ops);
+        mx4_setup_token<0>(j, false, 1.0f, xin, ops, 0, cw, lane, ring + (NS - 1) * slot_bytes);  // (768 bytes per step fit the 1024 of a slot's step)
+    }
 
-    // The two partial-sum areas are laid out for this job's own `hw`; the job this workgroup served before may have used
-    // another layout, and its last row sums may still be read by a slower wavefront: wait for everybody before writing
-    // (`fresh`: the workgroup's first job of the launch has nobody to wait for).
-    if (!fresh) __builtin_amdgcn_s_barrier();
     uint32_t n_use = 0;
     for (uint32_t tb = 0; tb < nt; tb += R) {
-        float *pb = part + parity * (R * 16 * nw_launch * hw);
+        float *pb = part + parity * (R * 16 * nw_launch);
         const uint32_t nbt = min((uint32_t)R, nt - tb);
         if (working) {
             for (uint32_t tl = 0; tl < nbt; tl++) {
@@ -1510,8 +1449,8 @@ __device__ __forceinline__ void run_mxfp4_mfma(const GemvJob &j, const Mx4Sel &s
                     }
                 }
                 n_use++;
-                // the three term sums of token kg for weight row jr
-                if (kg < hw) pb[(tl * 16 + jr) * PW + wv * hw + kg] = (D[0] + D[1]) + D[2];
+                // the three term sums for weight row jr
+                if (kg == 0) pb[(tl * 16 + jr) * PW + wv] = (D[0] + D[1]) + D[2];
             }
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -1519,17 +1458,14 @@ __device__ __forceinline__ void run_mxfp4_mfma(const GemvJob &j, const Mx4Sel &s
         asm volatile("" ::: "memory");
         const uint32_t row_base = (tile_a + tb) * 16;
         const uint32_t nwork = min(nwj, (steps + cw - 1) / cw);
-        // hw threads per weight row: thread h adds up token h's slot of every wavefront (the same order of additions
-        // per token whatever the number of tokens that share the job)
-        for (uint32_t rr = threadIdx.x >> hw_sh; rr < nbt * 16; rr += blockDim.x >> hw_sh) {
-            const uint32_t h = threadIdx.x & (hw - 1u);
+        for (uint32_t rr = threadIdx.x; rr < nbt * 16; rr += blockDim.x) {
             float s = 0.f;
-            for (uint32_t w = 0; w < nwork; w++) s += pb[rr * PW + w * hw + h];
+            for (uint32_t w = 0; w < nwork; w++) s += pb[rr * PW + w];
             const uint32_t row = row_base + rr;
-            if (h < ntok && row < rows) {
+            if (row < rows) {
                 if (!sel.ok[0]) s = 0.0f;  // an expert outside the bank: no contribution (its stand-in's bytes were read, not used)
                 else if (j.bias) s += ((const GLOBAL_AS float *)sel.bias[0])[(size_t)row * j.bias_step];
-                ((g_f32wp)(j.out + mx4_out_off(j, h)))[row] = s;
+                ((g_f32wp)j.out)[row] = s;
             }
         }
         parity ^= 1u;
@@ -2963,15 +2899,12 @@ __global__ void __launch_bounds__(kQ4kMaxWaves * 64) gemv_q4k_q8k_kernel(GemvLau
 __global__ void __launch_bounds__(kMx4MaxWaves * 64) gemv_mxfp4_mfma_kernel(GemvLaunch L) {
     extern __shared__ __attribute__((aligned(16))) uint8_t mx4_lds[];
     const job_cp jobs = job_table(L);
-    // (a job list built on the device brings its own count and pass total)
-    const uint32_t n_jobs = L.dyn ? (uint32_t)__builtin_amdgcn_readfirstlane(((const GLOBAL_AS uint32_t *)L.dyn)[0]) : L.n_jobs;
-    const uint64_t P = L.dyn ? (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane(((const GLOBAL_AS uint32_t *)L.dyn)[1]) : L.total_passes;
-    if (P == 0 || n_jobs == 0) return;
+    const uint32_t n_jobs = L.n_jobs;
+    const uint64_t P = L.total_passes;
     uint32_t p = (uint32_t)(P * blockIdx.x / gridDim.x);
     const uint32_t p_end = (uint32_t)(P * (blockIdx.x + 1) / gridDim.x);
     const uint32_t lo = first_job_of_share(L, jobs, n_jobs, p);
     uint32_t ji = lo, parity = 0;
-    bool fresh = true;  // no job of this launch has used the workgroup's LDS yet
     while (p < p_end) {
         GemvJob j = uniform_job(jobs + ji);
         Mx4Sel S;
@@ -3013,14 +2946,12 @@ __global__ void __launch_bounds__(kMx4MaxWaves * 64) gemv_mxfp4_mfma_kernel(Gemv
             }
         }
         const uint32_t seg_end = min(p_end, j.pass_begin + j.n_pass);
-        // a tile belongs to the workgroup whose share contains its first cost unit (the job's range opens with its
-        // start-up allowance, if it has one)
-        const uint32_t a = p - j.pass_begin, b = seg_end - j.pass_begin, cpt = j.cpt ? j.cpt : j.cpr, su = j.su;
-        const uint32_t tile_a = a > su ? (a - su + cpt - 1) / cpt : 0, tile_b = b > su ? (b - su + cpt - 1) / cpt : 0;
+        // a tile belongs to the workgroup whose share contains its first cost unit
+        const uint32_t a = p - j.pass_begin, b = seg_end - j.pass_begin, cpt = j.cpt ? j.cpt : j.cpr;
+        const uint32_t tile_a = (a + cpt - 1) / cpt, tile_b = (b + cpt - 1) / cpt;
         if (tile_a < tile_b) {
             if (j.combine_w) run_mxfp4_fold(j, S, tile_a, tile_b, mx4_lds, L.pad, parity);
-            else run_mxfp4_mfma(j, S, tile_a, tile_b, mx4_lds, L.pad, parity, fresh);
-            fresh = false;
+            else run_mxfp4_mfma(j, S, tile_a, tile_b, mx4_lds, L.pad, parity);
         }
         p = seg_end;
         ji++;
@@ -3258,7 +3189,6 @@ bool gemv_job_geometry(GemvJob &j, uint32_t threads) {
         if (tiles * steps * fold > 0x7FFFFFFFull) return false;
         j.n_pass = (uint32_t)(tiles * steps * fold);
         j.cpt = fold > 1 ? (uint32_t)(steps * fold) : 0;
-        j.su = 0;
         return true;
     }
     if (j.kind == KIND_Q6K_MFMA) {  // geometry and cost model as for the Q4_K matrix-core kernel

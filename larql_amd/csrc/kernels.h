@@ -41,21 +41,19 @@ struct GemvJob {
     // uses w + e*w_sel_stride, aux + e*aux_sel_stride (one bank of equally shaped matrices).
     const uint32_t *sel;
     uint64_t w_sel_stride, aux_sel_stride;
-    // Optional batch (bf16 / Q4_K gates, MXFP4 experts shared by up to four tokens): `batch` activations x + t*x_stride
-    // against the same weights, results to out + t*out_stride (strides in floats).  0 or 1 = a plain matvec.
-    // See gemv_batch_capacity.  The MXFP4 matrix-core kernel's tokens sit anywhere: token 1 at x + x_stride (which may
-    // wrap, i.e. be negative), tokens 2 and 3 at x + x_off[0], x + x_off[1]; results likewise with out_stride, out_off.
+    // Optional batch (bf16 / Q4_K gates): `batch` activations x + t*x_stride against the same weights, results to
+    // out + t*out_stride (strides in floats).  0 or 1 = a plain matvec.  See gemv_batch_capacity.  A job folded over experts
+    // (combine_w) has its activations 2 and 3 at x + x_off[0], x + x_off[1].
     uint32_t batch, pad2;
     uint64_t x_stride, out_stride;
-    int64_t x_off[2], out_off[2];
+    int64_t x_off[2];
     // Optional gated activation (MoE down projection, MXFP4 matrix-core kernel only): when `x_glu` is set the
     // activation is ClampedGlu(g = x[i], u = x_glu[i]) computed while the activations are prepared; x_glu == x means
     // that g and u are interleaved in x (g = x[2i], u = x[2i+1]: the result of a fused gate_up matrix walked in place).
     const float *x_glu;
     float glu_limit, glu_alpha;
-    // Optional cost model of the job in the launch's pass list (MXFP4 matrix-core kernel): the job's n_pass is
-    // su + tiles * cpt (a start-up allowance, then cpt units per 16-row tile); cpt == 0 means cpr units per tile, no allowance.
-    uint32_t cpt, su;
+    // Cost units per 16-row tile of a job folded over experts (0: cpr).
+    uint32_t cpt, pad3;
     // Optional selection inside the kernel (MXFP4 matrix-core kernel, one token): when `route_logits` is set the job
     // takes the expert of rank `route_rank` of Router::select over those logits (route_n experts <= 64, route_k <= 8,
     // policy as router_select_launch) where it would read *sel, and the workgroup that opens the job also writes the
@@ -84,7 +82,7 @@ struct GemvJob {
     // range of a wider matrix — w points at the range's first super-block of row 0.  0 = rows are packed (row_bytes).
     uint64_t row_stride;
 };
-static_assert(sizeof(GemvJob) % 16 == 0, "the descriptor is a whole number of 16-byte words (moe_plan_kernel stores it that way)");
+static_assert(sizeof(GemvJob) % 16 == 0, "job tables are arrays of 16-byte words");
 
 struct GemvLaunch {
     const GemvJob *table;  // device table, or null to use `inl`
@@ -92,9 +90,6 @@ struct GemvLaunch {
     uint64_t total_passes;
     uint32_t n_jobs;
     uint32_t pad;
-    // Optional: the job count and pass total live in device memory ({n_jobs, total_passes}, written by a kernel
-    // earlier on the stream) and override the two fields above.  MXFP4 matrix-core kernel only.
-    const uint32_t *dyn;
     // Optional: the first job of every workgroup's share ([grid] indices in device memory), so that a workgroup need not
     // search the jobs' pass ranges for it.
     const uint32_t *wg_first;
@@ -185,17 +180,34 @@ struct Moe1Args {
 bool moe1_geometry(Moe1Args &A, uint32_t *threads, size_t *lds);  // fills cw / nw / stages; false: not served
 hipError_t moe1_launch(hipStream_t s, const Moe1Args &A, bool down, uint32_t grid, uint32_t threads, size_t lds);
 
+// Several tokens through a bank of MXFP4 experts (moe_group.hip): a launch per projection stage over the slots (token, rank).
+constexpr uint32_t kMoeGroupMaxSlots = 4096, kMoeGroupMaxExperts = 1024;  // (the slots' ids and two counters per expert in LDS)
+struct MoeGroupArgs {
+    const uint32_t *experts;        // [slots], slot = token * k + rank; an id >= n_experts contributes nothing
+    uint32_t slots, k, n_experts;
+    uint32_t split;                 // gate/up stage: gate and up matrices apart (else one fused matrix, gate row 2i, up row 2i+1)
+    const uint8_t *w[2], *aux[2];   // expert 0's matrices; expert e's start e * stride bytes further on
+    uint64_t w_stride, aux_stride;
+    const float *bias;              // optional [n_experts, rows] (gate/up: interleaved whatever the weight layout)
+    uint32_t rows, kdim;            // of the (virtually fused) matrix
+    const uint16_t *terms_in;       // three bf16 terms of the activations: [term][in_rows][moe_terms_pad(kdim)]; gate/up: by token, down: by slot
+    uint32_t in_rows;
+    float glu_limit, glu_alpha;
+    uint16_t *terms_out;            // gate/up stage: the gated activation, [term][slots][moe_terms_pad(rows / 2)]
+    float *out;                     // down stage: [slots, rows]
+};
+__host__ __device__ constexpr size_t moe_terms_pad(size_t n) { return (n + 127) / 128 * 128; }  // elements per row of terms
+bool moe_group_serves(uint32_t rows, uint32_t kdim);
+hipError_t moe_group_launch(hipStream_t s, const MoeGroupArgs &A, bool down, uint32_t cu_count);
+// the tokens' selection (logits != nullptr) and the terms of their activations, terms[term][token][moe_terms_pad(hidden)]
+hipError_t moe_route_terms_launch(hipStream_t s, const float *logits, const float *bias, uint32_t tokens, uint32_t n_experts, uint32_t k, int policy,
+                                  uint32_t *experts, float *weights, const float *x, uint32_t hidden, uint16_t *terms);
+
 // MoE helpers
 constexpr uint32_t kRouterMaxExperts = 256;      // the selection kernel and the planner (four logits per lane)
 constexpr uint32_t kRouterInLaunchExperts = 64;  // a matvec launch that selects for itself (one logit per lane)
 hipError_t router_select_launch(hipStream_t s, const float *logits, const float *bias, uint32_t tokens, uint32_t n_experts, uint32_t k,
                                 int policy, uint32_t *experts, float *weights);
-// (logits != nullptr: the kernel selects the experts itself first — at most kRouterMaxExperts, top-kRouterMaxK — and writes experts / weights)
-hipError_t moe_plan_launch(hipStream_t s, const float *logits, const float *router_bias, int policy, float *weights, uint32_t *experts,
-                           uint32_t slots, uint32_t k, uint32_t n_experts, const GemvJob &tg,
-                           const GemvJob &tu, const GemvJob &td, uint64_t gu_w_stride, uint64_t gu_s_stride, uint64_t dn_w_stride,
-                           uint64_t dn_s_stride, uint32_t hidden, uint32_t inter, bool fused, uint32_t group, uint32_t g_grid, uint32_t d_grid,
-                           GemvJob *gu_table, uint32_t *gu_hdr, GemvJob *dn_table, uint32_t *dn_hdr, uint32_t *gu_first, uint32_t *dn_first);
 hipError_t clamped_glu_interleaved_launch(hipStream_t s, const float *gu, float *h, size_t n, float limit, float alpha);
 hipError_t clamped_glu_launch(hipStream_t s, const float *g, const float *u, float *h, size_t n, float limit, float alpha);
 hipError_t expert_scale_launch(hipStream_t s, float *weights, const uint32_t *experts, const float *scale, uint32_t n, uint32_t n_scale);

@@ -257,252 +257,6 @@ __global__ void weighted_sum_bias_kernel(const float *__restrict__ d, const floa
     out[(size_t)t * hidden + i] = acc;
 }
 
-// Job lists of an expert block, built on the device from the router's choice (no host round trip): the slots
-// (token, rank) that chose the same expert are grouped by `group` (2 or 4), in slot order, and every group becomes one
-// gate, one up and one down job whose activations share the expert's weights (GemvJob::batch = tokens in the group;
-// the other activations / results sit x_stride, x_off[] / out_stride, out_off[] floats away from the first).
-// tg / tu / td are the jobs of slot 0 with expert 0 (geometry filled in); tables: [gate jobs | up jobs], [down jobs];
-// headers: {job count, pass total}.  One block; a thread per slot, O(slots) work each.
-// `fused`: tg walks a fused gate_up matrix of 2*inter interleaved rows (no up jobs; a slot's results and the down
-// job's activation are 2*inter floats, gate and up values alternating).
-// With `logits` the kernel is the router as well (one launch fewer in front of the matvecs): a wavefront per token
-// selects as router_select_kernel does and writes `experts` / `weights` before the planning reads the choice.
-__global__ void __launch_bounds__(1024) moe_plan_kernel(const float *__restrict__ logits, const float *__restrict__ router_bias, int policy,
-                                                       float *__restrict__ weights, uint32_t *__restrict__ experts, uint32_t slots, uint32_t k, uint32_t n_experts,
-                                                       GemvJob tg, GemvJob tu, GemvJob td, uint64_t gu_w_stride, uint64_t gu_s_stride,
-                                                       uint64_t dn_w_stride, uint64_t dn_s_stride, uint32_t hidden, uint32_t inter, uint32_t fused,
-                                                       uint32_t group, uint32_t g_grid, uint32_t d_grid, GemvJob *__restrict__ gu_table,
-                                                       uint32_t *__restrict__ gu_hdr, GemvJob *__restrict__ dn_table, uint32_t *__restrict__ dn_hdr,
-                                                       uint32_t *__restrict__ gu_first, uint32_t *__restrict__ dn_first) {
-    __shared__ uint32_t first_job[1025];  // first job of expert e; [n_experts] = total
-    __shared__ uint32_t first_kind_a[1025], first_kind_b[1025];  // the jobs before expert e by kind: {full groups, of 1 slot}, {of 2, of 3}
-    __shared__ __attribute__((aligned(16))) uint32_t cnt[1024];  // slots per expert
-    __shared__ __attribute__((aligned(16))) uint32_t ex[4096];   // the router's choice, read once
-    __shared__ uint32_t first_slot[1025]; // slots of the experts before e
-    __shared__ uint16_t rank[4096];       // a slot's rank among the slots of its expert, in slot order
-    __shared__ uint16_t by_expert[4096];  // the slots ordered by (expert, rank)
-    const uint32_t t = threadIdx.x;
-    const uint32_t gsh = group == 4 ? 2u : 1u, gmask = group - 1;  // (group is 2 or 4: no divisions below)
-    for (uint32_t e = t; e < ((n_experts + 3u) & ~3u); e += blockDim.x) cnt[e] = 0;
-    if (logits) {
-        const uint32_t lane = t & 63u, tokens = slots / k;
-        for (uint32_t tok = t >> 6; tok < tokens; tok += blockDim.x >> 6) {
-            uint32_t sel_idx[kRouterMaxK];
-            float sel_w[kRouterMaxK];
-            router_select_any(logits + (size_t)tok * n_experts, router_bias, n_experts, k, policy, lane, sel_idx, sel_w);
-            if (lane == 0) {
-#pragma unroll
-                for (int r = 0; r < kRouterMaxK; r++)
-                    if ((uint32_t)r < k) {
-                        experts[(size_t)tok * k + r] = sel_idx[r];
-                        weights[(size_t)tok * k + r] = sel_w[r];
-                        ex[tok * k + r] = sel_idx[r];
-                    }
-            }
-        }
-        for (uint32_t s2 = slots + t; s2 < ((slots + 3u) & ~3u); s2 += blockDim.x) ex[s2] = 0xFFFFFFFFu;
-    } else {
-        for (uint32_t s = t; s < ((slots + 3u) & ~3u); s += blockDim.x) ex[s] = s < slots ? experts[s] : 0xFFFFFFFFu;
-    }
-    __syncthreads();
-    if (slots <= 64 && n_experts <= 64) {
-        // A block of up to 64 slots and 64 experts is planned by one wavefront without a barrier in between: lane s is
-        // slot s (its rank = the earlier lanes with the same expert, one ballot per expert), lane e is expert e (its
-        // count from the same ballots, the sums over the experts before it by a scan across the lanes).
-        if (t < 64) {
-            const uint32_t e = t < slots ? ex[t] : 0xFFFFFFFFu;
-            uint32_t r = 0, c = 0;
-            for (uint32_t q = 0; q < n_experts; q++) {
-                const uint64_t m = __ballot(e == q);
-                if (e == q) r = (uint32_t)__popcll(m & ((1ull << t) - 1ull));
-                if (t == q) c = (uint32_t)__popcll(m);
-            }
-            if (t < slots) rank[t] = (uint16_t)r;
-            if (t < n_experts) cnt[t] = c;
-            // what expert t adds to the sums (lanes from n_experts on add nothing): jobs | slots << 16, and the jobs by kind
-            // in one word (full groups, groups of 1, 2, 3 slots: a byte each, at most 64)
-            const uint32_t mm = c & gmask;
-            uint32_t js = ((c + gmask) >> gsh) | (c << 16);
-            uint32_t kk = (c >> gsh) | (mm == 1 ? 0x100u : 0u) | (mm == 2 ? 0x10000u : 0u) | (mm == 3 ? 0x1000000u : 0u);
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {  // inclusive sums over the lanes
-                const uint32_t a = (uint32_t)__shfl_up((int)js, o, 64), bq = (uint32_t)__shfl_up((int)kk, o, 64);
-                if (t >= (uint32_t)o) { js += a; kk += bq; }
-            }
-            // entry e = the experts before e: lane e - 1's inclusive sums (entry 0 = nothing, entry n_experts = everything)
-            const uint32_t at = t + 1;
-            if (at <= n_experts) {
-                first_job[at] = js & 0xFFFFu; first_slot[at] = js >> 16;
-                first_kind_a[at] = (kk & 0xFFu) | (((kk >> 8) & 0xFFu) << 16);
-                first_kind_b[at] = ((kk >> 16) & 0xFFu) | ((kk >> 24) << 16);
-            }
-            if (t == 0) { first_job[0] = 0; first_slot[0] = 0; first_kind_a[0] = 0; first_kind_b[0] = 0; }
-            // (the same wavefront reads what it has just written: LDS executes a wavefront's operations in order)
-            if (e < n_experts) by_expert[first_slot[e] + r] = (uint16_t)t;
-        }
-        __syncthreads();
-    } else {
-        // ranks: four earlier slots per LDS read, the reads of a round independent of each other
-        for (uint32_t s = t; s < slots; s += blockDim.x) {
-            const uint32_t e = ex[s];
-            uint32_t r = 0;
-    #pragma unroll 4
-            for (uint32_t q = 0; q < s; q += 4) {
-                const uint4 v = *reinterpret_cast<const uint4 *>(&ex[q]);
-                r += (v.x == e ? 1u : 0u) + (q + 1 < s && v.y == e ? 1u : 0u) + (q + 2 < s && v.z == e ? 1u : 0u) + (q + 3 < s && v.w == e ? 1u : 0u);
-            }
-            rank[s] = (uint16_t)r;
-            if (e < n_experts) atomicAdd(&cnt[e], 1u);
-        }
-        __syncthreads();
-        // Per expert: the jobs before it, counted by kind (full groups, and groups of 1, 2 or 3 slots), 16 bits a count.
-        for (uint32_t e = t; e <= n_experts; e += blockDim.x) {
-            uint32_t f = 0, ka = 0, kb = 0, fs = 0;
-            auto add = [&](uint32_t c) {
-                fs += c;
-                f += (c + gmask) >> gsh;
-                const uint32_t m = c & gmask;
-                ka += (c >> gsh) + (m == 1 ? 0x10000u : 0u);
-                kb += (m == 2 ? 1u : 0u) + (m == 3 ? 0x10000u : 0u);
-            };
-    #pragma unroll 2
-            for (uint32_t q = 0; q < e; q += 4) {
-                const uint4 v = *reinterpret_cast<const uint4 *>(&cnt[q]);
-                add(v.x);
-                if (q + 1 < e) add(v.y);
-                if (q + 2 < e) add(v.z);
-                if (q + 3 < e) add(v.w);
-            }
-            first_job[e] = f; first_kind_a[e] = ka; first_kind_b[e] = kb; first_slot[e] = fs;
-        }
-        __syncthreads();
-    }
-    const uint32_t n_jobs = first_job[n_experts];
-    // Cost of a job in a launch's pass list.  A workgroup prepares the activations of every job it takes a share of
-    // before the share's first tile: about 3 tiles' time for one token and 2 more for every further one (time
-    // stamps of the kernel), whether the share opens the job or not.  A job cut into n shares pays that n times, and
-    // n = 1 + tiles / (tiles per workgroup) on average: so a job costs one preparation up front (GemvJob::su) and each
-    // of its tiles carries the preparation's part, cpt = 4 * tpw + prep in quarter tiles where a tile's own time is
-    // 4 * tpw units (tpw = the launch's tiles per workgroup).  The workgroup that opens a job mid-share also lets its
-    // stream of weights run dry in between: 2 tiles more up front.  Launches whose workgroups walk more than 256
-    // tiles each leave the parts out (under 4 % of a share).
-    struct JobCost {  // of a job with m tokens, in one launch
-        uint32_t tiles, unit;  // unit = tpw, or 0 where the parts are left out
-        __device__ uint32_t prep(uint32_t m) const { return 12 + 8 * (m - 1); }
-        __device__ uint32_t cpt(uint32_t m) const { return unit ? 4 * unit + prep(m) : 4u; }
-        __device__ uint32_t su(uint32_t m) const { return (prep(m) + 8) * (unit ? unit : 1u); }
-        __device__ uint32_t job(uint32_t m) const { return su(m) + tiles * cpt(m); }
-    };
-    const auto cost_model = [&](uint32_t tiles, uint32_t grid, uint32_t lists) {
-        // (float arithmetic: a rough figure is all the model needs, and a 64-bit division is a hundred instructions)
-        const float tpw_f = (float)(lists * n_jobs) * (float)tiles / (float)max(grid, 1u);
-        const uint32_t tpw = tpw_f < 1.0f ? 1u : tpw_f > 256.0f ? 0u : (uint32_t)tpw_f;
-        return JobCost{tiles, tpw};
-    };
-    const uint32_t g_tiles = ((uint32_t)tg.rows + 15) / 16, d_tiles = ((uint32_t)td.rows + 15) / 16;
-    const JobCost gc = cost_model(g_tiles, g_grid, fused ? 1u : 2u), dc = cost_model(d_tiles, d_grid, 1u);
-    const auto jobs_cost = [&](const JobCost &c, uint32_t e) {  // the jobs of the experts before e
-        const uint32_t ka = first_kind_a[e], kb = first_kind_b[e];
-        return (ka & 0xFFFFu) * c.job(group) + (ka >> 16) * c.job(1) + (kb & 0xFFFFu) * c.job(2) + (kb >> 16) * c.job(3);
-    };
-    const uint32_t g_total = jobs_cost(gc, n_experts), d_total = jobs_cost(dc, n_experts);
-    if (!(slots <= 64 && n_experts <= 64)) {  // (the one-wavefront path has done this)
-        for (uint32_t s = t; s < slots; s += blockDim.x) {
-            const uint32_t e = ex[s];
-            if (e < n_experts) by_expert[first_slot[e] + rank[s]] = (uint16_t)s;
-        }
-    }
-    __syncthreads();
-    // Ranks that are multiples of `group` open a job, the `group - 1` that follow join it.  The three descriptors of a
-    // job (gate, up, down) are written by three different wavefronts: thread idx serves slot idx % span as kind idx / span.
-    const uint32_t span = (slots + 63u) & ~63u;
-    for (uint32_t idx = t; idx < 3 * span; idx += blockDim.x) {
-        const uint32_t which = idx / span, s1 = idx - which * span;  // (span is a multiple of 64: `which` is the same in a wavefront)
-        if (s1 >= slots || (which == 1 && fused)) continue;
-        const uint32_t e = ex[s1], r = rank[s1];
-        if (e >= n_experts || (r & gmask)) continue;
-        const uint32_t jb = first_job[e] + (r >> gsh);
-        const uint32_t nb = min(group, cnt[e] - r);
-        uint32_t sm[4];
-#pragma unroll
-        for (uint32_t q = 0; q < 4; q++) sm[q] = q < nb ? by_expert[first_slot[e] + r + q] : s1;
-        const uint32_t tok1 = s1 / k;
-        const size_t gs = fused ? 2 * (size_t)inter : (size_t)inter;  // floats of gate/up results per slot and half
-        const auto tok_off = [&](uint32_t q) { return ((int64_t)(sm[q] / k) - (int64_t)tok1) * (int64_t)hidden; };
-        const auto slot_off = [&](uint32_t q, size_t unit) { return ((int64_t)sm[q] - (int64_t)s1) * (int64_t)unit; };
-        // a job = the template's words with the fields that differ replaced, kept in registers as plain dwords
-        // and stored 16 bytes at a time
-        const auto emit = [&](GemvJob *dst, const GemvJob &tm, size_t w_off, size_t aux_off, size_t x_off, size_t out_off, bool x_by_token,
-                              size_t out_unit, uint32_t pass_begin, const JobCost &c) {
-            static_assert(sizeof(GemvJob) % 16 == 0 && alignof(GemvJob) == 8, "descriptor is a whole number of 16-byte stores");
-            constexpr int N = sizeof(GemvJob) / 4;
-            const uint32_t *src = reinterpret_cast<const uint32_t *>(&tm);
-            uint32_t d[N];
-#pragma unroll
-            for (int i = 0; i < N; i++) d[i] = src[i];
-            const auto put32 = [&](size_t byte_off, uint32_t v) { d[byte_off / 4] = v; };
-            const auto put64 = [&](size_t byte_off, uint64_t v) { d[byte_off / 4] = (uint32_t)v; d[byte_off / 4 + 1] = (uint32_t)(v >> 32); };
-            put64(offsetof(GemvJob, w), (uint64_t)(tm.w + w_off));
-            put64(offsetof(GemvJob, aux), (uint64_t)(tm.aux + aux_off));
-            put64(offsetof(GemvJob, x), (uint64_t)(tm.x + x_off));
-            put64(offsetof(GemvJob, out), (uint64_t)(tm.out + out_off));
-            if (tm.x_glu) put64(offsetof(GemvJob, x_glu), (uint64_t)(tm.x_glu + x_off));
-            if (tm.bias) put64(offsetof(GemvJob, bias), (uint64_t)(tm.bias + (size_t)e * tm.bias_sel_stride));  // this expert's bias row
-            put32(offsetof(GemvJob, batch), nb);
-            put64(offsetof(GemvJob, x_stride), (uint64_t)(x_by_token ? tok_off(1) : slot_off(1, gs)));
-            put64(offsetof(GemvJob, out_stride), (uint64_t)slot_off(1, out_unit));
-            put64(offsetof(GemvJob, x_off), (uint64_t)(x_by_token ? tok_off(2) : slot_off(2, gs)));
-            put64(offsetof(GemvJob, x_off) + 8, (uint64_t)(x_by_token ? tok_off(3) : slot_off(3, gs)));
-            put64(offsetof(GemvJob, out_off), (uint64_t)slot_off(2, out_unit));
-            put64(offsetof(GemvJob, out_off) + 8, (uint64_t)slot_off(3, out_unit));
-            put32(offsetof(GemvJob, pass_begin), pass_begin);
-            put32(offsetof(GemvJob, n_pass), c.job(nb));
-            put32(offsetof(GemvJob, cpt), c.cpt(nb));
-            put32(offsetof(GemvJob, su), c.su(nb));
-            uint4 *o = reinterpret_cast<uint4 *>(dst);  // (the tables are 16-byte aligned)
-#pragma unroll
-            for (int i = 0; i < N / 4; i++) o[i] = make_uint4(d[4 * i], d[4 * i + 1], d[4 * i + 2], d[4 * i + 3]);
-        };
-        // (the earlier jobs of this expert are all full groups)
-        const uint32_t g_begin = jobs_cost(gc, e) + (r >> gsh) * gc.job(group), d_begin = jobs_cost(dc, e) + (r >> gsh) * dc.job(group);
-        if (gu_first) {
-            // The first job of every workgroup's share (what a workgroup would otherwise find by bisection over the jobs'
-            // pass ranges, a dependent load per step): workgroup b starts at pass floor(P b / grid), so this job, whose
-            // passes are [begin, begin + cost), is the first of the workgroups from ceil(begin grid / P) up to that of its end.
-            const bool dn = which == 2;
-            const uint32_t grid = dn ? d_grid : g_grid;
-            const uint64_t P = dn ? (uint64_t)d_total : (uint64_t)g_total * (fused ? 1u : 2u);
-            const uint64_t begin = dn ? d_begin : (which == 1 ? g_total + g_begin : g_begin), end = begin + (dn ? dc.job(nb) : gc.job(nb));
-            const uint32_t b0 = (uint32_t)((begin * grid + P - 1) / P), b1 = min(grid, (uint32_t)((end * grid + P - 1) / P));
-            for (uint32_t bb = b0; bb < b1; bb++) (dn ? dn_first : gu_first)[bb] = (which == 1 ? n_jobs : 0u) + jb;
-        }
-        if (which == 0)
-            emit(gu_table + jb, tg, (size_t)e * gu_w_stride, (size_t)e * gu_s_stride, (size_t)tok1 * hidden, (size_t)s1 * gs, true, gs, g_begin, gc);
-        else if (which == 1)
-            emit(gu_table + n_jobs + jb, tu, (size_t)e * gu_w_stride, (size_t)e * gu_s_stride, (size_t)tok1 * hidden, (size_t)s1 * gs, true, gs,
-                 g_total + g_begin, gc);
-        else
-            emit(dn_table + jb, td, (size_t)e * dn_w_stride, (size_t)e * dn_s_stride, (size_t)s1 * gs, (size_t)s1 * hidden, false, hidden, d_begin, dc);
-    }
-    if (t == 0) {
-        gu_hdr[0] = fused ? n_jobs : 2 * n_jobs; gu_hdr[1] = fused ? g_total : 2 * g_total;
-        dn_hdr[0] = n_jobs; dn_hdr[1] = d_total;
-    }
-}
-
-hipError_t moe_plan_launch(hipStream_t s, const float *logits, const float *router_bias, int policy, float *weights, uint32_t *experts,
-                           uint32_t slots, uint32_t k, uint32_t n_experts, const GemvJob &tg,
-                           const GemvJob &tu, const GemvJob &td, uint64_t gu_w_stride, uint64_t gu_s_stride, uint64_t dn_w_stride,
-                           uint64_t dn_s_stride, uint32_t hidden, uint32_t inter, bool fused, uint32_t group, uint32_t g_grid, uint32_t d_grid, GemvJob *gu_table,
-                           uint32_t *gu_hdr, GemvJob *dn_table, uint32_t *dn_hdr, uint32_t *gu_first, uint32_t *dn_first) {
-    if (n_experts > 1024 || slots > 4096 || (group != 2 && group != 4)) return hipErrorInvalidValue;
-    // (a wavefront per token while selecting: 16 wavefronts when the kernel routes)
-    hipLaunchKernelGGL(moe_plan_kernel, dim3(1), dim3(logits ? 1024 : 256), 0, s, logits, router_bias, policy, weights, experts, slots, k, n_experts, tg, tu, td,
-                       gu_w_stride, gu_s_stride,
-                       dn_w_stride, dn_s_stride, hidden, inter, fused ? 1u : 0u, group, g_grid, d_grid, gu_table, gu_hdr, dn_table, dn_hdr, gu_first, dn_first);
-    return hipGetLastError();
-}
-
 hipError_t router_select_launch(hipStream_t s, const float *logits, const float *bias, uint32_t tokens, uint32_t n_experts, uint32_t k,
                                 int policy, uint32_t *experts, float *weights) {
     if (tokens == 0) return hipSuccess;

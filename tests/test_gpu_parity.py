@@ -1117,6 +1117,43 @@ def test_moe_mxfp4_routed_equals_select_then_block(be, fmt, T, E, hidden, inter,
         be.dev_moe_mxfp4_routed(b, x, T, k, 0, policy, e2, w2, o2, ws, wsb)
 
 
+@pytest.mark.parametrize("T,E,k,hidden,inter,interleaved,outside", [
+    (17, 4, 4, 384, 320, 1, False), (16, 4, 1, 384, 128, 0, False), (16, 4, 1, 160, 352, 1, True), (40, 4, 2, 1152, 160, 0, False), (33, 3, 3, 2880, 288, 1, False), (20, 3, 3, 4096, 128, 1, False),
+    (50, 2, 2, 5120, 128, 0, True), (3, 6, 4, 4128, 4128, 0, False), (1100, 5, 4, 256, 128, 1, False)])
+def test_moe_mxfp4_groups_of_sixteen_tokens(be, fmt, T, E, k, hidden, inter, interleaved, outside):
+    """Blocks whose experts have more than four tokens on average (groups of sixteen) and just not: row lengths of one to five
+    128-element steps per wavefront, ragged last steps, gate and up apart and fused, terms that do not fit the workspace
+    (k * inter < hidden), more slots than one launch takes, ids outside the bank.  Sampled tokens against the oracle at the
+    bound of the four-token test (1e-5), and every sampled token bit for bit what it is in a two-token block."""
+    rng = np.random.default_rng(T + hidden)
+    g_rows = 2 * inter if interleaved else inter
+    gp, gs = O.quantize_mxfp4((rng.standard_normal(E * g_rows * hidden) * 0.05).astype(F), E * g_rows, hidden)
+    dp, ds = O.quantize_mxfp4((rng.standard_normal(E * hidden * inter) * 0.05).astype(F), E * hidden, inter)
+    up, us = (None, None) if interleaved else O.quantize_mxfp4((rng.standard_normal(E * inter * hidden) * 0.05).astype(F), E * inter, hidden)
+    gub, db = (rng.standard_normal(E * 2 * inter) * 0.1).astype(F), (rng.standard_normal(E * hidden) * 0.1).astype(F)
+    x = rng.standard_normal((T, hidden)).astype(F)
+    ex = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.uint32)
+    wt = rng.random((T, k)).astype(F)
+    if outside:
+        ex[1, 0] = E + 3
+        ex[T - 1, k - 1] = 0xFFFFFFFF
+    dev = {n: be.to_device(a) for n, a in dict(gp=gp, gs=gs, dp=dp, ds=ds, gub=gub, db=db, x=x, ex=ex, wt=wt).items()}
+    du, dus = (None, None) if interleaved else (be.to_device(up), be.to_device(us))
+    b = fmt.Mxfp4Experts(dev["gp"], dev["gs"], du, dus, dev["dp"], dev["ds"], E, hidden, inter, 7.0, 1.702, interleaved, None, dev["gub"], dev["db"])
+    wsb = be.moe_mxfp4_workspace_bytes(T, k, hidden, inter)
+    ws, do, two = be.malloc(wsb), be.malloc(T * hidden * 4), be.malloc(2 * hidden * 4)
+    assert be.dev_moe_mxfp4(b, dev["x"], T, k, dev["ex"], dev["wt"], do, ws, wsb), be.last_error()
+    be.synchronize()
+    got = be.d2h(do, (T, hidden), F)
+    for t in sorted({0, 1, T // 2, T - 2}):
+        assert be.dev_moe_mxfp4(b, dev["x"] + t * hidden * 4, 2, k, dev["ex"] + t * k * 4, dev["wt"] + t * k * 4, two, ws, wsb)
+        be.synchronize()
+        assert np.array_equal(be.d2h(two, (2, hidden), F), got[t:t + 2]), t
+        want = O.moe_block_mxfp4(x[t:t + 1], ex[t:t + 1], wt[t:t + 1], (gp, gs), None if interleaved else (up, us), (dp, ds), E, hidden, inter,
+                                 interleaved=bool(interleaved), gate_up_bias=gub, down_bias=db)
+        assert rel_l2(got[t], want[0]) < 1e-5, t
+
+
 def test_moe_mxfp4_job_groups_of_every_size(be, fmt):
     """Experts chosen by 1, 2, 3, 4 and 5 slots: jobs of one, two, three and four tokens and a second job for the
     fifth.  Every token's result equals, bit for bit, what it is in a two-token block."""
