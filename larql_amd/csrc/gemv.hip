@@ -550,18 +550,22 @@ __device__ __forceinline__ void run_q4k(const GemvJob &j, uint32_t p0, uint32_t 
 // The dot products run on v_mfma_i32_16x16x64_i8, exactly, with the roles
 // swapped: the 16 "B" columns are the 16 weight rows of the tile and the "A"
 // rows carry the activation.  Per 256-wide column, x is scaled by a power of
-// two to 28-bit integers n = rint(x * 2^(27-e)) (2^e > max|x|) and n is split
-// into four balanced base-128 digits (int8 "limbs"); A row 4g + 2cl + i holds
-// limb i (first operand set) or limb 2+i (second set) of sub-block 2g+cl in
-// the k-slots that the sub-block's nibbles occupy in B, zero elsewhere.  Lane
-// (row j = lane%16, kq = lane/16) supplies, per 32-byte group, the low nibbles
-// of its bytes 8kq..8kq+7 in k-slots 0-7 and the high nibbles in slots 8-15
-// (three mask/shift instructions per 8 weights) and, after two MFMAs per group,
-// holds for weight row j and group g = kq the eight exact integer sums
-// nibbles.limb — it is the very lane that decodes that group's two scales and
-// mins from the header.  The limb sums are recombined in f32 (the only
-// rounding besides the final scale), so the result differs from an f32 FMA
-// chain over exact products only by the 2^-28 relative quantum of x.
+// two to 31-bit integers n = trunc(x * 2^(30-e)) (2^e > max|x|) and n is split
+// into four balanced base-256 digits (the bytes of n + 0x80808080, each less
+// 128: two instructions for all four).  Lane (row j = lane%16, kq = lane/16)
+// owns group kq of weight row j, 32 bytes of nibbles: MFMA (h, nib) takes the
+// low (nib = 0) or high nibbles of its bytes 16h..16h+15 in the lane's 16
+// k-slots, three mask/shift instructions per 8 weights.  A row 4g + l holds
+// digit l of the activations of group g in the k-slots of kq == g and zero
+// elsewhere, so all 16 A rows are in use, and after four MFMAs the lane holds
+// for its own row and group the four exact digit sums of both sub-blocks — it is
+// the very lane that decodes their scales and mins from the header.  Digits meet
+// pairwise in integers and once in f32 (the only rounding besides the final
+// scale), so the result differs from an f32 FMA chain over exact products only
+// by the 2^-30 relative quantum of x.  (The scheme before had the low and high
+// nibbles of a group in one MFMA and two digits per operand set: eight MFMAs and
+// 28 selects per column to mask the operands, and every activation was split by
+// two lanes.)  The digits reach the operand layout through 1 KB of LDS per column.
 // Value per row as q4k_matvec_into (larql-compute/src/cpu/ops/q4_common/
 // matvec_f32.rs:116-155): sum over sub-blocks of (d*sc)*dot(q,x) - (dmin*mn)*sum(x).
 //
@@ -579,107 +583,67 @@ constexpr int kQ4kBatchTiles = 4;  // 16-row tiles between two folds of the row 
 constexpr int kQ4kMaxColPasses = 4;
 constexpr int kQ4kMaxWaves = 10;  // with the ring, the partials and 4 prepared columns per wavefront this fills the 160 KB of LDS
 constexpr uint32_t kQ4kTileBytes = 16 * 144;
-constexpr uint32_t kQ4kColBytes = 1024 + 64;  // a column's activation limbs for 64 lanes, then {k, -, -, -, sums of 8 sub-blocks}
+constexpr uint32_t kQ4kColBytes = 1024 + 64;  // a column's digits (four planes of 256 bytes), then {2^(e-30), -, -, -, sums of its 8 sub-blocks}
+constexpr uint32_t kQ4kZeroBytes = 64;        // what the lanes outside an A row's group read
 
 struct Q4kCol {
-    uint32_t xq[4];        // this lane's 8 activations as int8 limbs: {limb i: 2 dwords, limb 2+i: 2 dwords}, i = lane & 1
-    float k;               // 2^(e-27): integer dot -> value
+    Q4kOp xm[4];           // A operand of MFMA 2h + nib
+    float k;               // 2^(e-30): integer dot -> value
     float sum_lo, sum_hi;  // sum of x over sub-blocks 2kq and 2kq+1
 };
 
-// A column's activations as loaded
-struct Q4kRaw { f32x4 v, a, b; };
-
-__device__ __forceinline__ Q4kRaw q4k_mfma_load_col(const float *x, uint32_t c, uint32_t lane) {
-    // A-operand row j = 4g + 2cl + i feeds sub-block m = j/2 = 2g+cl: elements 8kq..8kq+7 of it
-    const uint32_t j = lane & 15u, kq = lane >> 4, m = j >> 1;
-    g_f4p xc = (g_f4p)(x + (size_t)c * 256);
-    g_f4p xs = (g_f4p)(x + (size_t)c * 256 + m * 32 + 8 * kq);
-    Q4kRaw r;
-    r.v = xc[lane];  // 4 consecutive activations per lane: column max and per-sub-block sums (8 lanes each)
-    r.a = xs[0];
-    r.b = xs[1];
-    return r;
-}
-
-__device__ __forceinline__ Q4kCol q4k_mfma_finish_col(const Q4kRaw &r, uint32_t lane) {
-    const uint32_t j = lane & 15u, kq = lane >> 4;
-    float mx = wave_max_nonneg(fmaxf(fmaxf(fabsf(r.v.x), fabsf(r.v.y)), fmaxf(fabsf(r.v.z), fabsf(r.v.w))));
-    float sm = (r.v.x + r.v.y) + (r.v.z + r.v.w);
+// The digit planes of a column whose activations a wavefront holds four elements per lane (element 4*lane first), plane l
+// (l = 0: most significant) at planes + 256 l; its scale and this lane's sums.
+__device__ __forceinline__ void q4k_digits(const f32x4 v, uint32_t lane, uint8_t *planes, float &k, float &sum_lo, float &sum_hi) {
+    const float mx = wave_max_nonneg(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+    float sm = (v.x + v.y) + (v.z + v.w);
     // sum over the 8 lanes of a sub-block: the exchange pattern of a butterfly (partners 1, 2, 4 lanes away), by DPP
     sm = dpp_add<0xB1>(sm);   // quad_perm [1,0,3,2]
     sm = dpp_add<0x4E>(sm);   // quad_perm [2,3,0,1]
     sm = dpp_add<0x141>(sm);  // row_half_mirror: the other quad of the eight
-    Q4kCol col;
-    {   // sub-block m's sum sits in lanes 8m .. 8m+7; this lane wants sub-blocks 2kq and 2kq+1
-        float sb[8];
-#pragma unroll
-        for (int m = 0; m < 8; m++) sb[m] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sm), 8 * m));
-        col.sum_lo = kq == 0 ? sb[0] : (kq == 1 ? sb[2] : (kq == 2 ? sb[4] : sb[6]));
-        col.sum_hi = kq == 0 ? sb[1] : (kq == 1 ? sb[3] : (kq == 2 ? sb[5] : sb[7]));
-    }
+    // sub-blocks 2kq and 2kq+1 lie in the lower and upper eight lanes of this lane's row of 16
+    const float other = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, sm), 0x128, 0xF, 0xF, false));  // row_ror:8
+    sum_lo = (lane & 8u) ? other : sm;
+    sum_hi = (lane & 8u) ? sm : other;
     int ex = 0;
     if (mx > 0.f && mx < __builtin_inff()) (void)frexpf(mx, &ex);  // mx = f * 2^ex, f in [0.5, 1)
-    ex = max(-90, min(120, ex));
-    const float to_int = ldexpf(1.f, 27 - ex);  // |x| * to_int < 2^27
-    col.k = ldexpf(1.f, ex - 27);
-    const float e[8] = {r.a.x, r.a.y, r.a.z, r.a.w, r.b.x, r.b.y, r.b.z, r.b.w};
-    const uint32_t i = j & 1u;
-    uint32_t la[8], lb[8];  // limbs i and 2+i of the 8 elements, as unsigned bytes
+    ex = max(-90, ex);
+    const float to_int = ldexpf(1.f, 30 - ex);  // |x| * to_int < 2^30
+    k = ldexpf(1.f, ex - 30);
+    uint32_t u[4];
+    const float e[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-    for (int t = 0; t < 8; t++) {
-        // n = l0*128^3 + l1*128^2 + l2*128 + l3 with l1..l3 in [-64, 63], l0 in [-64, 64]
-        const int n = (int)__builtin_rintf(e[t] * to_int);
-        const int l3 = ((n + 64) & 127) - 64, n1 = (n - l3) >> 7;
-        const int l2 = ((n1 + 64) & 127) - 64, n2 = (n1 - l2) >> 7;
-        const int l1 = ((n2 + 64) & 127) - 64, l0 = (n2 - l1) >> 7;
-        la[t] = (uint32_t)(i ? l1 : l0) & 0xFFu;
-        lb[t] = (uint32_t)(i ? l3 : l2) & 0xFFu;
-    }
-    col.xq[0] = la[0] | (la[1] << 8) | (la[2] << 16) | (la[3] << 24);
-    col.xq[1] = la[4] | (la[5] << 8) | (la[6] << 16) | (la[7] << 24);
-    col.xq[2] = lb[0] | (lb[1] << 8) | (lb[2] << 16) | (lb[3] << 24);
-    col.xq[3] = lb[4] | (lb[5] << 8) | (lb[6] << 16) | (lb[7] << 24);
-    return col;
+    for (int t = 0; t < 4; t++) u[t] = (uint32_t)(int)(e[t] * to_int) + 0x80808080u;
+    // bytes of the four elements transposed into the four planes, 128 taken off each (a flip of its top bit)
+    const uint32_t a01 = __builtin_amdgcn_perm(u[1], u[0], 0x05010400u), b01 = __builtin_amdgcn_perm(u[1], u[0], 0x07030602u);
+    const uint32_t a23 = __builtin_amdgcn_perm(u[3], u[2], 0x05010400u), b23 = __builtin_amdgcn_perm(u[3], u[2], 0x07030602u);
+    uint32_t *p = reinterpret_cast<uint32_t *>(planes) + lane;
+    p[0] = __builtin_amdgcn_perm(b23, b01, 0x07060302u) ^ 0x80808080u;
+    p[64] = __builtin_amdgcn_perm(b23, b01, 0x05040100u) ^ 0x80808080u;
+    p[128] = __builtin_amdgcn_perm(a23, a01, 0x07060302u) ^ 0x80808080u;
+    p[192] = __builtin_amdgcn_perm(a23, a01, 0x05040100u) ^ 0x80808080u;
 }
 
-// xm[2g] / xm[2g+1]: A operands (limbs 0,1 / limbs 2,3) of the MFMAs of group g.  A lane is non-zero only in
-// its own group (j/4) and only in the k-slots of its sub-block's nibbles: 0-7 (low, cl = 0) or 8-15 (high).
-__device__ __forceinline__ void q4k_mfma_operands(Q4kOp (&xm)[8], const Q4kCol &col, uint32_t j) {
-    const uint32_t my_g = j >> 2, cl = (j >> 1) & 1u;
+// This lane's A operands: digit l of group g for row 4g + l = lane % 16 where the lane's k-slots are the group's, zeros elsewhere
+__device__ __forceinline__ void q4k_operands(Q4kOp (&xm)[4], const uint8_t *planes, const uint8_t *zeros, uint32_t lane) {
+    const uint32_t j = lane & 15u, kq = lane >> 4;
+    const uint8_t *p = (j >> 2) == kq ? planes + (j & 3u) * 256 + kq * 64 : zeros;
 #pragma unroll
-    for (int g = 0; g < 4; g++) {
-        const bool lo = my_g == (uint32_t)g && cl == 0, hi = my_g == (uint32_t)g && cl == 1;
-        xm[2 * g].u[0] = lo ? col.xq[0] : 0u; xm[2 * g].u[1] = lo ? col.xq[1] : 0u;
-        xm[2 * g].u[2] = hi ? col.xq[0] : 0u; xm[2 * g].u[3] = hi ? col.xq[1] : 0u;
-        xm[2 * g + 1].u[0] = lo ? col.xq[2] : 0u; xm[2 * g + 1].u[1] = lo ? col.xq[3] : 0u;
-        xm[2 * g + 1].u[2] = hi ? col.xq[2] : 0u; xm[2 * g + 1].u[3] = hi ? col.xq[3] : 0u;
-    }
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int nib = 0; nib < 2; nib++) xm[2 * h + nib].v = *reinterpret_cast<const i32x4 *>(p + 32 * nib + 16 * h);
 }
 
-// one wave-tile from its LDS slot: 16 rows x one super-block against the column's activations
-__device__ __forceinline__ float q4k_mfma_tile(const uint8_t *slot, const Q4kOp (&xm)[8], const Q4kCol &col, uint32_t j, uint32_t kq) {
-    const uint8_t *sp = slot + j * 144;
-    const u32x4 hdr = *reinterpret_cast<const u32x4 *>(sp);
-    u32x2 q[4];
+// one wave-tile: this lane's weight row and group (header, 32 bytes of nibbles) against the column's activations
+__device__ __forceinline__ float q4k_mfma_dot(const u32x4 hdr, const u32x4 q0, const u32x4 q1, const Q4kCol &col, uint32_t kq) {
+    i32x4 Dl = {0, 0, 0, 0}, Dh = {0, 0, 0, 0};
 #pragma unroll
-    for (int g = 0; g < 4; g++) q[g] = *reinterpret_cast<const u32x2 *>(sp + 16 + 32 * g + 8 * kq);
-    i32x4 Da = {0, 0, 0, 0}, Db = {0, 0, 0, 0};
-#pragma unroll
-    for (int g = 0; g < 4; g++) {
-        Q4kOp b;
-        b.u[0] = q[g].x & 0x0F0F0F0Fu; b.u[1] = q[g].y & 0x0F0F0F0Fu;
-        b.u[2] = (q[g].x >> 4) & 0x0F0F0F0Fu; b.u[3] = (q[g].y >> 4) & 0x0F0F0F0Fu;
-        Da = __builtin_amdgcn_mfma_i32_16x16x64_i8(xm[2 * g].v, b.v, Da, 0, 0, 0);
-        Db = __builtin_amdgcn_mfma_i32_16x16x64_i8(xm[2 * g + 1].v, b.v, Db, 0, 0, 0);
+    for (int h = 0; h < 2; h++) {
+        const u32x4 q = h ? q1 : q0;
+        const u32x4 lo = q & 0x0F0F0F0Fu, hi = (q >> 4) & 0x0F0F0F0Fu;
+        Dl = __builtin_amdgcn_mfma_i32_16x16x64_i8(col.xm[2 * h].v, __builtin_bit_cast(i32x4, lo), Dl, 0, 0, 0);
+        Dh = __builtin_amdgcn_mfma_i32_16x16x64_i8(col.xm[2 * h + 1].v, __builtin_bit_cast(i32x4, hi), Dh, 0, 0, 0);
     }
-    // this lane's group is g = kq.  Da = [lo.l0, lo.l1, hi.l0, hi.l1], Db = [lo.l2, lo.l3, hi.l2, hi.l3]
-    float dot_lo = __builtin_fmaf((float)Da[0], 128.f, (float)Da[1]);
-    float dot_hi = __builtin_fmaf((float)Da[2], 128.f, (float)Da[3]);
-    dot_lo = __builtin_fmaf(dot_lo, 128.f, (float)Db[0]);
-    dot_hi = __builtin_fmaf(dot_hi, 128.f, (float)Db[2]);
-    dot_lo = __builtin_fmaf(dot_lo, 128.f, (float)Db[1]) * col.k;
-    dot_hi = __builtin_fmaf(dot_hi, 128.f, (float)Db[3]) * col.k;
     // header fields as get_scale_min_k4 (matvec_f32.rs:124-131), two bytes at a time
     const float d = half_bits_to_float(hdr.x & 0xFFFFu), dmin = half_bits_to_float(hdr.x >> 16);
     const uint32_t sh = (kq & 1u) * 16u;
@@ -688,6 +652,9 @@ __device__ __forceinline__ float q4k_mfma_tile(const uint8_t *slot, const Q4kOp 
     const uint32_t sc2 = kq < 2 ? (a & 0x3F3Fu) : sc_hi2, mn2 = kq < 2 ? (b & 0x3F3Fu) : mn_hi2;
     const float sc_lo = d * (float)(sc2 & 0xFFu), sc_hi = d * (float)(sc2 >> 8);
     const float mn_lo = dmin * (float)(mn2 & 0xFFu), mn_hi = dmin * (float)(mn2 >> 8);
+    // a digit sum is at most 32 * 15 * 128 = 61440: two of them meet below 2^24, exact in f32
+    const float dot_lo = __builtin_fmaf((float)(Dl[0] * 256 + Dl[1]), 65536.f, (float)(Dl[2] * 256 + Dl[3])) * col.k;
+    const float dot_hi = __builtin_fmaf((float)(Dh[0] * 256 + Dh[1]), 65536.f, (float)(Dh[2] * 256 + Dh[3])) * col.k;
     float r = sc_lo * dot_lo - mn_lo * col.sum_lo;
     r += sc_hi * dot_hi - mn_hi * col.sum_hi;
     return r;
@@ -744,41 +711,42 @@ __device__ __forceinline__ void run_q4k_mfma(const GemvJob &j, uint32_t tile_a, 
     };
     // the activations of all this wavefront's columns are requested first and together (one memory round
     // trip, ahead of the weight tiles in the in-order return queue), then prepared while the tiles fly
-    Q4kRaw raw[kQ4kMaxColPasses];
+    f32x4 raw[kQ4kMaxColPasses];
 #pragma unroll
     for (int p = 0; p < kQ4kMaxColPasses; p++)
-        if ((uint32_t)p < np) raw[p] = q4k_mfma_load_col(j.x, wv + nwj * p, lane);
+        if ((uint32_t)p < np) raw[p] = ((g_f4p)(j.x + (size_t)(wv + nwj * p) * 256))[lane];
     if (np >= 1)
         for (int s = 0; s < NS - 1; s++) issue();
 
-    // Column state: in registers when the wavefront has one column; with several it is prepared once per
-    // job into this wavefront's own LDS area (1 KB of operands + 64 B of scales and sums per column) and
-    // fetched at every column change.
+    // Column state: in registers when the wavefront has one column (the ring's last slot, still free, is its scratch);
+    // with several it is prepared once per job into this wavefront's own LDS area and fetched at every column change.
     uint8_t *cols = lds + nw_launch * (NS * kQ4kTileBytes) + 2 * R * 16 * nw_launch * 4 * sizeof(float) +
-                    wv * (kQ4kMaxColPasses * kQ4kColBytes);
+                    wv * (kQ4kMaxColPasses * kQ4kColBytes + kQ4kZeroBytes);
     Q4kCol col;
-    Q4kOp xm[8];
     auto fetch_col = [&](uint32_t p) {
         const uint8_t *cp = cols + p * kQ4kColBytes;
-        const u32x4 xq = *reinterpret_cast<const u32x4 *>(cp + lane * 16);
+        q4k_operands(col.xm, cp, cols + kQ4kMaxColPasses * kQ4kColBytes, lane);
         const float2_t sm = *reinterpret_cast<const float2_t *>(cp + 1024 + 16 + kq * 8);
-        col.xq[0] = xq.x; col.xq[1] = xq.y; col.xq[2] = xq.z; col.xq[3] = xq.w;
         col.k = *reinterpret_cast<const float *>(cp + 1024);
         col.sum_lo = sm.x; col.sum_hi = sm.y;
-        q4k_mfma_operands(xm, col, jr);
     };
     if (np == 1) {
-        col = q4k_mfma_finish_col(raw[0], lane);
-        q4k_mfma_operands(xm, col, jr);
+        uint8_t *scratch = ring + (n_issue % NS) * kQ4kTileBytes;
+        reinterpret_cast<uint32_t *>(scratch + 1024)[lane & 15u] = 0u;
+        q4k_digits(raw[0], lane, scratch, col.k, col.sum_lo, col.sum_hi);
+        asm volatile("" ::: "memory");  // same wavefront: LDS executes its writes before the reads that follow
+        q4k_operands(col.xm, scratch, scratch + 1024, lane);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot is filled with weights next
     } else if (np > 1) {
+        reinterpret_cast<uint32_t *>(cols + kQ4kMaxColPasses * kQ4kColBytes)[lane & 15u] = 0u;
 #pragma unroll
         for (int p = 0; p < kQ4kMaxColPasses; p++) {
             if ((uint32_t)p < np) {
-                const Q4kCol c = q4k_mfma_finish_col(raw[p], lane);
                 uint8_t *cp = cols + p * kQ4kColBytes;
-                *reinterpret_cast<u32x4 *>(cp + lane * 16) = (u32x4){c.xq[0], c.xq[1], c.xq[2], c.xq[3]};
-                if (lane == 0) *reinterpret_cast<float *>(cp + 1024) = c.k;
-                if (jr == 0) *reinterpret_cast<float2_t *>(cp + 1024 + 16 + kq * 8) = (float2_t){c.sum_lo, c.sum_hi};
+                float ck, lo, hi;
+                q4k_digits(raw[p], lane, cp, ck, lo, hi);
+                if (lane == 0) *reinterpret_cast<float *>(cp + 1024) = ck;
+                if (jr == 0) *reinterpret_cast<float2_t *>(cp + 1024 + 16 + kq * 8) = (float2_t){lo, hi};
             }
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // own writes, own reads: program order is enough
@@ -801,7 +769,9 @@ __device__ __forceinline__ void run_q4k_mfma(const GemvJob &j, uint32_t tile_a, 
                         issue();
                         LARQL_WAIT_VMCNT(3 * (NS - 1));  // at most NS-1 younger wave-tiles still in flight: the oldest has landed
                         asm volatile("" ::: "memory");
-                        racc[tl] += q4k_mfma_tile(ring + (n_use % NS) * kQ4kTileBytes, xm, col, jr, kq);
+                        const uint8_t *sp = ring + (n_use % NS) * kQ4kTileBytes + jr * 144;
+                        const u32x4 *qp = reinterpret_cast<const u32x4 *>(sp + 16 + 32 * kq);
+                        racc[tl] += q4k_mfma_dot(*reinterpret_cast<const u32x4 *>(sp), qp[0], qp[1], col, kq);
                         n_use++;
                     }
                 }
@@ -3375,7 +3345,7 @@ size_t gemv_lds_bytes(const GemvJob *jobs, size_t n, uint32_t threads) {
         bool multi = false;  // some row needs several column passes: room for the prepared activations
         for (size_t i = 0; i < n; i++) multi = multi || jobs[i].k / 256 > (uint64_t)kQ4kMaxWaves;
         return nw * kQ4kStages * kQ4kTileBytes + 2 * (size_t)kQ4kBatchTiles * 16 * nw * 4 * sizeof(float) +
-               (multi ? nw * kQ4kMaxColPasses * kQ4kColBytes : 0);
+               (multi ? nw * (kQ4kMaxColPasses * kQ4kColBytes + kQ4kZeroBytes) : 0);
     }
     size_t m = 0;
     for (size_t i = 0; i < n; i++) {
