@@ -262,6 +262,13 @@ static size_t table_bytes_for(size_t n_jobs) { return n_jobs * sizeof(GemvJob) +
 
 int prepare_same_kind(larql_hip_ctx *c, GemvJob *live, size_t n_live, void *table_dst, PreparedLaunch &P, int stage_slot = -1) {
     P.kind = live[0].kind;
+    memset(&P.L, 0, sizeof P.L);
+    if (P.kind == KIND_Q4K_MFMA && gemv_q4k_short(live, n_live, (uint32_t)c->cu_count, &P.threads, &P.grid, &P.lds, &P.L.pad)) {
+        P.kind = KIND_Q4K_SHORT;
+        P.L.n_jobs = (uint32_t)n_live;
+        for (size_t i = 0; i < n_live; i++) P.L.inl[i] = live[i];
+        return LARQL_OK;
+    }
     P.threads = gemv_pick_threads(live, n_live);
     if (P.threads == 0) return fail(c, LARQL_UNSUPPORTED, "matvec: row length not supported by the gfx950 kernels");
     uint64_t total = 0;
@@ -293,7 +300,6 @@ int prepare_same_kind(larql_hip_ctx *c, GemvJob *live, size_t n_live, void *tabl
     }
     if (grid > total) grid = total;
     P.grid = (uint32_t)grid;
-    memset(&P.L, 0, sizeof P.L);
     P.L.total_passes = total;
     P.L.n_jobs = (uint32_t)n_live;
     P.L.pad = gemv_launch_param(live, n_live);

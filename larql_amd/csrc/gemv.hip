@@ -581,6 +581,7 @@ union Q4kOp { i32x4 v; uint32_t u[4]; };  // one MFMA operand: 16 int8 k-slots o
 constexpr int kQ4kStages = 4;      // wave-tiles in flight per wavefront (ring slots of 2304 B)
 constexpr int kQ4kBatchTiles = 4;  // 16-row tiles between two folds of the row partials
 constexpr int kQ4kMaxColPasses = 4;
+constexpr uint32_t kQ4kShortJobs = 4;  // matvecs of a short launch
 constexpr int kQ4kMaxWaves = 10;  // with the ring, the partials and 4 prepared columns per wavefront this fills the 160 KB of LDS
 constexpr uint32_t kQ4kTileBytes = 16 * 144;
 constexpr uint32_t kQ4kColBytes = 1024 + 64;  // a column's digits (four planes of 256 bytes), then {2^(e-30), -, -, -, sums of its 8 sub-blocks}
@@ -794,6 +795,104 @@ __device__ __forceinline__ void run_q4k_mfma(const GemvJob &j, uint32_t tile_a, 
             if (qd == 0 && row_base + rr < rows) ((g_f32wp)j.out)[row_base + rr] = s;
         }
         parity ^= 1u;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Q4_K, short launches: the matvecs of one stage of a token (q, k, v | o | gate, up | down), a few tiles per compute unit.
+//
+// Bound: latency.  Such a launch moves 3-30 MB (0.5-5 us) and depends on the one before it, so what counts is the chain
+// from a wavefront's first instruction to its last store.  The streaming kernel above walks it in steps (descriptor from a
+// 2 KB argument block, activation, a ring of tiles, a fold per batch, next tile); here a workgroup knows its whole work
+// from a small argument block, and every load of it leaves before anything is waited for: the activation's columns, then
+// all NT tiles x NP columns of the wavefront, straight into registers (a lane's header and 32 bytes of nibbles are three
+// 16-byte loads).  One barrier, one fold.  A tile is cut to `tile_rows` <= 16 rows so that all compute units get the same
+// share (2560 rows: 256 tiles of 10, where 16-row tiles kept 160 of 256 busy).
+// Same operands and the same order of additions per row as the streaming kernel: results are equal bit for bit.
+// ---------------------------------------------------------------------------
+struct Q4kShortArgs {
+    const float *x;
+    uint32_t cpr, nw, tile_rows, n_jobs;
+    const uint8_t *w[kQ4kShortJobs];
+    float *out[kQ4kShortJobs];
+    uint32_t rows[kQ4kShortJobs], tile_end[kQ4kShortJobs];  // tile_end: tiles of the jobs up to and with this one
+};
+
+template <int NT, int NP>
+__global__ void __launch_bounds__(kQ4kMaxWaves * 64) gemv_q4k_short_kernel(const Q4kShortArgs A) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t q4ks_lds[];
+    const uint32_t lane = threadIdx.x & 63u, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t jr = lane & 15u, kq = lane >> 4;
+    const uint32_t nw = A.nw, cpr = A.cpr, row_bytes = cpr * 144, TR = A.tile_rows;
+    const uint32_t tile0 = blockIdx.x * NT, tiles = A.tile_end[A.n_jobs - 1];
+
+    // columns wv, wv + nw, ... of this wavefront (one past the row's end reads the last column and is not used)
+    f32x4 raw[NP];
+#pragma unroll
+    for (int p = 0; p < NP; p++) raw[p] = ((g_f4p)(A.x + (size_t)min(wv + nw * p, cpr - 1) * 256))[lane];
+
+    // the tiles: job, first row, rows (a tile past the end is the last one again)
+    uint32_t job[NT], row0[NT], live[NT];
+    u32x4 hdr[NT][NP], q0[NT][NP], q1[NT][NP];
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        const uint32_t tile = min(tile0 + t, tiles - 1);
+        uint32_t ji = 0;
+#pragma unroll
+        for (uint32_t q = 0; q + 1 < kQ4kShortJobs; q++) ji += (q + 1 < A.n_jobs && tile >= A.tile_end[q]) ? 1u : 0u;
+        job[t] = ji;
+        row0[t] = (tile - (ji ? A.tile_end[ji - 1] : 0u)) * TR;
+        live[t] = tile0 + t < tiles ? min(TR, A.rows[ji] - row0[t]) : 0u;
+        const uint32_t row = row0[t] + min(jr, max(live[t], 1u) - 1);
+        const uint8_t *wr = A.w[ji] + (size_t)row * row_bytes;
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+            g_u4p blk = (g_u4p)(wr + min(wv + nw * p, cpr - 1) * 144);
+            hdr[t][p] = blk[0];
+            q0[t][p] = blk[1 + 2 * kq];
+            q1[t][p] = blk[2 + 2 * kq];
+        }
+    }
+
+    uint8_t *planes = q4ks_lds + wv * (NP * 1024), *zeros = q4ks_lds + nw * (NP * 1024);
+    float *part = reinterpret_cast<float *>(zeros + kQ4kZeroBytes);  // [NT * 16 rows][nw * 4]
+    reinterpret_cast<uint32_t *>(zeros)[lane & 15u] = 0u;           // (every wavefront the same zeros)
+    float k[NP], lo[NP], hi[NP];
+#pragma unroll
+    for (int p = 0; p < NP; p++) q4k_digits(raw[p], lane, planes + p * 1024, k[p], lo[p], hi[p]);
+    asm volatile("" ::: "memory");  // same wavefront: LDS executes its writes before the reads that follow
+    float racc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) racc[t] = 0.f;
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+        if (p == 0 || wv + nw * p < cpr) {
+            Q4kCol col;
+            q4k_operands(col.xm, planes + p * 1024, zeros, lane);
+            col.k = k[p]; col.sum_lo = lo[p]; col.sum_hi = hi[p];
+#pragma unroll
+            for (int t = 0; t < NT; t++) racc[t] += q4k_mfma_dot(hdr[t][p], q0[t][p], q1[t][p], col, kq);
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < NT; t++) part[(t * 16 + jr) * (nw * 4) + wv * 4 + kq] = racc[t];
+    __syncthreads();
+    // fold: 4 lanes per row, lane q sums the group-q partial of every wavefront in order
+    for (uint32_t rr = threadIdx.x >> 2; rr < NT * 16; rr += blockDim.x >> 2) {
+        const uint32_t qd = threadIdx.x & 3u;
+        float v[kQ4kMaxWaves];
+#pragma unroll
+        for (uint32_t w = 0; w < kQ4kMaxWaves; w++) v[w] = part[rr * (nw * 4) + min(w, nw - 1) * 4 + qd];
+        float s = v[0];
+#pragma unroll
+        for (uint32_t w = 1; w < kQ4kMaxWaves; w++) s = w < nw ? s + v[w] : s;
+        s = dpp_add<0xB1>(s);  // quad_perm [1,0,3,2]
+        s = dpp_add<0x4E>(s);  // quad_perm [2,3,0,1]
+        uint32_t ji = job[0], r0 = row0[0], n = live[0];
+#pragma unroll
+        for (uint32_t t = 1; t < NT; t++)
+            if ((rr >> 4) == t) { ji = job[t]; r0 = row0[t]; n = live[t]; }
+        if (qd == 0 && (rr & 15u) < n) ((g_f32wp)A.out[ji])[r0 + (rr & 15u)] = s;
     }
 }
 
@@ -3356,6 +3455,35 @@ size_t gemv_lds_bytes(const GemvJob *jobs, size_t n, uint32_t threads) {
     return m;
 }
 
+// A launch of matvecs against one activation that leaves every compute unit a few tiles (NT tiles x NP columns per
+// wavefront <= 10, all of them in registers) takes the short kernel: fills grid, threads, LDS and L.pad.
+static uint32_t q4k_short_np(uint64_t cpr) { const uint32_t nw = q4k_mfma_waves(cpr); return (uint32_t)((cpr + nw - 1) / nw); }
+bool gemv_q4k_short(const GemvJob *jobs, size_t n, uint32_t cu_count, uint32_t *threads, uint32_t *grid, size_t *lds, uint32_t *param) {
+    if (n == 0 || n > (size_t)kQ4kShortJobs) return false;
+    uint64_t rows = 0;
+    for (size_t i = 0; i < n; i++) {
+        const GemvJob &j = jobs[i];
+        if (j.kind != KIND_Q4K_MFMA || j.x != jobs[0].x || j.k != jobs[0].k || j.row_stride || j.sel || j.batch > 1) return false;
+        rows += j.rows;
+    }
+    const uint64_t cpr = jobs[0].k / 256;
+    const uint32_t nw = q4k_mfma_waves(cpr), np = q4k_short_np(cpr);
+    const uint64_t nt = (rows + 16ull * cu_count - 1) / (16ull * cu_count);
+    if (nt == 0 || nt * np > 10 || nt > 8) return false;
+    uint32_t tr = (uint32_t)((rows + cu_count * nt - 1) / (cu_count * nt));
+    uint64_t tiles = 0;
+    for (;; tr++) {  // (a job's last tile is ragged: a row more per tile where the tiles would spill over into another round)
+        tiles = 0;
+        for (size_t i = 0; i < n; i++) tiles += (jobs[i].rows + tr - 1) / tr;
+        if (tiles <= cu_count * nt || tr == 16) break;
+    }
+    *threads = nw * 64;
+    *grid = (uint32_t)((tiles + nt - 1) / nt);
+    *lds = (size_t)nw * np * 1024 + kQ4kZeroBytes + (size_t)nt * 16 * nw * 4 * sizeof(float);
+    *param = tr | (uint32_t)nt << 8 | np << 16;
+    return true;
+}
+
 uint32_t gemv_wgs_per_cu(int kind, uint32_t threads, size_t lds, uint32_t dflt) {
     if (kind != KIND_Q4K_MFMA && kind != KIND_MXFP4_MFMA && kind != KIND_BF16_MFMA && kind != KIND_Q4K_BATCH && kind != KIND_Q8_0_MFMA &&
         kind != KIND_Q4K_Q8K && kind != KIND_Q6K_MFMA)
@@ -3451,6 +3579,26 @@ hipError_t gemv_launch(hipStream_t stream, int kind, const GemvLaunch &L, uint32
                 attr_set_mx4 = true;
             }
             hipLaunchKernelGGL(gemv_mxfp4_mfma_kernel, dim3(grid), dim3(threads), lds, stream, L);
+            break;
+        }
+        case KIND_Q4K_SHORT: {
+            Q4kShortArgs A = {};
+            const uint32_t tr = L.pad & 0xFFu, nt = (L.pad >> 8) & 0xFFu, np = L.pad >> 16;
+            A.x = L.inl[0].x; A.cpr = (uint32_t)(L.inl[0].k / 256); A.nw = threads / 64; A.tile_rows = tr; A.n_jobs = L.n_jobs;
+            uint32_t tiles = 0;
+            for (uint32_t i = 0; i < L.n_jobs; i++) {
+                const GemvJob &j = L.inl[i];
+                tiles += (uint32_t)((j.rows + tr - 1) / tr);
+                A.w[i] = j.w; A.out[i] = j.out; A.rows[i] = (uint32_t)j.rows; A.tile_end[i] = tiles;
+            }
+#define LARQL_Q4K_SHORT(NT, NP) case (NT) | (NP) << 8: hipLaunchKernelGGL((gemv_q4k_short_kernel<NT, NP>), dim3(grid), dim3(threads), lds, stream, A); break;
+            switch (nt | np << 8) {
+                LARQL_Q4K_SHORT(1, 1) LARQL_Q4K_SHORT(2, 1) LARQL_Q4K_SHORT(3, 1) LARQL_Q4K_SHORT(4, 1) LARQL_Q4K_SHORT(5, 1) LARQL_Q4K_SHORT(6, 1)
+                LARQL_Q4K_SHORT(7, 1) LARQL_Q4K_SHORT(8, 1) LARQL_Q4K_SHORT(1, 2) LARQL_Q4K_SHORT(2, 2) LARQL_Q4K_SHORT(3, 2) LARQL_Q4K_SHORT(4, 2)
+                LARQL_Q4K_SHORT(5, 2) LARQL_Q4K_SHORT(1, 3) LARQL_Q4K_SHORT(2, 3) LARQL_Q4K_SHORT(3, 3) LARQL_Q4K_SHORT(1, 4) LARQL_Q4K_SHORT(2, 4)
+                default: return hipErrorInvalidValue;
+            }
+#undef LARQL_Q4K_SHORT
             break;
         }
         case KIND_Q4K_MFMA: {
