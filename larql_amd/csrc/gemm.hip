@@ -82,9 +82,9 @@ __global__ void __launch_bounds__(1024) q4k_gemm_prep_kernel(const void *__restr
     const uint32_t tok = blockIdx.x;
     const u32x4 *xb = reinterpret_cast<const u32x4 *>((const uint16_t *)x + (size_t)tok * hidden);
     const f32x4 *xf = reinterpret_cast<const f32x4 *>((const float *)x + (size_t)tok * hidden);
-    auto load8 = [&](uint32_t v, float (&o)[8]) {
+    auto load8 = [&](uint32_t v, float (&o)[8], const u32x4 *kept = nullptr) {
         if (x_is_bf16) {
-            const u32x4 r = xb[v];
+            const u32x4 r = kept ? *kept : xb[v];
             const uint32_t w[4] = {r.x, r.y, r.z, r.w};
 #pragma unroll
             for (int i = 0; i < 4; i++) {
@@ -96,13 +96,26 @@ __global__ void __launch_bounds__(1024) q4k_gemm_prep_kernel(const void *__restr
             o[0] = a.x; o[1] = a.y; o[2] = a.z; o[3] = a.w; o[4] = b.x; o[5] = b.y; o[6] = b.z; o[7] = b.w;
         }
     };
+    // KEEP vectors of a bf16 token stay in the thread's registers from the maximum to the conversion, requested together (the
+    // launch is a chain of round trips; 77 tokens of 15360: 5.9 us)
+    constexpr uint32_t KEEP = 2;
+    u32x4 kept[KEEP] = {};
     float mx = 0.f;
-    for (uint32_t v = t; v < nvec; v += blockDim.x) {
+    if (x_is_bf16) {
+#pragma unroll
+        for (uint32_t u = 0; u < KEEP; u++) kept[u] = xb[min(t + u * blockDim.x, nvec - 1)];
+    }
+    auto max8 = [&](uint32_t v, const u32x4 *k) {
         float o[8];
-        load8(v, o);
+        load8(v, o, k);
 #pragma unroll
         for (int i = 0; i < 8; i++) mx = fmaxf(mx, fabsf(o[i]));
+    };
+    if (x_is_bf16) {  // (a clamped vector is the token's own: it does not change the maximum)
+#pragma unroll
+        for (uint32_t u = 0; u < KEEP; u++) max8(0, &kept[u]);
     }
+    for (uint32_t v = t + (x_is_bf16 ? KEEP * blockDim.x : 0u); v < nvec; v += blockDim.x) max8(v, nullptr);
     for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
     if ((t & 63u) == 0) red[t >> 6] = mx;
     __syncthreads();
@@ -119,9 +132,9 @@ __global__ void __launch_bounds__(1024) q4k_gemm_prep_kernel(const void *__restr
     // workgroup copies of them for a super-block is one contiguous run
     u32x4 *oh = reinterpret_cast<u32x4 *>(xh);
     u32x4 *ol = xl ? reinterpret_cast<u32x4 *>(xl) : nullptr;
-    for (uint32_t v = t; v < nvec; v += blockDim.x) {  // nvec % 32 == 0: the four threads of a sub-block run together
+    auto convert = [&](uint32_t v, const u32x4 *k) {  // nvec % 32 == 0: the four threads of a sub-block run together
         float o[8];
-        load8(v, o);
+        load8(v, o, k);
         uint32_t hw[4] = {0u, 0u, 0u, 0u}, lw[4] = {0u, 0u, 0u, 0u};
         float sm = 0.f;
 #pragma unroll
@@ -149,28 +162,37 @@ __global__ void __launch_bounds__(1024) q4k_gemm_prep_kernel(const void *__restr
             const uint32_t pair = (uint32_t)__builtin_bit_cast(uint16_t, sh) | ((uint32_t)__builtin_bit_cast(uint16_t, sl) << 16);
             reinterpret_cast<uint32_t *>(sx)[((size_t)(v >> 5) * seq + tok) * 8 + ((v >> 2) & 7u)] = pair;
         }
+    };
+    if (x_is_bf16) {
+#pragma unroll
+        for (uint32_t u = 0; u < KEEP; u++)
+            if (t + u * blockDim.x < nvec) convert(t + u * blockDim.x, &kept[u]);
     }
+    for (uint32_t v = t + (x_is_bf16 ? KEEP * blockDim.x : 0u); v < nvec; v += blockDim.x) convert(v, nullptr);
     if (lo_seen && any_lo) *any_lo = 1;
 }
 
 // adds the partial slabs of a K-split in slab order and applies the token scale; VEC elements per thread (4 when
-// rows % 4 == 0 and everything is 16-byte aligned: the four are then of one token)
+// rows % 4 == 0 and everything is 16-byte aligned: the four are then of one token).
+// Bound: latency, then memory (the slabs come out of the last-level cache).  Eight slabs are requested together, so that a
+// launch costs splits / 8 round trips instead of `splits`; a request past the last slab reads the last one and is not added.
 template <int VEC>
 __global__ void __launch_bounds__(256) q4k_gemm_reduce_kernel(const float *__restrict__ partial, uint32_t splits, const float *__restrict__ tok_scale,
                                                               float *__restrict__ out, uint32_t rows, uint32_t seq, int accumulate) {
+    typedef float vec __attribute__((ext_vector_type(VEC)));
     const size_t n = (size_t)rows * seq, i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * VEC;
     if (i >= n) return;
     float s[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; e++) s[e] = 0.f;
-    for (uint32_t z = 0; z < splits; z++) {
-        if (VEC == 4) {
-            const f32x4 v = *reinterpret_cast<const f32x4 *>(partial + (size_t)z * n + i);
+    for (uint32_t z0 = 0; z0 < splits; z0 += 8) {
+        vec v[8];
 #pragma unroll
-            for (int e = 0; e < VEC; e++) s[e] += v[e];
-        } else {
-            s[0] += partial[(size_t)z * n + i];
-        }
+        for (uint32_t u = 0; u < 8; u++) v[u] = *reinterpret_cast<const vec *>(partial + (size_t)min(z0 + u, splits - 1) * n + i);
+#pragma unroll
+        for (uint32_t u = 0; u < 8; u++)
+#pragma unroll
+            for (int e = 0; e < VEC; e++) s[e] = z0 + u < splits ? s[e] + v[u][e] : s[e];
     }
     const float ts = tok_scale[i / rows];
     if (VEC == 4) {
@@ -919,9 +941,9 @@ __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *
 hipError_t q4k_gemm_prep_launch(hipStream_t s, const void *x, int x_is_bf16, uint32_t hidden, uint32_t seq, uint16_t *xh, uint16_t *xl,
                                 uint16_t *sx, float *tok_scale, int *any_lo, const uint8_t *w, uint32_t rows, int *rexp) {
     if (seq == 0 && !(rexp && rows)) return hipSuccess;  // (no tokens: only the rows' exponents, if they are asked for)
-    // a token per block; wide activations take more threads per token (two passes over the token: 256 threads on 15360
-    // elements are 15 dependent rounds of loads)
-    const uint32_t threads = hidden >= 8192 ? 1024u : 256u;
+    // a token per block; wide activations take more threads per token (two vectors of a thread stay in registers: 4096
+    // elements for 256 threads, 16384 for 1024)
+    const uint32_t threads = hidden > 4096 ? 1024u : 256u;
     const uint32_t row_blocks = rexp ? (rows + threads / 16 - 1) / (threads / 16) : 0;
     hipLaunchKernelGGL(q4k_gemm_prep_kernel, dim3(seq + row_blocks), dim3(threads), 0, s, x, x_is_bf16, hidden, xh, xl, sx, tok_scale, any_lo,
                        1, seq, w, rows, rexp);
@@ -929,14 +951,23 @@ hipError_t q4k_gemm_prep_launch(hipStream_t s, const void *x, int x_is_bf16, uin
 }
 
 
-// K-ranges per output tile so that a launch fills the CUs (1 = no split)
+// K-ranges per output tile (1 = no split), where one 256x128 workgroup runs per CU and the unsplit tiles leave CUs idle.
+// In tenths of a microsecond: a super-block of a tile takes 39, a split's
+// reduction 30 for the launch and 8 bytes per slab element at 4 TB/s.  The range count with the smallest sum is taken, any
+// number up to 32 whose workgroups all run at once (so the slabs stay below 256 tiles, 34 MB).  Doubling up to 8, the rule
+// before, kept 120 of 256 CUs on a 3840 x 15360 matrix with 77 tokens: with this one
+// (15 ranges), the reduction above and the kept activations of the preparation the call went from 46.4 to 36.2 us
+// (5.9 preparation, 27.3 GEMM, 4.8 reduction in the kernel trace).
 uint32_t q4k_gemm_splits(uint32_t rows, uint32_t hidden, uint32_t seq, uint32_t cu_count) {
-    const uint32_t nsb = hidden / 256;
-    uint32_t s = 1;
-    // one 256x128 workgroup per CU
-    const uint64_t tiles = (uint64_t)((rows + GM - 1) / GM) * ((seq + GN - 1) / GN);
-    while (s < 8 && tiles * s * 2 <= (uint64_t)cu_count && nsb / (s * 2) >= 4) s *= 2;
-    return s;
+    const uint64_t nsb = hidden / 256, tiles = (uint64_t)((rows + GM - 1) / GM) * ((seq + GN - 1) / GN);
+    uint64_t best = nsb * 39, splits = 1;
+    for (uint64_t z = 2; z <= 32 && z <= nsb && tiles * z <= cu_count; z++) {
+        const uint64_t per = (nsb + z - 1) / z;
+        if ((nsb + per - 1) / per != z) continue;  // (the same ranges as a smaller count)
+        const uint64_t cost = per * 39 + 30 + z * rows * seq * 8 / 400000;
+        if (cost < best) { best = cost; splits = z; }
+    }
+    return (uint32_t)splits;
 }
 
 // `rexp` (from q4k_gemm_prep_launch): the rows' scales ride in the f16 weight operand; without it the weight operand is

@@ -72,6 +72,38 @@ def test_q4k_matvec_activation_ranges(be, case):
         assert rel_l2(got, want) < TOL
 
 
+@pytest.mark.parametrize("rows,cols", [([1], 256), ([4096, 1], 256), ([10240, 10240, 9999, 17], 512), ([20000, 12767], 2560), ([2560, 1024, 1023], 2816),
+                                       ([10000, 10480], 2816), ([5, 12000], 5376), ([15], 10240), ([8000], 10240), ([8193], 10240), ([33], 8448)])
+def test_q4k_launches_of_a_few_tiles_per_compute_unit(be, fmt, rows, cols):
+    """One to four matvecs against one activation: one to eight tiles and one to four columns per wavefront, ragged last tiles,
+    column counts that leave wavefronts without a last column, and one size past the kernel's registers.  Bit for bit what the
+    same matvecs give among five in a launch (the streaming kernel), and the first and last rows against the oracle (the f32
+    sums of a row: TOL)."""
+    rng = np.random.default_rng(cols + sum(rows))
+    blocks = [rng.integers(0, 256, size=(r * cols // 256, 144), dtype=np.uint8) for r in rows]
+    for b in blocks:
+        b[:, 0:4] = np.array([0x00, 0x2C, 0x00, 0x28], np.uint8)   # d = 2^-4, dmin = 2^-5
+    x_h = rng.standard_normal(cols).astype(F)
+    x = be.to_device(x_h)
+    dw = [be.to_device(b.reshape(-1)) for b in blocks]
+
+    def outputs(more):
+        outs = [be.to_device(np.full(r + 1, 7.0, F)) for r in rows]
+        spare = be.malloc(4 * 4)
+        jobs = [(fmt.FMT_Q4_K, w, None, x, o, r, cols) for w, o, r in zip(dw, outs, rows)] + [(fmt.FMT_Q4_K, dw[0], None, x, spare, 1, cols)] * more
+        plan = be.plan_create(jobs)
+        assert plan and be.plan_run(plan), be.last_error()
+        be.synchronize()
+        be.plan_destroy(plan)
+        return [be.d2h(o, r + 1, F) for o, r in zip(outs, rows)]
+
+    for got, ref, b, r in zip(outputs(0), outputs(4), blocks, rows):
+        assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)) and got[r] == 7.0
+        for part in (slice(0, min(r, 40)), slice(max(0, r - 40), r)):
+            want = O.q4k_matvec(b.reshape(r, -1)[part].reshape(-1), x_h, part.stop - part.start, cols)
+            assert rel_l2(got[part], want) < TOL
+
+
 def test_q4k_matvec_refusals_follow_the_cpu_backend(be):
     w, x = weights(1, 3, 512)
     q = O.quantize_q4_k(w)
@@ -1618,6 +1650,25 @@ def test_q4k_gemm_mfma_matches_oracle(be, rows, hidden, seq):
     assert np.all((m[ok] * np.exp2(e[ok].astype(np.float64)) >= 0.5) & (m[ok] * np.exp2(e[ok].astype(np.float64)) < 1.0))
     with pytest.raises(Exception):                                               # the exponents are not optional here
         be.dev_q4k_gemm_prepared(dw, 0, dx, rows, hidden, seq, do2)
+
+
+@pytest.mark.parametrize("rows,hidden,seq", [(256, 8192, 3), (515, 5376, 129), (260, 9472, 40), (1, 15360, 1), (1000, 1024, 16), (128, 20992, 130)])
+def test_q4k_gemm_few_tiles_in_many_ranges_of_k(be, rows, hidden, seq):
+    """Range counts that are no power of two and up to 32 per tile, a shorter last range, rows no multiple of four (the one-element
+    reduction), tokens just past a tile, activations of one to three register vectors per thread."""
+    rng = np.random.default_rng(67 + rows)
+    q = O.quantize_q4_k((rng.standard_normal((rows, hidden)) * 0.02).astype(F))
+    xb = O.f32_to_bf16(rng.standard_normal((seq, hidden)).astype(F))
+    want = O.q4k_matmul(q, (xb.astype(np.uint32) << 16).view(F).reshape(seq, hidden), rows, hidden, seq)
+    dw, dx, do = be.to_device(q), be.to_device(xb), be.to_device(np.full(seq * rows, 7.0, F))
+    assert be.dev_q4k_gemm(dw, dx, rows, hidden, seq, do)
+    be.synchronize()
+    got = be.d2h(do, (seq, rows), F)
+    # the f16 roundings are independent errors of 3e-4 of a typical result, 0.02 sqrt(hidden) (a single result may itself be much
+    # smaller: one output of 15360 terms was 0.3 of it): six standard deviations per element, 5e-4 over many elements
+    size = 0.02 * np.sqrt(hidden)
+    err = np.abs(got.astype(np.float64) - want)
+    assert err.max() < 6 * 3e-4 * size and (err.size < 32 or np.sqrt((err ** 2).mean()) < 5e-4 * size)
 
 
 def test_q4k_gemm_row_scales_of_any_size_and_uneven_blocks(be):
