@@ -73,76 +73,80 @@ __device__ __forceinline__ uint32_t f32_to_f16_flush(float v) {
     return sign | ((uint32_t)new_exp << 10) | (mant >> 13);
 }
 
-// ---------------------------------------------------------------------------
-// quantize_q4_k — larql-compute/src/cpu/ops/q4_common/quantize.rs:89-189.
-// One wavefront per 256-element super-block; lane l owns elements 4l..4l+3
-// (all inside sub-block l/8).  min/max folds are order-independent, so the
-// wave reductions give the host's numbers exactly.
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ float wave_min_span(float v, int span) {
-    for (int o = 1; o < span; o <<= 1) v = fminf(v, __shfl_xor(v, o, 64));
-    return v;
-}
-__device__ __forceinline__ float wave_max_span(float v, int span) {
-    for (int o = 1; o < span; o <<= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
+// v of another lane of the same 16 (CTRL: a DPP quad_perm, row_half_mirror or row_mirror; every lane has a source)
+template <int CTRL> __device__ __forceinline__ uint32_t dpp_u32(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true); }
+template <int CTRL> __device__ __forceinline__ float dpp_f32(float v) { return u2f(dpp_u32<CTRL>(f2u(v))); }
+// sat_u8(clampf(roundf(v), 0, hi)) for an integer hi: clamped first (NaN -> 0), then half away from zero on a value >= 0
+__device__ __forceinline__ uint32_t round_u8(float v, float hi) {
+    const float c = __builtin_amdgcn_fmed3f(v, 0.0f, hi);
+    return (uint32_t)c + (__builtin_amdgcn_fractf(c) >= 0.5f ? 1u : 0u);
 }
 
+// ---------------------------------------------------------------------------
+// quantize_q4_k — larql-compute/src/cpu/ops/q4_common/quantize.rs:89-189.
+// Bound: memory (1 KB read, 144 bytes written per super-block) once the vector instructions per super-block are few:
+// sixteen lanes share one, lane (sub, b) = (lane % 16 / 2, lane % 2) holds sixteen elements of sub-block sub (its float4
+// 2i + b, i < 4), so that the five divisions, the folds (DPP within the sixteen lanes) and the header are paid once for
+// four super-blocks of a wavefront.  A wavefront per super-block with shuffles was bound by its ~300 instructions:
+// 10240 x 2560 took 47.8 us (2.5 TB/s), now 22.3 us (5.4 TB/s).  min/max folds are order-independent, so they give the host's numbers exactly.
+// ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) quantize_q4_k_kernel(const float *__restrict__ src, size_t n_sb,
                                                             uint8_t *__restrict__ dst) {
-    const uint32_t lane = threadIdx.x & 63u;
-    const size_t sb = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (sb >= n_sb) return;
-    const float4 v = reinterpret_cast<const float4 *>(src + sb * 256)[lane];
-    const float e[4] = {v.x, v.y, v.z, v.w};
-    const uint32_t sub = lane >> 3;  // 8 lanes per 32-element sub-block
-    float mn = fminf(fminf(e[0], e[1]), fminf(e[2], e[3]));
-    float mx = fmaxf(fmaxf(e[0], e[1]), fmaxf(e[2], e[3]));
-    mn = fminf(wave_min_span(mn, 8), 0.0f);
-    mx = fmaxf(wave_max_span(mx, 8), 0.0f);
+    const uint32_t lane = threadIdx.x & 15u, sub = lane >> 1, b = lane & 1u;
+    const size_t sb = (size_t)blockIdx.x * 16 + (threadIdx.x >> 4);
+    if (sb >= n_sb) return;  // (sixteen lanes leave together: the DPP exchanges stay among the rest)
+    const float4 *p = reinterpret_cast<const float4 *>(src + sb * 256) + sub * 8 + b;
+    float e[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) { const float4 v = p[2 * i]; e[i][0] = v.x; e[i][1] = v.y; e[i][2] = v.z; e[i][3] = v.w; }
+    float mn = e[0][0], mx = e[0][0];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) { mn = fminf(mn, e[i][c]); mx = fmaxf(mx, e[i][c]); }
+    mn = fminf(fminf(mn, dpp_f32<0xB1>(mn)), 0.0f);  // quad_perm [1,0,3,2]: the sub-block's other lane
+    mx = fmaxf(fmaxf(mx, dpp_f32<0xB1>(mx)), 0.0f);
     const float range = mx - mn;
-    // across the 8 sub-blocks (lanes differing in bits 3..5)
+    // across the 8 sub-blocks: quad_perm [2,3,0,1], row_half_mirror, row_mirror
     float gmr = range, gmin = mn;
-    for (int o = 8; o < 64; o <<= 1) {
-        gmr = fmaxf(gmr, __shfl_xor(gmr, o, 64));
-        gmin = fminf(gmin, __shfl_xor(gmin, o, 64));
-    }
+    gmr = fmaxf(gmr, dpp_f32<0x4E>(gmr));   gmin = fminf(gmin, dpp_f32<0x4E>(gmin));
+    gmr = fmaxf(gmr, dpp_f32<0x141>(gmr));  gmin = fminf(gmin, dpp_f32<0x141>(gmin));
+    gmr = fmaxf(gmr, dpp_f32<0x140>(gmr));  gmin = fminf(gmin, dpp_f32<0x140>(gmin));
     gmr = fmaxf(gmr, 0.0f);
     const float d = gmr > 0.0f ? gmr / (15.0f * 63.0f) : 0.0f;
     const float dmin = gmin < 0.0f ? -gmin / 63.0f : 0.0f;
-    const uint32_t q_scale = d > 0.0f ? sat_u8(clampf(roundf(range / (15.0f * d)), 0.0f, 63.0f)) : 0u;
-    const uint32_t q_min = dmin > 0.0f ? sat_u8(clampf(roundf(-mn / dmin), 0.0f, 63.0f)) : 0u;
+    const uint32_t q_scale = d > 0.0f ? round_u8(range / (15.0f * d), 63.0f) : 0u;
+    const uint32_t q_min = dmin > 0.0f ? round_u8(-mn / dmin, 63.0f) : 0u;
     const float sc = d * (float)q_scale;
     const float mnv = dmin * (float)q_min;
     const float inv = sc > 0.0f ? 1.0f / sc : 0.0f;
-    uint32_t enc = 0;  // 4 codes, one per byte
+    uint32_t w[4];  // the codes of float4 2i + b, one per byte, then joined with those of the pair's other sub-block
 #pragma unroll
-    for (int i = 0; i < 4; i++) enc |= sat_u8(clampf(roundf((e[i] + mnv) * inv), 0.0f, 15.0f)) << (8 * i);
+    for (int i = 0; i < 4; i++) {
+        uint32_t enc = 0;
+#pragma unroll
+        for (int c = 0; c < 4; c++) enc |= round_u8((e[i][c] + mnv) * inv, 15.0f) << (8 * c);
+        const uint32_t partner = dpp_u32<0x4E>(enc);  // same position, other sub-block of the pair (lane ^ 2)
+        w[i] = (sub & 1u) ? partner | (enc << 4) : enc | (partner << 4);
+    }
+    // group g = sub / 2 has 8 dwords, dword 2i + b in lane b's w[i]: the lanes of the even sub-block store dwords 0..3, those
+    // of the odd one 4..7, two neighbouring dwords each
+    const uint32_t u0 = (sub & 1u) ? w[2] : w[0], u1 = (sub & 1u) ? w[3] : w[1];
+    const uint32_t got = dpp_u32<0xB1>(b ? u0 : u1);
     uint8_t *o = dst + sb * 144;
-    // nibble bytes: group g = sub/2 pairs sub-block 2g (low) with 2g+1 (high); lane holds
-    // elements 4*(lane&7).. of its sub-block -> bytes g*32 + 4*(lane&7) ..+3
-    const uint32_t partner = (uint32_t)__shfl_xor((int)enc, 8, 64);  // same position, other sub-block of the pair
-    if ((sub & 1u) == 0) {
-        const uint32_t packed = enc | (partner << 4);
-        reinterpret_cast<uint32_t *>(o + 16 + (sub >> 1) * 32)[lane & 7u] = packed;
-    }
-    // header: lanes 0..7*8 hold the per-sub-block scale/min; gather them to lane 0
-    uint32_t qs[8], qm[8];
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-        qs[j] = (uint32_t)__shfl((int)q_scale, j * 8, 64);
-        qm[j] = (uint32_t)__shfl((int)q_min, j * 8, 64);
-    }
+    const uint2 pair = {b ? got : u0, b ? u1 : got};
+    *reinterpret_cast<uint2 *>(o + 16 + (sub >> 1) * 32 + (sub & 1u) * 16 + b * 8) = pair;
+    // header: every sub-block's bits, joined over the sixteen lanes
+    const uint32_t at = 8 * (sub & 3u);
+    const bool upper = sub >= 4;
+    uint32_t w1 = upper ? (q_scale >> 4) << (at + 6) : q_scale << at;
+    uint32_t w2 = upper ? (q_min >> 4) << (at + 6) : q_min << at;
+    uint32_t w3 = upper ? ((q_scale & 0x0Fu) | ((q_min & 0x0Fu) << 4)) << at : 0u;
+    w1 |= dpp_u32<0x4E>(w1);   w2 |= dpp_u32<0x4E>(w2);   w3 |= dpp_u32<0x4E>(w3);
+    w1 |= dpp_u32<0x141>(w1);  w2 |= dpp_u32<0x141>(w2);  w3 |= dpp_u32<0x141>(w3);
+    w1 |= dpp_u32<0x140>(w1);  w2 |= dpp_u32<0x140>(w2);  w3 |= dpp_u32<0x140>(w3);
     if (lane == 0) {
-        uint32_t w0 = f32_to_f16_trunc(d) | (f32_to_f16_trunc(dmin) << 16);
-        uint32_t w1 = 0, w2 = 0, w3 = 0;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            w1 |= ((qs[j] & 0x3Fu) | (((qs[j + 4] >> 4) & 3u) << 6)) << (8 * j);
-            w2 |= ((qm[j] & 0x3Fu) | (((qm[j + 4] >> 4) & 3u) << 6)) << (8 * j);
-            w3 |= ((qs[j + 4] & 0x0Fu) | ((qm[j + 4] & 0x0Fu) << 4)) << (8 * j);
-        }
-        uint4 h = {w0, w1, w2, w3};
+        const uint4 h = {f32_to_f16_trunc(d) | (f32_to_f16_trunc(dmin) << 16), w1, w2, w3};
         *reinterpret_cast<uint4 *>(o) = h;
     }
 }
@@ -157,6 +161,11 @@ __global__ void __launch_bounds__(256) quantize_q4_k_kernel(const float *__restr
 // qh[32h + l] = the top two bits of codes 128h + l + {0, 32, 64, 96}; then the 16
 // scales and the truncated f16 d (210 bytes, 2-byte aligned).
 // ---------------------------------------------------------------------------
+__device__ __forceinline__ float wave_max_span(float v, int span) {
+    for (int o = 1; o < span; o <<= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+    return v;
+}
+
 __global__ void __launch_bounds__(256) quantize_q6_k_kernel(const float *__restrict__ src, size_t n_sb, uint8_t *__restrict__ dst) {
     __shared__ uint8_t codes[4][256];
     const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
@@ -385,7 +394,7 @@ static inline dim3 blocks_for(size_t n, uint32_t t) { return dim3((uint32_t)((n 
 hipError_t quantize_q4_k_launch(hipStream_t s, const float *src, size_t n, uint8_t *dst) {
     const size_t n_sb = n / 256;
     if (n_sb == 0) return hipSuccess;
-    hipLaunchKernelGGL(quantize_q4_k_kernel, blocks_for(n_sb, 4), dim3(256), 0, s, src, n_sb, dst);
+    hipLaunchKernelGGL(quantize_q4_k_kernel, blocks_for(n_sb, 16), dim3(256), 0, s, src, n_sb, dst);
     return hipGetLastError();
 }
 hipError_t quantize_q6_k_launch(hipStream_t s, const float *src, size_t n, uint8_t *dst) {

@@ -757,6 +757,27 @@ def test_registered_region_serves_sub_slices(be):
 
 
 # ---------------------------------------------------------------- encoders
+@pytest.mark.parametrize("n_sb", [1, 3, 15, 16, 17, 21])
+def test_device_kquant_encoders_on_partial_workgroups_and_odd_blocks(be, n_sb):
+    """Super-block counts around a workgroup's sixteen, and blocks of every kind: wide ranges, one sign, halves (rounding ties),
+    constants, zeros, subnormals, infinities and NaN.  Byte for byte the oracle's."""
+    rng = np.random.default_rng(n_sb)
+    for special in ("finite", "odd"):
+        w = rng.standard_normal((n_sb, 256)).astype(F) * np.exp2(rng.integers(-20, 20, size=(n_sb, 1))).astype(F)
+        w[::4] = rng.integers(0, 127, size=w[::4].shape) * F(0.5)
+        w[n_sb // 2] = F(-0.75)
+        if special == "odd":
+            w[0, ::3] = F(1e-40)
+            w[n_sb - 1, 5], w[n_sb // 3, 70], w[n_sb // 2, 255], w[n_sb // 4, 32:64] = F(np.inf), F(-np.inf), F(np.nan), F(0)
+        src, dst = be.to_device(w.reshape(-1)), be.to_device(np.full(n_sb * 210 + 16, 0xA5, np.uint8))
+        for encode, want in ((be.dev_quantize_q4_k, O.quantize_q4_k(w.reshape(-1))), (be.dev_quantize_q6_k, O.quantize_q6_k(w.reshape(-1)))):
+            be.h2d(dst, np.full(n_sb * 210 + 16, 0xA5, np.uint8))
+            assert encode(src, w.size, dst)
+            be.synchronize()
+            got = be.d2h(dst, n_sb * 210 + 16, np.uint8)
+            assert np.array_equal(got[:want.size], np.asarray(want).reshape(-1)) and (got[want.size:] == 0xA5).all(), special
+
+
 def test_device_encoders_are_bit_exact(be):
     rng = np.random.default_rng(41)
     n = 256 * 4096
