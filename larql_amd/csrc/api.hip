@@ -260,6 +260,7 @@ struct PreparedLaunch {
 constexpr size_t kTableFirstMax = 4096;
 static size_t table_bytes_for(size_t n_jobs) { return n_jobs * sizeof(GemvJob) + kTableFirstMax * sizeof(uint32_t); }
 
+constexpr int kTableOnDevice = -2;  // stage_slot: a kernel ahead of the launch writes the table (JobTableSpec)
 int prepare_same_kind(larql_hip_ctx *c, GemvJob *live, size_t n_live, void *table_dst, PreparedLaunch &P, int stage_slot = -1) {
     P.kind = live[0].kind;
     memset(&P.L, 0, sizeof P.L);
@@ -309,9 +310,14 @@ int prepare_same_kind(larql_hip_ctx *c, GemvJob *live, size_t n_live, void *tabl
     } else {
         // the table: the jobs, then the first job of every workgroup's share (what a workgroup would otherwise find by
         // bisection over the jobs' pass ranges, a dependent load per step)
-        c->alloc_events++;
         const size_t job_bytes = n_live * sizeof(GemvJob);
         const bool with_first = grid >= 1 && grid <= (uint64_t)kTableFirstMax;
+        if (stage_slot == kTableOnDevice) {
+            P.L.table = (const GemvJob *)table_dst;
+            if (with_first) P.L.wg_first = (const uint32_t *)((const uint8_t *)table_dst + job_bytes);
+            return LARQL_OK;
+        }
+        c->alloc_events++;
         const size_t bytes = job_bytes + (with_first ? (size_t)grid * sizeof(uint32_t) : 0);
         std::vector<uint8_t> blob(bytes);
         memcpy(blob.data(), live, job_bytes);
@@ -2300,15 +2306,12 @@ static int moe_layer_enqueue(larql_hip_ctx *c, larql_hip_moe_layer *L, const flo
         const size_t aq_stride = dense ? ((inter * sizeof(float) + 255) & ~(size_t)255) : (q8k_bytes(ip) + 255) & ~(size_t)255;
         const size_t f_bytes = ((2 * slots * inter + slots * hidden) * sizeof(float) + 255) & ~(size_t)255;
         const size_t x_area = (dense && !pad_x) ? 0 : ((tokens * xq_stride + 255) & ~(size_t)255);
-        rc = ensure(c, L->ws, f_bytes + x_area + slots * aq_stride + 256); if (rc) return rc;
+        const size_t a_area = (slots * aq_stride + 255) & ~(size_t)255, gu_table = dense ? 0 : (table_bytes_for(2 * slots) + 255) & ~(size_t)255;
+        rc = ensure(c, L->ws, f_bytes + x_area + a_area + gu_table + (dense ? 0 : table_bytes_for(slots)) + 256); if (rc) return rc;
         float *g = (float *)L->ws.p, *u = g + slots * inter, *dd = u + slots * inter;
         uint8_t *xq = (dense && !pad_x) ? (uint8_t *)const_cast<float *>(x) : (uint8_t *)L->ws.p + f_bytes;
         uint8_t *aq = (uint8_t *)L->ws.p + f_bytes + x_area;
-        if (!dense)  // the route and the Q8_K expert input of every token: one launch
-            HIPCHECK(c, moe_kq_route_quant_launch(c->stream, logits, L->router_bias, (uint32_t)tokens, (uint32_t)E, (uint32_t)k, policy,
-                                                  L->per_expert_scale ? L->scale : nullptr, experts, weights, x, hidden, (uint32_t)hidden, (uint32_t)cols, xq,
-                                                  xq_stride));
-        else if (pad_x) HIPCHECK(c, pad_rows_f32_launch(c->stream, x, hidden, (uint32_t)hidden, (uint32_t)cols, (uint32_t)tokens, (float *)xq));
+        std::vector<GemvJob> down;
         jobs.clear();
         for (size_t s = 0; s < slots; s++) {
             GemvJob a = make_job(L->kq_kind, L->kq_gate, nullptr, xq + (s / k) * xq_stride, g + s * inter, inter, cols);
@@ -2317,23 +2320,48 @@ static int moe_layer_enqueue(larql_hip_ctx *c, larql_hip_moe_layer *L, const flo
             b.w = L->kq_up; b.out = u + s * inter;
             jobs.push_back(a);
             jobs.push_back(b);
+            a = make_job(L->kq_kind, L->kq_down, nullptr, aq + s * aq_stride, dd + s * hidden, hidden, ip);
+            a.sel = experts + s; a.w_sel_stride = L->kq_dn_stride; a.sel_count = (uint32_t)E;
+            down.push_back(a);
         }
-        rc = enqueue_jobs(c, jobs);
-        if (rc) return rc;
-        if (dense)
+        if (dense) {
+            if (pad_x) HIPCHECK(c, pad_rows_f32_launch(c->stream, x, hidden, (uint32_t)hidden, (uint32_t)cols, (uint32_t)tokens, (float *)xq));
+            rc = enqueue_jobs(c, jobs);
+            if (rc) return rc;
             HIPCHECK(c, moe_act_f32_launch(c->stream, g, u, (uint32_t)inter, (uint32_t)slots, experts, (uint32_t)E, L->kq_gub, L->gate_rule, L->glu_limit,
                                            L->glu_alpha, (float *)aq, aq_stride / sizeof(float)));
-        else
+            rc = enqueue_jobs(c, down);
+            if (rc) return rc;
+        } else {
+            // both launches' jobs are of one kind and one shape: their tables are written on the device by the launch that routes
+            PreparedLaunch P[2];
+            JobTableSpec T[2];
+            memset(T, 0, sizeof T);
+            std::vector<GemvJob> *list[2] = {&jobs, &down};
+            uint8_t *table = aq + a_area;
+            for (int i = 0; i < 2; i++, table += gu_table) {
+                std::vector<GemvJob> &v = *list[i];
+                rc = check_jobs(c, v); if (rc) return rc;
+                rc = prepare_same_kind(c, v.data(), v.size(), table, P[i], kTableOnDevice); if (rc) return rc;
+                if (!P[i].L.table) continue;  // few enough to travel with the launch
+                JobTableSpec &t = T[i];
+                t.base = v[0];
+                t.jobs = (GemvJob *)table; t.first = const_cast<uint32_t *>(P[i].L.wg_first);
+                t.n_jobs = (uint32_t)v.size(); t.per_slot = i == 0 ? 2 : 1; t.x_div = i == 0 ? (uint32_t)k : 1;
+                t.grid = P[i].grid; t.total = P[i].L.total_passes;
+                t.x_step = i == 0 ? xq_stride : aq_stride; t.out_step = i == 0 ? inter : hidden;
+                if (i == 0) { t.w_second = (uint64_t)(L->kq_up - L->kq_gate); t.out_second = slots * inter; }
+                if (v.back().pass_begin != (uint32_t)(v.size() - 1) * v[0].n_pass) return fail(c, LARQL_E_DEVICE, "moe_layer: matvecs of one shape with unequal passes");
+            }
+            // the route, the Q8_K expert input of every token and the tables: one launch
+            HIPCHECK(c, moe_kq_route_quant_launch(c->stream, logits, L->router_bias, (uint32_t)tokens, (uint32_t)E, (uint32_t)k, policy,
+                                                  L->per_expert_scale ? L->scale : nullptr, experts, weights, x, hidden, (uint32_t)hidden, (uint32_t)cols, xq,
+                                                  xq_stride, T));
+            HIPCHECK(c, gemv_launch(c->stream, P[0].kind, P[0].L, P[0].threads, P[0].grid, P[0].lds));
             HIPCHECK(c, moe_kq_act_q8k_launch(c->stream, g, u, (uint32_t)inter, (uint32_t)ip, (uint32_t)slots, experts, (uint32_t)E, L->kq_gub, L->gate_rule,
                                               L->glu_limit, L->glu_alpha, aq, aq_stride));
-        jobs.clear();
-        for (size_t s = 0; s < slots; s++) {
-            GemvJob a = make_job(L->kq_kind, L->kq_down, nullptr, aq + s * aq_stride, dd + s * hidden, hidden, ip);
-            a.sel = experts + s; a.w_sel_stride = L->kq_dn_stride; a.sel_count = (uint32_t)E;
-            jobs.push_back(a);
+            HIPCHECK(c, gemv_launch(c->stream, P[1].kind, P[1].L, P[1].threads, P[1].grid, P[1].lds));
         }
-        rc = enqueue_jobs(c, jobs);
-        if (rc) return rc;
         HIPCHECK(c, weighted_sum_bias_launch(c->stream, dd, weights, experts, (uint32_t)E, L->kq_db, out, (uint32_t)tokens, (uint32_t)k, (uint32_t)hidden));
         return LARQL_OK;
     }

@@ -220,9 +220,22 @@ hipError_t quantize_rows_to_q8k_launch(hipStream_t s, const float *src, size_t s
 hipError_t moe_kq_act_q8k_launch(hipStream_t s, const float *g, const float *u, uint32_t inter, uint32_t inter_padded, uint32_t slots,
                                  const uint32_t *experts, uint32_t n_experts, const float *gub, int rule, float limit, float alpha, uint8_t *dst,
                                  size_t dst_stride);
+// A job table that a kernel writes for the launches behind it: matvecs of one shape, `per_slot` (1 or 2) for each slot.  Job i
+// belongs to slot i / per_slot: its activation is the one of token slot / x_div, its expert the slot's.
+struct JobTableSpec {
+    GemvJob base;                     // job 0, with the launch's geometry
+    GemvJob *jobs;                    // null: no table
+    uint32_t *first;                  // the first job of each of `grid` workgroups' shares, or null
+    uint32_t n_jobs, per_slot, x_div, grid;
+    uint64_t total;                   // passes of the launch
+    uint64_t x_step;                  // bytes from token to token
+    uint64_t out_step;                // floats from slot to slot
+    uint64_t w_second, out_second;    // bytes / floats from a slot's first job to its second
+};
 hipError_t moe_kq_route_quant_launch(hipStream_t s, const float *logits, const float *bias, uint32_t tokens, uint32_t n_experts, uint32_t k, int policy,
                                      const float *scale, uint32_t *experts, float *weights, const float *src, size_t src_stride, uint32_t src_cols,
-                                     uint32_t cols, uint8_t *dst, size_t dst_stride);
+                                     uint32_t cols, uint8_t *dst, size_t dst_stride,
+                                     const JobTableSpec (&tables)[2]);
 hipError_t pad_rows_f32_launch(hipStream_t s, const float *src, size_t src_stride, uint32_t src_cols, uint32_t cols, uint32_t rows, float *dst);
 hipError_t moe_act_f32_launch(hipStream_t s, const float *g, const float *u, uint32_t inter, uint32_t slots, const uint32_t *experts, uint32_t n_experts,
                               const float *gub, int rule, float limit, float alpha, float *act, size_t act_stride);
