@@ -153,54 +153,69 @@ __global__ void __launch_bounds__(256) quantize_q4_k_kernel(const float *__restr
 
 // ---------------------------------------------------------------------------
 // quantize_q6_k — larql-compute/src/cpu/ops/q4_common/quantize.rs:198-276.
-// One wavefront per 256-element super-block; lane l owns elements 4l..4l+3, all
-// inside the 16-element sub-block l/4.  d = amax / (31*127); sub-block scale =
-// round(sub_max / (31 d)) as i8; code = round(v * (1 / (d * scale))) clamped to
+// Sixteen lanes per super-block, for the reason given at quantize_q4_k: lane l owns the 16-element sub-block l.
+// d = amax / (31*127); sub-block scale = round(sub_max / (31 d)) as i8; code = round(v * (1 / (d * scale))) clamped to
 // -32..31, biased by 32.  The 256 six-bit codes pass through LDS into ggml's
 // planar layout: ql[64h + p] = code[128h + p] & 15 | (code[128h + p + 64] & 15) << 4,
 // qh[32h + l] = the top two bits of codes 128h + l + {0, 32, 64, 96}; then the 16
-// scales and the truncated f16 d (210 bytes, 2-byte aligned).
+// scales and the truncated f16 d (210 bytes, 2-byte aligned).  10240 x 2560: 40.1 -> 22.2 us (5.7 TB/s).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ float wave_max_span(float v, int span) {
-    for (int o = 1; o < span; o <<= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
+// sat_i8(roundf(clampf(v, lo, hi))) for integers lo, hi: half away from zero, NaN -> 0
+__device__ __forceinline__ int round_i8(float v, float lo, float hi) {
+    const float c = v != v ? 0.0f : __builtin_amdgcn_fmed3f(v, lo, hi);
+    const int t = (int)c;
+    const float f = c - (float)t;  // exact
+    return t + (f >= 0.5f ? 1 : 0) - (f <= -0.5f ? 1 : 0);
 }
 
 __global__ void __launch_bounds__(256) quantize_q6_k_kernel(const float *__restrict__ src, size_t n_sb, uint8_t *__restrict__ dst) {
-    __shared__ uint8_t codes[4][256];
-    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
-    const size_t sb = (size_t)blockIdx.x * 4 + wv;
-    if (sb >= n_sb) return;  // (whole wavefronts leave together: no workgroup barrier below)
-    const float4 v = reinterpret_cast<const float4 *>(src + sb * 256)[lane];
-    const float e[4] = {v.x, v.y, v.z, v.w};
-    float sub_max = fmaxf(fmaxf(fabsf(e[0]), fabsf(e[1])), fmaxf(fabsf(e[2]), fabsf(e[3])));
-    sub_max = wave_max_span(sub_max, 4);
-    float amax = sub_max;
-    for (int o = 4; o < 64; o <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+    __shared__ __attribute__((aligned(16))) uint8_t codes[16][256];
+    const uint32_t lane = threadIdx.x & 15u, slot = threadIdx.x >> 4;
+    const size_t sb = (size_t)blockIdx.x * 16 + slot;
+    if (sb >= n_sb) return;  // (sixteen lanes leave together: no workgroup barrier below)
+    const float4 *p = reinterpret_cast<const float4 *>(src + sb * 256) + lane * 4;
+    float e[16];
+#pragma unroll
+    for (int i = 0; i < 4; i++) { const float4 v = p[i]; e[4 * i] = v.x; e[4 * i + 1] = v.y; e[4 * i + 2] = v.z; e[4 * i + 3] = v.w; }
+    float sub_max = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; i++) sub_max = fmaxf(sub_max, fabsf(e[i]));
+    float amax = sub_max;  // quad_perm [1,0,3,2] and [2,3,0,1], row_half_mirror, row_mirror
+    amax = fmaxf(amax, dpp_f32<0xB1>(amax));
+    amax = fmaxf(amax, dpp_f32<0x4E>(amax));
+    amax = fmaxf(amax, dpp_f32<0x141>(amax));
+    amax = fmaxf(amax, dpp_f32<0x140>(amax));
     const float d = amax / (31.0f * 127.0f);
     const float scf = d > 0.0f ? sub_max / (31.0f * d) : 0.0f;
-    const int sub_scale = sat_i8(clampf(roundf(scf), -128.0f, 127.0f));
+    const int sub_scale = round_i8(scf, -128.0f, 127.0f);
     const float sc = d * (float)sub_scale;
     const float inv = fabsf(sc) > 1e-10f ? 1.0f / sc : 0.0f;
+    uint32_t w[4];
 #pragma unroll
-    for (int i = 0; i < 4; i++) codes[wv][4 * lane + i] = (uint8_t)(sat_i8(clampf(roundf(e[i] * inv), -32.0f, 31.0f)) + 32);
+    for (int i = 0; i < 4; i++) {
+        w[i] = 0;
+#pragma unroll
+        for (int c = 0; c < 4; c++) w[i] |= (uint32_t)(round_i8(e[4 * i + c] * inv, -32.0f, 31.0f) + 32) << (8 * c);
+    }
+    uint8_t *c = codes[slot];
+    *reinterpret_cast<uint4 *>(c + 16 * lane) = make_uint4(w[0], w[1], w[2], w[3]);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const uint8_t *c = codes[wv];
     uint8_t *o = dst + sb * 210;
-    {   // ql bytes 2*lane, 2*lane + 1
-        const uint32_t i0 = 2 * lane, h = i0 >> 6, p = i0 & 63u;
-        const uint32_t b0 = (c[128 * h + p] & 15u) | ((c[128 * h + p + 64] & 15u) << 4);
-        const uint32_t b1 = (c[128 * h + p + 1] & 15u) | ((c[128 * h + p + 65] & 15u) << 4);
-        *reinterpret_cast<uint16_t *>(o + i0) = (uint16_t)(b0 | (b1 << 8));
+    const uint32_t h = lane >> 3, at = lane & 7u;
+    {   // ql bytes 8*lane .. 8*lane + 7
+        const uint2 lo = *reinterpret_cast<const uint2 *>(c + 128 * h + 8 * at), hi = *reinterpret_cast<const uint2 *>(c + 128 * h + 64 + 8 * at);
+        const uint2 q = {(lo.x & 0x0F0F0F0Fu) | ((hi.x & 0x0F0F0F0Fu) << 4), (lo.y & 0x0F0F0F0Fu) | ((hi.y & 0x0F0F0F0Fu) << 4)};
+        __builtin_memcpy(__builtin_assume_aligned(o + 8 * lane, 2), &q, 8);
     }
-    {   // qh byte `lane`
-        const uint32_t h = lane >> 5, l = lane & 31u, b = 128 * h + l;
-        o[128 + lane] = (uint8_t)(((c[b] >> 4) & 3u) | (((c[b + 32] >> 4) & 3u) << 2) | (((c[b + 64] >> 4) & 3u) << 4) | (((c[b + 96] >> 4) & 3u) << 6));
+    {   // qh bytes 4*lane .. 4*lane + 3
+        uint32_t q = 0;
+#pragma unroll
+        for (int u = 0; u < 4; u++) q |= ((*reinterpret_cast<const uint32_t *>(c + 128 * h + 32 * u + 4 * at) >> 4) & 0x03030303u) << (2 * u);
+        __builtin_memcpy(__builtin_assume_aligned(o + 128 + 4 * lane, 2), &q, 4);
     }
-    const int scale_of = __shfl(sub_scale, (int)((lane & 15u) * 4), 64);  // sub-block j lives in lanes 4j..4j+3
-    if (lane < 16) o[192 + lane] = (uint8_t)scale_of;
+    o[192 + lane] = (uint8_t)sub_scale;
     if (lane == 0) *reinterpret_cast<uint16_t *>(o + 208) = (uint16_t)f32_to_f16_trunc(d);
 }
 
