@@ -628,6 +628,8 @@ __device__ __forceinline__ void copy16_to_lds(const void *base, uint32_t lane_of
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(lane_off), "s"(bs) : "memory");  // (m0 is not the compiler's to allocate; nothing else in these kernels uses it)
 }
 
+// NB: blocks of 32 tokens that are multiplied (4 unless the prompt is shorter than the tile)
+template <int NB>
 __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *w, const uint16_t *xh, const uint16_t *sx, const int *__restrict__ rexp,
                                                                   const float *__restrict__ tok_scale, float *__restrict__ out,
                                                                   uint32_t rows, uint32_t hidden, uint32_t seq, int with_mins,
@@ -748,16 +750,16 @@ __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *
 #pragma unroll
     for (int j = 0; j < 2; j++) b_col[j] = ((kh * 4 + 2 * kgrp + (uint32_t)j) ^ ((row32 >> 1) & 7u)) << 4;
 
-    f32x16 acc[2][4];
+    f32x16 acc[2][NB];
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
-        for (int jj = 0; jj < 4; jj++)
+        for (int jj = 0; jj < NB; jj++)
 #pragma unroll
             for (int e = 0; e < 16; e++) acc[i][jj][e] = 0.f;
 
     uint32_t an[2][2][4];  // the weight operand of the step being prepared / multiplied: [row block][j][dword]
-    u32x4 breg[8];         // its activation operands: [j * 4 + token block]
+    u32x4 breg[8] = {};    // its activation operands: [j * 4 + token block]; blocks from NB on are neither read nor multiplied
 
     // ---- X(n): prepare step n (g: its position in super-block sbn): table entries at a super-block's first step, the
     //      activation operands into registers, the weight operand converted, and this wavefront's copy requests:
@@ -780,7 +782,7 @@ __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *
         // other wavefront's MFMAs when this wavefront is the older of the two, and eight reads in a row hold them up)
 #define LARQL_RD(G) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(breg[G]) : "v"((G) < 4 ? b0 : b1), "n"(((G) & 3) * 4096));
 #define LARQL_PIECE(G)                                                                                                      \
-        LARQL_RD(G)                                                                                                         \
+        if constexpr (((G) & 3) < NB) LARQL_RD(G)                                                                           \
         convert4(rq[(G) >> 2][(G) & 3], sp[(G) >> 2], an[(G) >> 2][((G) >> 1) & 1][2 * ((G) & 1)], an[(G) >> 2][((G) >> 1) & 1][2 * ((G) & 1) + 1]); \
         __builtin_amdgcn_sched_barrier(0);
         LARQL_PIECE(0) LARQL_PIECE(1) LARQL_PIECE(2) LARQL_PIECE(3) LARQL_PIECE(4) LARQL_PIECE(5) LARQL_PIECE(6) LARQL_PIECE(7)
@@ -808,15 +810,15 @@ __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *
     //      them in one wavefront: a token's sum is then formed in the same order whichever token block it sits in) ----
     auto multiply = [&](const int khc, const int g) {
         if (g == 1 && khc == 0 && with_mins) {
-            f16x8 amf[2], bmf[4];
+            f16x8 amf[2], bmf[NB];
 #pragma unroll
             for (int i = 0; i < 2; i++) amf[i] = *reinterpret_cast<const f16x8 *>(glds + G_AM_OFF + (wm + i * 32 + row32) * 32 + kgrp * 16);
 #pragma unroll
-            for (int jj = 0; jj < 4; jj++) bmf[jj] = *reinterpret_cast<const f16x8 *>(glds + G_BM_OFF + (jj * 32 + row32) * 32 + kgrp * 16);
+            for (int jj = 0; jj < NB; jj++) bmf[jj] = *reinterpret_cast<const f16x8 *>(glds + G_BM_OFF + (jj * 32 + row32) * 32 + kgrp * 16);
 #pragma unroll
             for (int i = 0; i < 2; i++)
 #pragma unroll
-                for (int jj = 0; jj < 4; jj++) acc[i][jj] = __builtin_amdgcn_mfma_f32_32x32x16_f16(amf[i], bmf[jj], acc[i][jj], 0, 0, 0);
+                for (int jj = 0; jj < NB; jj++) acc[i][jj] = __builtin_amdgcn_mfma_f32_32x32x16_f16(amf[i], bmf[jj], acc[i][jj], 0, 0, 0);
         }
         f16x8 af[2][2];
 #pragma unroll
@@ -827,7 +829,7 @@ __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *
         for (int G = 0; G < 8; G++)
 #pragma unroll
             for (int i = 0; i < 2; i++)
-                acc[i][G & 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i][G >> 2], __builtin_bit_cast(f16x8, breg[G]), acc[i][G & 3], 0, 0, 0);
+                if ((G & 3) < NB) acc[i][(G & 3) % NB] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i][G >> 2], __builtin_bit_cast(f16x8, breg[G]), acc[i][(G & 3) % NB], 0, 0, 0);
         __builtin_amdgcn_s_setprio(0);
     };
 
@@ -890,7 +892,7 @@ __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *
 #pragma unroll
         for (int i = 0; i < 2; i++)
 #pragma unroll
-            for (int jj = 0; jj < 4; jj++)
+            for (int jj = 0; jj < NB; jj++)
 #pragma unroll
                 for (int q = 0; q < 4; q++)  // registers 4q .. 4q+3 of a block: rows 8q + 4kgrp .. +3, token row32
                     *reinterpret_cast<f32x4 *>(blk + (jj * 32 + row32) * EP_LD + i * 32 + q * 8 + kgrp * 4) =
@@ -901,7 +903,7 @@ __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *
 #pragma unroll
         for (int i = 0; i < 2; i++)
 #pragma unroll
-            for (int jj = 0; jj < 4; jj++)
+            for (int jj = 0; jj < NB; jj++)
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
                     f32x4 *at = reinterpret_cast<f32x4 *>(blk + (jj * 32 + row32) * EP_LD + i * 32 + q * 8 + kgrp * 4);
@@ -982,15 +984,24 @@ hipError_t q4k_gemm_f16_launch(hipStream_t s, const uint8_t *w, const uint16_t *
     static std::atomic<bool> attr_set{false};  // dynamic LDS above 64 KB has to be allowed once per process
     if (!attr_set) {
         hipError_t e = hipFuncSetAttribute((const void *)q4k_gemm_exact_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        if (e == hipSuccess) e = hipFuncSetAttribute((const void *)q4k_gemm_pair_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        for (const void *k : {(const void *)q4k_gemm_pair_kernel<1>, (const void *)q4k_gemm_pair_kernel<2>, (const void *)q4k_gemm_pair_kernel<3>, (const void *)q4k_gemm_pair_kernel<4>})
+            if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         if (e != hipSuccess) return e;
         attr_set = true;
     }
     const dim3 grid((rows + GM - 1) / GM, (seq + GN - 1) / GN, z);
     float *slab = split ? partial : (float *)nullptr;
-    if (rexp)
-        hipLaunchKernelGGL(q4k_gemm_pair_kernel, grid, dim3(QTHREADS), G_LDS_BYTES, s, w, xh, sx, rexp, tok_scale, out, rows, hidden, seq,
-                           with_mins, accumulate, per, slab);
+    // a prompt of one token tile reads and multiplies only its blocks of 32 tokens (3840 x 15360 with 16 / 64 / 96 tokens: 32.5 / 36.4 /
+    // 37.2 us per call with all four blocks, 27.2 / 32.9 / 35.4 so); the copies stay whole, clamped to the last token
+#define LARQL_PAIR(NB) hipLaunchKernelGGL(q4k_gemm_pair_kernel<NB>, grid, dim3(QTHREADS), G_LDS_BYTES, s, w, xh, sx, rexp, tok_scale, out, rows, hidden, seq, \
+                                          with_mins, accumulate, per, slab)
+    if (rexp) {
+        if (seq <= 32) LARQL_PAIR(1);
+        else if (seq <= 64) LARQL_PAIR(2);
+        else if (seq <= 96) LARQL_PAIR(3);
+        else LARQL_PAIR(4);
+    }
+#undef LARQL_PAIR
     else
         hipLaunchKernelGGL(q4k_gemm_exact_kernel, grid, dim3(GTHREADS), G_LDS_BYTES, s, w, xh, sx, tok_scale, out, rows, hidden, seq, with_mins,
                            accumulate, per, slab);
