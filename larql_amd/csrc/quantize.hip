@@ -293,22 +293,37 @@ __device__ __forceinline__ int sat_i32(float v) {
     return (int)v;
 }
 
-__global__ void quantize_q4_0_kernel(const float *__restrict__ src, size_t n_blocks, uint8_t *__restrict__ dst) {
-    const size_t b = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= n_blocks) return;
-    const float *blk = src + b * 32;
+// Four lanes per block, lane q with elements 4q..4q+3 and 16+4q..+3 (which share its four bytes): whole lines per load and
+// store.  A thread per block (byte stores 18 bytes apart, every element loaded twice) took 93.8 us for
+// 10240 x 2560, this takes 20.0 (6.0 TB/s).
+__global__ void __launch_bounds__(256) quantize_q4_0_kernel(const float *__restrict__ src, size_t n_blocks, uint8_t *__restrict__ dst) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x, b = i >> 2;
+    if (b >= n_blocks) return;  // (four lanes leave together)
+    const uint32_t q = (uint32_t)i & 3u;
+    const float *blk = src + b * 32 + 4 * q;
+    float lo[4], hi[4];  // (the source may stand at any float, the result at any byte)
+    __builtin_memcpy(lo, blk, 16);
+    __builtin_memcpy(hi, blk + 16, 16);
     float amax = 0.0f;
-    for (int i = 0; i < 32; i++) amax = fmaxf(amax, fabsf(blk[i]));
+#pragma unroll
+    for (int c = 0; c < 4; c++) amax = fmaxf(amax, fmaxf(fabsf(lo[c]), fabsf(hi[c])));
+    amax = fmaxf(amax, dpp_f32<0xB1>(amax));  // quad_perm [1,0,3,2], [2,3,0,1]
+    amax = fmaxf(amax, dpp_f32<0x4E>(amax));
     const float scale = amax / 7.0f;
     const float inv = scale > 0.0f ? 1.0f / scale : 0.0f;
+    uint32_t w = 0;
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        int l = sat_i32(roundf(lo[c] * inv)) + 8, h = sat_i32(roundf(hi[c] * inv)) + 8;
+        l = l < 0 ? 0 : (l > 15 ? 15 : l);
+        h = h < 0 ? 0 : (h > 15 ? 15 : h);
+        w |= (uint32_t)(l | (h << 4)) << (8 * c);
+    }
     uint8_t *o = dst + b * 18;
-    const uint32_t h = f32_to_f16_flush(scale);
-    o[0] = (uint8_t)(h & 0xFF); o[1] = (uint8_t)(h >> 8);
-    for (int j = 0; j < 16; j++) {
-        int lo = sat_i32(roundf(blk[j] * inv)) + 8, hi = sat_i32(roundf(blk[j + 16] * inv)) + 8;
-        lo = lo < 0 ? 0 : (lo > 15 ? 15 : lo);
-        hi = hi < 0 ? 0 : (hi > 15 ? 15 : hi);
-        o[2 + j] = (uint8_t)(lo | (hi << 4));
+    __builtin_memcpy(o + 2 + 4 * q, &w, 4);
+    if (q == 0) {
+        const uint16_t h = (uint16_t)f32_to_f16_flush(scale);
+        __builtin_memcpy(o, &h, 2);
     }
 }
 
@@ -372,9 +387,18 @@ __global__ void quantize_mxfp4_kernel(const float *__restrict__ src, size_t n_gr
     reinterpret_cast<uint4 *>(packed)[g] = o;
 }
 
-__global__ void f32_to_bf16_kernel(const float *__restrict__ src, size_t n, uint16_t *__restrict__ dst) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) dst[i] = (uint16_t)(f2u(src[i]) >> 16);  // truncation, larql-models/src/quant/half.rs:107-109
+// Four elements per thread (one 16-byte load, one 8-byte store), the last few one by one: 10240 x 2560
+// 38.1 us with an element per thread, now 23.0 (6.8 TB/s).
+__global__ void __launch_bounds__(256) f32_to_bf16_kernel(const float *__restrict__ src, size_t n, uint16_t *__restrict__ dst) {
+    const size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+    if (i + 4 <= n) {
+        uint32_t v[4];  // truncation, larql-models/src/quant/half.rs:107-109
+        __builtin_memcpy(v, src + i, 16);
+        const uint32_t w[2] = {(v[0] >> 16) | (v[1] & 0xFFFF0000u), (v[2] >> 16) | (v[3] & 0xFFFF0000u)};
+        __builtin_memcpy(dst + i, w, 8);
+    } else {
+        for (size_t e = i; e < n; e++) dst[e] = (uint16_t)(f2u(src[e]) >> 16);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -439,13 +463,13 @@ hipError_t quantize_mxfp4_launch(hipStream_t s, const float *src, size_t rows, s
 }
 hipError_t f32_to_bf16_launch(hipStream_t s, const float *src, size_t n, uint16_t *dst) {
     if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(f32_to_bf16_kernel, blocks_for(n, 256), dim3(256), 0, s, src, n, dst);
+    hipLaunchKernelGGL(f32_to_bf16_kernel, blocks_for((n + 3) / 4, 256), dim3(256), 0, s, src, n, dst);
     return hipGetLastError();
 }
 hipError_t quantize_q4_0_launch(hipStream_t s, const float *src, size_t n, uint8_t *dst) {
     const size_t nb = n / 32;
     if (nb == 0) return hipSuccess;
-    hipLaunchKernelGGL(quantize_q4_0_kernel, blocks_for(nb, 256), dim3(256), 0, s, src, nb, dst);
+    hipLaunchKernelGGL(quantize_q4_0_kernel, blocks_for(nb * 4, 256), dim3(256), 0, s, src, nb, dst);
     return hipGetLastError();
 }
 hipError_t quantize_to_q8_launch(hipStream_t s, const float *src, size_t n, int8_t *q8, float *scales) {

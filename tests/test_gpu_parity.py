@@ -778,6 +778,30 @@ def test_device_kquant_encoders_on_partial_workgroups_and_odd_blocks(be, n_sb):
             assert np.array_equal(got[:want.size], np.asarray(want).reshape(-1)) and (got[want.size:] == 0xA5).all(), special
 
 
+@pytest.mark.parametrize("n", [32, 96, 2048 + 32, 64 * 33])
+def test_device_q4_0_and_bf16_encoders_at_any_alignment_and_length(be, n):
+    """Block counts around a workgroup's sixty-four, a length that leaves one to three elements to bf16's last thread, sources at
+    any float and results at any byte (Q4_0) or half-word (bf16), infinities, NaN and subnormals.  Byte for byte the oracle's."""
+    rng = np.random.default_rng(n)
+    w = rng.standard_normal(n + 8).astype(F)
+    w[3::32] = F(1e-40); w[n // 2] = F(np.inf); w[5] = F(np.nan); w[n - 32:n - 16] = 0
+    for skip in (0, 1, 2):
+        src = be.to_device(w) + 4 * skip
+        x = w[skip:skip + n]
+        dst = be.to_device(np.full(2 * n + 32, 0xA5, np.uint8))
+        assert be.dev_quantize_q4_0(src, n, dst + skip)
+        be.synchronize()
+        got, want = be.d2h(dst, 2 * n + 32, np.uint8), np.asarray(O.quantize_q4_0(x)).reshape(-1)
+        assert np.array_equal(got[skip:skip + want.size], want) and (got[skip + want.size:] == 0xA5).all()
+        for m in (n, n - 1, n - 2, n - 3):
+            be.h2d(dst, np.full(2 * n + 32, 0xA5, np.uint8))
+            assert be.dev_f32_to_bf16(src, m, dst + 2 * skip)
+            be.synchronize()
+            got = be.d2h(dst, 2 * n + 32, np.uint8)
+            assert np.array_equal(got[2 * skip:2 * (skip + m)].view(np.uint16), (x[:m].view(np.uint32) >> 16).astype(np.uint16))
+            assert (got[2 * (skip + m):] == 0xA5).all()
+
+
 def test_device_encoders_are_bit_exact(be):
     rng = np.random.default_rng(41)
     n = 256 * 4096
