@@ -448,7 +448,12 @@ static hipError_t topk_rows(hipStream_t stream, TopkArgs A, uint32_t batch, void
                      : topk_stage<false, kTopkCached, false, true, false>(stream, A, 1, batch);
     }
     const bool cached = A.n <= (uint32_t)(kTopkThreads * kTopkCached);
-    if (large) return cached ? topk_stage<BY_ABS, kTopkCached, true, false, false>(stream, A, 1, batch) : topk_stage<BY_ABS, 0, true, false, false>(stream, A, 1, batch);
+    if (large) {
+        // (the radix passes walk every round of the registers, empty or not: rows of up to 4096 take four instead of sixteen —
+        // a KNN call over 1254 features, K = 256: 20.8 us with sixteen, 17.9 with four, 19.3 streamed from memory)
+        if (A.n <= (uint32_t)(kTopkThreads * kTopkCached / 4)) return topk_stage<BY_ABS, kTopkCached / 4, true, false, false>(stream, A, 1, batch);
+        return cached ? topk_stage<BY_ABS, kTopkCached, true, false, false>(stream, A, 1, batch) : topk_stage<BY_ABS, 0, true, false, false>(stream, A, 1, batch);
+    }
     return cached ? topk_stage<BY_ABS, kTopkCached, false, false, false>(stream, A, 1, batch) : topk_stage<BY_ABS, 0, false, false, false>(stream, A, 1, batch);
 }
 
