@@ -778,6 +778,22 @@ def test_device_kquant_encoders_on_partial_workgroups_and_odd_blocks(be, n_sb):
             assert np.array_equal(got[:want.size], np.asarray(want).reshape(-1)) and (got[want.size:] == 0xA5).all(), special
 
 
+@pytest.mark.parametrize("n,k", [(65, 65), (300, 256), (4095, 200), (4096, 256), (4097, 256), (16384, 100)])
+def test_more_than_64_hits_of_rows_around_the_register_sizes(be, fmt, n, k):
+    """K above 64 over rows that four or sixteen registers a thread hold, ties among them: the order of (|score|, lower index
+    first) over the scores that the call itself left."""
+    rng = np.random.default_rng(n)
+    gate = np.repeat(rng.standard_normal(((n + 1) // 2, 256)).astype(F), 2, axis=0)[:n].copy()   # every score twice
+    dg, x = be.to_device(gate), be.to_device(rng.standard_normal((2, 256)).astype(F))
+    sc, idx, val, cnt = be.malloc(2 * n * 4), be.malloc(2 * k * 4), be.malloc(2 * k * 4), be.malloc(8)
+    assert be.dev_gate_knn(fmt.FMT_F32, dg, x, 2, n, 256, k, sc, idx, val, cnt), be.last_error()
+    be.synchronize()
+    s, i, v = be.d2h(sc, (2, n), F), be.d2h(idx, (2, k), np.uint32), be.d2h(val, (2, k), F)
+    for row in range(2):
+        want = np.lexsort((np.arange(n), -np.abs(s[row])))[:k]
+        assert np.array_equal(i[row], want) and np.array_equal(v[row], s[row][want])
+
+
 @pytest.mark.parametrize("n", [32, 96, 2048 + 32, 64 * 33])
 def test_device_q4_0_and_bf16_encoders_at_any_alignment_and_length(be, n):
     """Block counts around a workgroup's sixty-four, a length that leaves one to three elements to bf16's last thread, sources at
