@@ -496,12 +496,27 @@ int enqueue_jobs(larql_hip_ctx *c, std::vector<GemvJob> &jobs_in) {
     return LARQL_OK;
 }
 
-// top-K over rows of device scores, with the workspace that long rows are selected through
+// `ensure` for memory that a call is only faster with: false, and no error left behind, where there is none to be had
+bool ensure_optional(larql_hip_ctx *c, DevBuf &b, size_t bytes) {
+    c->alloc_events++;
+    if (bytes <= b.cap) return true;
+    if (b.p) (void)hipFree(b.p);
+    b.p = nullptr; b.cap = 0;
+    if (hipMalloc(&b.p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        b.p = nullptr;
+        return false;
+    }
+    b.cap = bytes;
+    return true;
+}
+
+// top-K over rows of device scores, with the workspace that long rows are selected through; without it they are streamed
 int run_topk(larql_hip_ctx *c, const float *scores, uint32_t batch, uint32_t n, uint32_t k, bool by_abs, uint32_t *idx, float *val,
              uint32_t *count, int *nan_flag) {
-    const size_t ws = topk_workspace_bytes(batch, n, k);
-    if (ws) { int rc = ensure(c, c->topk, ws); if (rc) return rc; }
-    HIPCHECK(c, topk_launch(c->stream, scores, batch, n, k, by_abs, idx, val, count, nan_flag, c->topk.p, ws));
+    size_t ws = topk_workspace_bytes(batch, n, k);
+    if (ws && !ensure_optional(c, c->topk, ws)) ws = 0;
+    HIPCHECK(c, topk_launch(c->stream, scores, batch, n, k, by_abs, idx, val, count, nan_flag, ws ? c->topk.p : nullptr, ws));
     return LARQL_OK;
 }
 

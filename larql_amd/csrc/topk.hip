@@ -389,8 +389,8 @@ __global__ void __launch_bounds__(kTopkThreads) __attribute__((amdgpu_num_sgpr(8
 }
 
 // How a row is cut.  A row that one workgroup can hold in registers is not: two launches cost 4 us more than one.  Above
-// that, K <= 64 takes chunks of 4096 (four scores a thread; 16 times as many where the chunks' winners would not fit the
-// merging workgroup's registers), a larger K chunks of 16384 while they shrink the row to a quarter at least.
+// that, K <= 64 takes chunks of 4096 (four scores a thread; of 16384 where the chunks' winners would not fit the
+// merging workgroup's registers), a larger K chunks of 16384.
 static uint32_t topk_chunk(uint32_t n, uint32_t k) {
     constexpr uint32_t held = kTopkThreads * kTopkCached, small = held / 4;
     if (n <= held) return n;
@@ -402,9 +402,23 @@ static uint32_t topk_chunk(uint32_t n, uint32_t k) {
     return k <= held / 4 && n <= 0x7FFFFFFFu ? held : n;
 }
 
-size_t topk_workspace_bytes(uint32_t batch, uint32_t n, uint32_t k) {
+// Bytes of workspace that one row's chunks leave their keys in (0: the row is not cut).
+static size_t topk_row_bytes(uint32_t n, uint32_t k) {
     const uint32_t chunk = n ? topk_chunk(n, k) : n;
-    return chunk == n ? 0 : (size_t)batch * ((n + chunk - 1) / chunk) * k * sizeof(uint64_t);
+    return chunk == n ? 0 : (size_t)((n + chunk - 1) / chunk) * k * sizeof(uint64_t);
+}
+
+// The workspace is bounded: a batch that needs more is selected in slices of rows (512 at least where K <= 64, and a multiple
+// of 256 where it holds so many: the merging launch of a slice is a workgroup per row), and a row that alone needs more is
+// streamed.
+constexpr size_t kTopkWorkspaceMax = 64u << 20;
+size_t topk_workspace_bytes(uint32_t batch, uint32_t n, uint32_t k) {
+    const size_t row = topk_row_bytes(n, k);
+    if (row == 0 || row > kTopkWorkspaceMax) return 0;
+    size_t rows = kTopkWorkspaceMax / row;
+    if (rows >= batch) rows = batch;
+    else if (rows > 256) rows -= rows % 256;
+    return row * rows;
 }
 
 // one launch over `batch` rows of `chunks` chunks each
@@ -428,12 +442,12 @@ static hipError_t topk_stage(hipStream_t stream, TopkArgs A, uint32_t chunks, ui
     return hipGetLastError();
 }
 
+// (workspace: room for the keys of all `batch` rows' chunks, or null: the rows are not cut)
 template <bool BY_ABS>
-static hipError_t topk_rows(hipStream_t stream, TopkArgs A, uint32_t batch, void *workspace, size_t workspace_bytes) {
+static hipError_t topk_rows(hipStream_t stream, TopkArgs A, uint32_t batch, void *workspace) {
     const bool large = A.k > 64 && A.n > 64;
-    const size_t need = topk_workspace_bytes(batch, A.n, A.k);
     A.chunk = A.n;
-    if (need && workspace && workspace_bytes >= need) {
+    if (workspace) {
         const uint32_t chunk = topk_chunk(A.n, A.k), chunks = (A.n + chunk - 1) / chunk;
         A.chunk = chunk;
         A.keys_out = (uint64_t *)workspace;
@@ -462,12 +476,16 @@ hipError_t topk_launch(hipStream_t stream, const float *scores, uint32_t batch, 
     if (k > kTopkMaxK) return hipErrorInvalidValue;
     TopkArgs A = {};
     A.scores_n = A.n = n; A.k = k; A.nan_flag = nan_flag;
-    for (uint32_t b0 = 0; b0 < batch; b0 += 65535) {  // (rows are the grid's y)
+    const size_t need = topk_workspace_bytes(batch, n, k);
+    if (need == 0 || workspace_bytes < need) workspace = nullptr;
+    const uint32_t slice = workspace ? std::min<uint32_t>(65535u, (uint32_t)(need / topk_row_bytes(n, k))) : 65535u;  // (rows are the grid's y)
+    for (uint32_t b0 = 0; b0 < batch; b0 += slice) {
+        const uint32_t rows = std::min(slice, batch - b0);
         A.scores = scores + (size_t)b0 * n;
         A.idx_out = idx_out + (size_t)b0 * k; A.val_out = val_out + (size_t)b0 * k; A.count_out = count_out + b0;
-        const hipError_t e = by_abs ? topk_rows<true>(stream, A, std::min(65535u, batch - b0), workspace, workspace_bytes)
-                                    : topk_rows<false>(stream, A, std::min(65535u, batch - b0), workspace, workspace_bytes);
+        const hipError_t e = by_abs ? topk_rows<true>(stream, A, rows, workspace) : topk_rows<false>(stream, A, rows, workspace);
         if (e != hipSuccess) return e;
+        if (rows == batch - b0) break;  // (b0 + slice may pass 2^32)
     }
     return hipSuccess;
 }

@@ -4,6 +4,7 @@ inputs.  Bars: quantised bytes bit-exact; matvec outputs within 1e-3 relative
 L2 (fp32 accumulate; measured ~1e-6, asserted at 2e-5 so a wrong scale or a
 dropped term cannot hide); top-K index sets identical except at score ties
 within 1e-5."""
+import ctypes as C
 import json
 import os
 
@@ -2026,6 +2027,40 @@ def test_top_k_of_rows_cut_into_chunks(be, fmt, n, k, case):
     valid = np.flatnonzero(np.isfinite(s16))
     want = valid[np.lexsort((valid, -s16[valid]))[:k]]
     assert [i for i, _ in got] == want.tolist()
+
+
+def _device_memory_free(fmt):
+    free, total = C.c_size_t(), C.c_size_t()
+    assert C.CDLL(fmt._lib.LIB_PATH).hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def test_top_k_of_many_long_rows_takes_bounded_memory(be, fmt):
+    """1500 rows of 44100 scores, 4096 hits each: the chunks' keys of all rows would take 147 MB; the selection goes through them in
+    slices of the 64 MB it may take.  Rows on both sides of every slice's end against the order of the scores."""
+    T, n, k, hidden = 1500, 44100, 4096, 32
+    rng = np.random.default_rng(8)
+    own = fmt.HipBackend()
+    try:
+        gate, x = own.to_device(rng.standard_normal((n, hidden)).astype(F)), own.to_device(rng.standard_normal((T, hidden)).astype(F))
+        sc, idx, val, cnt = own.malloc(T * n * 4), own.malloc(T * k * 4), own.malloc(T * k * 4), own.malloc(T * 4)
+        assert own.dev_gate_knn(fmt.FMT_F32, gate, x, T, n // 4, hidden, 8, sc, idx, val, cnt)   # (job tables: not what is looked at)
+        own.synchronize()
+        before = _device_memory_free(fmt)
+        assert own.dev_gate_knn(fmt.FMT_F32, gate, x, T, n, hidden, k, sc, idx, val, cnt), own.last_error()
+        own.synchronize()
+        assert before - _device_memory_free(fmt) < 72 << 20
+        assert (own.d2h(cnt, (T,), np.uint32) == k).all()
+        per = (64 << 20) // (3 * k * 8) // 256 * 256
+        for t in (0, per - 1, per, 2 * per - 1, 2 * per, T - 1):
+            s = own.d2h(sc + t * n * 4, (n,), F)
+            want = np.lexsort((np.arange(n), -np.abs(s)))[:k]
+            assert np.array_equal(own.d2h(idx + t * k * 4, (k,), np.uint32), want), t
+            assert np.array_equal(own.d2h(val + t * k * 4, (k,), F), s[want]), t
+        for p in (gate, x, sc, idx, val, cnt):
+            own.free(p)
+    finally:
+        own.close()
 
 
 def test_top_k_above_64_limits_and_by_value(be, fmt):
