@@ -388,10 +388,17 @@ __global__ void __launch_bounds__(kTopkThreads) __attribute__((amdgpu_num_sgpr(8
     }
 }
 
-// How a row is cut.  A row that one workgroup can hold in registers is not: two launches cost 4 us more than one.  Above
-// that, K <= 64 takes chunks of 4096 (four scores a thread; of 16384 where the chunks' winners would not fit the
-// merging workgroup's registers), a larger K chunks of 16384.
-static uint32_t topk_chunk(uint32_t n, uint32_t k) {
+// How a row of a batch is cut.  A row that one workgroup can hold in registers is not: two launches cost 4 us more than one.
+// Above that, K <= 64 takes chunks of 4096 (four scores a thread; of 16384 where the chunks' winners would not fit the
+// merging workgroup's registers).
+// A larger K takes chunks of 16384 where that is faster than streaming the row: a second launch and a second ordering of K
+// winners against ~1.7 us per thousand scores beyond the first 16384 that one workgroup would walk again and again.  The two
+// meet at 17408 + 5 K scores (one row, streamed / cut, us: 18000 scores, K = 65 44.1 / 42.8; 20000, 500 51.0 / 51.6; 20000, 1000
+// 55.4 / 60.8; 24000, 1000 61.7 / 61.0; 24000, 2000 68.2 / 75.9; 32768, 2000 84.4 / 76.8; the same within 5 % for 100 or 1000 rows).
+// Above K = 2048 the two orderings (a bitonic sort of 4096 keys is 35 us) take four chunks to pay for (32768, 4096 101.6 / 115.7;
+// 65536, 4096 157.1 / 127.9), and do not once the rows fill the chip by themselves (65536, 4096: 100 rows 315 / 300, 300 rows 722 / 731,
+// 1000 rows 2044 / 2242).
+static uint32_t topk_chunk(uint32_t batch, uint32_t n, uint32_t k) {
     constexpr uint32_t held = kTopkThreads * kTopkCached, small = held / 4;
     if (n <= held) return n;
     if (k <= 64) {
@@ -399,12 +406,13 @@ static uint32_t topk_chunk(uint32_t n, uint32_t k) {
             if ((uint64_t)((n + chunk - 1) / chunk) * k <= held) return chunk;
         return n;
     }
-    return k <= held / 4 && n <= 0x7FFFFFFFu ? held : n;
+    if (n > 0x7FFFFFFFu || k > held / 4) return n;
+    const bool cut = k <= held / 8 ? n >= held + 1024 + 5 * k : n > 3 * held && batch <= 128;
+    return cut ? held : n;
 }
 
 // Bytes of workspace that one row's chunks leave their keys in (0: the row is not cut).
-static size_t topk_row_bytes(uint32_t n, uint32_t k) {
-    const uint32_t chunk = n ? topk_chunk(n, k) : n;
+static size_t topk_row_bytes(uint32_t n, uint32_t k, uint32_t chunk) {
     return chunk == n ? 0 : (size_t)((n + chunk - 1) / chunk) * k * sizeof(uint64_t);
 }
 
@@ -413,7 +421,7 @@ static size_t topk_row_bytes(uint32_t n, uint32_t k) {
 // streamed.
 constexpr size_t kTopkWorkspaceMax = 64u << 20;
 size_t topk_workspace_bytes(uint32_t batch, uint32_t n, uint32_t k) {
-    const size_t row = topk_row_bytes(n, k);
+    const size_t row = topk_row_bytes(n, k, topk_chunk(batch, n, k));
     if (row == 0 || row > kTopkWorkspaceMax) return 0;
     size_t rows = kTopkWorkspaceMax / row;
     if (rows >= batch) rows = batch;
@@ -444,11 +452,11 @@ static hipError_t topk_stage(hipStream_t stream, TopkArgs A, uint32_t chunks, ui
 
 // (workspace: room for the keys of all `batch` rows' chunks, or null: the rows are not cut)
 template <bool BY_ABS>
-static hipError_t topk_rows(hipStream_t stream, TopkArgs A, uint32_t batch, void *workspace) {
+static hipError_t topk_rows(hipStream_t stream, TopkArgs A, uint32_t batch, uint32_t chunk, void *workspace) {
     const bool large = A.k > 64 && A.n > 64;
     A.chunk = A.n;
     if (workspace) {
-        const uint32_t chunk = topk_chunk(A.n, A.k), chunks = (A.n + chunk - 1) / chunk;
+        const uint32_t chunks = (A.n + chunk - 1) / chunk;
         A.chunk = chunk;
         A.keys_out = (uint64_t *)workspace;
         hipError_t e = large ? topk_stage<BY_ABS, kTopkCached, true, false, true>(stream, A, chunks, batch)
@@ -478,12 +486,13 @@ hipError_t topk_launch(hipStream_t stream, const float *scores, uint32_t batch, 
     A.scores_n = A.n = n; A.k = k; A.nan_flag = nan_flag;
     const size_t need = topk_workspace_bytes(batch, n, k);
     if (need == 0 || workspace_bytes < need) workspace = nullptr;
-    const uint32_t slice = workspace ? std::min<uint32_t>(65535u, (uint32_t)(need / topk_row_bytes(n, k))) : 65535u;  // (rows are the grid's y)
+    const uint32_t chunk = topk_chunk(batch, n, k);
+    const uint32_t slice = workspace ? std::min<uint32_t>(65535u, (uint32_t)(need / topk_row_bytes(n, k, chunk))) : 65535u;  // (rows are the grid's y)
     for (uint32_t b0 = 0; b0 < batch; b0 += slice) {
         const uint32_t rows = std::min(slice, batch - b0);
         A.scores = scores + (size_t)b0 * n;
         A.idx_out = idx_out + (size_t)b0 * k; A.val_out = val_out + (size_t)b0 * k; A.count_out = count_out + b0;
-        const hipError_t e = by_abs ? topk_rows<true>(stream, A, rows, workspace) : topk_rows<false>(stream, A, rows, workspace);
+        const hipError_t e = by_abs ? topk_rows<true>(stream, A, rows, chunk, workspace) : topk_rows<false>(stream, A, rows, chunk, workspace);
         if (e != hipSuccess) return e;
         if (rows == batch - b0) break;  // (b0 + slice may pass 2^32)
     }

@@ -1997,7 +1997,8 @@ def test_top_k_above_64(be, fmt, n, k):
         assert sorted(idx.tolist()) == list(range(n))
 
 
-@pytest.mark.parametrize("n,k,case", [(16385, 64, "normal"), (20480, 1, "normal"), (65537, 40, "ties"), (262144, 64, "ties"), (262145, 64, "sorted"),
+@pytest.mark.parametrize("n,k,case", [(16385, 64, "normal"), (17732, 65, "ties"), (17733, 65, "ties"), (27647, 2048, "ties"), (27648, 2048, "ties"),
+                                      (49152, 2049, "normal"), (49153, 2049, "ties"), (20480, 1, "normal"), (65537, 40, "ties"), (262144, 64, "ties"), (262145, 64, "sorted"),
                                       (300001, 16, "constant"), (1100000, 64, "normal"), (16385, 65, "normal"), (98305, 200, "ties"),
                                       (65536, 4096, "ties"), (40000, 5000, "normal"), (70000, 300, "few")])
 def test_top_k_of_rows_cut_into_chunks(be, fmt, n, k, case):
@@ -2036,9 +2037,9 @@ def _device_memory_free(fmt):
 
 
 def test_top_k_of_many_long_rows_takes_bounded_memory(be, fmt):
-    """1500 rows of 44100 scores, 4096 hits each: the chunks' keys of all rows would take 147 MB; the selection goes through them in
+    """2700 rows of 44100 scores, 2048 hits each: the chunks' keys of all rows would take 133 MB; the selection goes through them in
     slices of the 64 MB it may take.  Rows on both sides of every slice's end against the order of the scores."""
-    T, n, k, hidden = 1500, 44100, 4096, 32
+    T, n, k, hidden = 2700, 44100, 2048, 32
     rng = np.random.default_rng(8)
     own = fmt.HipBackend()
     try:
