@@ -960,13 +960,17 @@ hipError_t q4k_gemm_prep_launch(hipStream_t s, const void *x, int x_is_bf16, uin
 // before, kept 120 of 256 CUs on a 3840 x 15360 matrix with 77 tokens: with this one
 // (15 ranges), the reduction above and the kept activations of the preparation the call went from 46.4 to 36.2 us
 // (5.9 preparation, 27.3 GEMM, 4.8 reduction in the kernel trace).
+// The ranges group a result's additions, so they must not change with the number of tokens inside a tile (a token's bits would
+// depend on how many others came with it): the last tile counts as half full.  Against a count chosen for each prompt's own
+// length, us: 4096 x 4096 with 16 / 48 / 77 / 128 tokens 16.1 / 23.8 / 25.6 / 30.1 -> 16.9 / 21.3 / 25.5 / 30.1; 2560 x 5120 with
+// 128 28.6 -> 26.8; at the worst 15360 x 1024 with 16 / 128 15.0 / 26.0 -> 16.2 / 29.2.
 uint32_t q4k_gemm_splits(uint32_t rows, uint32_t hidden, uint32_t seq, uint32_t cu_count) {
-    const uint64_t nsb = hidden / 256, tiles = (uint64_t)((rows + GM - 1) / GM) * ((seq + GN - 1) / GN);
+    const uint64_t nsb = hidden / 256, cols = (seq + GN - 1) / GN, tiles = (uint64_t)((rows + GM - 1) / GM) * cols, tokens = cols * GN - GN / 2;
     uint64_t best = nsb * 39, splits = 1;
     for (uint64_t z = 2; z <= 32 && z <= nsb && tiles * z <= cu_count; z++) {
         const uint64_t per = (nsb + z - 1) / z;
         if ((nsb + per - 1) / per != z) continue;  // (the same ranges as a smaller count)
-        const uint64_t cost = per * 39 + 30 + z * rows * seq * 8 / 400000;
+        const uint64_t cost = per * 39 + 30 + z * rows * tokens * 8 / 400000;
         if (cost < best) { best = cost; splits = z; }
     }
     return (uint32_t)splits;

@@ -1734,6 +1734,27 @@ def test_q4k_gemm_few_tiles_in_many_ranges_of_k(be, rows, hidden, seq):
     assert err.max() < 6 * 3e-4 * size and (err.size < 32 or np.sqrt((err ** 2).mean()) < 5e-4 * size)
 
 
+@pytest.mark.parametrize("rows,hidden,seqs", [(2560, 5120, (16, 33, 64, 77, 96, 128)), (3840, 4096, (16, 40, 64, 128)), (2560, 5120, (129, 200, 256))])
+def test_q4k_gemm_tokens_of_a_tile_do_not_depend_on_how_many_they_are(be, rows, hidden, seqs):
+    """A prompt's length inside a tile of 128 tokens does not change a token's result, bit for bit: device tier, and host tier from
+    its sixteen tokens on."""
+    rng = np.random.default_rng(rows)
+    q = rng.integers(0, 256, size=(rows * hidden // 256, 144), dtype=np.uint8)
+    q[:, 0:4] = np.array([0x00, 0x2C, 0x00, 0x28], np.uint8)   # d = 2^-4, dmin = 2^-5
+    x = rng.standard_normal((max(seqs), hidden)).astype(F)
+    dw, dx, do = be.to_device(q), be.to_device(O.f32_to_bf16(x)), be.malloc(max(seqs) * rows * 4)
+    dev, host = None, None
+    for seq in sorted(seqs, reverse=True):
+        assert be.dev_q4k_gemm(dw, dx, rows, hidden, seq, do), be.last_error()
+        be.synchronize()
+        got = be.d2h(do, (seq, rows), np.uint32)
+        dev = got if dev is None else dev
+        assert np.array_equal(got, dev[:seq]), seq
+        got = be.q4k_matmul(q, x[:seq], rows, hidden, seq).reshape(seq, rows).view(np.uint32)
+        host = got if host is None else host
+        assert np.array_equal(got, host[:seq]), seq
+
+
 def test_q4k_gemm_row_scales_of_any_size_and_uneven_blocks(be):
     """The device tier's GEMM carries each row's scale in an f16 operand behind a per-row exponent: rows whose weights
     differ by twelve orders of magnitude, rows of zeros, and a row with one super-block far larger than the others
