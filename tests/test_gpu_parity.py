@@ -1715,7 +1715,7 @@ def test_q4k_gemm_mfma_matches_oracle(be, rows, hidden, seq):
 
 
 @pytest.mark.parametrize("rows,hidden,seq", [(256, 8192, 3), (515, 5376, 129), (260, 9472, 40), (1, 15360, 1), (1000, 1024, 16), (128, 20992, 130), (300, 1024, 64),
-                                             (300, 1024, 96), (70, 768, 97)])
+                                             (300, 1024, 96), (70, 768, 97), (20, 4096, 9), (20, 4352, 9), (20, 8192, 9), (20, 8448, 9)])
 def test_q4k_gemm_few_tiles_in_many_ranges_of_k(be, rows, hidden, seq):
     """Range counts that are no power of two and up to 32 per tile, a shorter last range, rows no multiple of four (the one-element
     reduction), tokens just past a tile, activations of one to three register vectors per thread."""
