@@ -3460,7 +3460,10 @@ size_t gemv_lds_bytes(const GemvJob *jobs, size_t n, uint32_t threads) {
 // A launch of matvecs against one activation that leaves every compute unit a few tiles takes the short kernel: fills grid,
 // threads, LDS and L.pad.  The line is NT tiles x NP columns per wavefront <= 10: a lane keeps twelve registers of each, 120
 // next to the operands.  With more the streaming kernel's ring hides its set-up behind the stream (238 matvecs in one launch:
-// 5.8 TB/s); the stages of a token, from one to five tiles, took 4.0-8.0 us here and 6.1-12.5 us there.
+// 5.8 TB/s).  Streaming / short kernel on the same launch, us: one tile of 512 / 2560 / 10240 elements 3.8 / 3.2, 5.0 / 3.2, 7.7 / 6.1;
+// eight tiles of 512 / 1024 / 2560 5.8 / 5.7, 5.7 / 5.4, 10.8 / 9.9; at the line 5120 elements x five tiles 13.4 / 12.1, 7680 x three
+// 12.1 / 11.3, 10240 x two 10.7 / 10.6.  Rows of one super-block have one wavefront per workgroup, which walks its tiles alone:
+// one to four tiles 3.8 / 3.2, 3.9 / 3.3, 3.8 / 3.8, 4.0 / 4.3, six 4.1 / 5.4, so the line is three there.
 static uint32_t q4k_short_np(uint64_t cpr) { const uint32_t nw = q4k_mfma_waves(cpr); return (uint32_t)((cpr + nw - 1) / nw); }
 bool gemv_q4k_short(const GemvJob *jobs, size_t n, uint32_t cu_count, uint32_t *threads, uint32_t *grid, size_t *lds, uint32_t *param) {
     if (n == 0 || n > (size_t)kQ4kShortJobs) return false;
@@ -3473,7 +3476,7 @@ bool gemv_q4k_short(const GemvJob *jobs, size_t n, uint32_t cu_count, uint32_t *
     const uint64_t cpr = jobs[0].k / 256;
     const uint32_t nw = q4k_mfma_waves(cpr), np = q4k_short_np(cpr);
     const uint64_t nt = (rows + 16ull * cu_count - 1) / (16ull * cu_count);
-    if (nt == 0 || nt * np > 10 || nt > 8) return false;
+    if (nt == 0 || nt * np > 10 || nt > (cpr == 1 ? 3u : 8u)) return false;
     uint32_t tr = (uint32_t)((rows + cu_count * nt - 1) / (cu_count * nt));
     uint64_t tiles = 0;
     for (;; tr++) {  // (a job's last tile is ragged: a row more per tile where the tiles would spill over into another round)

@@ -74,7 +74,8 @@ def test_q4k_matvec_activation_ranges(be, case):
 
 
 @pytest.mark.parametrize("rows,cols", [([1], 256), ([4096, 1], 256), ([10240, 10240, 9999, 17], 512), ([20000, 12767], 2560), ([2560, 1024, 1023], 2816),
-                                       ([10000, 10480], 2816), ([5, 12000], 5376), ([15], 10240), ([8000], 10240), ([8193], 10240), ([33], 8448)])
+                                       ([10000, 10480], 2816), ([5, 12000], 5376), ([15], 10240), ([8000], 10240), ([8193], 10240), ([33], 8448),
+                                       ([12000, 288], 256), ([12288, 1], 256), ([32768], 512), ([32769], 512)])
 def test_q4k_launches_of_a_few_tiles_per_compute_unit(be, fmt, rows, cols):
     """One to four matvecs against one activation: one to eight tiles and one to four columns per wavefront, ragged last tiles,
     column counts that leave wavefronts without a last column, and one size past the kernel's registers.  Bit for bit what the
