@@ -158,7 +158,7 @@ __global__ void __launch_bounds__(256) quantize_q4_k_kernel(const float *__restr
 // -32..31, biased by 32.  The 256 six-bit codes pass through LDS into ggml's
 // planar layout: ql[64h + p] = code[128h + p] & 15 | (code[128h + p + 64] & 15) << 4,
 // qh[32h + l] = the top two bits of codes 128h + l + {0, 32, 64, 96}; then the 16
-// scales and the truncated f16 d (210 bytes, 2-byte aligned).  10240 x 2560: 40.1 -> 22.2 us (5.7 TB/s).
+// scales and the truncated f16 d (210 bytes, 2-byte aligned).  10240 x 2560, call behind call: 32.8 -> 19.5 us (6.5 TB/s).
 // ---------------------------------------------------------------------------
 // sat_i8(roundf(clampf(v, lo, hi))) for integers lo, hi: half away from zero, NaN -> 0
 __device__ __forceinline__ int round_i8(float v, float lo, float hi) {
@@ -439,7 +439,7 @@ hipError_t quantize_q4_k_launch(hipStream_t s, const float *src, size_t n, uint8
 hipError_t quantize_q6_k_launch(hipStream_t s, const float *src, size_t n, uint8_t *dst) {
     const size_t n_sb = n / 256;
     if (n_sb == 0) return hipSuccess;
-    hipLaunchKernelGGL(quantize_q6_k_kernel, blocks_for(n_sb, 4), dim3(256), 0, s, src, n_sb, dst);
+    hipLaunchKernelGGL(quantize_q6_k_kernel, blocks_for(n_sb, 16), dim3(256), 0, s, src, n_sb, dst);
     return hipGetLastError();
 }
 hipError_t quantize_q8_0_launch(hipStream_t s, const float *src, size_t n, uint8_t *dst) {
