@@ -3428,8 +3428,10 @@ size_t gemv_lds_bytes(const GemvJob *jobs, size_t n, uint32_t threads) {
     }
     if (n > 0 && jobs[0].kind == KIND_MXFP4_MFMA) {
         const size_t nw = threads / 64;
-        // ring + two partial-sum areas of up to four sums (tokens, or folded experts) per weight row and wavefront
-        return nw * kMx4Stages * gemv_launch_param(jobs, n) + 2 * (size_t)kMx4BatchTiles * 16 * nw * 4 * sizeof(float);
+        // ring + two areas of partial sums: one sum per weight row and wavefront, four where a job folds experts
+        uint32_t sums = 1;
+        for (size_t i = 0; i < n; i++) if (jobs[i].combine_w) sums = 4;
+        return nw * kMx4Stages * gemv_launch_param(jobs, n) + 2 * (size_t)kMx4BatchTiles * 16 * nw * sums * sizeof(float);
     }
     if (n > 0 && jobs[0].kind == KIND_Q4K_Q8K) {  // rings + one partial per (row, super-block), double-buffered
         const size_t nw = threads / 64;
