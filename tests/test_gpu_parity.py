@@ -2052,6 +2052,35 @@ def test_top_k_of_rows_cut_into_chunks(be, fmt, n, k, case):
     assert [i for i, _ in got] == want.tolist()
 
 
+@pytest.mark.parametrize("T,n,k", [(3, 20000, 64), (2, 40000, 1), (3, 30000, 200), (2, 262144, 64), (130, 17000, 64), (2, 60000, 3000), (129, 49200, 2100)])
+def test_top_k_of_several_long_rows(be, fmt, T, n, k):
+    """Rows that are selected in two launches (and, in the last case, streamed because there are many), several of them and each with
+    scores of its own, every score twice: the order of (|score|, lower index first) over the scores that the call itself left, row by
+    row.  Then a NaN in a late chunk: the flag is raised, and everything else stays where it was."""
+    rng = np.random.default_rng(n + k)
+    gate = np.repeat(rng.standard_normal((n // 2, 32)).astype(F), 2, axis=0)
+    dg, x = be.to_device(gate), be.to_device(rng.standard_normal((T, 32)).astype(F))
+    sc, idx, val, cnt = be.malloc(T * n * 4), be.malloc(T * k * 4), be.malloc(T * k * 4), be.malloc(T * 4)
+    be.dev_take_nan_flag()
+
+    def run():
+        assert be.dev_gate_knn(fmt.FMT_F32, dg, x, T, n, 32, k, sc, idx, val, cnt), be.last_error()
+        be.synchronize()
+        return be.d2h(sc, (T, n), F), be.d2h(idx, (T, k), np.uint32), be.d2h(val, (T, k), F), be.d2h(cnt, (T,), np.uint32)
+
+    s, i, v, c = run()
+    assert (c == k).all() and not be.dev_take_nan_flag()
+    for row in sorted({0, 1, T // 2, T - 1}):
+        want = np.lexsort((np.arange(n), -np.abs(s[row])))[:k]
+        assert np.array_equal(i[row], want) and np.array_equal(v[row], s[row][want]), row
+    late = int(np.setdiff1d(np.arange(n - 200, n), i.reshape(-1))[0])   # (an index that no row took)
+    gate[late] = np.nan
+    be.h2d(dg, gate)
+    s2, i2, v2, c2 = run()
+    assert np.isnan(s2[:, late]).all() and be.dev_take_nan_flag() and not be.dev_take_nan_flag()
+    assert np.array_equal(i2, i) and np.array_equal(v2, v) and np.array_equal(c2, c)
+
+
 def _device_memory_free(fmt):
     free, total = C.c_size_t(), C.c_size_t()
     assert C.CDLL(fmt._lib.LIB_PATH).hipMemGetInfo(C.byref(free), C.byref(total)) == 0

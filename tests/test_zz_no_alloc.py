@@ -69,6 +69,30 @@ def test_static_entry_equals_the_allocating_one_on_two_calls_in_a_row(be, name):
             assert sorted(i for i, _ in want) == sorted(int(i) for i in ib[b])
 
 
+@pytest.mark.parametrize("name", ["q4_0", "f32"])
+@pytest.mark.parametrize("batch,n,k", [(2, 40000, 64), (8, 16384, 64), (7, 16400, 64), (3, 40000, 1000), (1, 131072, 64), (2, 65536, 2048),
+                                       (1, 65536, 4096), (1, 100000, 4096)])
+def test_static_entry_selects_long_rows_through_the_q8_area(be, name, batch, n, k):
+    """Rows above 16384 scores: the selection's workspace is the scratch array's Q8 area, which a Q4_0 gate's activation has just
+    been read from.  It holds exactly what (2, 65536, 2048) and (1, 65536, 4096) need; the last shape needs more and is streamed.
+    Twice in a row: what the selection left there does not matter to the next call."""
+    import larql_amd as fmt
+    rng = np.random.default_rng(n + k)
+    w = (rng.standard_normal((n, 64)) * 0.02).astype(F)
+    f, enc = encode(fmt, name, w)
+    gd = be.to_device(np.ascontiguousarray(enc))
+    try:
+        for _ in range(2):
+            x = rng.standard_normal((batch, 64)).astype(F)
+            (ia, va), (ib, vb), cnt, scores = both(be, f, gd, x, batch, n, 64, k)
+            assert np.array_equal(ia, ib) and np.array_equal(va, vb) and list(cnt) == [k] * batch
+            for b in range(batch):
+                want = np.lexsort((np.arange(n), -np.abs(scores[b])))[:k]
+                assert np.array_equal(ib[b], want) and np.array_equal(vb[b], scores[b][want].view(np.uint32))
+    finally:
+        be.free(gd)
+
+
 def test_static_entry_refuses_what_does_not_fit(be):
     import larql_amd as fmt
     assert be.static_scratch_bytes() == 131072 * 4 + 256 + 8 * 16384 + 8 * 16384 // 32 * 4
