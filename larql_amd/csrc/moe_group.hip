@@ -9,7 +9,8 @@
 // in LDS and are added in wavefront order.  A token's additions are those of a group of any size, so a result does not
 // depend on who else is in the block, bit for bit.
 //   * TG = 16: one A operand per term, 16 tokens each: three MFMAs share a converted weight operand.  The operands of all
-//     steps stay in registers (12 CW times 4 VGPRs).
+//     steps stay in registers (12 CW times 4 VGPRs; with four steps, rows of 3073 to 4096 elements, all 256 are taken and 9 or 12
+//     values go through scratch: its loads and stores only make the counted waits stricter).
 //   * TG = 4: one A operand holds four tokens' terms (row 4t + i = term i of token t): a third of the MFMAs and operand
 //     loads, for blocks whose experts have few tokens each.
 // The activations arrive as terms, split once (moe_route_terms_kernel, and this kernel's gate/up stage for the down stage):
@@ -17,7 +18,7 @@
 //
 // No job table: a workgroup counts the slots (token, rank) per expert in LDS from the router's choice (at most 4096 ids),
 // which gives it the list of groups and its share of their row tiles; a planning launch on one workgroup took 43 us for 512
-// slots.  128 tokens over 32 experts, top-4, 2880 x 2880: see moe_group_launch.
+// slots.  Figures: see mg_launch_stage.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -358,9 +359,21 @@ static hipError_t mg_launch(hipStream_t s, const MoeGroupArgs &A, uint32_t cu_co
     return hipGetLastError();
 }
 
+// Groups of sixteen tokens once an expert has more than four on average, five with four steps per wavefront.  Same block with
+// groups of four / of sixteen, us (routing included; biases), by slots per expert:
+//   1024 x 1024, 32 experts, top-4   4: 32.6 / 32.9    5: 34.7 / 33.5    6: 37.1 / 34.0    8: 43.8 / 36.0
+//   2048 x 2048, 32 experts, top-4   4: 63.3 / 61.9    5: 74.4 / 62.5    6: 80.1 / 63.9    8: 96.1 / 68.2
+//   2880 x 2880, 32 experts, top-4   2: 93.4 / 107.0   4: 120.3 / 122.8  5: 131.2 / 124.2  6: 144.3 / 125.6   8: 179.8 / 126.1
+//   3328 x 3328, 16 experts, top-2   5: 86.1 / 93.1    6: 100.7 / 94.7   7: 105.7 / 97.6
+//   4096 x 4096, 16 experts, top-2   2: 85.6 / 107.9   4: 107.7 / 118.4  5: 119.4 / 122.6  5.5: 128.4 / 121.8  8: 171.4 / 133.5
+// The job tables before, where four tokens shared a job (2880 / 4096 as above): 2 tokens 47.1 -> 33.4 / 47.2 -> 32.2, 8 tokens
+// 95.0 -> 74.5 / 80.0 -> 58.3, 16 tokens 118.7 -> 93.9 / 114.7 -> 84.8, 64 tokens - / 234.8 -> 133.2, 128 tokens 400 -> 164 / 375.9 -> 169.1;
+// 5120 x 5120, 16 experts, top-4, groups of four only: 2 tokens 85.6 -> 74.2, 16 213.9 -> 196.5, 64 582.9 -> 591.1, 128 1054 -> 996.
 template <bool DOWN>
-static hipError_t mg_launch_stage(hipStream_t s, const MoeGroupArgs &A, uint32_t cu_count, bool wide) {
-    switch (mg_steps_per_wave(A.kdim)) {
+static hipError_t mg_launch_stage(hipStream_t s, const MoeGroupArgs &A, uint32_t cu_count) {
+    const uint32_t cw = mg_steps_per_wave(A.kdim);
+    const bool wide = A.slots > (cw == 4 ? 5u : 4u) * A.n_experts;
+    switch (cw) {
         case 1: return wide ? mg_launch<DOWN, 1, 16>(s, A, cu_count) : mg_launch<DOWN, 1, 4>(s, A, cu_count);
         case 2: return wide ? mg_launch<DOWN, 2, 16>(s, A, cu_count) : mg_launch<DOWN, 2, 4>(s, A, cu_count);
         case 3: return wide ? mg_launch<DOWN, 3, 16>(s, A, cu_count) : mg_launch<DOWN, 3, 4>(s, A, cu_count);
@@ -373,11 +386,7 @@ static hipError_t mg_launch_stage(hipStream_t s, const MoeGroupArgs &A, uint32_t
 hipError_t moe_group_launch(hipStream_t s, const MoeGroupArgs &A, bool down, uint32_t cu_count) {
     if (!moe_group_serves(A.rows, A.kdim) || A.slots == 0 || A.slots > kMoeGroupMaxSlots || A.n_experts == 0 || A.n_experts > kMoeGroupMaxExperts)
         return hipErrorInvalidValue;
-    // Sixteen tokens a group once an expert has more than four on average (32 experts, top-4, 2880 x 2880, biases; us per
-    // block, groups of four / of sixteen / the job-table kernels before): 16 tokens 94 / 109 / 118, 32 tokens 121 / 122 / 154,
-    // 64 tokens 178 / 126 / 237, 128 tokens 290 / 163 / 396, 512 tokens 830 / 410 / 1353.
-    const bool wide = A.slots > 4 * A.n_experts;
-    return down ? mg_launch_stage<true>(s, A, cu_count, wide) : mg_launch_stage<false>(s, A, cu_count, wide);
+    return down ? mg_launch_stage<true>(s, A, cu_count) : mg_launch_stage<false>(s, A, cu_count);
 }
 
 }  // namespace larql

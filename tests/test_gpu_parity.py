@@ -1214,9 +1214,10 @@ def test_moe_mxfp4_routed_equals_select_then_block(be, fmt, T, E, hidden, inter,
 
 @pytest.mark.parametrize("T,E,k,hidden,inter,interleaved,outside", [
     (17, 4, 4, 384, 320, 1, False), (16, 4, 1, 384, 128, 0, False), (16, 4, 1, 160, 352, 1, True), (40, 4, 2, 1152, 160, 0, False), (33, 3, 3, 2880, 288, 1, False), (20, 3, 3, 4096, 128, 1, False),
-    (50, 2, 2, 5120, 128, 0, True), (3, 6, 4, 4128, 4128, 0, False), (1100, 5, 4, 256, 128, 1, False)])
+    (50, 2, 2, 5120, 128, 0, True), (3, 6, 4, 4128, 4128, 0, False), (1100, 5, 4, 256, 128, 1, False),
+    (20, 8, 2, 3328, 128, 1, False), (21, 8, 2, 3328, 128, 1, False), (7, 3, 2, 256, 3136, 1, False), (8, 3, 2, 256, 3136, 1, False)])
 def test_moe_mxfp4_groups_of_sixteen_tokens(be, fmt, T, E, k, hidden, inter, interleaved, outside):
-    """Blocks whose experts have more than four tokens on average (groups of sixteen) and just not: row lengths of one to five
+    """Blocks whose experts have more than four tokens on average (groups of sixteen; five with rows of 3073 to 4096) and just not: row lengths of one to five
     128-element steps per wavefront, ragged last steps, gate and up apart and fused, terms that do not fit the workspace
     (k * inter < hidden), more slots than one launch takes, ids outside the bank.  Sampled tokens against the oracle at the
     bound of the four-token test (1e-5), and every sampled token bit for bit what it is in a two-token block."""
