@@ -218,8 +218,12 @@ __global__ void __launch_bounds__(512) moe_group_kernel(const MoeGroupArgs A) {
                     const bool odd = r & 1u;
                     const float in = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, odd ? s.x : s.y), CTRL, 0xF, 0xF, false));
                     const uint32_t token = 2 * p + (odd ? 1u : 0u);
+                    float act = clamped_glu(odd ? in : s.x, odd ? s.y : in, A.glu_limit, A.glu_alpha);
+                    // (the terms are those of the f32 value, as in the one-token kernels: its last product would else be fused
+                    // into their first subtraction)
+                    asm volatile("" : "+v"(act));
                     uint32_t t3[3];
-                    mx4_terms(clamped_glu(odd ? in : s.x, odd ? s.y : in, A.glu_limit, A.glu_alpha), 0.0f, t3);
+                    mx4_terms(act, 0.0f, t3);
                     if (token < ntok) {
                         const size_t opad = moe_terms_pad(A.rows / 2), plane = slots * opad;
                         GLOBAL_AS uint16_t *tp = (GLOBAL_AS uint16_t *)A.terms_out + gl[token] * opad + moe_term_at(row >> 1);

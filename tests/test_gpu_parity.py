@@ -1250,6 +1250,35 @@ def test_moe_mxfp4_groups_of_sixteen_tokens(be, fmt, T, E, k, hidden, inter, int
         assert rel_l2(got[t], want[0]) < 1e-5, t
 
 
+@pytest.mark.parametrize("k,hidden,inter,interleaved", [(1, 384, 320, 1), (1, 2880, 160, 0), (5, 384, 320, 1), (5, 1152, 352, 0), (8, 160, 1152, 1)])
+def test_moe_mxfp4_token_among_others_equals_the_token_alone(be, fmt, k, hidden, inter, interleaved):
+    """A token's result, bit for bit, whether it comes alone or with others (few: groups of four; many: groups of sixteen).  With up to
+    four experts per token the two-launch path of a token alone weights the activations instead of the sums and adds in another order:
+    equal where there is one expert of weight one."""
+    T, E = 40, 9
+    rng = np.random.default_rng(hidden + k)
+    g_rows = 2 * inter if interleaved else inter
+    bank = [O.quantize_mxfp4((rng.standard_normal(E * r * c) * 0.05).astype(F), E * r, c) for r, c in ((g_rows, hidden), (hidden, inter))]
+    up = (None, None) if interleaved else O.quantize_mxfp4((rng.standard_normal(E * inter * hidden) * 0.05).astype(F), E * inter, hidden)
+    gub, db = (rng.standard_normal(E * 2 * inter) * 0.1).astype(F), (rng.standard_normal(E * hidden) * 0.1).astype(F)
+    ex = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.uint32)
+    p = [be.to_device(a) if a is not None else None for a in (*bank[0], *up, *bank[1], gub, db, rng.standard_normal((T, hidden)).astype(F), ex,
+                                                               np.ones((T, k), F) if k == 1 else rng.random((T, k)).astype(F))]
+    b = fmt.Mxfp4Experts(*p[:6], E, hidden, inter, 7.0, 1.702, interleaved, None, p[6], p[7])
+    wsb = be.moe_mxfp4_workspace_bytes(T, k, hidden, inter)
+    ws, out = be.malloc(wsb), be.malloc(T * hidden * 4)
+
+    def block(t, n):
+        assert be.dev_moe_mxfp4(b, p[8] + t * hidden * 4, n, k, p[9] + t * k * 4, p[10] + t * k * 4, out, ws, wsb), be.last_error()
+        be.synchronize()
+        return be.d2h(out, (n, hidden), np.uint32)
+
+    many, few = block(0, T), block(7, 3)
+    assert np.array_equal(many[7:10], few)
+    for t in (0, 7, 9, T - 1):
+        assert np.array_equal(block(t, 1)[0], many[t]), t
+
+
 def test_moe_mxfp4_job_groups_of_every_size(be, fmt):
     """Experts chosen by 1, 2, 3, 4 and 5 slots: jobs of one, two, three and four tokens and a second job for the
     fifth.  Every token's result equals, bit for bit, what it is in a two-token block."""
