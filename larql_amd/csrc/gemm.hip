@@ -959,8 +959,8 @@ hipError_t q4k_gemm_prep_launch(hipStream_t s, const void *x, int x_is_bf16, uin
 // reduction 30 for the launch and 8 bytes per slab element at 4 TB/s.  The range count with the smallest sum is taken, any
 // number up to 32 whose workgroups all run at once (so the slabs stay below 256 tiles, 34 MB).  Doubling up to 8, the rule
 // before, kept 120 of 256 CUs on a 3840 x 15360 matrix with 77 tokens: with this one
-// (15 ranges), the reduction above and the kept activations of the preparation the call went from 46.4 to 36.2 us
-// (5.9 preparation, 27.3 GEMM, 4.8 reduction in the kernel trace).
+// (15 ranges), the reduction above and the kept activations of the preparation the call went from 46.4 to 36.2 us, and with
+// blocks of 32 tokens (q4k_gemm_f16_launch) to 33.7 (6 preparation, 26 GEMM, 5 reduction in the kernel trace).
 // The ranges group a result's additions, so they must not change with the number of tokens inside a tile (a token's bits would
 // depend on how many others came with it): the last tile counts as half full.  Against a count chosen for each prompt's own
 // length, us: 4096 x 4096 with 16 / 48 / 77 / 128 tokens 16.1 / 23.8 / 25.6 / 30.1 -> 16.9 / 21.3 / 25.5 / 30.1; 2560 x 5120 with

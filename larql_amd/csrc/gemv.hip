@@ -810,7 +810,7 @@ __device__ __forceinline__ void run_q4k_mfma(const GemvJob &j, uint32_t tile_a, 
 // share (2560 rows: 256 tiles of 10, where 16-row tiles kept 160 of 256 busy).
 // Same operands and the same order of additions per row as the streaming kernel: results are equal bit for bit.
 // Per dependent launch in a 34-layer token (2560 wide; streaming kernel before): gate/up 20480 x 2560 11 -> 8.0 us (3.7 TB/s),
-// down 2560 x 10240 12.5 -> 6.2, q/k/v 4096 x 2560 7 -> 4.5, o 2560 x 2048 6.1 -> 4.0; the token 1221 -> 883 us.
+// down 2560 x 10240 12.5 -> 6.1, q/k/v 4096 x 2560 7 -> 4.5, o 2560 x 2048 6.1 -> 4.6; the token 1221 -> 883 us.
 // ---------------------------------------------------------------------------
 struct Q4kShortArgs {
     const float *x;

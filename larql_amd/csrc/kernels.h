@@ -207,7 +207,7 @@ hipError_t moe_route_terms_launch(hipStream_t s, const float *logits, const floa
                                   uint32_t *experts, float *weights, const float *x, uint32_t hidden, uint16_t *terms);
 
 // MoE helpers
-constexpr uint32_t kRouterMaxExperts = 256;      // the selection kernel and the planner (four logits per lane)
+constexpr uint32_t kRouterMaxExperts = 256;      // the selection kernels (four logits per lane)
 constexpr uint32_t kRouterInLaunchExperts = 64;  // a matvec launch that selects for itself (one logit per lane)
 hipError_t router_select_launch(hipStream_t s, const float *logits, const float *bias, uint32_t tokens, uint32_t n_experts, uint32_t k,
                                 int policy, uint32_t *experts, float *weights);

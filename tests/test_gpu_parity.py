@@ -1069,7 +1069,7 @@ def _moe_oracle(c, experts, weights):
 def test_moe_mxfp4_block_matches_oracle(be, fmt, T, E, hidden, inter, biases, interleaved):
     """The expert block (gate/up + bias -> ClampedGlu -> down + bias -> weighted sum) against the checker's block, whose
     composition is pinned on the reference's GPT-OSS fixture; with and without biases, both bank layouts, one token
-    (the down projection folds experts and weighted sum) and several (device-built job lists); 96-wide rows take the
+    (the down projection folds experts and weighted sum) and several (groups found on the device); 96-wide rows take the
     kernels without matrix-core support."""
     rng = np.random.default_rng(59 + T + E)
     k = 4
@@ -1125,8 +1125,8 @@ def test_moe_mxfp4_expert_id_outside_the_bank_is_skipped(be, fmt, T, hidden, int
 
 
 def test_moe_mxfp4_tokens_sharing_an_expert_equal_single_token_calls(be, fmt):
-    """Slots that chose the same expert are served up to four at a time from one read of its weights; a token's result
-    must not depend on who it shared a job with: the 13-token block equals, bit for bit, the two-token blocks of its
+    """Slots that chose the same expert share a read of its weights; a token's result
+    must not depend on who it shared it with: the 13-token block equals, bit for bit, the two-token blocks of its
     neighbouring tokens."""
     rng = np.random.default_rng(83)
     T, E, hidden, inter, k = 13, 6, 384, 320, 4          # 52 slots over 6 experts: full groups, leftovers of one to three, far-apart companions
@@ -1280,7 +1280,7 @@ def test_moe_mxfp4_token_among_others_equals_the_token_alone(be, fmt, k, hidden,
 
 
 def test_moe_mxfp4_job_groups_of_every_size(be, fmt):
-    """Experts chosen by 1, 2, 3, 4 and 5 slots: jobs of one, two, three and four tokens and a second job for the
+    """Experts chosen by 1, 2, 3, 4 and 5 slots: groups of one, two, three and four tokens and a second group for the
     fifth.  Every token's result equals, bit for bit, what it is in a two-token block."""
     rng = np.random.default_rng(97)
     E, hidden, inter, k = 6, 384, 320, 2
@@ -1376,7 +1376,7 @@ def test_moe_mxfp4_interleaved_gate_up_bank_equals_separate_banks(be, fmt, T, E,
     (1, 4, 96, 64, "interleaved", True, True),            # rows the matrix-core kernels do not take
     (1, 128, 384, 320, "interleaved", False, True),       # 128 experts, top-8 (Gemma 4 26B-A4B's count): one token
     (6, 128, 384, 320, "halves", True, True),             # ... several tokens, per-expert scale
-    (3, 128, 384, 320, "interleaved", False, False),      # ... the planner selects
+    (3, 128, 384, 320, "interleaved", False, False),      # ... the launch that splits the activations selects
 ])
 def test_moe_layer_from_per_expert_slices_with_router_projection(be, fmt, T, E, hidden, inter, layout, per_expert, renorm):
     """MoeLayerWeights as the reference brings it (pipeline/moe.rs:469-541): per-expert gate+up / down slices in
