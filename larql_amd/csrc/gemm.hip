@@ -955,23 +955,24 @@ hipError_t q4k_gemm_prep_launch(hipStream_t s, const void *x, int x_is_bf16, uin
 
 
 // K-ranges per output tile (1 = no split), where one 256x128 workgroup runs per CU and the unsplit tiles leave CUs idle.
-// In tenths of a microsecond: a super-block of a tile takes 39, a split's
-// reduction 30 for the launch and 8 bytes per slab element at 4 TB/s.  The range count with the smallest sum is taken, any
+// In tenths of a microsecond: a super-block of a tile takes 45, a split's
+// reduction 50 for the launch and 8 bytes per slab element at 4 TB/s.  The range count with the smallest sum is taken, any
 // number up to 32 whose workgroups all run at once (so the slabs stay below 256 tiles, 34 MB).  Doubling up to 8, the rule
 // before, kept 120 of 256 CUs on a 3840 x 15360 matrix with 77 tokens: with this one
 // (15 ranges), the reduction above and the kept activations of the preparation the call went from 46.4 to 36.2 us, and with
 // blocks of 32 tokens (q4k_gemm_f16_launch) to 33.7 (6 preparation, 26 GEMM, 5 reduction in the kernel trace).
 // The ranges group a result's additions, so they must not change with the number of tokens inside a tile (a token's bits would
-// depend on how many others came with it): the last tile counts as half full.  Against a count chosen for each prompt's own
-// length, us: 4096 x 4096 with 16 / 48 / 77 / 128 tokens 16.1 / 23.8 / 25.6 / 30.1 -> 16.9 / 21.3 / 25.5 / 30.1; 2560 x 5120 with
-// 128 28.6 -> 26.8; at the worst 15360 x 1024 with 16 / 128 15.0 / 26.0 -> 16.2 / 29.2.
+// depend on how many others came with it): the last tile counts as five eighths full.
+// Fitted on calls of 170 shapes (512 to 15360 rows, 1024 to 15360 elements, 16 to 512 tokens) at every range count: 0.5 % above
+// each shape's best on average; at the worst 15360 x 1024 with 16 tokens 18.1 us unsplit and 14.9 with 4 ranges (with 128 tokens 26.0
+// unsplit and 29.2 with 2), 4096 x 4096 with 16 16.9 with 8 and 16.1 with 16, 8000 x 2048 with 512 41.6 unsplit and 39.4 with 2.
 uint32_t q4k_gemm_splits(uint32_t rows, uint32_t hidden, uint32_t seq, uint32_t cu_count) {
-    const uint64_t nsb = hidden / 256, cols = (seq + GN - 1) / GN, tiles = (uint64_t)((rows + GM - 1) / GM) * cols, tokens = cols * GN - GN / 2;
-    uint64_t best = nsb * 39, splits = 1;
+    const uint64_t nsb = hidden / 256, cols = (seq + GN - 1) / GN, tiles = (uint64_t)((rows + GM - 1) / GM) * cols, tokens = cols * GN - GN * 3 / 8;
+    uint64_t best = nsb * 45, splits = 1;
     for (uint64_t z = 2; z <= 32 && z <= nsb && tiles * z <= cu_count; z++) {
         const uint64_t per = (nsb + z - 1) / z;
         if ((nsb + per - 1) / per != z) continue;  // (the same ranges as a smaller count)
-        const uint64_t cost = per * 39 + 30 + z * rows * tokens * 8 / 400000;
+        const uint64_t cost = per * 45 + 50 + z * rows * tokens * 8 / 400000;
         if (cost < best) { best = cost; splits = z; }
     }
     return (uint32_t)splits;
