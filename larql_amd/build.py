@@ -14,7 +14,8 @@ LIB = os.path.join(HERE, "liblarql_hip.so")
 SOURCES = ["gemv.hip", "topk.hip", "quantize.hip", "moe.hip", "moe_group.hip", "gemm.hip", "api.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["-O3", "-std=c++17", "--offload-arch=gfx950", "-fPIC", "-Wall",
-         "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+         "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+         "-mllvm", "-amdgpu-kernarg-preload-count=14"]  # plain scalar arguments arrive in registers
 
 
 def build(verbose: bool = False) -> str:

@@ -812,56 +812,75 @@ __device__ __forceinline__ void run_q4k_mfma(const GemvJob &j, uint32_t tile_a, 
 // Per dependent launch in a 34-layer token (2560 wide; streaming kernel before): gate/up 20480 x 2560 11 -> 8.0 us (3.7 TB/s),
 // down 2560 x 10240 12.5 -> 6.1, q/k/v 4096 x 2560 7 -> 4.5, o 2560 x 2048 6.1 -> 4.6; the token 1221 -> 883 us.
 // ---------------------------------------------------------------------------
-struct Q4kShortArgs {
-    const float *x;
-    uint32_t cpr, nw, tile_rows, n_jobs;
-    const uint8_t *w[kQ4kShortJobs];
-    float *out[kQ4kShortJobs];
-    uint32_t rows[kQ4kShortJobs], tile_end[kQ4kShortJobs];  // tile_end: tiles of the jobs up to and with this one
+// The argument block is fourteen dwords that the hardware puts into scalar registers before a wavefront starts (kernel-argument
+// preload: plain scalar arguments, from the first on), then what is needed late or by a fourth matvec.  Read from a structure,
+// the arguments took five scalar loads that waited for one another (job count, last tile, job's first tile, rows, address)
+// before the first weight was asked for.
+constexpr uint32_t kQ4kShortFour = 1u << 24;  // geom: columns per row | wavefronts << 8 | rows per tile << 16 | a fourth matvec
+
+struct Q4kShortLate {  // behind the preloaded arguments
+    float *out[4];
+    const uint8_t *w3;
+    uint32_t begin3, rows3;
 };
+constexpr uint32_t kQ4kShortLateAt = 56;
+typedef const __attribute__((address_space(4))) Q4kShortLate *q4k_short_late_p;
 
 template <int NT, int NP>
-__global__ void __launch_bounds__(kQ4kMaxWaves * 64) gemv_q4k_short_kernel(const Q4kShortArgs A) {
+__global__ void __launch_bounds__(kQ4kMaxWaves * 64)
+    gemv_q4k_short_kernel(const float *x, const uint8_t *w0, const uint8_t *w1, const uint8_t *w2, uint32_t geom, uint32_t begin1, uint32_t begin2,
+                          uint32_t rows0, uint32_t rows1, uint32_t rows2,  // begin: a matvec's first tile (2^32 - 1: there is none)
+                          const Q4kShortLate) {  // (read through the kernarg pointer below)
     extern __shared__ __attribute__((aligned(16))) uint8_t q4ks_lds[];
     const uint32_t lane = threadIdx.x & 63u, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t jr = lane & 15u, kq = lane >> 4;
-    const uint32_t nw = A.nw, cpr = A.cpr, row_bytes = cpr * 144, TR = A.tile_rows;
-    const uint32_t tile0 = blockIdx.x * NT, tiles = A.tile_end[A.n_jobs - 1];
+    const uint32_t cpr = geom & 0xFFu, nw = (geom >> 8) & 0xFFu, TR = (geom >> 16) & 0xFFu, row_bytes = cpr * 144;
+    constexpr uint32_t PW = kQ4kMaxWaves * 4;
 
     // columns wv, wv + nw, ... of this wavefront (one past the row's end reads the last column and is not used)
     f32x4 raw[NP];
 #pragma unroll
-    for (int p = 0; p < NP; p++) raw[p] = ((g_f4p)(A.x + (size_t)min(wv + nw * p, cpr - 1) * 256))[lane];
+    for (int p = 0; p < NP; p++) raw[p] = ((g_f4p)(x + min(wv + nw * p, cpr - 1) * 256))[lane];
 
-    // the tiles: job, first row, rows (a tile past the end is the last one again)
+    // the tiles: matvec, first row, rows (a tile past the last matvec's end reads its last row again)
     uint32_t job[NT], row0[NT], live[NT];
     u32x4 hdr[NT][NP], q0[NT][NP], q1[NT][NP];
+    q4k_short_late_p late = (q4k_short_late_p)((const __attribute__((address_space(4))) uint8_t *)__builtin_amdgcn_kernarg_segment_ptr() + kQ4kShortLateAt);
 #pragma unroll
     for (int t = 0; t < NT; t++) {
-        const uint32_t tile = min(tile0 + t, tiles - 1);
-        uint32_t ji = 0;
-#pragma unroll
-        for (uint32_t q = 0; q + 1 < kQ4kShortJobs; q++) ji += (q + 1 < A.n_jobs && tile >= A.tile_end[q]) ? 1u : 0u;
-        job[t] = ji;
-        row0[t] = (tile - (ji ? A.tile_end[ji - 1] : 0u)) * TR;
-        live[t] = tile0 + t < tiles ? min(TR, A.rows[ji] - row0[t]) : 0u;
-        const uint32_t row = row0[t] + min(jr, max(live[t], 1u) - 1);
-        const uint8_t *wr = A.w[ji] + (size_t)row * row_bytes;
+        const uint32_t tile = blockIdx.x * NT + t;
+        const bool second = tile >= begin1, third = tile >= begin2;
+        const uint8_t *w = third ? w2 : second ? w1 : w0;
+        uint32_t rows = third ? rows2 : second ? rows1 : rows0, begin = third ? begin2 : second ? begin1 : 0u;
+        job[t] = third ? 2u : second ? 1u : 0u;
+        if (geom & kQ4kShortFour) {
+            if (tile >= late->begin3) { w = late->w3; rows = late->rows3; begin = late->begin3; job[t] = 3u; }
+        }
+        row0[t] = (tile - begin) * TR;
+        live[t] = row0[t] < rows ? min(TR, rows - row0[t]) : 0u;
+        const uint32_t at = min(row0[t] + min(jr, TR - 1), rows - 1) * row_bytes;  // (a short launch's matrices are far below 4 GB)
 #pragma unroll
         for (int p = 0; p < NP; p++) {
-            g_u4p blk = (g_u4p)(wr + min(wv + nw * p, cpr - 1) * 144);
+            g_u4p blk = (g_u4p)(w + (at + min(wv + nw * p, cpr - 1) * 144));
             hdr[t][p] = blk[0];
             q0[t][p] = blk[1 + 2 * kq];
             q1[t][p] = blk[2 + 2 * kq];
         }
     }
+    // (the results' addresses are asked for here, beside the weights: neither ahead of them nor behind the barrier)
+    asm volatile("" : "+s"(late) :: "memory");
+    float *out[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) out[t] = late->out[job[t]];
 
     uint8_t *planes = q4ks_lds + wv * (NP * 1024), *zeros = q4ks_lds + nw * (NP * 1024);
-    float *part = reinterpret_cast<float *>(zeros + kQ4kZeroBytes);  // [NT * 16 rows][nw * 4]
+    float *part = reinterpret_cast<float *>(zeros + kQ4kZeroBytes);  // [NT * 16 rows][kQ4kMaxWaves * 4]
     reinterpret_cast<uint32_t *>(zeros)[lane & 15u] = 0u;           // (every wavefront the same zeros)
     float k[NP], lo[NP], hi[NP];
 #pragma unroll
     for (int p = 0; p < NP; p++) q4k_digits(raw[p], lane, planes + p * 1024, k[p], lo[p], hi[p]);
+#pragma unroll
+    for (int t = 0; t < NT; t++) asm volatile("" : "+s"(out[t]));
     asm volatile("" ::: "memory");  // same wavefront: LDS executes its writes before the reads that follow
     float racc[NT];
 #pragma unroll
@@ -877,24 +896,28 @@ __global__ void __launch_bounds__(kQ4kMaxWaves * 64) gemv_q4k_short_kernel(const
         }
     }
 #pragma unroll
-    for (int t = 0; t < NT; t++) part[(t * 16 + jr) * (nw * 4) + wv * 4 + kq] = racc[t];
+    for (int t = 0; t < NT; t++) part[(t * 16 + jr) * PW + wv * 4 + kq] = racc[t];
+    // (x + -0.0 is x, so the places of wavefronts that there are not need no test in the fold)
+    for (uint32_t w = wv + nw; w < kQ4kMaxWaves; w += nw)
+#pragma unroll
+        for (int t = 0; t < NT; t++) part[(t * 16 + jr) * PW + w * 4 + kq] = -0.f;
     __syncthreads();
     // fold: 4 lanes per row, lane q sums the group-q partial of every wavefront in order
-    for (uint32_t rr = threadIdx.x >> 2; rr < NT * 16; rr += blockDim.x >> 2) {
+    for (uint32_t rr = threadIdx.x >> 2; rr < NT * 16; rr += nw * 16) {
         const uint32_t qd = threadIdx.x & 3u;
-        float v[kQ4kMaxWaves];
+        const float *pr = part + rr * PW + qd;
+        float s = pr[0];
 #pragma unroll
-        for (uint32_t w = 0; w < kQ4kMaxWaves; w++) v[w] = part[rr * (nw * 4) + min(w, nw - 1) * 4 + qd];
-        float s = v[0];
-#pragma unroll
-        for (uint32_t w = 1; w < kQ4kMaxWaves; w++) s = w < nw ? s + v[w] : s;
+        for (int w = 1; w < kQ4kMaxWaves; w++) s += pr[w * 4];
         s = dpp_add<0xB1>(s);  // quad_perm [1,0,3,2]
         s = dpp_add<0x4E>(s);  // quad_perm [2,3,0,1]
-        uint32_t ji = job[0], r0 = row0[0], n = live[0];
+        float *o = out[0] + row0[0];
+        uint32_t n = live[0];
 #pragma unroll
         for (uint32_t t = 1; t < NT; t++)
-            if ((rr >> 4) == t) { ji = job[t]; r0 = row0[t]; n = live[t]; }
-        if (qd == 0 && (rr & 15u) < n) ((g_f32wp)A.out[ji])[r0 + (rr & 15u)] = s;
+            if ((rr >> 4) == t) { o = out[t] + row0[t]; n = live[t]; }
+        if (qd == 0 && (rr & 15u) < n) ((g_f32wp)o)[rr & 15u] = s;
+        if (NT == 1) break;  // (nw >= 1: one round)
     }
 }
 
@@ -3488,7 +3511,7 @@ bool gemv_q4k_short(const GemvJob *jobs, size_t n, uint32_t cu_count, uint32_t *
     }
     *threads = nw * 64;
     *grid = (uint32_t)((tiles + nt - 1) / nt);
-    *lds = (size_t)nw * np * 1024 + kQ4kZeroBytes + (size_t)nt * 16 * nw * 4 * sizeof(float);
+    *lds = (size_t)nw * np * 1024 + kQ4kZeroBytes + (size_t)nt * 16 * kQ4kMaxWaves * 4 * sizeof(float);
     *param = tr | (uint32_t)nt << 8 | np << 16;
     return true;
 }
@@ -3591,16 +3614,22 @@ hipError_t gemv_launch(hipStream_t stream, int kind, const GemvLaunch &L, uint32
             break;
         }
         case KIND_Q4K_SHORT: {
-            Q4kShortArgs A = {};
             const uint32_t tr = L.pad & 0xFFu, nt = (L.pad >> 8) & 0xFFu, np = L.pad >> 16;
-            A.x = L.inl[0].x; A.cpr = (uint32_t)(L.inl[0].k / 256); A.nw = threads / 64; A.tile_rows = tr; A.n_jobs = L.n_jobs;
-            uint32_t tiles = 0;
-            for (uint32_t i = 0; i < L.n_jobs; i++) {
+            const uint8_t *w[kQ4kShortJobs] = {};
+            float *out[kQ4kShortJobs] = {};
+            uint32_t rows[kQ4kShortJobs] = {}, begin[kQ4kShortJobs], tiles = 0;
+            for (uint32_t i = 0; i < kQ4kShortJobs; i++) {
+                begin[i] = i < L.n_jobs ? tiles : ~0u;
+                if (i >= L.n_jobs) continue;
                 const GemvJob &j = L.inl[i];
+                w[i] = j.w; out[i] = j.out; rows[i] = (uint32_t)j.rows;
                 tiles += (uint32_t)((j.rows + tr - 1) / tr);
-                A.w[i] = j.w; A.out[i] = j.out; A.rows[i] = (uint32_t)j.rows; A.tile_end[i] = tiles;
             }
-#define LARQL_Q4K_SHORT(NT, NP) case (NT) | (NP) << 8: hipLaunchKernelGGL((gemv_q4k_short_kernel<NT, NP>), dim3(grid), dim3(threads), lds, stream, A); break;
+            const uint32_t geom = (uint32_t)(L.inl[0].k / 256) | (threads / 64) << 8 | tr << 16 | (L.n_jobs > 3 ? kQ4kShortFour : 0u);
+            const Q4kShortLate late = {{out[0], out[1], out[2], out[3]}, w[3], begin[3], rows[3]};
+#define LARQL_Q4K_SHORT(NT, NP) case (NT) | (NP) << 8: \
+                hipLaunchKernelGGL((gemv_q4k_short_kernel<NT, NP>), dim3(grid), dim3(threads), lds, stream, L.inl[0].x, w[0], w[1], w[2], geom, begin[1], begin[2], \
+                                   rows[0], rows[1], rows[2], late); break;
             switch (nt | np << 8) {
                 LARQL_Q4K_SHORT(1, 1) LARQL_Q4K_SHORT(2, 1) LARQL_Q4K_SHORT(3, 1) LARQL_Q4K_SHORT(4, 1) LARQL_Q4K_SHORT(5, 1) LARQL_Q4K_SHORT(6, 1)
                 LARQL_Q4K_SHORT(7, 1) LARQL_Q4K_SHORT(8, 1) LARQL_Q4K_SHORT(1, 2) LARQL_Q4K_SHORT(2, 2) LARQL_Q4K_SHORT(3, 2) LARQL_Q4K_SHORT(4, 2)
