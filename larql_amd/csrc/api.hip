@@ -264,8 +264,8 @@ constexpr int kTableOnDevice = -2;  // stage_slot: a kernel ahead of the launch 
 int prepare_same_kind(larql_hip_ctx *c, GemvJob *live, size_t n_live, void *table_dst, PreparedLaunch &P, int stage_slot = -1) {
     P.kind = live[0].kind;
     memset(&P.L, 0, sizeof P.L);
-    if (P.kind == KIND_Q4K_MFMA && gemv_q4k_short(live, n_live, (uint32_t)c->cu_count, &P.threads, &P.grid, &P.lds, &P.L.pad)) {
-        P.kind = KIND_Q4K_SHORT;
+    if (gemv_short(live, n_live, (uint32_t)c->cu_count, &P.threads, &P.grid, &P.lds, &P.L.pad)) {
+        P.kind = KIND_SHORT;
         P.L.n_jobs = (uint32_t)n_live;
         for (size_t i = 0; i < n_live; i++) P.L.inl[i] = live[i];
         return LARQL_OK;

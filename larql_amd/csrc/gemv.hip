@@ -581,7 +581,6 @@ union Q4kOp { i32x4 v; uint32_t u[4]; };  // one MFMA operand: 16 int8 k-slots o
 constexpr int kQ4kStages = 4;      // wave-tiles in flight per wavefront (ring slots of 2304 B)
 constexpr int kQ4kBatchTiles = 4;  // 16-row tiles between two folds of the row partials
 constexpr int kQ4kMaxColPasses = 4;
-constexpr uint32_t kQ4kShortJobs = 4;  // matvecs of a short launch
 constexpr int kQ4kMaxWaves = 10;  // with the ring, the partials and 4 prepared columns per wavefront this fills the 160 KB of LDS
 constexpr uint32_t kQ4kTileBytes = 16 * 144;
 constexpr uint32_t kQ4kColBytes = 1024 + 64;  // a column's digits (four planes of 256 bytes), then {2^(e-30), -, -, -, sums of its 8 sub-blocks}
@@ -799,129 +798,6 @@ __device__ __forceinline__ void run_q4k_mfma(const GemvJob &j, uint32_t tile_a, 
 }
 
 // ---------------------------------------------------------------------------
-// Q4_K, short launches: the matvecs of one stage of a token (q, k, v | o | gate, up | down), a few tiles per compute unit.
-//
-// Bound: latency.  Such a launch moves 3-30 MB (0.5-5 us) and depends on the one before it, so what counts is the chain
-// from a wavefront's first instruction to its last store.  The streaming kernel above walks it in steps (descriptor from a
-// 2 KB argument block, activation, a ring of tiles, a fold per batch, next tile); here a workgroup knows its whole work
-// from a small argument block, and every load of it leaves before anything is waited for: the activation's columns, then
-// all NT tiles x NP columns of the wavefront, straight into registers (a lane's header and 32 bytes of nibbles are three
-// 16-byte loads).  One barrier, one fold.  A tile is cut to `tile_rows` <= 16 rows so that all compute units get the same
-// share (2560 rows: 256 tiles of 10, where 16-row tiles kept 160 of 256 busy).
-// Same operands and the same order of additions per row as the streaming kernel: results are equal bit for bit.
-// Per dependent launch in a 34-layer token (2560 wide; streaming kernel before): gate/up 20480 x 2560 11 -> 8.0 us (3.7 TB/s),
-// down 2560 x 10240 12.5 -> 6.1, q/k/v 4096 x 2560 7 -> 4.5, o 2560 x 2048 6.1 -> 4.6; the token 1221 -> 883 us.
-// ---------------------------------------------------------------------------
-// The argument block is fourteen dwords that the hardware puts into scalar registers before a wavefront starts (kernel-argument
-// preload: plain scalar arguments, from the first on), then what is needed late or by a fourth matvec.  Read from a structure,
-// the arguments took five scalar loads that waited for one another (job count, last tile, job's first tile, rows, address)
-// before the first weight was asked for.
-constexpr uint32_t kQ4kShortFour = 1u << 24;  // geom: columns per row | wavefronts << 8 | rows per tile << 16 | a fourth matvec
-
-struct Q4kShortLate {  // behind the preloaded arguments
-    float *out[4];
-    const uint8_t *w3;
-    uint32_t begin3, rows3;
-};
-constexpr uint32_t kQ4kShortLateAt = 56;
-typedef const __attribute__((address_space(4))) Q4kShortLate *q4k_short_late_p;
-
-template <int NT, int NP>
-__global__ void __launch_bounds__(kQ4kMaxWaves * 64)
-    gemv_q4k_short_kernel(const float *x, const uint8_t *w0, const uint8_t *w1, const uint8_t *w2, uint32_t geom, uint32_t begin1, uint32_t begin2,
-                          uint32_t rows0, uint32_t rows1, uint32_t rows2,  // begin: a matvec's first tile (2^32 - 1: there is none)
-                          const Q4kShortLate) {  // (read through the kernarg pointer below)
-    extern __shared__ __attribute__((aligned(16))) uint8_t q4ks_lds[];
-    const uint32_t lane = threadIdx.x & 63u, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t jr = lane & 15u, kq = lane >> 4;
-    const uint32_t cpr = geom & 0xFFu, nw = (geom >> 8) & 0xFFu, TR = (geom >> 16) & 0xFFu, row_bytes = cpr * 144;
-    constexpr uint32_t PW = kQ4kMaxWaves * 4;
-
-    // columns wv, wv + nw, ... of this wavefront (one past the row's end reads the last column and is not used)
-    f32x4 raw[NP];
-#pragma unroll
-    for (int p = 0; p < NP; p++) raw[p] = ((g_f4p)(x + min(wv + nw * p, cpr - 1) * 256))[lane];
-
-    // the tiles: matvec, first row, rows (a tile past the last matvec's end reads its last row again)
-    uint32_t job[NT], row0[NT], live[NT];
-    u32x4 hdr[NT][NP], q0[NT][NP], q1[NT][NP];
-    q4k_short_late_p late = (q4k_short_late_p)((const __attribute__((address_space(4))) uint8_t *)__builtin_amdgcn_kernarg_segment_ptr() + kQ4kShortLateAt);
-#pragma unroll
-    for (int t = 0; t < NT; t++) {
-        const uint32_t tile = blockIdx.x * NT + t;
-        const bool second = tile >= begin1, third = tile >= begin2;
-        const uint8_t *w = third ? w2 : second ? w1 : w0;
-        uint32_t rows = third ? rows2 : second ? rows1 : rows0, begin = third ? begin2 : second ? begin1 : 0u;
-        job[t] = third ? 2u : second ? 1u : 0u;
-        if (geom & kQ4kShortFour) {
-            if (tile >= late->begin3) { w = late->w3; rows = late->rows3; begin = late->begin3; job[t] = 3u; }
-        }
-        row0[t] = (tile - begin) * TR;
-        live[t] = row0[t] < rows ? min(TR, rows - row0[t]) : 0u;
-        const uint32_t at = min(row0[t] + min(jr, TR - 1), rows - 1) * row_bytes;  // (a short launch's matrices are far below 4 GB)
-#pragma unroll
-        for (int p = 0; p < NP; p++) {
-            g_u4p blk = (g_u4p)(w + (at + min(wv + nw * p, cpr - 1) * 144));
-            hdr[t][p] = blk[0];
-            q0[t][p] = blk[1 + 2 * kq];
-            q1[t][p] = blk[2 + 2 * kq];
-        }
-    }
-    // (the results' addresses are asked for here, beside the weights: neither ahead of them nor behind the barrier)
-    asm volatile("" : "+s"(late) :: "memory");
-    float *out[NT];
-#pragma unroll
-    for (int t = 0; t < NT; t++) out[t] = late->out[job[t]];
-
-    uint8_t *planes = q4ks_lds + wv * (NP * 1024), *zeros = q4ks_lds + nw * (NP * 1024);
-    float *part = reinterpret_cast<float *>(zeros + kQ4kZeroBytes);  // [NT * 16 rows][kQ4kMaxWaves * 4]
-    reinterpret_cast<uint32_t *>(zeros)[lane & 15u] = 0u;           // (every wavefront the same zeros)
-    float k[NP], lo[NP], hi[NP];
-#pragma unroll
-    for (int p = 0; p < NP; p++) q4k_digits(raw[p], lane, planes + p * 1024, k[p], lo[p], hi[p]);
-#pragma unroll
-    for (int t = 0; t < NT; t++) asm volatile("" : "+s"(out[t]));
-    asm volatile("" ::: "memory");  // same wavefront: LDS executes its writes before the reads that follow
-    float racc[NT];
-#pragma unroll
-    for (int t = 0; t < NT; t++) racc[t] = 0.f;
-#pragma unroll
-    for (int p = 0; p < NP; p++) {
-        if (p == 0 || wv + nw * p < cpr) {
-            Q4kCol col;
-            q4k_operands(col.xm, planes + p * 1024, zeros, lane);
-            col.k = k[p]; col.sum_lo = lo[p]; col.sum_hi = hi[p];
-#pragma unroll
-            for (int t = 0; t < NT; t++) racc[t] += q4k_mfma_dot(hdr[t][p], q0[t][p], q1[t][p], col, kq);
-        }
-    }
-#pragma unroll
-    for (int t = 0; t < NT; t++) part[(t * 16 + jr) * PW + wv * 4 + kq] = racc[t];
-    // (x + -0.0 is x, so the places of wavefronts that there are not need no test in the fold)
-    for (uint32_t w = wv + nw; w < kQ4kMaxWaves; w += nw)
-#pragma unroll
-        for (int t = 0; t < NT; t++) part[(t * 16 + jr) * PW + w * 4 + kq] = -0.f;
-    __syncthreads();
-    // fold: 4 lanes per row, lane q sums the group-q partial of every wavefront in order
-    for (uint32_t rr = threadIdx.x >> 2; rr < NT * 16; rr += nw * 16) {
-        const uint32_t qd = threadIdx.x & 3u;
-        const float *pr = part + rr * PW + qd;
-        float s = pr[0];
-#pragma unroll
-        for (int w = 1; w < kQ4kMaxWaves; w++) s += pr[w * 4];
-        s = dpp_add<0xB1>(s);  // quad_perm [1,0,3,2]
-        s = dpp_add<0x4E>(s);  // quad_perm [2,3,0,1]
-        float *o = out[0] + row0[0];
-        uint32_t n = live[0];
-#pragma unroll
-        for (uint32_t t = 1; t < NT; t++)
-            if ((rr >> 4) == t) { o = out[t] + row0[t]; n = live[t]; }
-        if (qd == 0 && (rr & 15u) < n) ((g_f32wp)o)[rr & 15u] = s;
-        if (NT == 1) break;  // (nw >= 1: one round)
-    }
-}
-
-// ---------------------------------------------------------------------------
 // Q6_K on the matrix cores: the scheme of the Q4_K kernel above for 210-byte super-blocks (q6k_matvec::dispatch,
 // larql-compute/src/cpu/ops/q6k_matvec.rs:45-91: per 16-element group sub = sum (q - 32) * x; acc += (d * sc) * sub).
 //
@@ -997,17 +873,9 @@ __device__ __forceinline__ void q6k_mfma_fetch_col(Q6kCol &col, const uint8_t *c
     col.k = *reinterpret_cast<const float *>(cp + 1024 + 64);
 }
 
-// one wave-tile from its LDS slot: 16 rows x one super-block against the column's activations
-__device__ __forceinline__ float q6k_mfma_tile(const uint8_t *slot, const Q6kCol &col, uint32_t j, uint32_t kq) {
-    const uint8_t *sp = slot + j * kQ6kPitch;
-    u32x4 ql[2], qh[2];
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-        ql[h] = *reinterpret_cast<const u32x4 *>(sp + 64 * h + 16 * kq);
-        qh[h] = *reinterpret_cast<const u32x4 *>(sp + 128 + 32 * h + 16 * (kq & 1u));
-    }
-    const u32x4 scs = *reinterpret_cast<const u32x4 *>(sp + 192);
-    const float d = half_bits_to_float(*reinterpret_cast<const uint32_t *>(slot + 16 * kQ6kPitch + 16 * j + 12) >> 16);
+// one wave-tile: 16 rows x one super-block against the column's activations.  A lane holds its 16-byte pieces of ql and qh of
+// both halves, the scales and d of its weight row.
+__device__ __forceinline__ float q6k_mfma_dot(const u32x4 (&ql)[2], const u32x4 (&qh)[2], const u32x4 scs, float d, const Q6kCol &col, uint32_t kq) {
     // top bits: MFMA 2h wants bits s0, s0+1 of the qh bytes in bits 4-5 (a left shift by 4 - s0), MFMA 2h+1 bits
     // s0+4, s0+5 (a right shift by s0); what crosses a byte boundary falls outside the mask
     const uint32_t s0 = 2u * (kq >> 1), sl = 4u - s0;
@@ -1030,6 +898,19 @@ __device__ __forceinline__ float q6k_mfma_tile(const uint8_t *slot, const Q6kCol
         acc = __builtin_fmaf(sc, __builtin_fmaf(dot, col.k, col.sumx[m]), acc);  // (sumx holds -32 * the group's sum of x)
     }
     return d * acc;
+}
+
+// ... from its LDS slot
+__device__ __forceinline__ float q6k_mfma_tile(const uint8_t *slot, const Q6kCol &col, uint32_t j, uint32_t kq) {
+    const uint8_t *sp = slot + j * kQ6kPitch;
+    u32x4 ql[2], qh[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        ql[h] = *reinterpret_cast<const u32x4 *>(sp + 64 * h + 16 * kq);
+        qh[h] = *reinterpret_cast<const u32x4 *>(sp + 128 + 32 * h + 16 * (kq & 1u));
+    }
+    const u32x4 scs = *reinterpret_cast<const u32x4 *>(sp + 192);
+    return q6k_mfma_dot(ql, qh, scs, half_bits_to_float(*reinterpret_cast<const uint32_t *>(slot + 16 * kQ6kPitch + 16 * j + 12) >> 16), col, kq);
 }
 
 // tiles [tile_a, tile_b) of one job, columns innermost (the workgroup reads whole rows); `parity` flips per batch
@@ -1141,6 +1022,180 @@ __device__ __forceinline__ void run_q6k_mfma(const GemvJob &j, uint32_t tile_a, 
             if (qd == 0 && row_base + rr < rows) ((g_f32wp)j.out)[row_base + rr] = s;
         }
         parity ^= 1u;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Short launches of Q4_K or Q6_K: the matvecs of one stage of a token (q, k, v | o | gate, up | down), a few tiles per compute unit.
+//
+// Bound: latency.  Such a launch moves 3-30 MB (0.5-5 us) and depends on the one before it, so what counts is the chain
+// from a wavefront's first instruction to its last store.  The streaming kernels above walk it in steps (descriptor from a
+// 2 KB argument block, activation, a ring of tiles, a fold per batch, next tile); here a workgroup knows its whole work
+// from a few arguments, and every load of it leaves before anything is waited for: the activation's columns, then
+// all NT tiles x NP columns of the wavefront, straight into registers (Q4_K: a lane's header and 32 bytes of nibbles are three
+// 16-byte loads; Q6_K: ql and qh of both halves and the scales are five, and two bytes of d).  One barrier, one fold.  A tile is
+// cut to `tile_rows` <= 16 rows so that all compute units get the same share (2560 rows: 256 tiles of 10, where 16-row tiles kept
+// 160 of 256 busy).  Same operands and the same order of additions per row as the streaming kernels: results are equal bit for bit.
+//
+// The argument block is fourteen dwords that the hardware puts into scalar registers before a wavefront starts (kernel-argument
+// preload: plain scalar arguments, from the first on), then what is needed late or by a fourth matvec.  Read from a structure,
+// the arguments took five scalar loads that waited for one another (job count, last tile, job's first tile, rows, address)
+// before the first weight was asked for.  Per dependent launch in a 34-layer token 2560 wide, with the structure / with preload:
+// q/k/v 4096 x 2560 4.1 / 3.25 us, o 2560 x 2048 4.0 / 3.15, gate/up 20480 x 2560 8.4 / 7.8 (3.8 TB/s), down 2560 x 10240 6.0 / 6.0
+// (the streaming kernel: 7, 6.1, 11, 12.5); a launch of one tile 2.1.
+//
+// More wavefronts than the streaming kernel's (sixteen of one or two columns for rows of 11 to 32 super-blocks, each column's partial
+// in LDS for the fold) were measured: 2560 x 4096 3.8 -> 4.0 us, 2560 x 5120 4.1 -> 4.5, 8192 x 7680 8.8 -> 9.4, 2560 x 10240 5.9 -> 6.6;
+// 12288 x 3840 7.2 -> 7.0 alone.
+// Q6_K: its super-blocks lie 2 bytes off, which costs the direct loads more per byte than the streaming kernel's copies: it gains
+// where the columns are one per wavefront (rows of up to ten super-blocks) and the tiles up to four: 2560 x 2560 6.9 -> 4.2, 8192 x
+// 2560 9.0 -> 6.8, 16384 x 2560 11.9 -> 11.3, 20480 x 2560 13.1 -> 13.6 (streaming -> short).
+// ---------------------------------------------------------------------------
+constexpr uint32_t kShortJobs = 4;       // matvecs of a launch
+// geom: columns per row | wavefronts << 8 | rows per tile << 13 | a fourth matvec << 18
+constexpr uint32_t kShortFour = 1u << 18;
+struct ShortLate {  // behind the preloaded arguments
+    float *out[4];
+    const uint8_t *w3;
+    uint32_t begin3, rows3;
+};
+constexpr uint32_t kShortLateAt = 56;
+typedef const __attribute__((address_space(4))) ShortLate *short_late_p;
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));  // (Q6_K super-blocks are 2-byte aligned)
+
+template <bool Q6> struct ShortTile;
+template <> struct ShortTile<false> {
+    static constexpr uint32_t kBlock = 144, kColBytes = 1024;
+    u32x4 hdr, q0, q1;
+    __device__ __forceinline__ void load(const uint8_t *p, uint32_t kq) {
+        g_u4p blk = (g_u4p)p;
+        hdr = blk[0];
+        q0 = blk[1 + 2 * kq];
+        q1 = blk[2 + 2 * kq];
+    }
+};
+template <> struct ShortTile<true> {
+    static constexpr uint32_t kBlock = 210, kColBytes = 1024 + 80;
+    u32x4 ql[2], qh[2], sc;
+    uint32_t d;
+    __device__ __forceinline__ void load(const uint8_t *p, uint32_t kq) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            ql[h] = *(const GLOBAL_AS u32x4_a2 *)(p + 64 * h + 16 * kq);
+            qh[h] = *(const GLOBAL_AS u32x4_a2 *)(p + 128 + 32 * h + 16 * (kq & 1u));
+        }
+        sc = *(const GLOBAL_AS u32x4_a2 *)(p + 192);
+        d = *(const GLOBAL_AS uint16_t *)(p + 208);
+    }
+};
+
+template <bool Q6, int NT, int NP>
+__global__ void __launch_bounds__(kQ4kMaxWaves * 64)
+    gemv_short_kernel(const float *x, const uint8_t *w0, const uint8_t *w1, const uint8_t *w2, uint32_t geom, uint32_t begin1, uint32_t begin2,
+                      uint32_t rows0, uint32_t rows1, uint32_t rows2,  // begin: a matvec's first tile (2^32 - 1: there is none)
+                      const ShortLate) {                               // (read through the kernarg pointer below)
+    extern __shared__ __attribute__((aligned(16))) uint8_t short_lds[];
+    typedef ShortTile<Q6> Tile;
+    constexpr uint32_t PW = kQ4kMaxWaves * 4 + 4;  // partials: [NT * 16 rows][ten wavefronts' four]; the pitch keeps 16 rows off each other's banks
+    const uint32_t lane = threadIdx.x & 63u, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t jr = lane & 15u, kq = lane >> 4;
+    const uint32_t cpr = geom & 0xFFu, nw = (geom >> 8) & 0x1Fu, TR = (geom >> 13) & 0x1Fu, row_bytes = cpr * Tile::kBlock;
+
+    // columns wv, wv + nw, ... of this wavefront (one past the row's end reads the last column and is not used)
+    f32x4 raw[NP];
+#pragma unroll
+    for (int p = 0; p < NP; p++) raw[p] = ((g_f4p)(x + min(wv + nw * p, cpr - 1) * 256))[lane];
+
+    // the tiles: matvec, first row, rows (a tile past the last matvec's end reads its last row again)
+    uint32_t job[NT], row0[NT], live[NT];
+    Tile tile[NT][NP];
+    short_late_p late = (short_late_p)((const __attribute__((address_space(4))) uint8_t *)__builtin_amdgcn_kernarg_segment_ptr() + kShortLateAt);
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        const uint32_t ti = blockIdx.x * NT + t;
+        const bool second = ti >= begin1, third = ti >= begin2;
+        const uint8_t *w = third ? w2 : second ? w1 : w0;
+        uint32_t rows = third ? rows2 : second ? rows1 : rows0, begin = third ? begin2 : second ? begin1 : 0u;
+        job[t] = third ? 2u : second ? 1u : 0u;
+        if (geom & kShortFour) {
+            if (ti >= late->begin3) { w = late->w3; rows = late->rows3; begin = late->begin3; job[t] = 3u; }
+        }
+        row0[t] = (ti - begin) * TR;
+        live[t] = row0[t] < rows ? min(TR, rows - row0[t]) : 0u;
+        const uint32_t at = min(row0[t] + min(jr, TR - 1), rows - 1) * row_bytes;  // (a short launch's matrices are far below 4 GB)
+#pragma unroll
+        for (int p = 0; p < NP; p++) tile[t][p].load(w + (at + min(wv + nw * p, cpr - 1) * Tile::kBlock), kq);
+    }
+    // (the results' addresses are asked for here, beside the weights: neither ahead of them nor behind the barrier)
+    asm volatile("" : "+s"(late) :: "memory");
+    float *out[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) out[t] = late->out[job[t]];
+
+    uint8_t *planes = short_lds + wv * (NP * Tile::kColBytes), *zeros = short_lds + nw * (NP * Tile::kColBytes);
+    float *part = reinterpret_cast<float *>(zeros + kQ4kZeroBytes);
+    float k[NP], lo[NP], hi[NP];
+    if constexpr (!Q6) reinterpret_cast<uint32_t *>(zeros)[lane & 15u] = 0u;  // (every wavefront the same zeros)
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+        if constexpr (Q6) q6k_mfma_prepare_col(raw[p], lane, planes + p * Tile::kColBytes);
+        else q4k_digits(raw[p], lane, planes + p * Tile::kColBytes, k[p], lo[p], hi[p]);
+    }
+#pragma unroll
+    for (int t = 0; t < NT; t++) asm volatile("" : "+s"(out[t]));
+    asm volatile("" ::: "memory");  // same wavefront: LDS executes its writes before the reads that follow
+
+    float racc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) racc[t] = 0.f;
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+        if (p == 0 || wv + nw * p < cpr) {
+            auto dots = [&](auto &col) {
+#pragma unroll
+                for (int t = 0; t < NT; t++) {
+                    float v;
+                    if constexpr (Q6) v = q6k_mfma_dot(tile[t][p].ql, tile[t][p].qh, tile[t][p].sc, half_bits_to_float(tile[t][p].d), col, kq);
+                    else v = q4k_mfma_dot(tile[t][p].hdr, tile[t][p].q0, tile[t][p].q1, col, kq);
+                    racc[t] += v;
+                }
+            };
+            if constexpr (Q6) {
+                Q6kCol col;
+                q6k_mfma_fetch_col(col, planes + p * Tile::kColBytes, jr, kq);
+                dots(col);
+            } else {
+                Q4kCol col;
+                q4k_operands(col.xm, planes + p * Tile::kColBytes, zeros, lane);
+                col.k = k[p]; col.sum_lo = lo[p]; col.sum_hi = hi[p];
+                dots(col);
+            }
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < NT; t++) part[(t * 16 + jr) * PW + wv * 4 + kq] = racc[t];
+    // the places of wavefronts that there are not hold zeros, so that the fold needs no tests (a partial is 0 + something, and so
+    // never -0: adding +0 changes nothing)
+    for (uint32_t w = wv + nw; w < kQ4kMaxWaves; w += nw)
+#pragma unroll
+        for (int t = 0; t < NT; t++) part[(t * 16 + jr) * PW + w * 4 + kq] = 0.f;
+    __syncthreads();
+    // fold: 4 lanes per row, lane q sums the group-q partial of every wavefront in order
+    for (uint32_t rr = threadIdx.x >> 2; rr < NT * 16; rr += nw * 16) {
+        const uint32_t qd = threadIdx.x & 3u;
+        const float *pr = part + rr * PW + qd;
+        float s = pr[0];
+#pragma unroll
+        for (int w = 1; w < kQ4kMaxWaves; w++) s += pr[w * 4];
+        s = dpp_add<0xB1>(s);  // quad_perm [1,0,3,2]
+        s = dpp_add<0x4E>(s);  // quad_perm [2,3,0,1]
+        float *o = out[0] + row0[0];
+        uint32_t n = live[0];
+#pragma unroll
+        for (uint32_t t = 1; t < NT; t++)
+            if ((rr >> 4) == t) { o = out[t] + row0[t]; n = live[t]; }
+        if (qd == 0 && (rr & 15u) < n) ((g_f32wp)o)[rr & 15u] = s;
+        if (NT == 1) break;  // (nw >= 1: one round)
     }
 }
 
@@ -3488,20 +3543,21 @@ size_t gemv_lds_bytes(const GemvJob *jobs, size_t n, uint32_t threads) {
 // 5.8 TB/s).  Streaming / short kernel on the same launch, us: one tile of 512 / 2560 / 10240 elements 3.8 / 3.2, 5.0 / 3.2, 7.7 / 6.1;
 // eight tiles of 512 / 1024 / 2560 5.8 / 5.7, 5.7 / 5.4, 10.8 / 9.9; at the line 5120 elements x five tiles 13.4 / 12.1, 7680 x three
 // 12.1 / 11.3, 10240 x two 10.7 / 10.6.  Rows of one super-block have one wavefront per workgroup, which walks its tiles alone:
-// one to four tiles 3.8 / 3.2, 3.9 / 3.3, 3.8 / 3.8, 4.0 / 4.3, six 4.1 / 5.4, so the line is three there.
-static uint32_t q4k_short_np(uint64_t cpr) { const uint32_t nw = q4k_mfma_waves(cpr); return (uint32_t)((cpr + nw - 1) / nw); }
-bool gemv_q4k_short(const GemvJob *jobs, size_t n, uint32_t cu_count, uint32_t *threads, uint32_t *grid, size_t *lds, uint32_t *param) {
-    if (n == 0 || n > (size_t)kQ4kShortJobs) return false;
+// one to four tiles 3.8 / 3.2, 3.9 / 3.3, 3.8 / 3.8, 4.0 / 4.3, six 4.1 / 5.4, so the line is three there.  Q6_K: one column per
+// wavefront and up to four tiles (the figures at the kernel).
+bool gemv_short(const GemvJob *jobs, size_t n, uint32_t cu_count, uint32_t *threads, uint32_t *grid, size_t *lds, uint32_t *param) {
+    if (n == 0 || n > (size_t)kShortJobs) return false;
+    const bool q6 = jobs[0].kind == KIND_Q6K_MFMA;
+    if (!q6 && jobs[0].kind != KIND_Q4K_MFMA) return false;
     uint64_t rows = 0;
     for (size_t i = 0; i < n; i++) {
         const GemvJob &j = jobs[i];
-        if (j.kind != KIND_Q4K_MFMA || j.x != jobs[0].x || j.k != jobs[0].k || j.row_stride || j.sel || j.batch > 1) return false;
+        if (j.kind != jobs[0].kind || j.x != jobs[0].x || j.k != jobs[0].k || j.row_stride || j.sel || j.batch > 1) return false;
         rows += j.rows;
     }
-    const uint64_t cpr = jobs[0].k / 256;
-    const uint32_t nw = q4k_mfma_waves(cpr), np = q4k_short_np(cpr);
-    const uint64_t nt = (rows + 16ull * cu_count - 1) / (16ull * cu_count);
-    if (nt == 0 || nt * np > 10 || nt > (cpr == 1 ? 3u : 8u)) return false;
+    const uint64_t cpr = jobs[0].k / 256, nt = (rows + 16ull * cu_count - 1) / (16ull * cu_count);
+    const uint32_t nw = q6 ? q6k_mfma_waves(cpr) : q4k_mfma_waves(cpr), np = (uint32_t)((cpr + nw - 1) / nw);
+    if (nt == 0 || nt > (cpr == 1 ? 3u : 8u) || (q6 ? np > 1 || nt > 4 : nt * np > 10)) return false;
     uint32_t tr = (uint32_t)((rows + cu_count * nt - 1) / (cu_count * nt));
     uint64_t tiles = 0;
     for (;; tr++) {  // (a job's last tile is ragged: a row more per tile where the tiles would spill over into another round)
@@ -3511,9 +3567,39 @@ bool gemv_q4k_short(const GemvJob *jobs, size_t n, uint32_t cu_count, uint32_t *
     }
     *threads = nw * 64;
     *grid = (uint32_t)((tiles + nt - 1) / nt);
-    *lds = (size_t)nw * np * 1024 + kQ4kZeroBytes + (size_t)nt * 16 * kQ4kMaxWaves * 4 * sizeof(float);
-    *param = tr | (uint32_t)nt << 8 | np << 16;
+    *lds = (size_t)nw * np * (q6 ? ShortTile<true>::kColBytes : ShortTile<false>::kColBytes) + kQ4kZeroBytes +
+           (size_t)nt * 16 * (kQ4kMaxWaves * 4 + 4) * sizeof(float);
+    *param = tr | (uint32_t)nt << 8 | np << 12;
     return true;
+}
+
+static hipError_t gemv_short_launch(hipStream_t stream, const GemvLaunch &L, uint32_t threads, uint32_t grid, size_t lds) {
+    const uint32_t tr = L.pad & 0xFFu, nt = (L.pad >> 8) & 0xFu, np = (L.pad >> 12) & 7u;
+    const bool q6 = L.inl[0].kind == KIND_Q6K_MFMA;
+    const uint8_t *w[kShortJobs] = {};
+    ShortLate late = {};
+    uint32_t rows[kShortJobs] = {}, begin[kShortJobs], tiles = 0;
+    for (uint32_t i = 0; i < kShortJobs; i++) {
+        begin[i] = i < L.n_jobs ? tiles : ~0u;
+        if (i >= L.n_jobs) continue;
+        const GemvJob &j = L.inl[i];
+        w[i] = j.w; late.out[i] = j.out; rows[i] = (uint32_t)j.rows;
+        tiles += (uint32_t)((j.rows + tr - 1) / tr);
+    }
+    late.w3 = w[3]; late.begin3 = begin[3]; late.rows3 = rows[3];
+    const uint32_t geom = (uint32_t)(L.inl[0].k / 256) | (threads / 64) << 8 | tr << 13 | (L.n_jobs > 3 ? kShortFour : 0u);
+#define LARQL_SHORT(Q6, NT, NP) case (Q6) | (NT) << 1 | (NP) << 5: \
+        hipLaunchKernelGGL((gemv_short_kernel<Q6, NT, NP>), dim3(grid), dim3(threads), lds, stream, L.inl[0].x, w[0], w[1], w[2], geom, begin[1], begin[2], \
+                           rows[0], rows[1], rows[2], late); break;
+    switch ((q6 ? 1u : 0u) | nt << 1 | np << 5) {
+        LARQL_SHORT(0, 1, 1) LARQL_SHORT(0, 2, 1) LARQL_SHORT(0, 3, 1) LARQL_SHORT(0, 4, 1) LARQL_SHORT(0, 5, 1) LARQL_SHORT(0, 6, 1) LARQL_SHORT(0, 7, 1)
+        LARQL_SHORT(0, 8, 1) LARQL_SHORT(0, 1, 2) LARQL_SHORT(0, 2, 2) LARQL_SHORT(0, 3, 2) LARQL_SHORT(0, 4, 2) LARQL_SHORT(0, 5, 2) LARQL_SHORT(0, 1, 3)
+        LARQL_SHORT(0, 2, 3) LARQL_SHORT(0, 3, 3) LARQL_SHORT(0, 1, 4) LARQL_SHORT(0, 2, 4)
+        LARQL_SHORT(1, 1, 1) LARQL_SHORT(1, 2, 1) LARQL_SHORT(1, 3, 1) LARQL_SHORT(1, 4, 1)
+        default: return hipErrorInvalidValue;
+    }
+#undef LARQL_SHORT
+    return hipGetLastError();
 }
 
 uint32_t gemv_wgs_per_cu(int kind, uint32_t threads, size_t lds, uint32_t dflt) {
@@ -3613,32 +3699,7 @@ hipError_t gemv_launch(hipStream_t stream, int kind, const GemvLaunch &L, uint32
             hipLaunchKernelGGL(gemv_mxfp4_mfma_kernel, dim3(grid), dim3(threads), lds, stream, L);
             break;
         }
-        case KIND_Q4K_SHORT: {
-            const uint32_t tr = L.pad & 0xFFu, nt = (L.pad >> 8) & 0xFFu, np = L.pad >> 16;
-            const uint8_t *w[kQ4kShortJobs] = {};
-            float *out[kQ4kShortJobs] = {};
-            uint32_t rows[kQ4kShortJobs] = {}, begin[kQ4kShortJobs], tiles = 0;
-            for (uint32_t i = 0; i < kQ4kShortJobs; i++) {
-                begin[i] = i < L.n_jobs ? tiles : ~0u;
-                if (i >= L.n_jobs) continue;
-                const GemvJob &j = L.inl[i];
-                w[i] = j.w; out[i] = j.out; rows[i] = (uint32_t)j.rows;
-                tiles += (uint32_t)((j.rows + tr - 1) / tr);
-            }
-            const uint32_t geom = (uint32_t)(L.inl[0].k / 256) | (threads / 64) << 8 | tr << 16 | (L.n_jobs > 3 ? kQ4kShortFour : 0u);
-            const Q4kShortLate late = {{out[0], out[1], out[2], out[3]}, w[3], begin[3], rows[3]};
-#define LARQL_Q4K_SHORT(NT, NP) case (NT) | (NP) << 8: \
-                hipLaunchKernelGGL((gemv_q4k_short_kernel<NT, NP>), dim3(grid), dim3(threads), lds, stream, L.inl[0].x, w[0], w[1], w[2], geom, begin[1], begin[2], \
-                                   rows[0], rows[1], rows[2], late); break;
-            switch (nt | np << 8) {
-                LARQL_Q4K_SHORT(1, 1) LARQL_Q4K_SHORT(2, 1) LARQL_Q4K_SHORT(3, 1) LARQL_Q4K_SHORT(4, 1) LARQL_Q4K_SHORT(5, 1) LARQL_Q4K_SHORT(6, 1)
-                LARQL_Q4K_SHORT(7, 1) LARQL_Q4K_SHORT(8, 1) LARQL_Q4K_SHORT(1, 2) LARQL_Q4K_SHORT(2, 2) LARQL_Q4K_SHORT(3, 2) LARQL_Q4K_SHORT(4, 2)
-                LARQL_Q4K_SHORT(5, 2) LARQL_Q4K_SHORT(1, 3) LARQL_Q4K_SHORT(2, 3) LARQL_Q4K_SHORT(3, 3) LARQL_Q4K_SHORT(1, 4) LARQL_Q4K_SHORT(2, 4)
-                default: return hipErrorInvalidValue;
-            }
-#undef LARQL_Q4K_SHORT
-            break;
-        }
+        case KIND_SHORT: return gemv_short_launch(stream, L, threads, grid, lds);
         case KIND_Q4K_MFMA: {
             static std::atomic<bool> attr_set{false};  // dynamic LDS above 64 KB has to be allowed once per process
             if (!attr_set) {

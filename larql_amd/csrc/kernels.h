@@ -17,7 +17,7 @@ enum GemvKind : int32_t {
     KIND_Q4K_Q8K = 13,   // Q4_K weights against a Q8_K activation (integer dots on the matrix cores); x = the Q8_K device layout
     KIND_Q6K_Q8K = 14,   // Q6_K weights against a Q8_K activation (K-slice kernel, v_dot4)
     KIND_Q6K_MFMA = 15,  // internal: Q6_K rows short enough for the matrix-core kernel
-    KIND_Q4K_SHORT = 16  // internal: a launch of KIND_Q4K_MFMA jobs that leaves every compute unit a few tiles (gemv_q4k_short)
+    KIND_SHORT = 16      // internal: a launch of KIND_Q4K_MFMA or KIND_Q6K_MFMA jobs that leaves every compute unit a few tiles (gemv_short)
 };
 
 constexpr int kGemvMaxThreads = 512;
@@ -103,7 +103,7 @@ bool gemv_refine_costs(GemvJob *jobs, size_t n, uint32_t grid);
 uint32_t gemv_pick_threads(const GemvJob *jobs, size_t n);
 size_t gemv_lds_bytes(const GemvJob *jobs, size_t n, uint32_t threads);
 int gemv_effective_kind(const GemvJob &j);
-bool gemv_q4k_short(const GemvJob *jobs, size_t n, uint32_t cu_count, uint32_t *threads, uint32_t *grid, size_t *lds, uint32_t *param);
+bool gemv_short(const GemvJob *jobs, size_t n, uint32_t cu_count, uint32_t *threads, uint32_t *grid, size_t *lds, uint32_t *param);
 uint32_t gemv_batch_capacity(int kind, uint64_t k);  // activations one job may carry (1: no batched kernel for this shape)
 uint32_t gemv_launch_param(const GemvJob *jobs, size_t n);  // goes into GemvLaunch::pad
 uint32_t gemv_wgs_per_cu(int kind, uint32_t threads, size_t lds, uint32_t dflt);

@@ -2233,3 +2233,37 @@ def test_dense_gemv_multi_is_one_submission_of_the_single_calls(be, half):
     bad = list(mats[:3]) + [(mats[3][0][:-1], mats[3][1], k)]
     assert multi(bad, x) is None
     assert multi([(mats[0][0], shapes[0], k - 64)], x) is None            # k must equal x.len()
+
+
+@pytest.mark.parametrize("fmt_name,k", [("Q4_K", k) for k in (256, 2304, 2560, 3840, 7680, 10240)] +
+                         [("Q6_K", k) for k in (256, 768, 2304, 2560, 2816)])
+def test_short_launches_equal_the_streaming_kernel_bit_for_bit(be, fmt, fmt_name, k):
+    """One to four matvecs against one activation (the short kernel while they leave a compute unit a few tiles) and the same matvecs
+    among six (the streaming kernel): every row's additions are in the same order.  Row counts around the tiles of one and more
+    per compute unit, matvecs that end inside a workgroup's tiles, a single row; rows of one to forty super-blocks (a wavefront has one to
+    four of them; Q6_K: the short kernel up to ten)."""
+    f, block, enc = (fmt.FMT_Q4_K, 144, be.dev_quantize_q4_k) if fmt_name == "Q4_K" else (fmt.FMT_Q6_K, 210, be.dev_quantize_q6_k)
+    most = 9100
+    src, w, x = be.malloc(most * k * 4), be.malloc(most * (k // 256) * block + 64), be.malloc(k * 4)
+    be.dev_fill_normal(src, most * k, 1234 + k, 0.02)
+    assert enc(src, most * k, w)
+    be.dev_fill_normal(x, k, 77, 1.0)
+    outs = [be.malloc(most * 4) for _ in range(6)]
+    for sizes in [(1,), (17,), (2560,), (4096,), (4097,), (8200,), (2048, 1024, 1024), (3000, 5, 1300), (4500, 4500), (100, 1, 700, 2000),
+                  (1500, 2500, 2000, 2900)]:
+        first = np.cumsum([0] + [-(-r // 8) * 8 for r in sizes[:-1]])  # (matrices start at 16 bytes)
+        mats = [(f, w + int(a) * (k // 256) * block, None, x, r, k) for a, r in zip(first, sizes)]
+        got = []
+        for n in (len(sizes), 6):
+            for o in outs:
+                be.h2d(o, np.full(most, np.nan, F))
+            plan = be.plan_create([(*mats[i % len(mats)][:4], outs[i], *mats[i % len(mats)][4:]) for i in range(n)])
+            assert plan is not None, be.last_error()
+            assert be.plan_run(plan)
+            be.synchronize()
+            got.append([be.d2h(outs[i], sizes[i], F).view(np.uint32) for i in range(len(sizes))])
+            be.plan_destroy(plan)
+        for i, (a, b) in enumerate(zip(*got)):
+            assert np.array_equal(a, b), (sizes, i)
+    for p in [src, w, x] + outs:
+        be.free(p)
