@@ -325,7 +325,7 @@ int prepare_same_kind(larql_hip_ctx *c, GemvJob *live, size_t n_live, void *tabl
             uint32_t *first = (uint32_t *)(blob.data() + job_bytes);
             size_t ji = 0;
             for (uint64_t b = 0; b < grid; b++) {
-                const uint64_t pb = total * b / grid;
+                const uint64_t pb = total / grid * b + std::min<uint64_t>(b, total % grid);  // (as the kernels cut the passes)
                 while (ji + 1 < n_live && (uint64_t)live[ji + 1].pass_begin <= pb) ji++;
                 first[b] = (uint32_t)ji;
             }

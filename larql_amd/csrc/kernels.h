@@ -85,9 +85,15 @@ struct GemvJob {
 };
 static_assert(sizeof(GemvJob) % 16 == 0, "job tables are arrays of 16-byte words");
 
+struct GemvInline {
+    GemvJob job[kInlineJobs];
+    GemvJob &operator[](size_t i) { return job[i]; }
+    const GemvJob &operator[](size_t i) const { return job[i]; }
+};
+
 struct GemvLaunch {
     const GemvJob *table;  // device table, or null to use `inl`
-    GemvJob inl[kInlineJobs];
+    GemvInline inl;
     uint64_t total_passes;
     uint32_t n_jobs;
     uint32_t pad;

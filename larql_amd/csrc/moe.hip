@@ -155,7 +155,10 @@ __device__ __forceinline__ void write_job_table(const JobTableSpec &T, uint32_t 
         j.pass_begin = i * T.base.n_pass;
         T.jobs[i] = j;
     }
-    if (T.first && i < T.grid) T.first[i] = min((uint32_t)(T.total * i / T.grid) / T.base.n_pass, T.n_jobs - 1);
+    if (T.first && i < T.grid) {  // (as the kernels cut the passes)
+        const uint32_t total = (uint32_t)T.total, pass = total / T.grid * i + min(i, total % T.grid);
+        T.first[i] = min(pass / T.base.n_pass, T.n_jobs - 1);
+    }
 }
 
 __global__ void __launch_bounds__(256) moe_kq_route_quant_kernel(const float *__restrict__ logits, const float *__restrict__ bias, uint32_t n_experts, uint32_t k,
