@@ -28,6 +28,7 @@
 #include <algorithm>
 
 #include "kernels.h"
+#include "kq.h"
 #include "mx4.h"
 #include "router.h"
 
@@ -37,12 +38,6 @@ typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef float float2_t __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ half2_t as_half2(uint32_t u) { return __builtin_bit_cast(half2_t, u); }
-__device__ __forceinline__ float half_bits_to_float(uint32_t lo16) {
-    // hardware f16 -> f32 conversion; f16 subnormals are preserved (the f16
-    // denormal mode is on for HIP kernels), which the Q4_K scales rely on.
-    return (float)__builtin_bit_cast(_Float16, (uint16_t)lo16);
-}
-
 template <int CTRL>
 __device__ __forceinline__ float dpp_add(float v) {
     int moved = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true);
@@ -574,15 +569,11 @@ __device__ __forceinline__ void run_q4k(const GemvJob &j, uint32_t p0, uint32_t 
 // Row partials meet in LDS every kQ4kBatchTiles tiles: part[row][wave*4 + g],
 // folded in a fixed order that depends only on the row length.
 // ---------------------------------------------------------------------------
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-union Q4kOp { i32x4 v; uint32_t u[4]; };  // one MFMA operand: 16 int8 k-slots of a lane
 
 constexpr int kQ4kStages = 4;      // wave-tiles in flight per wavefront (ring slots of 2304 B)
 constexpr int kQ4kBatchTiles = 4;  // 16-row tiles between two folds of the row partials
 constexpr int kQ4kMaxColPasses = 4;
 constexpr int kQ4kMaxWaves = 10;  // with the ring, the partials and 4 prepared columns per wavefront this fills the 160 KB of LDS
-constexpr uint32_t kQ4kTileBytes = 16 * 144;
 constexpr uint32_t kQ4kColBytes = 1024 + 64;  // a column's digits (four planes of 256 bytes), then {2^(e-30), -, -, -, sums of its 8 sub-blocks}
 constexpr uint32_t kQ4kZeroBytes = 64;        // what the lanes outside an A row's group read
 

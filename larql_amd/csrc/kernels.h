@@ -212,6 +212,22 @@ hipError_t moe_group_launch(hipStream_t s, const MoeGroupArgs &A, bool down, uin
 hipError_t moe_route_terms_launch(hipStream_t s, const float *logits, const float *bias, uint32_t tokens, uint32_t n_experts, uint32_t k, int policy,
                                   uint32_t *experts, float *weights, const float *x, uint32_t hidden, uint16_t *terms);
 
+// The slots of a call through a bank of Q4_K experts against Q8_K activations (moe_kq_group.hip): `n_mats` matrices of one shape per
+// expert (gate and up, or down) in one launch, each read once per group of slots.
+struct MoeKqGroupArgs {
+    const uint32_t *experts;       // [slots], slot = token * k + rank; an id >= n_experts leaves its results as they are
+    uint32_t slots, n_experts, n_mats;
+    uint32_t rows, cols;           // of every matrix; columns in super-blocks of 256
+    uint32_t x_div;                // slot s reads the activation s / x_div
+    const uint8_t *w[2];           // expert 0's matrices; expert e's start e * w_stride bytes further on
+    uint64_t w_stride;
+    const uint8_t *x;              // Q8_K activations (q8k_bytes), x_stride bytes apart
+    uint64_t x_stride;
+    float *out[2];                 // [slots, rows] of each matrix
+};
+bool moe_kq_group_serves(uint32_t rows, uint32_t cols, uint32_t n_experts, uint32_t slots);
+hipError_t moe_kq_group_launch(hipStream_t s, const MoeKqGroupArgs &A, uint32_t cu_count);
+
 // MoE helpers
 constexpr uint32_t kRouterMaxExperts = 256;      // the selection kernels (four logits per lane)
 constexpr uint32_t kRouterInLaunchExperts = 64;  // a matvec launch that selects for itself (one logit per lane)

@@ -25,6 +25,7 @@
 #include <algorithm>
 #include <atomic>
 
+#include "expert_groups.h"
 #include "kernels.h"
 #include "mx4.h"
 #include "router.h"
@@ -58,44 +59,22 @@ __global__ void __launch_bounds__(512) moe_group_kernel(const MoeGroupArgs A) {
     float *part = reinterpret_cast<float *>(mg_lds + nw * (NS * slot_bytes));  // [2][R][nw][16 rows][TG tokens]
     const uint32_t part_floats = R * nw * 16 * TG;
     float *lbias = part + 2 * part_floats;                                    // [2][R * 16]: the biases of a batch's rows
-    uint32_t *cnt = reinterpret_cast<uint32_t *>(lbias + 2 * R * 16);         // slots per expert
-    uint32_t *before = cnt + nE;                                              // groups of the experts before; [nE]: all
-    uint16_t *list = reinterpret_cast<uint16_t *>(before + nE + 1);           // [2][16]: the slots of a group
-    uint16_t *ex = list + 32;                                                 // [slots]: the router's choice
+    ExpertGroups G;
+    G.cnt = reinterpret_cast<uint32_t *>(lbias + 2 * R * 16);
+    G.before = G.cnt + nE;
+    uint16_t *list = reinterpret_cast<uint16_t *>(G.before + nE + 1);         // [2][16]: the slots of a group
+    G.ex = list + 32;
     const uint32_t step0 = wv * CW;  // (below `steps`: the launch has no more wavefronts than K-ranges)
 
-    // 1. slots per expert, groups before each expert (an id outside the bank belongs to nobody)
-    for (uint32_t e = tid; e < nE; e += blockDim.x) cnt[e] = 0;
-    __syncthreads();
-    for (uint32_t s = tid; s < slots; s += blockDim.x) {
-        const uint32_t e = ((const GLOBAL_AS uint32_t *)A.experts)[s];
-        ex[s] = e < nE ? (uint16_t)e : (uint16_t)0xFFFFu;
-        if (e < nE) atomicAdd(&cnt[e], 1u);
-    }
-    __syncthreads();
-    if (wv == 0) {
-        uint32_t run = 0;
-        for (uint32_t base = 0; base < nE; base += 64) {
-            const uint32_t e = base + lane, g = e < nE ? (cnt[e] + TG - 1) / TG : 0u;
-            uint32_t incl = g;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const uint32_t t = (uint32_t)__shfl_up((int)incl, o, 64);
-                if (lane >= (uint32_t)o) incl += t;
-            }
-            if (e < nE) before[e] = run + incl - g;
-            run += (uint32_t)__shfl((int)incl, 63, 64);
-        }
-        if (lane == 0) before[nE] = run;
-    }
-    __syncthreads();
+    // 1. slots per expert, groups before each expert
+    expert_groups_count<TG>(G, A.experts, slots, nE, tid, lane, wv);
 
     // 2. this workgroup's share of the list (group, 16-row tile).  Workgroups are dealt to the eight XCDs in turn: an XCD
     //    takes neighbouring shares, whose groups' operands then sit in its L2.
     //    A group opens with kStart units of its own: who meets a second group in its share starts twice (list, operands, first
     //    tiles), so it gets that many tiles fewer.
-        constexpr uint32_t kStart = TG == 16 ? 6 : 4;
-    const uint32_t per_group = tpm + kStart, units = before[nE] * per_group, grid = gridDim.x;
+    constexpr uint32_t kStart = TG == 16 ? 6 : 4;
+    const uint32_t per_group = tpm + kStart, units = G.before[nE] * per_group, grid = gridDim.x;
     const uint32_t share = (grid & 7u) ? blockIdx.x : (blockIdx.x & 7u) * (grid >> 3) + (blockIdx.x >> 3);
     uint32_t v = (uint32_t)((uint64_t)units * share / grid);
     const uint32_t v_end = (uint32_t)((uint64_t)units * (share + 1) / grid);
@@ -121,14 +100,8 @@ __global__ void __launch_bounds__(512) moe_group_kernel(const MoeGroupArgs A) {
         v += a1 - a0;
         if (a1 <= kStart) continue;
         const uint32_t t0 = max(a0, kStart) - kStart, nt = a1 - kStart - t0;
-        uint32_t e = 0;
-        for (uint32_t base = 0; base < nE; base += 64) {
-            const uint32_t q = base + lane;
-            const uint64_t m = __ballot(q < nE && before[min(q, nE)] <= gi && gi < before[min(q + 1, nE)]);
-            if (m) { e = base + (uint32_t)__builtin_ctzll(m); break; }
-        }
-        e = __builtin_amdgcn_readfirstlane(e);
-        const uint32_t lo = (gi - before[e]) * TG, ntok = min(cnt[e] - lo, (uint32_t)TG);
+        const uint32_t e = expert_of_group(G, nE, gi, lane);
+        const uint32_t lo = (gi - G.before[e]) * TG, ntok = min(G.cnt[e] - lo, (uint32_t)TG);
 
         // 3. the first tiles leave
         const uint8_t *wp = mat + (size_t)e * A.w_stride + (size_t)(t0 * tile_rows + lane_row) * row_bytes;
@@ -154,18 +127,7 @@ __global__ void __launch_bounds__(512) moe_group_kernel(const MoeGroupArgs A) {
         // 4. the group's slots: those of rank lo .. lo+TG-1 among the expert's, in slot order (every wavefront finds them
         //    for itself and writes the same list)
         uint16_t *const gl = list + lpar * 16;
-        {
-            uint32_t run = 0;
-            for (uint32_t base = 0; base < slots; base += 64) {
-                const bool is = base + lane < slots && ex[min(base + lane, slots - 1)] == e;
-                const uint64_t m = __ballot(is);
-                const uint32_t rank = run + (uint32_t)__popcll(m & ((1ull << lane) - 1ull)) - lo;
-                if (is && rank < (uint32_t)TG) gl[rank] = (uint16_t)(base + lane);
-                run += (uint32_t)__popcll(m);
-                if (run >= lo + TG) break;
-            }
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        expert_group_slots<TG>(G, slots, e, lo, gl, lane);
 
         // 5. the A operands of the wavefront's K-range
         BfOp a[NT][CW][4];

@@ -2267,3 +2267,14 @@ def test_short_launches_equal_the_streaming_kernel_bit_for_bit(be, fmt, fmt_name
             assert np.array_equal(a, b), (sizes, i)
     for p in [src, w, x] + outs:
         be.free(p)
+
+
+@pytest.mark.parametrize("T,E,k,hidden,cols,inter", [
+    (9, 1, 1, 272, 512, 300),      # one expert with nine slots: a group of eight and one of one; ragged last tiles of gate and up
+    (16, 2, 2, 256, 256, 17),      # two full groups per expert; a tile and one row, rows of one super-block
+    (3, 4, 4, 1040, 3072, 40),     # twelve super-blocks: the most that the grouped kernel takes
+    (2, 4, 2, 256, 3328, 48),      # thirteen: a matvec per slot
+])
+@pytest.mark.parametrize("wfmt", ["q4k", "q6k"])
+def test_moe_layer_k_quant_slots_share_an_expert(be, fmt, T, E, k, hidden, cols, inter, wfmt):
+    test_moe_layer_over_a_k_quant_bank_matches_the_integer_expert_path(be, fmt, T, E, k, hidden, cols, inter, wfmt, 1, True, False)
