@@ -1974,7 +1974,7 @@ static int moe_mxfp4_block(larql_hip_ctx *c, const larql_hip_mxfp4_experts *bank
             b.out = d;
             HIPCHECK(c, moe_group_launch(c->stream, a, false, (uint32_t)c->cu_count));
             HIPCHECK(c, moe_group_launch(c->stream, b, true, (uint32_t)c->cu_count));
-            HIPCHECK(c, weighted_sum_launch(c->stream, d, weights + s0, experts + s0, (uint32_t)bank->n_experts, out + t0 * hidden, (uint32_t)nt,
+            HIPCHECK(c, weighted_sum_launch(c->stream, d, weights + s0, experts + s0, (uint32_t)bank->n_experts, nullptr, out + t0 * hidden, (uint32_t)nt,
                                             (uint32_t)k, (uint32_t)hidden));
         }
         return LARQL_OK;
@@ -2035,7 +2035,7 @@ static int moe_mxfp4_block(larql_hip_ctx *c, const larql_hip_mxfp4_experts *bank
     }
     rc = enqueue_jobs(c, jobs);
     if (rc) return rc;
-    HIPCHECK(c, weighted_sum_launch(c->stream, d, weights, experts, (uint32_t)bank->n_experts, out, (uint32_t)tokens, (uint32_t)k, (uint32_t)hidden));
+    HIPCHECK(c, weighted_sum_launch(c->stream, d, weights, experts, (uint32_t)bank->n_experts, nullptr, out, (uint32_t)tokens, (uint32_t)k, (uint32_t)hidden));
     return LARQL_OK;
 }
 
@@ -2349,7 +2349,7 @@ static int moe_layer_enqueue(larql_hip_ctx *c, larql_hip_moe_layer *L, const flo
             b.x = aq; b.x_stride = aq_stride;
             b.out[0] = dd;
             HIPCHECK(c, moe_kq_group_launch(c->stream, b, (uint32_t)c->cu_count));
-            HIPCHECK(c, weighted_sum_bias_launch(c->stream, dd, weights, experts, (uint32_t)E, L->kq_db, out, (uint32_t)tokens, (uint32_t)k, (uint32_t)hidden));
+            HIPCHECK(c, weighted_sum_launch(c->stream, dd, weights, experts, (uint32_t)E, L->kq_db, out, (uint32_t)tokens, (uint32_t)k, (uint32_t)hidden));
             return LARQL_OK;
         }
         std::vector<GemvJob> down;
@@ -2403,7 +2403,7 @@ static int moe_layer_enqueue(larql_hip_ctx *c, larql_hip_moe_layer *L, const flo
                                               L->glu_limit, L->glu_alpha, aq, aq_stride));
             HIPCHECK(c, gemv_launch(c->stream, P[1].kind, P[1].L, P[1].threads, P[1].grid, P[1].lds));
         }
-        HIPCHECK(c, weighted_sum_bias_launch(c->stream, dd, weights, experts, (uint32_t)E, L->kq_db, out, (uint32_t)tokens, (uint32_t)k, (uint32_t)hidden));
+        HIPCHECK(c, weighted_sum_launch(c->stream, dd, weights, experts, (uint32_t)E, L->kq_db, out, (uint32_t)tokens, (uint32_t)k, (uint32_t)hidden));
         return LARQL_OK;
     }
     if (!L->per_expert_scale) return moe_mxfp4_block(c, &L->bank, x, tokens, k, experts, weights, out, L->ws.p, wsb, logits, policy);

@@ -262,9 +262,7 @@ hipError_t moe_kq_route_quant_launch(hipStream_t s, const float *logits, const f
 hipError_t pad_rows_f32_launch(hipStream_t s, const float *src, size_t src_stride, uint32_t src_cols, uint32_t cols, uint32_t rows, float *dst);
 hipError_t moe_act_f32_launch(hipStream_t s, const float *g, const float *u, uint32_t inter, uint32_t slots, const uint32_t *experts, uint32_t n_experts,
                               const float *gub, int rule, float limit, float alpha, float *act, size_t act_stride);
-hipError_t weighted_sum_bias_launch(hipStream_t s, const float *d, const float *weights, const uint32_t *experts, uint32_t n_experts,
-                                    const float *bias, float *out, uint32_t tokens, uint32_t k, uint32_t hidden);
-hipError_t weighted_sum_launch(hipStream_t s, const float *d, const float *weights, const uint32_t *experts, uint32_t n_experts, float *out,
+hipError_t weighted_sum_launch(hipStream_t s, const float *d, const float *weights, const uint32_t *experts, uint32_t n_experts, const float *bias, float *out,
                                uint32_t tokens, uint32_t k, uint32_t hidden);
 
 }  // namespace larql

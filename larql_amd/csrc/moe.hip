@@ -64,26 +64,36 @@ __global__ void expert_scale_kernel(float *__restrict__ weights, const uint32_t 
     if (e < n_scale) weights[i] *= scale[e];
 }
 
-// out[t] = sum over the token's k selected experts, in selection order, of w * down-output
-// (larql-compute/src/cpu/ops/moe/forward.rs:266-270).  A slot whose expert id lies outside the bank is skipped
-// (forward.rs:203-208): its rows of `d` were never written and are not read.
-__global__ void weighted_sum_kernel(const float *__restrict__ d, const float *__restrict__ weights, const uint32_t *__restrict__ experts,
-                                    uint32_t n_experts, float *__restrict__ out, uint32_t k, uint32_t hidden) {
-    const uint32_t t = blockIdx.y;
+// out[t] = sum over the token's k slots, in selection order, of w * (down output + the expert's down bias, where there is one)
+// (larql-compute/src/cpu/ops/moe/forward.rs:220-228, 266-270: add_down_bias, then `*a += w * v`).  A slot whose expert id lies
+// outside the bank adds nothing (forward.rs:203-208): its row of `d` holds nothing, and its bias is the bank's first.
+// Bound: latency.  K is the number of slots (0: any, four at a time), so that the ids and weights come in one scalar read each and
+// all rows of `d` are asked for together.
+template <int K, bool BIAS>
+__global__ void __launch_bounds__(256) weighted_sum_kernel(const float *__restrict__ d, const float *__restrict__ weights, const uint32_t *__restrict__ experts,
+                                                          float *__restrict__ out, uint32_t n_experts, uint32_t k_any, uint32_t hidden,
+                                                          const float *__restrict__ bias) {
+    const uint32_t t = blockIdx.y, k = K ? (uint32_t)K : k_any;
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= hidden) return;
+    constexpr int C = K ? K : 4;
     float acc = 0.0f;
-    for (uint32_t r0 = 0; r0 < k; r0 += 4) {  // four loads in flight, added in selection order
-        float w[4], v[4];
+    for (uint32_t r0 = 0; r0 < k; r0 += C) {
+        uint32_t e[C];
+        float w[C], v[C];
 #pragma unroll
-        for (uint32_t q = 0; q < 4; q++) {
-            const bool in = r0 + q < k && experts[(size_t)t * k + r0 + q] < n_experts;
-            w[q] = in ? weights[(size_t)t * k + r0 + q] : 0.0f;
-            v[q] = in ? d[((size_t)t * k + r0 + q) * hidden + i] : 0.0f;
+        for (int q = 0; q < C; q++) {
+            const size_t s = (size_t)t * k + (K ? (uint32_t)q : min(r0 + q, k - 1));
+            e[q] = experts[s];
+            w[q] = weights[s];
+            v[q] = d[s * hidden + i];
         }
 #pragma unroll
-        for (uint32_t q = 0; q < 4; q++)
-            if (r0 + q < k && experts[(size_t)t * k + r0 + q] < n_experts) acc += w[q] * v[q];
+        for (int q = 0; q < C; q++) {
+            if (BIAS) v[q] += bias[(size_t)(e[q] < n_experts ? e[q] : 0u) * hidden + i];
+            const float with = acc + w[q] * v[q];
+            acc = (K || r0 + q < k) && e[q] < n_experts ? with : acc;
+        }
     }
     out[(size_t)t * hidden + i] = acc;
 }
@@ -99,17 +109,25 @@ __device__ __forceinline__ int q8k_code(float t) {
     return r != r ? 0 : (int)r;
 }
 __device__ __forceinline__ void q8k_block(const float (&v)[4], uint32_t &codes, float &scale, int &sum) {
-    float amax = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));  // fmaxf ignores a NaN operand, as f32::max does
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
+    const float amax = wave_fmax(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));  // fmaxf ignores a NaN operand, as f32::max does
     scale = amax > 0.0f ? amax / 127.0f : 0.0f;
     const float inv = scale > 0.0f ? 1.0f / scale : 0.0f;
     const int q0 = q8k_code(v[0] * inv), q1 = q8k_code(v[1] * inv), q2 = q8k_code(v[2] * inv), q3 = q8k_code(v[3] * inv);
     sum = q0 + q1 + q2 + q3;
-    sum += __shfl_xor(sum, 1);
-    sum += __shfl_xor(sum, 2);
-    sum += __shfl_xor(sum, 4);
+    sum += __builtin_amdgcn_update_dpp(0, sum, 0xB1, 0xF, 0xF, true);   // quad_perm [1,0,3,2]
+    sum += __builtin_amdgcn_update_dpp(0, sum, 0x4E, 0xF, 0xF, true);   // quad_perm [2,3,0,1]
+    sum += __builtin_amdgcn_update_dpp(0, sum, 0x141, 0xF, 0xF, true);  // row_half_mirror: the other quad of the eight
     codes = ((uint32_t)q0 & 0xFFu) | (((uint32_t)q1 & 0xFFu) << 8) | (((uint32_t)q2 & 0xFFu) << 16) | (((uint32_t)q3 & 0xFFu) << 24);
+}
+// four elements of a row of `n` floats from j on, zeros past its end; `vec`: every row starts at 16 bytes and n % 4 == 0
+__device__ __forceinline__ void load4(float (&v)[4], const float *row, uint32_t j, uint32_t n, bool vec) {
+    if (vec) {
+        const float4 f = j < n ? *reinterpret_cast<const float4 *>(row + j) : make_float4(0.f, 0.f, 0.f, 0.f);
+        v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
+    } else {
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) v[i] = j + i < n ? row[j + i] : 0.0f;
+    }
 }
 // the device layout of a Q8_K activation of `cols` elements at `o`: [cols codes | cols/256 f32 scales | cols/32 i16 sums]
 __device__ __forceinline__ void q8k_store(uint8_t *o, uint32_t cols, uint32_t sb, uint32_t lane, uint32_t codes, float scale, int sum) {
@@ -138,10 +156,12 @@ __global__ void __launch_bounds__(256) quantize_rows_to_q8k_kernel(const float *
 
 // Token `blockIdx.x`'s route and its expert input in one launch (they do not depend on one another): wavefront 0 selects
 // as router_select_kernel does and applies MoeExpertScalePolicy::PerExpert where a scale table is given (as
-// expert_scale_kernel does); the four wavefronts then quantise the token's row as quantize_rows_to_q8k_kernel does.
+// expert_scale_kernel does) while the others, a wavefront per super-block up to eleven, quantise the token's row as
+// quantize_rows_to_q8k_kernel does (four wavefronts, the first of them after its selection: 9.0 -> 6.1 us for 16 tokens of 2816).
 // The workgroups behind the tokens write the job tables of the two matvec launches that follow, a thread per job and per share:
 // they are uniform, so the host need not build and upload them (two copies of 70 and 35 KB that the stream waited for,
 // 22 us each in a layer of 150 us with 16 tokens, 128 experts and top-8, now 107 us).
+constexpr uint32_t kRouteQuantWaves = 12;
 struct JobTables { JobTableSpec t[2]; };
 __device__ __forceinline__ void write_job_table(const JobTableSpec &T, uint32_t i) {
     if (!T.jobs) return;
@@ -161,7 +181,7 @@ __device__ __forceinline__ void write_job_table(const JobTableSpec &T, uint32_t 
     }
 }
 
-__global__ void __launch_bounds__(256) moe_kq_route_quant_kernel(const float *__restrict__ logits, const float *__restrict__ bias, uint32_t n_experts, uint32_t k,
+__global__ void __launch_bounds__(kRouteQuantWaves * 64) moe_kq_route_quant_kernel(const float *__restrict__ logits, const float *__restrict__ bias, uint32_t n_experts, uint32_t k,
                                                                 int policy, const float *__restrict__ scale, uint32_t *__restrict__ experts,
                                                                 float *__restrict__ weights, const float *__restrict__ src, size_t src_stride,
                                                                 uint32_t src_cols, uint32_t cols, uint8_t *__restrict__ dst, size_t dst_stride, uint32_t tokens,
@@ -188,15 +208,15 @@ __global__ void __launch_bounds__(256) moe_kq_route_quant_kernel(const float *__
         }
     }
     const float *s = src + (size_t)t * src_stride;
-    for (uint32_t sb = wave; sb < cols / 256; sb += 4) {
-        const uint32_t j = sb * 256 + 4 * lane;
-        float v[4];
-#pragma unroll
-        for (uint32_t i = 0; i < 4; i++) v[i] = j + i < src_cols ? s[j + i] : 0.0f;
-        uint32_t codes; float sc; int sum;
-        q8k_block(v, codes, sc, sum);
-        q8k_store(dst + (size_t)t * dst_stride, cols, sb, lane, codes, sc, sum);
-    }
+    const bool vec = ((src_stride | src_cols) & 3u) == 0 && ((uintptr_t)src & 15u) == 0;
+    if (wave > 0)
+        for (uint32_t sb = wave - 1; sb < cols / 256; sb += (blockDim.x >> 6) - 1) {
+            float v[4];
+            load4(v, s, sb * 256 + 4 * lane, src_cols, vec);
+            uint32_t codes; float sc; int sum;
+            q8k_block(v, codes, sc, sum);
+            q8k_store(dst + (size_t)t * dst_stride, cols, sb, lane, codes, sc, sum);
+        }
 }
 
 // Row `blockIdx.y` of src ([rows, src_cols] floats, src_stride apart) zero-padded to `cols` floats at dst + row * cols:
@@ -241,16 +261,17 @@ __global__ void __launch_bounds__(256) moe_kq_act_q8k_kernel(const float *__rest
     const uint32_t e = experts[slot];
     const float *b = (gub && e < n_experts) ? gub + (size_t)e * 2 * inter : nullptr;
     const uint32_t j = sb * 256 + 4 * lane;
-    float v[4];
-#pragma unroll
-    for (uint32_t i = 0; i < 4; i++) {
-        v[i] = 0.0f;
-        if (j + i < inter) {
-            const float gv = g[(size_t)slot * inter + j + i] + (b ? b[2 * (j + i)] : 0.0f);
-            const float uv = u[(size_t)slot * inter + j + i] + (b ? b[2 * (j + i) + 1] : 0.0f);
-            v[i] = moe_combine(rule, gv, uv, limit, alpha);
-        }
+    const bool vec = (inter & 3u) == 0 && (((uintptr_t)g | (uintptr_t)u | (uintptr_t)gub) & 15u) == 0;
+    float v[4], gv[4], uv[4], b0[4] = {0.f, 0.f, 0.f, 0.f}, b1[4] = {0.f, 0.f, 0.f, 0.f};
+    load4(gv, g + (size_t)slot * inter, j, inter, vec);
+    load4(uv, u + (size_t)slot * inter, j, inter, vec);
+    if (b) {
+        load4(b0, b, 2 * j, 2 * inter, vec);
+        load4(b1, b, 2 * j + 4, 2 * inter, vec);
     }
+    const float bias[8] = {b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[3]};
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++) v[i] = j + i < inter ? moe_combine(rule, gv[i] + bias[2 * i], uv[i] + bias[2 * i + 1], limit, alpha) : 0.0f;
     uint32_t codes; float scale; int sum;
     q8k_block(v, codes, scale, sum);
     q8k_store(dst + (size_t)slot * dst_stride, inter_padded, sb, lane, codes, scale, sum);
@@ -268,24 +289,6 @@ __global__ void __launch_bounds__(256) moe_act_f32_kernel(const float *__restric
     const float gv = g[(size_t)slot * inter + j] + (b ? b[2 * j] : 0.0f);
     const float uv = u[(size_t)slot * inter + j] + (b ? b[2 * j + 1] : 0.0f);
     act[(size_t)slot * act_stride + j] = moe_combine(rule, gv, uv, limit, alpha);
-}
-
-// out[t] = sum over the token's k slots, in selection order, of w * (down output + the expert's down bias)
-// (forward.rs:220-228: add_down_bias, then `*a += w * v`); a slot whose expert lies outside the bank is skipped.
-__global__ void weighted_sum_bias_kernel(const float *__restrict__ d, const float *__restrict__ weights, const uint32_t *__restrict__ experts,
-                                         uint32_t n_experts, const float *__restrict__ bias, float *__restrict__ out, uint32_t k, uint32_t hidden) {
-    const uint32_t t = blockIdx.y;
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= hidden) return;
-    float acc = 0.0f;
-    for (uint32_t r = 0; r < k; r++) {
-        const uint32_t e = experts[(size_t)t * k + r];
-        if (e >= n_experts) continue;
-        float v = d[((size_t)t * k + r) * hidden + i];
-        if (bias) v += bias[(size_t)e * hidden + i];
-        acc += weights[(size_t)t * k + r] * v;
-    }
-    out[(size_t)t * hidden + i] = acc;
 }
 
 hipError_t router_select_launch(hipStream_t s, const float *logits, const float *bias, uint32_t tokens, uint32_t n_experts, uint32_t k,
@@ -333,7 +336,8 @@ hipError_t moe_kq_route_quant_launch(hipStream_t s, const float *logits, const f
     uint32_t writers = 0;
     for (const JobTableSpec &t : T.t)
         if (t.jobs) writers = std::max(writers, std::max(t.n_jobs, t.first ? t.grid : 0u));
-    hipLaunchKernelGGL(moe_kq_route_quant_kernel, dim3(tokens + (writers + 255) / 256), dim3(256), 0, s, logits, bias, n_experts, k, policy, scale, experts, weights, src,
+    const uint32_t threads = 64 * std::min(kRouteQuantWaves, 1 + cols / 256);
+    hipLaunchKernelGGL(moe_kq_route_quant_kernel, dim3(tokens + (writers + threads - 1) / threads), dim3(threads), 0, s, logits, bias, n_experts, k, policy, scale, experts, weights, src,
                        src_stride, src_cols, cols, dst, dst_stride, tokens, T);
     return hipGetLastError();
 }
@@ -349,17 +353,23 @@ hipError_t moe_act_f32_launch(hipStream_t s, const float *g, const float *u, uin
                        act, act_stride);
     return hipGetLastError();
 }
-hipError_t weighted_sum_bias_launch(hipStream_t s, const float *d, const float *weights, const uint32_t *experts, uint32_t n_experts,
-                                    const float *bias, float *out, uint32_t tokens, uint32_t k, uint32_t hidden) {
-    if (tokens == 0 || hidden == 0) return hipSuccess;
-    hipLaunchKernelGGL(weighted_sum_bias_kernel, dim3((hidden + 255) / 256, tokens), dim3(256), 0, s, d, weights, experts, n_experts, bias, out, k, hidden);
-    return hipGetLastError();
-}
-
-hipError_t weighted_sum_launch(hipStream_t s, const float *d, const float *weights, const uint32_t *experts, uint32_t n_experts, float *out,
+hipError_t weighted_sum_launch(hipStream_t s, const float *d, const float *weights, const uint32_t *experts, uint32_t n_experts, const float *bias, float *out,
                                uint32_t tokens, uint32_t k, uint32_t hidden) {
     if (tokens == 0 || hidden == 0) return hipSuccess;
-    hipLaunchKernelGGL(weighted_sum_kernel, dim3((hidden + 255) / 256, tokens), dim3(256), 0, s, d, weights, experts, n_experts, out, k, hidden);
+    const dim3 grid((hidden + 255) / 256, tokens);
+#define LARQL_WSUM(K) \
+    if (bias) hipLaunchKernelGGL((weighted_sum_kernel<K, true>), grid, dim3(256), 0, s, d, weights, experts, out, n_experts, k, hidden, bias); \
+    else hipLaunchKernelGGL((weighted_sum_kernel<K, false>), grid, dim3(256), 0, s, d, weights, experts, out, n_experts, k, hidden, bias)
+    switch (k) {
+        case 1: LARQL_WSUM(1); break;
+        case 2: LARQL_WSUM(2); break;
+        case 3: LARQL_WSUM(3); break;
+        case 4: LARQL_WSUM(4); break;
+        case 6: LARQL_WSUM(6); break;
+        case 8: LARQL_WSUM(8); break;
+        default: LARQL_WSUM(0);
+    }
+#undef LARQL_WSUM
     return hipGetLastError();
 }
 

@@ -261,22 +261,24 @@ __global__ void __launch_bounds__(512) moe_group_kernel(const MoeGroupArgs A) {
     LARQL_WAIT_VMCNT(0);
 }
 
-// Token `blockIdx.x`'s selection (with `logits`: Router::select by wavefront 0) and its activation as three bf16 terms,
-// terms[term][token][moe_terms_pad(hidden)].
-__global__ void __launch_bounds__(256) moe_route_terms_kernel(const float *__restrict__ logits, const float *__restrict__ bias, uint32_t n_experts,
-                                                             uint32_t k, int policy, uint32_t *__restrict__ experts, float *__restrict__ weights,
-                                                             const float *__restrict__ x, uint32_t hidden, uint16_t *__restrict__ terms) {
+// Token `blockIdx.x`'s selection (with `logits`: Router::select by wavefront 0) and, by the other four wavefronts beside it, its
+// activation as three bf16 terms, terms[term][token][moe_terms_pad(hidden)].  (The selection behind its wavefront's share of the
+// terms: 6.1 us for 128 tokens of 2880, so 4.8.)
+__global__ void __launch_bounds__(320) moe_route_terms_kernel(const float *__restrict__ logits, const float *__restrict__ bias, uint32_t n_experts,
+                                                             uint32_t k, int policy, uint32_t tokens, uint32_t *__restrict__ experts,
+                                                             float *__restrict__ weights, const float *__restrict__ x, uint16_t *__restrict__ terms, uint32_t hidden) {
     const uint32_t t = blockIdx.x, lane = threadIdx.x & 63u;
-    const size_t pad = moe_terms_pad(hidden), plane = gridDim.x * pad;
-    for (uint32_t i = threadIdx.x * 4; i < hidden; i += blockDim.x * 4) {  // (hidden % 32 == 0)
-        const f32x4 v = *reinterpret_cast<const f32x4 *>(x + (size_t)t * hidden + i);
-        uint32_t a[3], b[3];
-        mx4_terms(v.x, v.y, a);
-        mx4_terms(v.z, v.w, b);
+    if (threadIdx.x >= 64) {
+        const size_t pad = moe_terms_pad(hidden), plane = tokens * pad;
+        for (uint32_t i = (threadIdx.x - 64) * 4; i < hidden; i += 1024) {  // (hidden % 32 == 0)
+            const f32x4 v = *reinterpret_cast<const f32x4 *>(x + (size_t)t * hidden + i);
+            uint32_t a[3], b[3];
+            mx4_terms(v.x, v.y, a);
+            mx4_terms(v.z, v.w, b);
 #pragma unroll
-        for (int q = 0; q < 3; q++) *reinterpret_cast<uint2 *>(terms + q * plane + t * pad + moe_term_at(i)) = make_uint2(a[q], b[q]);
-    }
-    if (logits && threadIdx.x < 64) {
+            for (int q = 0; q < 3; q++) *reinterpret_cast<uint2 *>(terms + q * plane + t * pad + moe_term_at(i)) = make_uint2(a[q], b[q]);
+        }
+    } else if (logits) {
         uint32_t sel_idx[kRouterMaxK];
         float sel_w[kRouterMaxK];
         router_select_any(logits + (size_t)t * n_experts, bias, n_experts, k, policy, lane, sel_idx, sel_w);
@@ -293,7 +295,7 @@ __global__ void __launch_bounds__(256) moe_route_terms_kernel(const float *__res
 
 hipError_t moe_route_terms_launch(hipStream_t s, const float *logits, const float *bias, uint32_t tokens, uint32_t n_experts, uint32_t k, int policy,
                                   uint32_t *experts, float *weights, const float *x, uint32_t hidden, uint16_t *terms) {
-    hipLaunchKernelGGL(moe_route_terms_kernel, dim3(tokens), dim3(256), 0, s, logits, bias, n_experts, k, policy, experts, weights, x, hidden, terms);
+    hipLaunchKernelGGL(moe_route_terms_kernel, dim3(tokens), dim3(320), 0, s, logits, bias, n_experts, k, policy, tokens, experts, weights, x, terms, hidden);
     return hipGetLastError();
 }
 
