@@ -20,16 +20,14 @@
 // wavefront orders them best-first with a bitonic sort done by cross-lane
 // shuffles.  Cost is a handful of passes over the row, whatever its order.
 // Rows of up to 16384 scores (every gate matrix) are read once: a thread keeps
-// its up to 16 ordered scores in registers, and a bound with at least 64 scores
-// at or above it (the smallest maximum of 64 slices of the row) usually leaves
-// a few hundred candidates, which are ranked directly; the radix passes remain
-// for rows with more than 1024 candidates.
+// its up to 16 ordered scores in registers, and for K up to 256 a bound with at
+// least K scores at or above it (the K-th largest maximum of 128 slices of the
+// row, of 512 for K above 64) leaves little more than K candidates, which are
+// ranked directly; the radix passes remain for rows with more than 1024 of them.
 // Longer rows (a vocabulary) are selected in two launches: every chunk of a row
 // leaves its own K best keys, sorted, in a workspace, and one workgroup per row
 // selects among those.  One workgroup cannot keep enough loads in flight for a
-// 262144-score row (405 us on one CU, six passes over 1 MB); 64 chunks of 4096
-// plus the merge of their 64 x 64 keys take 18 us together (the lm_head call over
-// 262144 x 2560: 562 -> 174 us).
+// 262144-score row (405 us on one CU, six passes over 1 MB).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -83,6 +81,16 @@ __device__ __forceinline__ uint64_t sort_desc(uint64_t key, uint32_t lane) {
     return key;
 }
 
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true));   // quad_perm [1,0,3,2]
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true));   // quad_perm [2,3,0,1]
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, true));  // row_half_mirror
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, true));  // row_mirror
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false)); // row_bcast:15 into rows 1 and 3
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false)); // row_bcast:31 into rows 2 and 3
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
 template <bool BY_ABS>
 __device__ __forceinline__ uint64_t make_key(float s, uint32_t idx, int *nan_flag) {
     const uint32_t bits = __builtin_bit_cast(uint32_t, s);
@@ -99,7 +107,8 @@ __device__ __forceinline__ uint64_t make_key(float s, uint32_t idx, int *nan_fla
 }
 
 constexpr int kTopkCached = 16;  // rounds of 64 scores per wavefront held in registers
-constexpr int kTopkCandidates = kTopkThreads;  // candidates of the short way: one per thread
+constexpr int kTopkCandidates = 1024;  // of the short way
+constexpr uint32_t kTopkShortK = 256;   // winners that the short way bounds
 
 // What a workgroup selects from: `n` scores of a row, cut into chunks of `chunk` (chunk == n: the whole row), or — KEYS_IN —
 // the row's `n` keys that the chunks' workgroups left.  A chunk's workgroup leaves keys (KEYS_OUT): its K best, best
@@ -113,6 +122,7 @@ struct TopkArgs {
     uint32_t *count_out;
     int *nan_flag;
     uint32_t scores_n, n, chunk, k, cap;
+    uint32_t by_value;         // (a score then comes out of its key)
 };
 
 // ROUNDS: scores per thread held in registers (0: streamed on every pass).
@@ -124,15 +134,16 @@ struct TopkArgs {
 // until half of the first one's wavefronts had left — more rows than CUs then ran in two rounds)
 template <bool BY_ABS, int ROUNDS, bool LARGE, bool KEYS_IN, bool KEYS_OUT>
 __global__ void __launch_bounds__(kTopkThreads) __attribute__((amdgpu_num_sgpr(80))) topk_kernel(const TopkArgs A) {
-    constexpr bool CACHED = ROUNDS > 0, SHORT_WAY = CACHED && !LARGE;  // (the candidate short cut bounds 64 winners only)
+    constexpr bool CACHED = ROUNDS > 0, SHORT_WAY = CACHED;
+    constexpr int GROUPS = LARGE ? 512 : 128, PL = GROUPS / 64;  // slices of the row that bound the K-th score; maxima per lane
     extern __shared__ __attribute__((aligned(16))) uint64_t big[];  // LARGE: cap keys
     __shared__ uint32_t hist[256];
     __shared__ uint32_t wave_ties[kTopkWaves];
     __shared__ uint64_t winners[64];
     __shared__ uint32_t sh_prefix, sh_need, sh_nwin, sh_ncand;
-    __shared__ uint32_t group_max[64];
-    __shared__ __attribute__((aligned(16))) uint64_t cand[SHORT_WAY ? kTopkCandidates + 4 : 1];
-    __shared__ uint32_t rank_sh[SHORT_WAY ? kTopkCandidates : 1];  // ranks counted in shares (short way)
+    __shared__ uint32_t group_max[SHORT_WAY ? GROUPS : 1];
+    __shared__ __attribute__((aligned(16))) uint64_t cand[SHORT_WAY ? kTopkCandidates : 1];
+    __shared__ float cand_score[SHORT_WAY && BY_ABS && !KEYS_OUT ? kTopkCandidates : 1];  // (by |score| a key has lost the sign)
     const uint32_t row = blockIdx.y, tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t k = A.k, cap = A.cap, first = blockIdx.x * A.chunk, n = min(A.chunk, A.n - first);
     int *const nan_flag = A.nan_flag;
@@ -145,17 +156,23 @@ __global__ void __launch_bounds__(kTopkThreads) __attribute__((amdgpu_num_sgpr(8
     const uint32_t w0 = min(n, wave * perw), w1 = min(n, w0 + perw);
 
     // winner number `rank` of the row (or of the chunk)
-    auto emit = [&](uint32_t rank, uint64_t key) {
+    auto put = [&](uint32_t rank, uint64_t key, float score) {
         if (KEYS_OUT) {
             kout[rank] = key;
         } else {
-            const uint32_t idx = ~(uint32_t)key;
-            A.idx_out[(size_t)row * k + rank] = idx;
-            A.val_out[(size_t)row * k + rank] = srow[idx];
+            A.idx_out[(size_t)row * k + rank] = ~(uint32_t)key;
+            A.val_out[(size_t)row * k + rank] = score;
         }
+    };
+    auto emit = [&](uint32_t rank, uint64_t key) {
+        const uint32_t ord = (uint32_t)(key >> 32);
+        if (KEYS_OUT) put(rank, key, 0.f);
+        else if (A.by_value) put(rank, key, __builtin_bit_cast(float, (ord & 0x80000000u) ? ord & 0x7FFFFFFFu : ~ord));
+        else put(rank, key, srow[~(uint32_t)key]);
     };
     // index i as a key: its ordered score (0: nothing there) and the low word, from the register copy or from memory
     uint32_t cache[CACHED ? ROUNDS : 1], low[KEYS_IN && CACHED ? ROUNDS : 1];
+    float raw[CACHED ? ROUNDS : 1];
     if (CACHED && KEYS_IN) {
         uint64_t raw[CACHED ? ROUNDS : 1];
 #pragma unroll
@@ -168,7 +185,6 @@ __global__ void __launch_bounds__(kTopkThreads) __attribute__((amdgpu_num_sgpr(8
     } else if (CACHED) {
         // every load leaves before the first score is looked at (a load inside a condition is waited for where it
         // stands: sixteen round trips instead of one); an index past the wavefront's range reads the row's last score
-        float raw[CACHED ? ROUNDS : 1];
 #pragma unroll
         for (int it = 0; it < ROUNDS; it++) raw[it] = s[min(w0 + it * 64 + lane, n - 1)];
 #pragma unroll
@@ -197,41 +213,59 @@ __global__ void __launch_bounds__(kTopkThreads) __attribute__((amdgpu_num_sgpr(8
     };
 
     if (tid < 64) winners[tid] = 0;
-    if (LARGE)
-        for (uint32_t i = tid; i < cap; i += kTopkThreads) big[i] = 0;
     if (tid == 0) { sh_prefix = 0; sh_need = k; sh_nwin = 0; sh_ncand = 0; }
-    if (SHORT_WAY) {
-        // ---- short way for a row held in registers.  The 64 groups of 16 lanes each own a slice of the row; the
-        //      smallest of the 64 group maxima, L, has at least 64 scores at or above it (one per group), so the
-        //      winners are among the scores >= L: a few hundred of a typical row.  Those are collected and each one
-        //      counts the candidates with a larger key: that count is its place in the output.  A row whose
-        //      candidates do not fit (sorted input, a group without valid scores) takes the radix passes below. ----
+    if (SHORT_WAY && k <= kTopkShortK) {
+        // ---- short way for a row held in registers.  Every group of neighbouring lanes owns a slice of the row; at least k
+        //      scores lie at or above L, the k-th largest of the group maxima (one per group): little more than k of a typical
+        //      row (128 groups, k = 64: ~90; the smallest of 64 maxima, the bound before, left ~300-500, and ranking them was a
+        //      third of the kernel).  Those are collected, and each one's place in the output is the number of candidates
+        //      above it.  A row whose candidates do not fit (many equal scores, too few valid ones) takes the radix passes below.
+        //      gate-KNN calls over 10240 features, before / now: K = 64 13.9 / 9.9 us, K = 8 13.8 / 9.5, K = 256 (radix passes
+        //      before) 25.2 / 13.8 ----
         uint32_t gmax = 0;
 #pragma unroll
         for (int it = 0; it < ROUNDS; it++) gmax = max(gmax, cache[it]);
+        for (uint32_t i = tid; i < (uint32_t)kTopkCandidates; i += kTopkThreads) cand[i] = 0;
         if (KEYS_IN) {
-            // a chunk's keys stand best first: slices of every fourth lane each hold one of the four best of every chunk
-            // (slices of 16 neighbours would leave the worst of a chunk to themselves and bound nothing)
+            // a chunk's keys stand best first: slices of every eighth (32nd) lane each hold one of the best of every chunk
+            // (slices of neighbours would leave the worst of a chunk to themselves and bound nothing)
 #pragma unroll
-            for (int o = 4; o < 64; o <<= 1) gmax = max(gmax, (uint32_t)__shfl_xor((int)gmax, o, 64));
-            if (lane < 4u) group_max[wave * 4 + lane] = gmax;
+            for (int o = 64 / (1024 / GROUPS); o < 64; o <<= 1) gmax = max(gmax, (uint32_t)__shfl_xor((int)gmax, o, 64));
+            if (lane < GROUPS / kTopkWaves) group_max[wave * (GROUPS / kTopkWaves) + lane] = gmax;
         } else {
             // (reductions by DPP row operations: a few cycles each, where a cross-lane shuffle costs an LDS round trip)
-            gmax = max(gmax, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)gmax, 0xB1, 0xF, 0xF, true));   // quad_perm [1,0,3,2]
-            gmax = max(gmax, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)gmax, 0x4E, 0xF, 0xF, true));   // quad_perm [2,3,0,1]
-            gmax = max(gmax, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)gmax, 0x141, 0xF, 0xF, true));  // row_half_mirror
-            gmax = max(gmax, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)gmax, 0x140, 0xF, 0xF, true));  // row_mirror
-            if ((lane & 15u) == 0) group_max[wave * 4 + (lane >> 4)] = gmax;
+            gmax = max(gmax, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)gmax, 0xB1, 0xF, 0xF, true));       // quad_perm [1,0,3,2]
+            if (!LARGE) {
+                gmax = max(gmax, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)gmax, 0x4E, 0xF, 0xF, true));   // quad_perm [2,3,0,1]
+                gmax = max(gmax, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)gmax, 0x141, 0xF, 0xF, true));  // row_half_mirror
+            }
+            if ((lane & (1024 / GROUPS - 1)) == 0) group_max[tid / (1024 / GROUPS)] = gmax;
         }
         __syncthreads();
-        uint32_t L = group_max[lane];
-        L = min(L, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)L, 0xB1, 0xF, 0xF, false));
-        L = min(L, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)L, 0x4E, 0xF, 0xF, false));
-        L = min(L, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)L, 0x141, 0xF, 0xF, false));
-        L = min(L, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)L, 0x140, 0xF, 0xF, false));
-        L = min(L, (uint32_t)__builtin_amdgcn_update_dpp((int)L, (int)L, 0x142, 0xA, 0xF, false));     // row_bcast:15 into rows 1 and 3
-        L = min(L, (uint32_t)__builtin_amdgcn_update_dpp((int)L, (int)L, 0x143, 0xC, 0xF, false));     // row_bcast:31 into rows 2 and 3
-        L = (uint32_t)__builtin_amdgcn_readlane((int)L, 63);
+        // The k-th largest maximum, every wavefront for itself: from the highest bit in which the largest and the smallest differ,
+        // a bit of L is set where k maxima still lie at or above it.  Fourteen bits: a bound may lie lower than the exact one.
+        uint32_t gm[PL], top = 0, bottom = ~0u;
+#pragma unroll
+        for (int q = 0; q < PL; q++) {
+            gm[q] = group_max[q * 64 + lane];
+            top = max(top, gm[q]);
+            bottom = min(bottom, gm[q]);
+        }
+        top = wave_max_u32(top);
+        bottom = ~wave_max_u32(~bottom);
+        uint32_t L = bottom;
+        if (top != bottom) {
+            const int high = 31 - __builtin_clz(top ^ bottom);
+            L = top & ~((2u << high) - 1u);  // (bits that all maxima share; high = 31: none)
+            for (int b = high; b >= 0 && b > high - 14; b--) {
+                const uint32_t trial = L | (1u << b);
+                uint32_t have = 0;
+#pragma unroll
+                for (int q = 0; q < PL; q++) have += (uint32_t)__popcll(__ballot(gm[q] >= trial));
+                if (have >= k) L = trial;
+            }
+        }
+        // (L = 0: fewer than k groups hold a score)
         if (L != 0) {
             // a wavefront reserves room for all its candidates at once, then places them round by round
             uint32_t mine = 0;
@@ -245,48 +279,45 @@ __global__ void __launch_bounds__(kTopkThreads) __attribute__((amdgpu_num_sgpr(8
                 const bool c = cache[it] >= L;
                 const uint64_t m = __ballot(c);
                 const uint32_t pos = base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-                if (c && pos < (uint32_t)kTopkCandidates) cand[pos] = ((uint64_t)cache[it] << 32) | low_word(it);
+                if (c && pos < (uint32_t)kTopkCandidates) {
+                    cand[pos] = ((uint64_t)cache[it] << 32) | low_word(it);
+                    if (BY_ABS && !KEYS_OUT && !KEYS_IN) cand_score[pos] = raw[it];
+                }
                 base += (uint32_t)__popcll(m);
             }
             __syncthreads();
             const uint32_t nc = sh_ncand;
             if (nc <= (uint32_t)kTopkCandidates) {  // (uniform over the workgroup)
-                // (the list is read four keys at a time: zero keys, below every real one, fill it up to a multiple of four)
-                if (tid < 4) cand[nc + tid] = 0;
-                // A candidate's rank = the candidates above it.  The threads beyond the list take part: with the list
-                // rounded up to a power of two, thread t counts for candidate t % that over the t / that -th share of
-                // the list, and the shares meet in an LDS counter (half as long for the usual 300-500 candidates).
-                uint32_t ncr = 64;
-                while (ncr < nc) ncr <<= 1;
-                const uint32_t parts = (uint32_t)kTopkThreads / ncr, ci = tid & (ncr - 1u), part = tid / ncr;
-                if (parts > 1 && tid < nc) rank_sh[tid] = 0;
-                __syncthreads();
-                uint64_t key = 0;
-                uint32_t rank = 0;
-                if (ci < nc) {
-                    key = cand[ci];
-                    typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
-                    const u64x2 *c2 = reinterpret_cast<const u64x2 *>(cand);
-                    const uint32_t quads = (nc + 3) / 4, per = (quads + parts - 1) / parts;
-                    const uint32_t j0 = part * per, j1 = min(quads, j0 + per);
+                // A candidate's rank = the candidates above it: eight neighbouring lanes each count an eighth of the list, read two
+                // keys at a time (zero keys, below every real one, stand behind it).
+                typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
+                const u64x2 *c2 = reinterpret_cast<const u64x2 *>(cand);
+                const uint32_t pairs = (nc + 15) / 16;  // of an eighth
+                for (uint32_t c0 = 0; c0 < nc; c0 += kTopkThreads / 8) {
+                    const uint32_t ci = c0 + (tid >> 3);
+                    const uint64_t key = cand[min(ci, nc - 1)];
+                    uint32_t rank = 0;
 #pragma unroll 2
-                    for (uint32_t j = j0; j < j1; j++) {
-                        const u64x2 a = c2[2 * j], b = c2[2 * j + 1];
-                        rank += (a.x > key ? 1u : 0u) + (a.y > key ? 1u : 0u) + (b.x > key ? 1u : 0u) + (b.y > key ? 1u : 0u);
+                    for (uint32_t j = 0; j < pairs; j++) {
+                        const u64x2 a = c2[j * 8 + (tid & 7u)];
+                        rank += (a.x > key ? 1u : 0u) + (a.y > key ? 1u : 0u);
                     }
-                    if (parts > 1 && rank != 0) atomicAdd(&rank_sh[ci], rank);
+                    rank += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)rank, 0xB1, 0xF, 0xF, true);   // quad_perm [1,0,3,2]
+                    rank += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)rank, 0x4E, 0xF, 0xF, true);   // quad_perm [2,3,0,1]
+                    rank += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)rank, 0x141, 0xF, 0xF, true);  // row_half_mirror
+                    if ((tid & 7u) == 0 && ci < nc && rank < k) {
+                        if (BY_ABS && !KEYS_OUT && !KEYS_IN) put(rank, key, cand_score[ci]);
+                        else emit(rank, key);
+                    }
                 }
-                if (parts > 1) {
-                    __syncthreads();
-                    if (tid < nc) rank = rank_sh[tid];
-                }
-                if (tid < nc && rank < k) emit(rank, key);  // (tid < nc: ci == tid, the key is this thread's candidate)
-                if (!KEYS_OUT && tid == 0) A.count_out[row] = min(k, nc);  // (a chunk's nc is at least 64)
+                if (!KEYS_OUT && tid == 0) A.count_out[row] = min(k, nc);  // (nc >= k: a chunk leaves k keys)
                 return;
             }
         }
         __syncthreads();
     }
+    if (LARGE)
+        for (uint32_t i = tid; i < cap; i += kTopkThreads) big[i] = 0;
     // ---- radix select of the k-th largest ordered score: 8 bits per pass, top byte first ----
     for (int pass = 0; pass < 4; pass++) {
         const int sh = 24 - 8 * pass;
@@ -389,22 +420,23 @@ __global__ void __launch_bounds__(kTopkThreads) __attribute__((amdgpu_num_sgpr(8
 }
 
 // How a row of a batch is cut.  A row that one workgroup can hold in registers is not: two launches cost 4 us more than one.
-// Above that, K <= 64 takes chunks of 4096 (four scores a thread; of 16384 where the chunks' winners would not fit the
-// merging workgroup's registers).
+// Above that, K <= 256 (the short way) takes chunks of 4096 (four scores a thread; of 16384 where the chunks' winners would not fit
+// the merging workgroup's registers): streamed or cut at 16384 / cut at 4096, us per lm_head call, K = 200:
+// 16400 scores 105 / 60, 32768 103 / 56, 262144 116 / 68; 18000 scores, 1 / 100 / 1000 rows 45 / 21, 63 / 42, 246 / 216.
 // A larger K takes chunks of 16384 where that is faster than streaming the row: a second launch and a second ordering of K
 // winners against ~1.7 us per thousand scores beyond the first 16384 that one workgroup would walk again and again.  The two
-// meet at 17408 + 5 K scores (one row, streamed / cut, us: 18000 scores, K = 65 44.1 / 42.8; 20000, 500 51.0 / 51.6; 20000, 1000
-// 55.4 / 60.8; 24000, 1000 61.7 / 61.0; 24000, 2000 68.2 / 75.9; 32768, 2000 84.4 / 76.8; the same within 5 % for 100 or 1000 rows).
+// meet at 17408 + 5 K scores (one row, streamed / cut, us: 20000, 500 51.0 / 51.6; 20000, 1000 55.4 / 60.8; 24000, 1000 61.7 / 61.0;
+// 24000, 2000 68.2 / 75.9; 32768, 2000 84.4 / 76.8; the same within 5 % for 100 or 1000 rows).
 // Above K = 2048 the two orderings (a bitonic sort of 4096 keys is 35 us) take four chunks to pay for (32768, 4096 101.6 / 115.7;
 // 65536, 4096 157.1 / 127.9), and do not once the rows fill the chip by themselves (65536, 4096: 100 rows 315 / 300, 300 rows 722 / 731,
 // 1000 rows 2044 / 2242).
 static uint32_t topk_chunk(uint32_t batch, uint32_t n, uint32_t k) {
     constexpr uint32_t held = kTopkThreads * kTopkCached, small = held / 4;
     if (n <= held) return n;
-    if (k <= 64) {
+    if (k <= kTopkShortK) {
         for (uint32_t chunk : {small, held})
             if ((uint64_t)((n + chunk - 1) / chunk) * k <= held) return chunk;
-        return n;
+        if (k <= 64) return n;
     }
     if (n > 0x7FFFFFFFu || k > held / 4) return n;
     const bool cut = k <= held / 8 ? n >= held + 1024 + 5 * k : n > 3 * held && batch <= 128;
@@ -459,13 +491,17 @@ static hipError_t topk_rows(hipStream_t stream, TopkArgs A, uint32_t batch, uint
         const uint32_t chunks = (A.n + chunk - 1) / chunk;
         A.chunk = chunk;
         A.keys_out = (uint64_t *)workspace;
-        hipError_t e = large ? topk_stage<BY_ABS, kTopkCached, true, false, true>(stream, A, chunks, batch)
+        hipError_t e = large ? (chunk <= kTopkThreads * kTopkCached / 4 ? topk_stage<BY_ABS, kTopkCached / 4, true, false, true>(stream, A, chunks, batch)
+                                                                         : topk_stage<BY_ABS, kTopkCached, true, false, true>(stream, A, chunks, batch))
                        : chunk <= kTopkThreads * kTopkCached / 4 ? topk_stage<BY_ABS, kTopkCached / 4, false, false, true>(stream, A, chunks, batch)
                                                                  : topk_stage<BY_ABS, kTopkCached, false, false, true>(stream, A, chunks, batch);
         if (e != hipSuccess) return e;
         A.keys_in = A.keys_out;
         A.n = A.chunk = chunks * A.k;
         if (A.n > kTopkThreads * kTopkCached) return topk_stage<false, 0, true, true, false>(stream, A, 1, batch);
+        if (A.n <= kTopkThreads * kTopkCached / 4)
+            return large ? topk_stage<false, kTopkCached / 4, true, true, false>(stream, A, 1, batch)
+                         : topk_stage<false, kTopkCached / 4, false, true, false>(stream, A, 1, batch);
         return large ? topk_stage<false, kTopkCached, true, true, false>(stream, A, 1, batch)
                      : topk_stage<false, kTopkCached, false, true, false>(stream, A, 1, batch);
     }
@@ -483,7 +519,7 @@ hipError_t topk_launch(hipStream_t stream, const float *scores, uint32_t batch, 
                        uint32_t *idx_out, float *val_out, uint32_t *count_out, int *nan_flag, void *workspace, size_t workspace_bytes) {
     if (k > kTopkMaxK) return hipErrorInvalidValue;
     TopkArgs A = {};
-    A.scores_n = A.n = n; A.k = k; A.nan_flag = nan_flag;
+    A.scores_n = A.n = n; A.k = k; A.nan_flag = nan_flag; A.by_value = by_abs ? 0u : 1u;
     const size_t need = topk_workspace_bytes(batch, n, k);
     if (need == 0 || workspace_bytes < need) workspace = nullptr;
     const uint32_t chunk = topk_chunk(batch, n, k);

@@ -2278,3 +2278,39 @@ def test_short_launches_equal_the_streaming_kernel_bit_for_bit(be, fmt, fmt_name
 @pytest.mark.parametrize("wfmt", ["q4k", "q6k"])
 def test_moe_layer_k_quant_slots_share_an_expert(be, fmt, T, E, k, hidden, cols, inter, wfmt):
     test_moe_layer_over_a_k_quant_bank_matches_the_integer_expert_path(be, fmt, T, E, k, hidden, cols, inter, wfmt, 1, True, False)
+
+
+@pytest.mark.parametrize("case", ["normal", "narrow", "coarse", "constant", "wide", "few"])
+def test_top_k_bounds_by_slices_of_the_row(be, fmt, case):
+    """The short way's bound (the K-th largest maximum of 128 slices, of 512 above K = 64; fourteen bits of it) over rows whose scores
+    differ in the last bits, are equal in large blocks, span the whole range of f32, or fill only some slices, by |score| and by
+    value (infinities and NaN skipped there), K on both sides of 64 and of 256.  Ties go to the lower index: one right answer."""
+    rng = np.random.default_rng(len(case))
+    for n in (130, 520, 4097, 10240, 16385, 20000):
+        sc = {"normal": rng.standard_normal(n), "narrow": 100.0 + rng.random(n) * 1e-3, "coarse": np.round(rng.standard_normal(n) * 2) / 2,
+              "constant": np.full(n, -0.75), "wide": rng.standard_normal(n) * np.exp2(rng.integers(-120, 120, n)),
+              "few": np.where(rng.random(n) < 0.03, rng.standard_normal(n), 0.0)}[case].astype(F)
+        sc[::7] *= F(-1.0)
+        gate = np.zeros((n, 32), F)
+        gate[:, 0] = sc
+        x = np.zeros(32, F)
+        x[0] = 1.0
+        by_abs = np.lexsort((np.arange(n), -np.abs(sc)))
+        # the same through a Q8_0 head: one f16 scale and one code per row
+        with np.errstate(over="ignore"):
+            d = sc.astype(np.float16)
+        d[5::50], d[6::50] = np.float16(np.inf), np.float16(np.nan)
+        blocks = np.zeros((n, 34), np.uint8)
+        blocks[:, :2] = d.view(np.uint8).reshape(n, 2)
+        blocks[:, 2] = 3
+        blocks = np.concatenate([blocks, np.zeros((n, 7 * 34), np.uint8)], axis=1)
+        x8 = np.zeros(256, F)
+        x8[0] = 1.0
+        val = d.astype(F) * F(3)
+        ok = np.flatnonzero(np.isfinite(val))
+        by_value = ok[np.lexsort((ok, -val[ok]))]
+        for k in (1, 64, 65, 200, 256, 257):
+            hits = be.gate_knn(fmt.FMT_F32, gate, x, n, 32, k)
+            assert [i for i, _ in hits] == by_abs[:k].tolist() and [v for _, v in hits] == sc[by_abs[:k]].tolist(), (n, k)
+            hits = be.q8_0_gemv_topk(blocks, x8, n, 256, k)
+            assert [i for i, _ in hits] == by_value[:k].tolist() and [v for _, v in hits] == val[by_value[:k]].tolist(), (n, k)
