@@ -45,13 +45,28 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 
+// Reductions by data-parallel primitives (a few cycles each; a cross-lane shuffle is a trip through LDS hardware).  Lanes without a
+// source bring 0: the values are non-negative.
+template <int CTRL, int ROW_MASK = 0xF>
+__device__ __forceinline__ float dpp_move(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, ROW_MASK, 0xF, true));
+}
+template <int CTRL, int ROW_MASK = 0xF>
+__device__ __forceinline__ float dpp_max(float v) { return fmaxf(v, dpp_move<CTRL, ROW_MASK>(v)); }
+__device__ __forceinline__ float row16_max(float v) {
+    v = dpp_max<0xB1>(v);     // quad_perm [1,0,3,2]
+    v = dpp_max<0x4E>(v);     // quad_perm [2,3,0,1]
+    v = dpp_max<0x141>(v);    // row_half_mirror
+    return dpp_max<0x140>(v); // row_mirror
+}
+
 // one block per token: scale, f16 terms, sub-block sums.  `x_is_bf16`: 16-bit inputs (exact in one term).
 // A thread takes 8 consecutive elements at a time (one or two 16-byte loads); four neighbouring threads hold a
 // 32-element sub-block.
-__global__ void __launch_bounds__(1024) q4k_gemm_prep_kernel(const void *__restrict__ x, int x_is_bf16, uint32_t hidden,
-                                                            uint16_t *__restrict__ xh, uint16_t *__restrict__ xl,
-                                                            uint16_t *__restrict__ sx, float *__restrict__ tok_scale,
-                                                            int *__restrict__ any_lo, int swap12, uint32_t seq,
+// (The arguments that a block's first loads wait for are the first fourteen dwords, which are in registers when it starts.)
+__global__ void __launch_bounds__(1024) q4k_gemm_prep_kernel(const void *__restrict__ x, uint32_t hidden, uint32_t seq, int x_is_bf16, int swap12,
+                                                            uint16_t *__restrict__ xh, uint16_t *__restrict__ sx, float *__restrict__ tok_scale,
+                                                            uint16_t *__restrict__ xl, int *__restrict__ any_lo,
                                                             const uint8_t *__restrict__ w, uint32_t rows, int *__restrict__ rexp) {
     __shared__ float red[16];
     const uint32_t t = threadIdx.x, nvec = hidden >> 3;  // hidden % 256 == 0
@@ -71,7 +86,7 @@ __global__ void __launch_bounds__(1024) q4k_gemm_prep_kernel(const void *__restr
                     m = fmaxf(m, fmaxf(fabsf(half_to_float(h[u] & 0xFFFFu)), 0.0625f * fabsf(half_to_float(h[u] >> 16))));
             }
         }
-        for (int o = 8; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+        m = row16_max(m);
         if (row < rows && (t & 15u) == 0) {
             int e = 0;
             if (m > 0.f && m < __builtin_inff()) (void)frexpf(m, &e);
@@ -116,8 +131,10 @@ __global__ void __launch_bounds__(1024) q4k_gemm_prep_kernel(const void *__restr
         for (uint32_t u = 0; u < KEEP; u++) max8(0, &kept[u]);
     }
     for (uint32_t v = t + (x_is_bf16 ? KEEP * blockDim.x : 0u); v < nvec; v += blockDim.x) max8(v, nullptr);
-    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-    if ((t & 63u) == 0) red[t >> 6] = mx;
+    mx = row16_max(mx);
+    mx = dpp_max<0x142, 0xA>(mx);  // row_bcast:15 into rows 1 and 3
+    mx = dpp_max<0x143, 0xC>(mx);  // row_bcast:31 into rows 2 and 3: lane 63 holds the wavefront's
+    if ((t & 63u) == 63) red[t >> 6] = mx;
     __syncthreads();
     mx = 0.f;
     for (uint32_t wv = 0; wv < (blockDim.x >> 6); wv++) mx = fmaxf(mx, red[wv]);
@@ -153,8 +170,8 @@ __global__ void __launch_bounds__(1024) q4k_gemm_prep_kernel(const void *__restr
         const size_t at = (size_t)tok * nvec + v;
         oh[at] = (u32x4){hw[0], hw[1], hw[2], hw[3]};
         if (ol) ol[at] = (u32x4){lw[0], lw[1], lw[2], lw[3]};
-        sm += __shfl_xor(sm, 1);
-        sm += __shfl_xor(sm, 2);
+        sm += dpp_move<0xB1>(sm);  // quad_perm [1,0,3,2]
+        sm += dpp_move<0x4E>(sm);  // quad_perm [2,3,0,1]
         sm *= 0.03125f;  // stored as Sx/32 so that 32 x 2^14 stays inside f16; the min operand carries the 32
         if ((t & 3u) == 0) {
             const _Float16 sh = (_Float16)sm;
@@ -882,41 +899,43 @@ __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *
 
     // The pair adds its partial sums through LDS, where the results also take the shape in which a store instruction
     // writes whole lines: a row group's 64-row x 128-token block as [token][row] (token rows padded to 68 floats: the
-    // lanes of a write phase hit different banks) in the pair's own 34 KB; wavefront 1 parks, wavefront 0 adds its own
-    // and parks the sum, then every lane of the pair stores 16 bytes of a 256-byte run of one token.
+    // lanes of a write phase hit different banks) in the pair's own 34 KB; each parks the 32 rows of the other and adds its
+    // own 32 to what the other parked, then every lane of the pair stores 16 bytes of a 256-byte run of one token.
+    const uint32_t rc = (lane & 15u) * 4, r = row0 + wm + rc;
+    float back[4];  // 2^-E of this lane's four rows (asked for here: behind the barriers nothing would hide the trip)
+#pragma unroll
+    for (int e = 0; e < 4; e++) back[e] = ldexpf(1.f, -rexp[min(r + e, rows - 1)]);
     __builtin_amdgcn_s_barrier();  // nobody's copies are still landing in what becomes somebody's block
     asm volatile("" ::: "memory");
     constexpr uint32_t EP_LD = G_EP_LD;
     float *blk = reinterpret_cast<float *>(glds) + wq * (GN * EP_LD);
-    if (kh) {
+    auto park = [&](auto I) {
+        constexpr int i = decltype(I)::value;
 #pragma unroll
-        for (int i = 0; i < 2; i++)
+        for (int jj = 0; jj < NB; jj++)
 #pragma unroll
-            for (int jj = 0; jj < NB; jj++)
+            for (int q = 0; q < 4; q++)  // registers 4q .. 4q+3 of a block: rows 8q + 4kgrp .. +3, token row32
+                *reinterpret_cast<f32x4 *>(blk + (jj * 32 + row32) * EP_LD + i * 32 + q * 8 + kgrp * 4) =
+                    (f32x4){acc[i][jj][4 * q], acc[i][jj][4 * q + 1], acc[i][jj][4 * q + 2], acc[i][jj][4 * q + 3]};
+    };
+    auto add_own = [&](auto I) {
+        constexpr int i = decltype(I)::value;
 #pragma unroll
-                for (int q = 0; q < 4; q++)  // registers 4q .. 4q+3 of a block: rows 8q + 4kgrp .. +3, token row32
-                    *reinterpret_cast<f32x4 *>(blk + (jj * 32 + row32) * EP_LD + i * 32 + q * 8 + kgrp * 4) =
-                        (f32x4){acc[i][jj][4 * q], acc[i][jj][4 * q + 1], acc[i][jj][4 * q + 2], acc[i][jj][4 * q + 3]};
-    }
+        for (int jj = 0; jj < NB; jj++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                f32x4 *at = reinterpret_cast<f32x4 *>(blk + (jj * 32 + row32) * EP_LD + i * 32 + q * 8 + kgrp * 4);
+                const f32x4 other = *at;
+                *at = (f32x4){acc[i][jj][4 * q] + other[0], acc[i][jj][4 * q + 1] + other[1], acc[i][jj][4 * q + 2] + other[2], acc[i][jj][4 * q + 3] + other[3]};
+            }
+    };
+    if (kh) park(std::integral_constant<int, 0>{});
+    else park(std::integral_constant<int, 1>{});
     __syncthreads();
-    if (!kh) {
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-            for (int jj = 0; jj < NB; jj++)
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    f32x4 *at = reinterpret_cast<f32x4 *>(blk + (jj * 32 + row32) * EP_LD + i * 32 + q * 8 + kgrp * 4);
-                    const f32x4 other = *at;
-                    *at = (f32x4){acc[i][jj][4 * q] + other[0], acc[i][jj][4 * q + 1] + other[1], acc[i][jj][4 * q + 2] + other[2], acc[i][jj][4 * q + 3] + other[3]};
-                }
-    }
+    if (kh) add_own(std::integral_constant<int, 1>{});
+    else add_own(std::integral_constant<int, 0>{});
     __syncthreads();
     const bool vec_ok = (rows & 3u) == 0 && (((uintptr_t)(partial ? partial : out)) & 15u) == 0;
-    const uint32_t rc = (lane & 15u) * 4, r = row0 + wm + rc;
-    float back[4];  // 2^-E of this lane's four rows
-#pragma unroll
-    for (int e = 0; e < 4; e++) back[e] = ldexpf(1.f, -rexp[min(r + e, rows - 1)]);
 #pragma unroll 4
     for (int it = 0; it < 16; it++) {
         const uint32_t tl = (kh * 16 + it) * 4 + (lane >> 4), tok = tok0 + tl;
@@ -948,8 +967,8 @@ hipError_t q4k_gemm_prep_launch(hipStream_t s, const void *x, int x_is_bf16, uin
     // x 4352 with 2048 tokens 52.2 us a call, with 512 threads 47.5, and no less with 16)
     const uint32_t threads = hidden > 8192 ? 1024u : hidden > 4096 ? 512u : 256u;
     const uint32_t row_blocks = rexp ? (rows + threads / 16 - 1) / (threads / 16) : 0;
-    hipLaunchKernelGGL(q4k_gemm_prep_kernel, dim3(seq + row_blocks), dim3(threads), 0, s, x, x_is_bf16, hidden, xh, xl, sx, tok_scale, any_lo,
-                       1, seq, w, rows, rexp);
+    hipLaunchKernelGGL(q4k_gemm_prep_kernel, dim3(seq + row_blocks), dim3(threads), 0, s, x, hidden, seq, x_is_bf16, 1, xh, sx, tok_scale, xl,
+                       any_lo, w, rows, rexp);
     return hipGetLastError();
 }
 
