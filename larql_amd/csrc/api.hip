@@ -2325,8 +2325,9 @@ static int moe_layer_enqueue(larql_hip_ctx *c, larql_hip_moe_layer *L, const flo
         float *g = (float *)L->ws.p, *u = g + slots * inter, *dd = u + slots * inter;
         uint8_t *xq = (dense && !pad_x) ? (uint8_t *)const_cast<float *>(x) : (uint8_t *)L->ws.p + f_bytes;
         uint8_t *aq = (uint8_t *)L->ws.p + f_bytes + x_area;
-        if (L->kq_kind == KIND_Q4K_Q8K && hidden <= 0xFFFFFFFFull && inter <= 0xFFFFFFFFull && moe_kq_group_serves((uint32_t)inter, (uint32_t)(cols / 256), (uint32_t)E, (uint32_t)slots) &&
-            moe_kq_group_serves((uint32_t)hidden, (uint32_t)(ip / 256), (uint32_t)E, (uint32_t)slots)) {
+        const bool q6 = L->kq_kind == KIND_Q6K_Q8K;
+        if (!dense && moe_kq_group_serves(q6, (uint32_t)inter, (uint32_t)(cols / 256), (uint32_t)E, (uint32_t)slots) &&
+            moe_kq_group_serves(q6, (uint32_t)hidden, (uint32_t)(ip / 256), (uint32_t)E, (uint32_t)slots)) {
             // slots that chose the same expert share its weights
             const JobTableSpec none[2] = {};
             HIPCHECK(c, moe_kq_route_quant_launch(c->stream, logits, L->router_bias, (uint32_t)tokens, (uint32_t)E, (uint32_t)k, policy,
@@ -2338,7 +2339,7 @@ static int moe_layer_enqueue(larql_hip_ctx *c, larql_hip_moe_layer *L, const flo
             a.w[0] = L->kq_gate; a.w[1] = L->kq_up; a.w_stride = L->kq_gu_stride;
             a.x = xq; a.x_stride = xq_stride;
             a.out[0] = g; a.out[1] = u;
-            HIPCHECK(c, moe_kq_group_launch(c->stream, a, (uint32_t)c->cu_count));
+            HIPCHECK(c, moe_kq_group_launch(c->stream, q6, a, (uint32_t)c->cu_count));
             HIPCHECK(c, moe_kq_act_q8k_launch(c->stream, g, u, (uint32_t)inter, (uint32_t)ip, (uint32_t)slots, experts, (uint32_t)E, L->kq_gub, L->gate_rule,
                                               L->glu_limit, L->glu_alpha, aq, aq_stride));
             MoeKqGroupArgs b = {};
@@ -2347,7 +2348,7 @@ static int moe_layer_enqueue(larql_hip_ctx *c, larql_hip_moe_layer *L, const flo
             b.w[0] = L->kq_down; b.w_stride = L->kq_dn_stride;
             b.x = aq; b.x_stride = aq_stride;
             b.out[0] = dd;
-            HIPCHECK(c, moe_kq_group_launch(c->stream, b, (uint32_t)c->cu_count));
+            HIPCHECK(c, moe_kq_group_launch(c->stream, q6, b, (uint32_t)c->cu_count));
             HIPCHECK(c, weighted_sum_launch(c->stream, dd, weights, experts, (uint32_t)E, L->kq_db, out, (uint32_t)tokens, (uint32_t)k, (uint32_t)hidden));
             return LARQL_OK;
         }

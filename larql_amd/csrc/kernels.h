@@ -212,7 +212,7 @@ hipError_t moe_group_launch(hipStream_t s, const MoeGroupArgs &A, bool down, uin
 hipError_t moe_route_terms_launch(hipStream_t s, const float *logits, const float *bias, uint32_t tokens, uint32_t n_experts, uint32_t k, int policy,
                                   uint32_t *experts, float *weights, const float *x, uint32_t hidden, uint16_t *terms);
 
-// The slots of a call through a bank of Q4_K experts against Q8_K activations (moe_kq_group.hip): `n_mats` matrices of one shape per
+// The slots of a call through a bank of Q4_K (q6: Q6_K) experts against Q8_K activations (moe_kq_group.hip): `n_mats` matrices of one shape per
 // expert (gate and up, or down) in one launch, each read once per group of slots.
 struct MoeKqGroupArgs {
     const uint32_t *experts;       // [slots], slot = token * k + rank; an id >= n_experts leaves its results as they are
@@ -225,8 +225,8 @@ struct MoeKqGroupArgs {
     uint64_t x_stride;
     float *out[2];                 // [slots, rows] of each matrix
 };
-bool moe_kq_group_serves(uint32_t rows, uint32_t cols, uint32_t n_experts, uint32_t slots);
-hipError_t moe_kq_group_launch(hipStream_t s, const MoeKqGroupArgs &A, uint32_t cu_count);
+bool moe_kq_group_serves(bool q6, uint32_t rows, uint32_t cols, uint32_t n_experts, uint32_t slots);
+hipError_t moe_kq_group_launch(hipStream_t s, bool q6, const MoeKqGroupArgs &A, uint32_t cu_count);
 
 // MoE helpers
 constexpr uint32_t kRouterMaxExperts = 256;      // the selection kernels (four logits per lane)
