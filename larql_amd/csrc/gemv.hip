@@ -1782,48 +1782,57 @@ __device__ __forceinline__ void run_mxfp4_fold(const GemvJob &j, const Mx4Sel &s
 //                  set, each expert's tile meets the whole set and lane (j, rq) keeps expert rq's sums, scaled by the
 //                  expert's routing weight; the experts meet in the fold of the row partials, the biases (weighted)
 //                  join there.  Without `terms` (gate and up apart) the activations are gated and split here.
+// What bounds a launch is its chain of waits: arguments, selection, first tile, fold.  So the arguments that the first loads need
+// are in registers when a wavefront starts (the rest of the block is read beside those loads), the host does the divisions of the
+// shares, a fold has all its partials on their way before it adds the first, and the biases of the first fold's rows are asked for
+// with the first tile.  2880 x 2880, 32 experts, k = 4, both launches: 21.3 us before, 19.2 with all four; 53 MB of weights take
+// 8.1 us at 6.5 TB/s.
 // ---------------------------------------------------------------------------
 constexpr int kMoe1BatchTiles = 4;
 constexpr int moe1_stages(int cw) { return cw <= 3 ? 3 : 3; }  // ring slots per wavefront that fit the LDS beside the partials
 constexpr uint32_t moe1_slot_bytes(int cw) { return (uint32_t)cw * kMx4StepBytes + (cw > 4 ? 512u : 256u); }  // steps, then a scale dword per lane (two with five steps)
+constexpr uint32_t kMoe1Apart = 1u << 16, kMoe1Terms = 1u << 17;  // geom: experts | wavefronts << 8 | gate and up apart | `act` are terms
 __device__ const uint32_t kMoe1Zeros[4] = {0u, 0u, 0u, 0u};      // what an operand lane without an activation loads
 
 // CW: 128-element steps per wavefront (the row length decides); NS: ring slots per wavefront
 template <bool DOWN, int CW, int NS>
-__global__ void __launch_bounds__(kMx4MaxWaves * 64) moe1_kernel(const Moe1Args A) {
+__global__ void __launch_bounds__(kMx4MaxWaves * 64)
+    moe1_kernel(const float *logits, const float *router_bias, uint32_t *experts, const void *act, uint32_t n_experts, uint32_t kdim, uint32_t geom,
+                uint32_t tpm, uint32_t share, uint32_t rest,  // (in registers when the wavefront starts; act: the terms, or A.x)
+                const Moe1Args A) {
     extern __shared__ __attribute__((aligned(16))) uint8_t m1_lds[];
     constexpr int R = DOWN ? kMoe1BatchTiles : 2 * kMoe1BatchTiles;  // row tiles between two folds of the row partials
     constexpr uint32_t cw = CW, slot_bytes = moe1_slot_bytes(CW);
     const uint32_t lane = threadIdx.x & 63u, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t nw_launch = blockDim.x >> 6;
     const uint32_t jr = lane & 15u, kg = lane >> 4;
-    const uint32_t kdim = A.kdim, nb = kdim / 32, row_bytes = nb * 16, steps = (kdim + 127) / 128, nwj = A.nw;
-    const uint32_t rows = A.rows, nq = min(A.k, kMoe1MaxK), TR = A.tile_rows;  // (rows per tile: 16, or fewer to share a short result out evenly)
+    const uint32_t nb = kdim / 32, row_bytes = nb * 16, steps = (kdim + 127) / 128, nwj = (geom >> 8) & 0xFFu;
+    const uint32_t rows = A.rows, nq = geom & 0xFFu, TR = A.tile_rows, n_mats = (geom & kMoe1Apart) ? 2u : 1u;  // (rows per tile: 16, or fewer to share a short result out evenly)
     uint8_t *ring = m1_lds + wv * (NS * slot_bytes);
     float *part = reinterpret_cast<float *>(m1_lds + nw_launch * (NS * slot_bytes));
     const uint32_t step0 = wv * cw;
     const bool working = wv < nwj && step0 < steps;
 
     // 0. what the selection needs: the logits, or the selection as stored where an earlier launch made it
-    const bool has_logit = A.logits && lane < A.n_experts;
-    float logit = has_logit ? ((const GLOBAL_AS float *)A.logits)[lane] : 0.0f;
-    if (has_logit && A.router_bias) logit += ((const GLOBAL_AS float *)A.router_bias)[lane];
-    const uint32_t ev = (!A.logits && lane < nq) ? ((const GLOBAL_AS uint32_t *)A.experts)[lane] : 0u;
-    const float wl = (!A.logits && DOWN && lane < nq) ? ((const GLOBAL_AS float *)A.weights)[lane] : 0.0f;
+    const bool has_logit = logits && lane < n_experts;
+    float logit = has_logit ? ((const GLOBAL_AS float *)logits)[lane] : 0.0f;
+    if (has_logit && router_bias) logit += ((const GLOBAL_AS float *)router_bias)[lane];
+    const uint32_t ev = (!logits && lane < nq) ? ((const GLOBAL_AS uint32_t *)experts)[lane] : 0u;
+    const float wl = (!logits && DOWN && lane < nq) ? ((const GLOBAL_AS float *)A.weights)[lane] : 0.0f;
 
     // 1. the activations of this wavefront's K-range: nothing they need has to be waited for
     GemvJob jx = {};  // (the fields the activation helpers read)
-    jx.k = kdim; jx.x = A.x; jx.x_glu = A.x_glu; jx.glu_limit = A.glu_limit; jx.glu_alpha = A.glu_alpha;
+    jx.k = kdim; jx.x = (const float *)act; jx.x_glu = A.x_glu; jx.glu_limit = A.glu_limit; jx.glu_alpha = A.glu_alpha;
     if (DOWN) { jx.batch = nq; jx.x_stride = A.x_slot_stride; jx.x_off[0] = (int64_t)(2 * A.x_slot_stride); jx.x_off[1] = (int64_t)(3 * A.x_slot_stride); }
     Mx4In xin[kMx4MaxSteps];
     Mx4Ops ops;
-    const bool pre = DOWN && A.terms != nullptr;  // the activations arrive as operand terms
+    const bool pre = DOWN && (geom & kMoe1Terms) != 0;  // the activations arrive as operand terms
     auto load_operands = [&]() {
         // lane (row i = 4q + term, kg): eight consecutive bf16 of term plane `term`, slot q, per MFMA; a lane without an
         // activation (fourth row of a slot, slot >= k, elements past the row end) reads zeros
         const uint32_t tq = jr >> 2, term = jr & 3u;
         const bool mine = working && tq < nq && term < 3u;
-        const uint16_t *tp = A.terms + ((size_t)term * nq + tq) * A.terms_kpad;
+        const uint16_t *tp = (const uint16_t *)act + ((size_t)term * nq + tq) * A.terms_kpad;
 #pragma unroll
         for (int s = 0; s < CW; s++) {
 #pragma unroll
@@ -1847,12 +1856,12 @@ __global__ void __launch_bounds__(kMx4MaxWaves * 64) moe1_kernel(const Moe1Args 
     uint32_t e[kMoe1MaxK];
     float cwt[kMoe1MaxK];
     bool ok[kMoe1MaxK];
-    if (A.logits) {
+    if (logits) {
         uint32_t idx[kRouterMaxK];
         float wt[kRouterMaxK];
-        const bool writer = A.experts && blockIdx.x == 0 && wv == 0;  // (wave-uniform)
-        if (writer || DOWN) router_select_lane<true>(logit, A.n_experts, nq, A.policy, lane, idx, wt);
-        else router_select_lane<false>(logit, A.n_experts, nq, A.policy, lane, idx, wt);
+        const bool writer = experts && blockIdx.x == 0 && wv == 0;  // (wave-uniform)
+        if (writer || DOWN) router_select_lane<true>(logit, n_experts, nq, A.policy, lane, idx, wt);
+        else router_select_lane<false>(logit, n_experts, nq, A.policy, lane, idx, wt);
 #pragma unroll
         for (int q = 0; q < (int)kMoe1MaxK; q++) {
             e[q] = __builtin_amdgcn_readfirstlane(idx[q]);
@@ -1861,7 +1870,7 @@ __global__ void __launch_bounds__(kMx4MaxWaves * 64) moe1_kernel(const Moe1Args 
         if (writer && lane == 0) {
 #pragma unroll
             for (int r = 0; r < (int)kMoe1MaxK; r++)
-                if ((uint32_t)r < nq) { A.experts[r] = idx[r]; A.weights[r] = wt[r]; }
+                if ((uint32_t)r < nq) { experts[r] = idx[r]; A.weights[r] = wt[r]; }
         }
     } else {
 #pragma unroll
@@ -1874,25 +1883,27 @@ __global__ void __launch_bounds__(kMx4MaxWaves * 64) moe1_kernel(const Moe1Args 
     const uint8_t *wq[kMoe1MaxK], *sq[kMoe1MaxK];
 #pragma unroll
     for (int q = 0; q < (int)kMoe1MaxK; q++) {
-        ok[q] = (uint32_t)q < nq && e[q] < A.n_experts;
+        ok[q] = (uint32_t)q < nq && e[q] < n_experts;
         e[q] = ok[q] ? e[q] : 0u;
         cwt[q] = ok[q] ? cwt[q] : 0.0f;
         wq[q] = A.w[0] + (size_t)e[q] * A.w_stride;
         sq[q] = A.aux[0] + (size_t)e[q] * A.aux_stride;
     }
     // (second matrix of a slot: the same expert in the up bank)
-    const size_t m1_w = A.n_mats == 2 ? (size_t)(A.w[1] - A.w[0]) : 0, m1_s = A.n_mats == 2 ? (size_t)(A.aux[1] - A.aux[0]) : 0;
+    const size_t m1_w = n_mats == 2 ? (size_t)(A.w[1] - A.w[0]) : 0, m1_s = n_mats == 2 ? (size_t)(A.aux[1] - A.aux[0]) : 0;
     auto expert_of = [&](uint32_t q) { return q == 1 ? e[1] : (q == 2 ? e[2] : (q == 3 ? e[3] : e[0])); };
     auto ok_of = [&](uint32_t q) { return q == 1 ? ok[1] : (q == 2 ? ok[2] : (q == 3 ? ok[3] : ok[0])); };
     auto weight_of = [&](uint32_t q) { return q == 1 ? cwt[1] : (q == 2 ? cwt[2] : (q == 3 ? cwt[3] : cwt[0])); };
 
     // 3. this workgroup's share.  Gate/up: row tiles [va, vb) of the list (slot, matrix, row tile); down: row tiles of
     // the result, each met by the k experts in turn (expert innermost).
-    const uint32_t tpm = (rows + TR - 1) / TR;
-    const uint32_t n_units = DOWN ? tpm : nq * A.n_mats * tpm;
-    const uint32_t va = n_units * blockIdx.x / gridDim.x, vb = n_units * (blockIdx.x + 1) / gridDim.x;  // (the host keeps the products below 2^32)
+    const uint32_t va = share * blockIdx.x + min(blockIdx.x, rest), vb = va + share + (blockIdx.x < rest ? 1u : 0u);
     if (va >= vb) return;
     const uint32_t nt = vb - va, n_virtual = DOWN ? nt * nq : nt;
+
+    uint32_t seg0 = 0, t0 = va;  // the share's first segment (slot, matrix) and row tile of it
+    if (!DOWN)
+        while (t0 >= tpm) { t0 -= tpm; seg0++; }
 
     // per-lane parts of a wave-tile's addresses: the lane's row within the tile and its block of each step
     // (a block past the row end is the row's last block again: its activations are zeros, so it adds nothing)
@@ -1907,14 +1918,14 @@ __global__ void __launch_bounds__(kMx4MaxWaves * 64) moe1_kernel(const Moe1Args 
     const uint32_t tile_w = TR * row_bytes, tile_s = TR * nb;
 
     // issue cursor: (segment = slot * n_mats + matrix, row tile) / (row tile, expert)
-    uint32_t it_seg = DOWN ? 0u : va / tpm, it_t = DOWN ? va : va - (va / tpm) * tpm, it_q = 0, it_left = n_virtual, slot_i = 0;
+    uint32_t it_seg = seg0, it_t = t0, it_q = 0, it_left = n_virtual, slot_i = 0;
     // the loads of the cursor's wave-tile (every lane takes part: no branch sits between the loads, so what is in flight
     // can be counted; lanes whose step does not exist copy a neighbouring block that nothing reads)
     auto issue_loads = [&]() {
-        const uint32_t q = DOWN ? it_q : (A.n_mats == 2 ? it_seg >> 1 : it_seg);
+        const uint32_t q = DOWN ? it_q : (n_mats == 2 ? it_seg >> 1 : it_seg);
         const uint8_t *wbase = q == 1 ? wq[1] : (q == 2 ? wq[2] : (q == 3 ? wq[3] : wq[0]));
         const uint8_t *sbase = q == 1 ? sq[1] : (q == 2 ? sq[2] : (q == 3 ? sq[3] : sq[0]));
-        if (!DOWN && A.n_mats == 2 && (it_seg & 1u)) { wbase += m1_w; sbase += m1_s; }
+        if (!DOWN && n_mats == 2 && (it_seg & 1u)) { wbase += m1_w; sbase += m1_s; }
         wbase += (size_t)it_t * tile_w;
         sbase += (size_t)it_t * tile_s;
         // lanes past the tile's last row (a tile of fewer than 16 rows, a ragged last tile) read that row again
@@ -1939,12 +1950,35 @@ __global__ void __launch_bounds__(kMx4MaxWaves * 64) moe1_kernel(const Moe1Args 
         it_left--;
         advance();
     };
+    // The biases of the first batch's rows, one row a thread of the fold (they are on their way with the tiles; a fold that
+    // asked for them at the end of a launch of one batch waited for memory once more).
+    const uint32_t rr0 = DOWN ? threadIdx.x >> 2 : threadIdx.x;
+    const bool has_bias = A.bias[0] != nullptr;
+    float bias0[DOWN ? kMoe1MaxK : 1];
+    auto load_bias = [&](uint32_t seg, uint32_t t, uint32_t jt, float (&to)[DOWN ? kMoe1MaxK : 1]) {
+        const uint32_t row = min(t * TR + jt, rows - 1);
+        if (DOWN) {
+#pragma unroll
+            for (int q = 0; q < (int)kMoe1MaxK; q++)
+                to[DOWN ? q : 0] = ((const GLOBAL_AS float *)A.bias[0])[(size_t)e[q] * A.bias_stride + (size_t)row * A.bias_step];
+        } else {
+            const uint32_t q = n_mats == 2 ? seg >> 1 : seg;
+            to[0] = ((const GLOBAL_AS float *)(n_mats == 2 && (seg & 1u) ? A.bias[1] : A.bias[0]))[(size_t)expert_of(q) * A.bias_stride + (size_t)row * A.bias_step];
+        }
+    };
+    auto first_biases = [&]() {
+        uint32_t seg = seg0, t = t0 + (rr0 >> 4);
+        if (!DOWN)
+            while (t >= tpm) { t -= tpm; seg++; }
+        if (rr0 < nt * 16) load_bias(seg, t, rr0 & 15u, bias0);
+    };
     // the first NS-1 wave-tiles without a branch around their loads (a share of fewer tiles reads its last one again)
     if (working) {
 #pragma unroll
         for (int s = 0; s + 1 < NS; s++) {
             issue_loads();
             if (it_left > 1) { it_left--; advance(); } else it_left = 0;
+            if (s == 0 && has_bias) first_biases();
             if (s == 0 && pre) load_operands();  // behind the first tile: they return in order, the tile first
         }
     }
@@ -1968,9 +2002,10 @@ __global__ void __launch_bounds__(kMx4MaxWaves * 64) moe1_kernel(const Moe1Args 
     constexpr uint32_t hw = DOWN ? 4u : 1u;  // partial sums per weight row and wavefront (down: one per expert)
     const uint32_t PW = nwj * hw, nwork = min(nwj, (steps + cw - 1) / cw);
     uint32_t use_i = 0, parity = 0;
-    uint32_t f_seg = DOWN ? 0u : va / tpm, f_t = DOWN ? va : va - (va / tpm) * tpm;  // the fold's cursor: first tile of the batch
+    uint32_t f_seg = seg0, f_t = t0;  // the fold's cursor: first tile of the batch
     uint32_t tl = 0, cq = 0;   // row tile within the batch, expert within the tile
     float acc = 0.f;
+    bool first = working;  // the first batch's biases are in registers
     for (uint32_t v = 0; v < n_virtual; v++) {
         float *pb = part + parity * (R * 16 * nw_launch * hw);
         if (working) {
@@ -2014,15 +2049,20 @@ __global__ void __launch_bounds__(kMx4MaxWaves * 64) moe1_kernel(const Moe1Args 
             for (uint32_t rr = threadIdx.x >> 2; rr < tl * 16; rr += blockDim.x >> 2) {
                 const uint32_t h = threadIdx.x & 3u;
                 float s = 0.f;
-                for (uint32_t w = 0; w < nwork; w++) s += pb[rr * PW + w * hw + h];
+                float pv[kMx4MaxWaves];  // (all on their way before the first is added)
+#pragma unroll
+                for (uint32_t w = 0; w < kMx4MaxWaves; w++) pv[w] = pb[rr * PW + min(w, nwork - 1) * hw + h];
+#pragma unroll
+                for (uint32_t w = 0; w < kMx4MaxWaves; w++) s = w < nwork ? s + pv[w] : s;
                 s = dpp_add<0xB1>(s);  // quad_perm [1,0,3,2]: experts 0+1, 2+3
                 s = dpp_add<0x4E>(s);  // quad_perm [2,3,0,1]: all four
                 const uint32_t jt = rr & 15u, row = (f_t + (rr >> 4)) * TR + jt;
                 if (h == 0 && jt < TR && row < rows) {
-                    if (A.bias[0]) {  // + sum_q w_q * bias_q[row], in selection order
+                    if (has_bias) {  // + sum_q w_q * bias_q[row], in selection order
+                        if (!(first && rr == rr0)) load_bias(0, f_t + (rr >> 4), jt, bias0);
 #pragma unroll
                         for (int q = 0; q < (int)kMoe1MaxK; q++)
-                            if (ok[q]) s += cwt[q] * ((const GLOBAL_AS float *)A.bias[0])[(size_t)e[q] * A.bias_stride + (size_t)row * A.bias_step];
+                            if (ok[q]) s += cwt[q] * bias0[DOWN ? q : 0];
                     }
                     ((g_f32wp)A.out[0])[row] = s;
                 }
@@ -2031,17 +2071,21 @@ __global__ void __launch_bounds__(kMx4MaxWaves * 64) moe1_kernel(const Moe1Args 
         } else {
             for (uint32_t rr = threadIdx.x; rr < tl * 16; rr += blockDim.x) {
                 float s = 0.f;
-                for (uint32_t w = 0; w < nwork; w++) s += pb[rr * PW + w];
+                float pv[kMx4MaxWaves];
+#pragma unroll
+                for (uint32_t w = 0; w < kMx4MaxWaves; w++) pv[w] = pb[rr * PW + min(w, nwork - 1)];
+#pragma unroll
+                for (uint32_t w = 0; w < kMx4MaxWaves; w++) s = w < nwork ? s + pv[w] : s;
                 // the tile of this row: `rr / 16` tiles past the batch's first
                 uint32_t seg = f_seg, t = f_t + (rr >> 4);
                 while (t >= tpm) { t -= tpm; seg++; }
-                const uint32_t q = A.n_mats == 2 ? seg >> 1 : seg, m = A.n_mats == 2 ? (seg & 1u) : 0u;
+                const uint32_t q = n_mats == 2 ? seg >> 1 : seg, m = n_mats == 2 ? (seg & 1u) : 0u;
                 const uint32_t jt = rr & 15u, row = t * TR + jt;
                 const bool live = jt < TR && row < rows;
                 if (live) {
-                    const float *bias = m ? A.bias[1] : A.bias[0];
+                    if (has_bias && !(first && rr == rr0)) load_bias(seg, t, jt, bias0);
                     if (!ok_of(q)) s = 0.0f;  // an expert outside the bank: no contribution (its stand-in's bytes were read, not used)
-                    else if (bias) s += ((const GLOBAL_AS float *)bias)[(size_t)expert_of(q) * A.bias_stride + (size_t)row * A.bias_step];
+                    else if (has_bias) s += bias0[0];
                 }
                 if (A.terms) {
                     // rows 2i (gate) and 2i+1 (up) sit in neighbouring lanes (rows and the block size are even)
@@ -2062,6 +2106,7 @@ __global__ void __launch_bounds__(kMx4MaxWaves * 64) moe1_kernel(const Moe1Args 
             while (f_t >= tpm) { f_t -= tpm; f_seg++; }
         }
         tl = 0;
+        first = false;
         parity ^= 1u;
     }
     LARQL_WAIT_VMCNT(0);
@@ -3614,7 +3659,11 @@ static hipError_t moe1_launch_cw(hipStream_t s, const Moe1Args &A, uint32_t grid
         if (e != hipSuccess) return e;
         attr_set = true;
     }
-    hipLaunchKernelGGL((moe1_kernel<DOWN, CW, moe1_stages(CW)>), dim3(grid), dim3(threads), lds, s, A);
+    const uint32_t tpm = (A.rows + A.tile_rows - 1) / A.tile_rows, units = DOWN ? tpm : A.k * A.n_mats * tpm;
+    const uint32_t geom = A.k | (A.nw << 8) | (A.n_mats == 2 ? kMoe1Apart : 0u) | (DOWN && A.terms ? kMoe1Terms : 0u);
+    const void *act = DOWN && A.terms ? (const void *)A.terms : (const void *)A.x;
+    hipLaunchKernelGGL((moe1_kernel<DOWN, CW, moe1_stages(CW)>), dim3(grid), dim3(threads), lds, s, A.logits, A.router_bias, A.experts, act, A.n_experts,
+                       A.kdim, geom, tpm, units / grid, units % grid, A);
     return hipGetLastError();
 }
 

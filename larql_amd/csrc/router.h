@@ -9,21 +9,18 @@ namespace larql {
 // Reductions over the wavefront by data-parallel primitives (four steps inside the rows of 16 lanes, two row
 // broadcasts, then lane 63 holds the result): a few cycles per step, where a cross-lane shuffle costs an LDS round trip.
 template <int CTRL, int ROW_MASK, bool BOUND>
-__device__ __forceinline__ uint64_t dpp_max_u64(uint64_t v) {  // lanes without a source read 0: the identity here
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, CTRL, ROW_MASK, 0xF, BOUND);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), CTRL, ROW_MASK, 0xF, BOUND);
-    const uint64_t other = ((uint64_t)hi << 32) | lo;
+__device__ __forceinline__ uint32_t dpp_max_u32(uint32_t v) {  // lanes without a source read 0: the identity here
+    const uint32_t other = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROW_MASK, 0xF, BOUND);
     return other > v ? other : v;
 }
-__device__ __forceinline__ uint64_t wave_max_u64(uint64_t v) {
-    v = dpp_max_u64<0xB1, 0xF, true>(v);    // quad_perm [1,0,3,2]
-    v = dpp_max_u64<0x4E, 0xF, true>(v);    // quad_perm [2,3,0,1]
-    v = dpp_max_u64<0x141, 0xF, true>(v);   // row_half_mirror
-    v = dpp_max_u64<0x140, 0xF, true>(v);   // row_mirror
-    v = dpp_max_u64<0x142, 0xA, false>(v);  // row_bcast:15 into rows 1 and 3
-    v = dpp_max_u64<0x143, 0xC, false>(v);  // row_bcast:31 into rows 2 and 3
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, 63), hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), 63);
-    return ((uint64_t)hi << 32) | lo;
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+    v = dpp_max_u32<0xB1, 0xF, true>(v);    // quad_perm [1,0,3,2]
+    v = dpp_max_u32<0x4E, 0xF, true>(v);    // quad_perm [2,3,0,1]
+    v = dpp_max_u32<0x141, 0xF, true>(v);   // row_half_mirror
+    v = dpp_max_u32<0x140, 0xF, true>(v);   // row_mirror
+    v = dpp_max_u32<0x142, 0xA, false>(v);  // row_bcast:15 into rows 1 and 3
+    v = dpp_max_u32<0x143, 0xC, false>(v);  // row_bcast:31 into rows 2 and 3
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 template <int CTRL, int ROW_MASK, bool BOUND>
 __device__ __forceinline__ float dpp_fmax(float v) {  // lanes without a source read -inf
@@ -56,10 +53,11 @@ __device__ __forceinline__ void router_select_lane(float l, uint32_t n_experts, 
                                                    uint32_t (&sel_idx)[kRouterMaxK], float (&sel_w)[kRouterMaxK]) {
     const bool has = lane < n_experts;
     l = has ? l : 0.0f;
-    // orderable key: logit bits made monotone, then ~index so the lower index wins a tie; 0 = absent
+    // orderable key: logit bits made monotone.  A rank is the largest key that is left (one fused maximum a step of the
+    // reduction, where a 64-bit key with the index in it took five instructions) and the lowest lane that holds it.
     const uint32_t bits = __builtin_bit_cast(uint32_t, l);
     const uint32_t ord = (bits & 0x80000000u) ? ~bits : (bits | 0x80000000u);
-    uint64_t key = has ? (((uint64_t)ord << 32) | (uint32_t)(~lane)) : 0;
+    bool left = has;
     float ex = 0.0f, denom = 0.0f;
     if (WEIGHTS) {
         const float dmax = wave_fmax(has ? l : -__builtin_inff());
@@ -72,11 +70,11 @@ __device__ __forceinline__ void router_select_lane(float l, uint32_t n_experts, 
     for (int r = 0; r < kRouterMaxK; r++) {
         sel_idx[r] = 0; sel_ex[r] = 0.0f;
         if ((uint32_t)r < k) {
-            const uint64_t best = wave_max_u64(key);
-            const uint32_t idx = ~(uint32_t)best & 63u;  // (k <= n_experts: a key is always left; the mask keeps the lane index in range regardless)
+            const uint32_t best = wave_max_u32(left ? ord : 0u);
+            const uint32_t idx = (uint32_t)__builtin_ctzll(__ballot(left && ord == best) | (1ull << 63));  // (k <= n_experts: a key is always left)
             sel_idx[r] = idx;
             if (WEIGHTS) sel_ex[r] = lane_value(ex, idx);
-            if (lane == idx) key = 0;
+            if (lane == idx) left = false;
         }
     }
     if (WEIGHTS && policy != 0) {
@@ -105,7 +103,8 @@ __device__ __forceinline__ void router_select_wide(const float *logits, const fl
                                                    uint32_t (&sel_idx)[kRouterMaxK], float (&sel_w)[kRouterMaxK]) {
     constexpr int S = kRouterWideSlots;
     float ex[S];
-    uint64_t key[S];
+    uint32_t key[S];
+    bool left[S];
     float l[S], lmax = -__builtin_inff();
 #pragma unroll
     for (int s = 0; s < S; s++) {
@@ -115,7 +114,8 @@ __device__ __forceinline__ void router_select_wide(const float *logits, const fl
         if (has) l[s] = bias ? logits[e] + bias[e] : logits[e];
         const uint32_t bits = __builtin_bit_cast(uint32_t, l[s]);
         const uint32_t ord = (bits & 0x80000000u) ? ~bits : (bits | 0x80000000u);
-        key[s] = has ? (((uint64_t)ord << 32) | (uint32_t)(~e)) : 0;
+        key[s] = has ? ord : 0u;
+        left[s] = has;
         lmax = has ? fmaxf(lmax, l[s]) : lmax;
     }
     float denom = 0.0f;
@@ -137,11 +137,16 @@ __device__ __forceinline__ void router_select_wide(const float *logits, const fl
     for (int r = 0; r < kRouterMaxK; r++) {
         sel_idx[r] = 0; sel_ex[r] = 0.0f;
         if ((uint32_t)r < k) {
-            uint64_t mine = key[0];
+            uint32_t mine = key[0];
 #pragma unroll
             for (int s = 1; s < S; s++) mine = key[s] > mine ? key[s] : mine;
-            const uint64_t best = wave_max_u64(mine);
-            const uint32_t idx = ~(uint32_t)best & (uint32_t)(64 * S - 1);             // (k <= n_experts: a key is always left)
+            const uint32_t best = wave_max_u32(mine);
+            uint32_t idx = 64 * S - 1;                                                 // (k <= n_experts: a key is always left)
+#pragma unroll
+            for (int s = S - 1; s >= 0; s--) {
+                const uint64_t at = __ballot(left[s] && key[s] == best);
+                idx = at ? 64u * (uint32_t)s + (uint32_t)__builtin_ctzll(at) : idx;
+            }
             const uint32_t slot = idx >> 6, owner = idx & 63u;                         // the same in every lane
             sel_idx[r] = idx;
             if (WEIGHTS) {
@@ -152,7 +157,7 @@ __device__ __forceinline__ void router_select_wide(const float *logits, const fl
             }
 #pragma unroll
             for (int s = 0; s < S; s++)
-                if (lane == owner && slot == (uint32_t)s) key[s] = 0;
+                if (lane == owner && slot == (uint32_t)s) { key[s] = 0; left[s] = false; }
         }
     }
     if (WEIGHTS && policy != 0) {

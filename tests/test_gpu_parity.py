@@ -2314,3 +2314,10 @@ def test_top_k_bounds_by_slices_of_the_row(be, fmt, case):
             assert [i for i, _ in hits] == by_abs[:k].tolist() and [v for _, v in hits] == sc[by_abs[:k]].tolist(), (n, k)
             hits = be.q8_0_gemv_topk(blocks, x8, n, 256, k)
             assert [i for i, _ in hits] == by_value[:k].tolist() and [v for _, v in hits] == val[by_value[:k]].tolist(), (n, k)
+
+
+@pytest.mark.parametrize("E,hidden,inter,interleaved", [(4, 256, 4352, 1), (4, 256, 4352, 0), (4, 5120, 320, 1), (5, 160, 160, 0), (5, 160, 160, 1)])
+def test_moe_mxfp4_one_token_folds_after_the_first(be, fmt, E, hidden, inter, interleaved):
+    """One token, biases: workgroups with more row tiles than a fold takes (whose later folds ask for their own biases), the widest
+    row (two result tiles a workgroup) and shares that are unequal or of one tile."""
+    test_moe_mxfp4_block_matches_oracle(be, fmt, 1, E, hidden, inter, True, interleaved)
