@@ -158,9 +158,9 @@ __global__ void __launch_bounds__(256) quantize_rows_to_q8k_kernel(const float *
 // as router_select_kernel does and applies MoeExpertScalePolicy::PerExpert where a scale table is given (as
 // expert_scale_kernel does) while the others, a wavefront per super-block up to eleven, quantise the token's row as
 // quantize_rows_to_q8k_kernel does (four wavefronts, the first of them after its selection: 9.0 -> 6.1 us for 16 tokens of 2816).
-// The workgroups behind the tokens write the job tables of the two matvec launches that follow, a thread per job and per share:
-// they are uniform, so the host need not build and upload them (two copies of 70 and 35 KB that the stream waited for,
-// 22 us each in a layer of 150 us with 16 tokens, 128 experts and top-8, now 107 us).
+// Where the matvecs run as a job per slot (rows or calls beyond the grouped kernel), the workgroups behind the tokens write the job
+// tables of the two launches that follow, a thread per job and per share: they are uniform, so the host need not build and upload
+// them (two copies of 70 and 35 KB that the stream waited for, 22 us each with 16 tokens, 128 experts and top-8).
 constexpr uint32_t kRouteQuantWaves = 12;
 struct JobTables { JobTableSpec t[2]; };
 __device__ __forceinline__ void write_job_table(const JobTableSpec &T, uint32_t i) {
