@@ -46,15 +46,18 @@ __device__ const uint32_t kMgZeros[4] = {0u, 0u, 0u, 0u};  // what an operand la
 __device__ __forceinline__ uint32_t moe_term_at(uint32_t e) { return (e & ~127u) | ((e & 24u) << 2) | ((e & 96u) >> 2) | (e & 7u); }
 
 template <bool DOWN, int CW, int TG>
-__global__ void __launch_bounds__(512) moe_group_kernel(const MoeGroupArgs A) {
+__global__ void __launch_bounds__(512)
+    moe_group_kernel(const uint32_t *experts, uint32_t slots, uint32_t nE, uint32_t kdim, uint32_t rows,
+                     uint32_t grid,  // (in registers when the wavefront starts: the way to the experts' ids)
+                     const MoeGroupArgs A) {
     extern __shared__ __attribute__((aligned(16))) uint8_t mg_lds[];
     constexpr int NS = kMgStages, R = mg_tiles(CW, TG), NT = TG == 16 ? 3 : 1, TP = TG / 2;  // NT: A operands, TP: pairs of tokens
     constexpr uint32_t slot_bytes = mg_slot_bytes(CW);
     constexpr int L = CW + 1 + (CW > 4);  // copies per tile
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wv = __builtin_amdgcn_readfirstlane(tid >> 6), nw = blockDim.x >> 6;
     const uint32_t jr = lane & 15u, kg = lane >> 4;
-    const uint32_t kdim = A.kdim, nb = kdim / 32, row_bytes = nb * 16, steps = (kdim + 127) / 128;
-    const uint32_t slots = A.slots, nE = A.n_experts, tpm = A.rows / 16;
+    const uint32_t nb = kdim / 32, row_bytes = nb * 16, steps = (kdim + 127) / 128;
+    const uint32_t tpm = rows / 16;
     uint8_t *ring = mg_lds + wv * (NS * slot_bytes);
     float *part = reinterpret_cast<float *>(mg_lds + nw * (NS * slot_bytes));  // [2][R][nw][16 rows][TG tokens]
     const uint32_t part_floats = R * nw * 16 * TG;
@@ -67,17 +70,17 @@ __global__ void __launch_bounds__(512) moe_group_kernel(const MoeGroupArgs A) {
     const uint32_t step0 = wv * CW;  // (below `steps`: the launch has no more wavefronts than K-ranges)
 
     // 1. slots per expert, groups before each expert
-    expert_groups_count<TG>(G, A.experts, slots, nE, tid, lane, wv);
+    expert_groups_count<TG>(G, experts, slots, nE, tid, lane, wv);
 
     // 2. this workgroup's share of the list (group, 16-row tile).  Workgroups are dealt to the eight XCDs in turn: an XCD
     //    takes neighbouring shares, whose groups' operands then sit in its L2.
     //    A group opens with kStart units of its own: who meets a second group in its share starts twice (list, operands, first
     //    tiles), so it gets that many tiles fewer.
     constexpr uint32_t kStart = TG == 16 ? 6 : 4;
-    const uint32_t per_group = tpm + kStart, units = G.before[nE] * per_group, grid = gridDim.x;
+    const uint32_t per_group = tpm + kStart, units = __builtin_amdgcn_readfirstlane(G.before[nE]) * per_group;
     const uint32_t share = (grid & 7u) ? blockIdx.x : (blockIdx.x & 7u) * (grid >> 3) + (blockIdx.x >> 3);
-    uint32_t v = (uint32_t)((uint64_t)units * share / grid);
-    const uint32_t v_end = (uint32_t)((uint64_t)units * (share + 1) / grid);
+    uint32_t v, v_end;
+    expert_group_share(units, share, grid, v, v_end);
 
     // per-lane parts of a tile's addresses: the block of each step, clamped into the row (a step past the row end meets
     // zero activations), and where its scale byte lies in the slot
@@ -172,8 +175,8 @@ __global__ void __launch_bounds__(512) moe_group_kernel(const MoeGroupArgs A) {
                 const uint32_t row = (f_tile + tile) * 16 + r;
                 if (A.bias) { const float bv = f_bias[tile * 16 + r]; s.x += bv; s.y += bv; }
                 if (DOWN) {
-                    if (2 * p < ntok) ((g_f32wp)A.out)[(size_t)gl[2 * p] * A.rows + row] = s.x;
-                    if (2 * p + 1 < ntok) ((g_f32wp)A.out)[(size_t)gl[2 * p + 1] * A.rows + row] = s.y;
+                    if (2 * p < ntok) ((g_f32wp)A.out)[(size_t)gl[2 * p] * rows + row] = s.x;
+                    if (2 * p + 1 < ntok) ((g_f32wp)A.out)[(size_t)gl[2 * p + 1] * rows + row] = s.y;
                 } else {
                     // the thread of a gate row (even) gates its first token, the one of the up row, TP lanes on, the second
                     constexpr int CTRL = TP == 8 ? 0x128 : 0x4E;  // row_ror:8 / quad_perm [2,3,0,1]
@@ -187,7 +190,7 @@ __global__ void __launch_bounds__(512) moe_group_kernel(const MoeGroupArgs A) {
                     uint32_t t3[3];
                     mx4_terms(act, 0.0f, t3);
                     if (token < ntok) {
-                        const size_t opad = moe_terms_pad(A.rows / 2), plane = slots * opad;
+                        const size_t opad = moe_terms_pad(rows / 2), plane = slots * opad;
                         GLOBAL_AS uint16_t *tp = (GLOBAL_AS uint16_t *)A.terms_out + gl[token] * opad + moe_term_at(row >> 1);
                         tp[0] = (uint16_t)t3[0]; tp[plane] = (uint16_t)t3[1]; tp[2 * plane] = (uint16_t)t3[2];
                     }
@@ -203,7 +206,7 @@ __global__ void __launch_bounds__(512) moe_group_kernel(const MoeGroupArgs A) {
             // would be waited for behind every tile in flight.  This copy is older than the tiles that may still fly when
             // the batch's last tile is waited for, so it has landed by then; anywhere else it only makes a wait stricter.
             if (A.bias && wv == turn) {
-                const float *bp = A.bias + (size_t)e * A.rows + (t0 + tb) * 16;
+                const float *bp = A.bias + (size_t)e * rows + (t0 + tb) * 16;
 #pragma unroll
                 for (int q = 0; q < (R * 16 + 63) / 64; q++)
                     if (q * 64 + lane < (uint32_t)R * 16)
@@ -323,7 +326,8 @@ static hipError_t mg_launch(hipStream_t s, const MoeGroupArgs &A, uint32_t cu_co
                        (2 * (size_t)A.n_experts + 1) * sizeof(uint32_t) + (32 + (size_t)A.slots) * sizeof(uint16_t);
     if (lds > 160 * 1024) return hipErrorInvalidValue;
     const uint32_t per_cu = std::max<uint32_t>(1, std::min<uint32_t>((160 * 1024) / (uint32_t)lds, 8 / nw));
-    hipLaunchKernelGGL((moe_group_kernel<DOWN, CW, TG>), dim3(cu_count * per_cu), dim3(nw * 64), lds, s, A);
+    hipLaunchKernelGGL((moe_group_kernel<DOWN, CW, TG>), dim3(cu_count * per_cu), dim3(nw * 64), lds, s, A.experts, A.slots, A.n_experts, A.kdim, A.rows,
+                       cu_count * per_cu, A);
     return hipGetLastError();
 }
 

@@ -95,15 +95,20 @@ __device__ __forceinline__ KgCol6 kg_load_col6(const uint8_t *const (&of)[4], ui
 }
 
 template <bool Q6>
-__global__ void __launch_bounds__(kKgMaxWaves * 64) moe_kq_group_kernel(const MoeKqGroupArgs A, const uint32_t ways) {
+__global__ void __launch_bounds__(kKgMaxWaves * 64)
+    moe_kq_group_kernel(const uint32_t *experts, uint32_t slots, uint32_t nE, uint32_t cols, uint32_t ways, uint32_t rows,
+                        uint32_t grid,  // (in registers when the wavefront starts: the way to the experts' ids)
+                        const MoeKqGroupArgs A) {
 #pragma clang fp contract(off)
     extern __shared__ __attribute__((aligned(16))) uint8_t kg_lds[];
     typedef KgFormat<Q6> F;
     constexpr int NS = F::kStages, R = F::kTiles, L = F::kCopies, SET = Q6 ? 4 : 2, NSET = kKgSlots / SET;  // SET: slots that share an operand
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wv = __builtin_amdgcn_readfirstlane(tid >> 6), cols = A.cols, nw = cols * ways;
-    const uint32_t col_i = wv % cols, way = wv / cols, kRows = ways * (R * 16);
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wv = __builtin_amdgcn_readfirstlane(tid >> 6), nw = cols * ways;
+    const uint32_t kRows = ways * (R * 16);
+    uint32_t col_i = wv, way = 0;
+    while (col_i >= cols) { col_i -= cols; way++; }
     const uint32_t jr = lane & 15u, kq = lane >> 4;
-    const uint32_t nE = A.n_experts, slots = A.slots, rows = A.rows, row_bytes = cols * F::kBlock;
+    const uint32_t row_bytes = cols * F::kBlock;
     uint8_t *ring = kg_lds + wv * (NS * F::kTileBytes);
     float *part = reinterpret_cast<float *>(kg_lds + nw * (NS * F::kTileBytes));  // [2][column][slot][kRows]
     const uint32_t part_floats = cols * kKgSlots * kRows;
@@ -112,14 +117,14 @@ __global__ void __launch_bounds__(kKgMaxWaves * 64) moe_kq_group_kernel(const Mo
     G.before = G.cnt + nE;
     uint16_t *list = reinterpret_cast<uint16_t *>(G.before + nE + 1);  // [2][8]
     G.ex = list + 2 * kKgSlots;
-    expert_groups_count<kKgSlots>(G, A.experts, slots, nE, tid, lane, wv);
+    expert_groups_count<kKgSlots>(G, experts, slots, nE, tid, lane, wv);
 
     // this workgroup's share of the list (group, 16-row tile); a group opens with kStart units of its own, what its start costs
     constexpr uint32_t kStart = 3;
-    const uint32_t tpm = (rows + 15) / 16, per_group = tpm * A.n_mats + kStart, units = G.before[nE] * per_group, grid = gridDim.x;
+    const uint32_t tpm = (rows + 15) / 16, per_group = tpm * A.n_mats + kStart, units = __builtin_amdgcn_readfirstlane(G.before[nE]) * per_group;
     const uint32_t share = (grid & 7u) ? blockIdx.x : (blockIdx.x & 7u) * (grid >> 3) + (blockIdx.x >> 3);  // neighbours on one XCD
-    uint32_t v = (uint32_t)((uint64_t)units * share / grid);
-    const uint32_t v_end = (uint32_t)((uint64_t)units * (share + 1) / grid);
+    uint32_t v, v_end;
+    expert_group_share(units, share, grid, v, v_end);
 
     // lane's pieces of a wave-tile: row and place there.  Q4_K: 16-byte unit u = row * 9 + piece, the last 256 bytes dword by dword;
     // Q6_K: u = row * 13 + piece (u < 208), and lanes 16..31 of the fourth copy bring the end of row lane - 16
@@ -326,7 +331,8 @@ static hipError_t kg_launch(hipStream_t s, const MoeKqGroupArgs &A, uint32_t cu_
         allowed = true;
     }
     const uint32_t ways = kg_ways<Q6>(A.cols, A.n_experts, A.slots);
-    hipLaunchKernelGGL(moe_kq_group_kernel<Q6>, dim3(cu_count), dim3(A.cols * ways * 64), kg_lds_bytes<Q6>(A.cols, ways, A.n_experts, A.slots), s, A, ways);
+    hipLaunchKernelGGL(moe_kq_group_kernel<Q6>, dim3(cu_count), dim3(A.cols * ways * 64), kg_lds_bytes<Q6>(A.cols, ways, A.n_experts, A.slots), s, A.experts, A.slots,
+                       A.n_experts, A.cols, ways, A.rows, cu_count, A);
     return hipGetLastError();
 }
 
