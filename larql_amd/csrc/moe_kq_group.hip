@@ -287,10 +287,11 @@ __global__ void __launch_bounds__(kKgMaxWaves * 64)
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
-            // a lane per (slot, row): super-blocks in order.  `ways` wavefronts hold the rows of a batch, so the slots go round `cols`
-            // sets of them
-            const uint32_t rr = (wv % ways) * 64 + lane, tile = tb + rr / 16, m = tile >= tpm ? 1u : 0u, row = (tile - m * tpm) * 16 + (rr & 15u);
-            for (uint32_t s = wv / ways; s < ns; s += cols) {
+            // A lane per (slot, row): super-blocks in order.  A batch has kRows rows, R * 16 per way; a wavefront takes 64 / (R * 16)
+            // slots of one way's rows (Q4_K: one slot; Q6_K: two of 32 rows each), and the slots go round `cols` sets of wavefronts.
+            constexpr uint32_t kWayRows = R * 16, kFoldSlots = 64 / kWayRows;
+            const uint32_t rr = (wv % ways) * kWayRows + lane % kWayRows, tile = tb + rr / 16, m = tile >= tpm ? 1u : 0u, row = (tile - m * tpm) * 16 + (rr & 15u);
+            for (uint32_t s = (wv / ways) * kFoldSlots + lane / kWayRows; s < ns; s += cols * kFoldSlots) {
                 const float *pv = pb + s * kRows + rr;
                 float acc = 0.f;
 #pragma unroll 4

@@ -2280,6 +2280,56 @@ def test_moe_layer_k_quant_slots_share_an_expert(be, fmt, T, E, k, hidden, cols,
     test_moe_layer_over_a_k_quant_bank_matches_the_integer_expert_path(be, fmt, T, E, k, hidden, cols, inter, wfmt, 1, True, False)
 
 
+def _k_quant_layer(be, fmt, seed, T, E, k, hidden, inter, wfmt):
+    """A k-quant layer and inputs for T tokens: (layer, router input, x, gate_up bytes, down bytes)."""
+    rng = np.random.default_rng(seed)
+    quant = O.quantize_q4_k if wfmt == "q4k" else O.quantize_q6_k
+    gate_up = [quant((rng.standard_normal((2 * inter, hidden)) * 0.05).astype(F)) for _ in range(E)]
+    down = [quant((rng.standard_normal((hidden, -(-inter // 256) * 256)) * 0.05).astype(F)) for _ in range(E)]
+    router_w = (rng.standard_normal((E, hidden)) * 0.05).astype(F)
+    x = rng.standard_normal((T, hidden)).astype(F)
+    layer = be.moe_layer_create(gate_up, down, None, None, router_w, k, hidden, inter, fmt.MOE_ROWS_CONTIGUOUS_HALVES,
+                                expert_scales=fmt.MOE_SCALES_INLINE, expert_data_format=fmt.FMT_Q4_K if wfmt == "q4k" else fmt.FMT_Q6_K, gate_rule=1)
+    assert layer, be.last_error()
+    return layer, (x * F(0.5) + F(0.25)).astype(F), x, gate_up, down
+
+
+def _same_in_calls_of(be, layer, rin, x, k, step, whole):
+    """Calls of `step` tokens give the rows of `whole`, one call over all of them, bit for bit."""
+    out, experts, weights = whole
+    for t in range(0, len(x), step):
+        part = be.moe_layer_forward(layer, rin[t:t + step], x[t:t + step], k)
+        assert part is not None, be.last_error()
+        assert np.array_equal(part[1], experts[t:t + step]) and np.array_equal(part[2].view(np.uint32), weights[t:t + step].view(np.uint32)), t
+        assert np.array_equal(part[0].view(np.uint32), out[t:t + step].view(np.uint32)), t
+
+
+@pytest.mark.parametrize("T,E,k,hidden,inter", [
+    (128, 8, 4, 1792, 768),     # gate and up: rows of seven super-blocks, one way; down: three, four ways
+    (128, 12, 8, 1024, 512),    # ... four super-blocks, three ways; two, six ways
+    (96, 24, 8, 2560, 256),     # ... ten super-blocks, one way; one, twelve ways
+])
+@pytest.mark.parametrize("wfmt", ["q4k", "q6k"])
+def test_moe_layer_k_quant_groups_over_many_tiles(be, fmt, T, E, k, hidden, inter, wfmt):
+    """Shares of several groups, and of more tiles than a workgroup takes between two folds (both sets of partial sums, every ring
+    slot used again, a fold's last rows beside the next batch's first), against the same tokens two at a time, whose shares are a
+    fraction of that, bit for bit, and against the checker."""
+    layer, rin, x, gate_up, down = _k_quant_layer(be, fmt, 4000 + T + hidden, T, E, k, hidden, inter, wfmt)
+    whole = be.moe_layer_forward(layer, rin, x, k)
+    assert whole is not None, be.last_error()
+    out, experts, weights = whole
+    # what the sizes are for: tiles (of 16 rows) a workgroup has in a launch, and the most that it takes in one batch
+    cus = int(be.device_info().split(" CUs")[0].split()[-1])
+    groups = int(sum(-(-int(n) // 8) for n in np.bincount(experts.reshape(-1))))
+    ways_tiles = 4 if wfmt == "q4k" else 2
+    for tiles, cols in ((2 * (inter // 16), hidden // 256), (hidden // 16, inter // 256)):
+        assert groups * tiles // cus > ways_tiles * (12 // cols), (groups, tiles, cols)
+    _same_in_calls_of(be, layer, rin, x, k, 2, whole)
+    want = O.moe_block_kq(x[:3], experts[:3], weights[:3], gate_up, down, hidden, hidden, inter, 4 if wfmt == "q4k" else 6, None, None, 1)
+    assert rel_l2(out[:3], want) < 2e-4
+    be.moe_layer_destroy(layer)
+
+
 @pytest.mark.parametrize("case", ["normal", "narrow", "coarse", "constant", "wide", "few"])
 def test_top_k_bounds_by_slices_of_the_row(be, fmt, case):
     """The short way's bound (the K-th largest maximum of 128 slices, of 512 above K = 64; fourteen bits of it) over rows whose scores
