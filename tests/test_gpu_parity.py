@@ -1199,7 +1199,7 @@ def test_moe_mxfp4_routed_equals_select_then_block(be, fmt, T, E, hidden, inter,
     assert be.dev_moe_mxfp4(b, x, T, k, e1, w1, o1, ws, wsb)
     be.synchronize()
     want = (be.d2h(e1, (T, k), np.uint32), be.d2h(w1, (T, k), F), be.d2h(o1, (T, hidden), F))
-    for rep in range(2):                                   # (the second call finds its job tables already on the device)
+    for rep in range(2):
         assert be.dev_moe_mxfp4_routed(b, x, T, k, dl, policy, e2, w2, o2, ws, wsb)
         be.synchronize()
         got = (be.d2h(e2, (T, k), np.uint32), be.d2h(w2, (T, k), F), be.d2h(o2, (T, hidden), F))
@@ -1444,7 +1444,7 @@ def test_moe_layer_from_per_expert_slices_with_router_projection(be, fmt, T, E, 
     (1, 6, 2, 2816, 2816, 704, "q4k", 1, False, False),    # Gemma 4 26B-A4B's real expert shape
     (4, 5, 3, 512, 512, 320, "q6k", 2, True, False),       # a Q6_K bank, SiLU
     (1, 4, 2, 256, 768, 256, "q6k", 1, False, True),
-    (300, 8, 2, 256, 256, 256, "q4k", 2, True, False),     # many tokens: 600 slots, job tables of 1200 and 600 entries
+    (300, 8, 2, 256, 256, 256, "q4k", 2, True, False),     # many tokens: 600 slots in groups of eight
 ])
 def test_moe_layer_over_a_k_quant_bank_matches_the_integer_expert_path(be, fmt, T, E, k, hidden, cols, inter, wfmt, rule, biases, per_expert):
     """MoeLayerWeights with expert_data_format Q4_K / Q6_K (Inline scales, ContiguousHalves rows): cpu_moe_forward's
@@ -1481,7 +1481,7 @@ def test_moe_layer_over_a_k_quant_bank_matches_the_integer_expert_path(be, fmt, 
     assert rel_l2(out, want_out) < 2e-4
     dx, dr, do = be.to_device(x), be.to_device(rin), be.malloc(T * hidden * 4)
     de, dw_ = be.malloc(T * k * 4), be.malloc(T * k * 4)
-    for rep in range(2):                                   # (the second call finds its job tables already on the device)
+    for rep in range(2):
         assert be.dev_moe_layer_forward(layer, dr, dx, T, do, de, dw_)
         be.synchronize()
         assert np.array_equal(be.d2h(do, (T, hidden), F).view(np.uint32), out.view(np.uint32))
@@ -2273,7 +2273,9 @@ def test_short_launches_equal_the_streaming_kernel_bit_for_bit(be, fmt, fmt_name
     (9, 1, 1, 272, 512, 300),      # one expert with nine slots: a group of eight and one of one; ragged last tiles of gate and up
     (16, 2, 2, 256, 256, 17),      # two full groups per expert; a tile and one row, rows of one super-block
     (3, 4, 4, 1040, 3072, 40),     # twelve super-blocks: the most that the grouped kernel takes
-    (2, 4, 2, 256, 3328, 48),      # thirteen: a matvec per slot
+    (2, 4, 2, 256, 3328, 48),      # thirteen: a matvec per slot, eight and four jobs (they travel with the launch)
+    (5, 4, 2, 272, 3328, 48),      # ... twenty and ten: tables that the routing launch writes on the device
+    (150, 6, 3, 256, 3328, 24),    # ... 900 and 450, several writing workgroups
 ])
 @pytest.mark.parametrize("wfmt", ["q4k", "q6k"])
 def test_moe_layer_k_quant_slots_share_an_expert(be, fmt, T, E, k, hidden, cols, inter, wfmt):
@@ -2327,6 +2329,22 @@ def test_moe_layer_k_quant_groups_over_many_tiles(be, fmt, T, E, k, hidden, inte
     _same_in_calls_of(be, layer, rin, x, k, 2, whole)
     want = O.moe_block_kq(x[:3], experts[:3], weights[:3], gate_up, down, hidden, hidden, inter, 4 if wfmt == "q4k" else 6, None, None, 1)
     assert rel_l2(out[:3], want) < 2e-4
+    be.moe_layer_destroy(layer)
+
+
+@pytest.mark.parametrize("hidden,inter", [(256, 40), (1536, 272), (2816, 24)])
+@pytest.mark.parametrize("wfmt", ["q4k", "q6k"])
+def test_moe_layer_k_quant_groups_equal_a_matvec_per_slot(be, fmt, hidden, inter, wfmt):
+    """A call of more than 4096 slots runs a matvec per slot, from job tables that the routing launch writes on the device; calls of
+    less share an expert's weights between its slots: the same bits."""
+    T, E, k = 520, 12, 8
+    layer, rin, x, gate_up, down = _k_quant_layer(be, fmt, 5000 + hidden, T, E, k, hidden, inter, wfmt)
+    whole = be.moe_layer_forward(layer, rin, x, k)
+    assert whole is not None, be.last_error()
+    assert whole[1].size > 4096
+    _same_in_calls_of(be, layer, rin, x, k, 130, whole)
+    want = O.moe_block_kq(x[:3], whole[1][:3], whole[2][:3], gate_up, down, hidden, hidden, inter, 4 if wfmt == "q4k" else 6, None, None, 1)
+    assert rel_l2(whole[0][:3], want) < 2e-4
     be.moe_layer_destroy(layer)
 
 
