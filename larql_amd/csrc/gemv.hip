@@ -3612,6 +3612,7 @@ static hipError_t gemv_short_launch(hipStream_t stream, const GemvLaunch &L, uin
     }
     late.w3 = w[3]; late.begin3 = begin[3]; late.rows3 = rows[3];
     const uint32_t geom = (uint32_t)(L.inl[0].k / 256) | (threads / 64) << 8 | tr << 13 | (L.n_jobs > 3 ? kShortFour : 0u);
+    static_assert(LastParam<decltype(gemv_short_kernel<false, 1, 1>)>::offset() == kShortLateAt, "read through the kernarg pointer");
 #define LARQL_SHORT(Q6, NT, NP) case (Q6) | (NT) << 1 | (NP) << 5: \
         hipLaunchKernelGGL((gemv_short_kernel<Q6, NT, NP>), dim3(grid), dim3(threads), lds, stream, L.inl[0].x, w[0], w[1], w[2], geom, begin[1], begin[2], \
                            rows[0], rows[1], rows[2], late); break;
@@ -3687,7 +3688,8 @@ hipError_t moe1_launch(hipStream_t s, const Moe1Args &A, bool down, uint32_t gri
 
 hipError_t gemv_launch(hipStream_t stream, int kind, const GemvLaunch &L, uint32_t threads, uint32_t grid, size_t lds) {
     const uint32_t share = grid ? (uint32_t)(L.total_passes / grid) : 0, rest = grid ? (uint32_t)(L.total_passes % grid) : 0;
-#define LARQL_JOBS_LAUNCH(KERNEL) \
+#define LARQL_JOBS_LAUNCH(KERNEL)                                                                                    \
+    static_assert(LastParam<decltype(KERNEL)>::offset() == kInlineAt, "the jobs are read through the kernarg pointer"); \
     hipLaunchKernelGGL(KERNEL, dim3(grid), dim3(threads), lds, stream, L.table, L.wg_first, share, rest, L.n_jobs, L.pad, L.inl)
     switch (kind) {
         case KIND_Q8_0_MFMA: {

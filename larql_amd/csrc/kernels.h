@@ -6,6 +6,17 @@
 
 namespace larql {
 
+// Where a kernel's last parameter lies in its argument block (parameters are laid out as the members of a structure are): for the
+// kernels that read that one through the kernarg pointer.
+template <class F> struct LastParam;
+template <class... P> struct LastParam<void(P...)> {
+    static constexpr size_t offset() {
+        size_t at = 0, end = 0;
+        ((at = (end + alignof(P) - 1) / alignof(P) * alignof(P), end = at + sizeof(P)), ...);
+        return at;
+    }
+};
+
 enum GemvKind : int32_t {
     KIND_Q4K = 0, KIND_Q8_0 = 1, KIND_MXFP4 = 2, KIND_Q4_0 = 3, KIND_BF16 = 4, KIND_F16 = 5, KIND_F32 = 6,
     KIND_Q4K_MFMA = 7,   // internal: Q4_K rows short enough for the matrix-core kernel (see gemv_effective_kind)
