@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "mx4.h"
+#include "wave.h"
 
 namespace larql {
 
@@ -13,17 +14,6 @@ struct ExpertGroups {
     uint32_t *cnt, *before;
     uint16_t *ex;
 };
-
-// inclusive sums over a wavefront by data-parallel primitives (a shuffle goes through LDS hardware, a round trip per step)
-__device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t v) {
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false);  // row_shr:1
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false);  // row_shr:2
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false);  // row_shr:4
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false);  // row_shr:8
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
-    return v;
-}
 
 // Counts the slots per expert and the groups of up to TG slots before each expert; an id outside the bank belongs to nobody.
 // The whole workgroup calls it; it ends with a barrier.

@@ -13,6 +13,7 @@
 #include <stdlib.h>
 
 #include "kernels.h"
+#include "wave.h"
 
 namespace larql {
 
@@ -44,21 +45,6 @@ __device__ __forceinline__ float half_to_float(uint32_t lo16) { return (float)__
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-
-// Reductions by data-parallel primitives (a few cycles each; a cross-lane shuffle is a trip through LDS hardware).  Lanes without a
-// source bring 0: the values are non-negative.
-template <int CTRL, int ROW_MASK = 0xF>
-__device__ __forceinline__ float dpp_move(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, ROW_MASK, 0xF, true));
-}
-template <int CTRL, int ROW_MASK = 0xF>
-__device__ __forceinline__ float dpp_max(float v) { return fmaxf(v, dpp_move<CTRL, ROW_MASK>(v)); }
-__device__ __forceinline__ float row16_max(float v) {
-    v = dpp_max<0xB1>(v);     // quad_perm [1,0,3,2]
-    v = dpp_max<0x4E>(v);     // quad_perm [2,3,0,1]
-    v = dpp_max<0x141>(v);    // row_half_mirror
-    return dpp_max<0x140>(v); // row_mirror
-}
 
 // one block per token: scale, f16 terms, sub-block sums.  `x_is_bf16`: 16-bit inputs (exact in one term).
 // A thread takes 8 consecutive elements at a time (one or two 16-byte loads); four neighbouring threads hold a
