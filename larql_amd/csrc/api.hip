@@ -282,12 +282,21 @@ int prepare_same_kind(larql_hip_ctx *c, GemvJob *live, size_t n_live, void *tabl
     }
     P.lds = gemv_lds_bytes(live, n_live, P.threads);
     uint64_t grid = (uint64_t)c->cu_count * (uint64_t)gemv_wgs_per_cu(P.kind, P.threads, P.lds, (uint32_t)c->wgs_per_cu);
-    if (P.kind == KIND_Q4K_MFMA || P.kind == KIND_Q4K_Q8K) {
-        // A launch with fewer 16-row tiles than workgroups: one workgroup per tile (and one more per job for its set-up
+    if (P.kind == KIND_Q4K_MFMA || P.kind == KIND_Q4K_Q8K || P.kind == KIND_Q6K_MFMA || P.kind == KIND_MXFP4_MFMA || P.kind == KIND_Q8_0_MFMA ||
+        P.kind == KIND_BF16_MFMA || P.kind == KIND_Q4K_BATCH) {
+        // A launch with fewer 16-row tiles than workgroups: one workgroup per tile (and more per job for its set-up
         // allowance), so that the tiles sit on consecutive workgroups — spread over the XCDs and CUs — and not on every
-        // n-th one, where two of them can meet on a CU while others stand idle (a 3072 x 1024 matvec alone: 5.3 -> 4.3 us).
+        // n-th one, where two of them can meet on a CU while others stand idle, or all of them on one XCD or two
+        // (every n-th / consecutive, us, weights from HBM: Q4_K 3072 x 1024 5.3 / 4.3; Q6_K 16384 x 256 6.7 / 4.7, 4096 x 2816
+        // 11.5 / 7.2; MXFP4 4096 x 512 8.4 / 5.35, 4096 x 2304 12.6 / 7.6; Q8_0 12288 x 512 6.8 / 5.8, 4096 x 1280 8.8 / 5.7;
+        // a launch of 4 to 64 tiles up to 5 % the other way: Q8_0 three of 64 x 2048 5.3 / 5.6).
         uint64_t tiles = 0;
-        for (size_t ji = 0; ji < n_live; ji++) tiles += (live[ji].rows + 15) / 16 + 1;
+        for (size_t ji = 0; ji < n_live; ji++) {
+            const GemvJob &j = live[ji];
+            // (Q4_K: the costs are refined below, where a share's set-up becomes part of its tiles; one workgroup is enough)
+            const uint32_t set_up = P.kind == KIND_Q6K_MFMA ? (j.pad2 + j.pad - 1) / j.pad : P.kind == KIND_Q4K_MFMA || P.kind == KIND_Q4K_Q8K ? 1 : 0;
+            tiles += (j.rows + 15) / 16 + set_up;
+        }
         if (grid > tiles) grid = tiles;
     }
     // the share-out's cost model wants to know how long a workgroup's share is: a second pass over the costs
