@@ -1038,9 +1038,8 @@ __device__ __forceinline__ void run_q6k_mfma(const GemvJob &j, uint32_t tile_a, 
 // More wavefronts than the streaming kernel's (sixteen of one or two columns for rows of 11 to 32 super-blocks, each column's partial
 // in LDS for the fold) were measured: 2560 x 4096 3.8 -> 4.0 us, 2560 x 5120 4.1 -> 4.5, 8192 x 7680 8.8 -> 9.4, 2560 x 10240 5.9 -> 6.6;
 // 12288 x 3840 7.2 -> 7.0 alone.
-// Q6_K: its super-blocks lie 2 bytes off, which costs the direct loads more per byte than the streaming kernel's copies: it gains
-// where the columns are one per wavefront (rows of up to ten super-blocks) and the tiles up to four: 2560 x 2560 6.9 -> 4.2, 8192 x
-// 2560 9.0 -> 6.8, 16384 x 2560 11.9 -> 11.3, 20480 x 2560 13.1 -> 13.6 (streaming -> short).
+// Q6_K: its super-blocks lie 2 bytes off, which costs the direct loads more per byte than the streaming kernel's copies, so it has
+// fewer tiles (the lines and both sides at gemv_short).
 // ---------------------------------------------------------------------------
 constexpr uint32_t kShortJobs = 4;       // matvecs of a launch
 // geom: columns per row | wavefronts << 8 | rows per tile << 13 | a fourth matvec << 18
@@ -3567,8 +3566,13 @@ size_t gemv_lds_bytes(const GemvJob *jobs, size_t n, uint32_t threads) {
 // 5.8 TB/s).  Streaming / short kernel on the same launch, us: one tile of 512 / 2560 / 10240 elements 3.8 / 3.2, 5.0 / 3.2, 7.7 / 6.1;
 // eight tiles of 512 / 1024 / 2560 5.8 / 5.7, 5.7 / 5.4, 10.8 / 9.9; at the line 5120 elements x five tiles 13.4 / 12.1, 7680 x three
 // 12.1 / 11.3, 10240 x two 10.7 / 10.6.  Rows of one super-block have one wavefront per workgroup, which walks its tiles alone:
-// one to four tiles 3.8 / 3.2, 3.9 / 3.3, 3.8 / 3.8, 4.0 / 4.3, six 4.1 / 5.4, so the line is three there.  Q6_K: one column per
-// wavefront and up to four tiles (the figures at the kernel).
+// one to four tiles 3.8 / 3.2, 3.9 / 3.3, 3.8 / 3.8, 4.0 / 4.3, six 4.1 / 5.4, so the line is three there.
+// Q6_K: one column per wavefront, so rows of up to ten super-blocks.  Streaming / short, us, with the weights from HBM | from the
+// last-level cache: four tiles of 512 to 1536 elements (16384 rows) 5.8 / 4.3 | 4.6 / 4.3 at 512, 11.0 / 7.55 | 8.55 / 7.45 at 1536; two
+// tiles (8192 rows) 7.0 / 6.5 | 5.8 / 6.1 at 1792, 7.3 / 5.8 | 5.8 / 5.6 at 2048, 8.2 / 6.9 | 6.4 / 6.6 at 2560; three (12288 rows) 8.0 / 8.7 |
+// 6.4 / 8.4 at 1792, 8.1 / 7.7 | 6.5 / 7.6 at 2048, 9.5 / 9.1 | 7.3 / 8.9 at 2560.  So four tiles up to six super-blocks (more were not
+// tried) and two above, where three would gain less from HBM than they lose from the cache.  Rows of nine super-blocks, every second
+// of which starts between two dwords: one tile (4096 rows) 6.9 / 5.4 | 5.9 / 5.05, two 7.9 / 8.2 | 6.6 / 7.9.
 bool gemv_short(const GemvJob *jobs, size_t n, uint32_t cu_count, uint32_t *threads, uint32_t *grid, size_t *lds, uint32_t *param) {
     if (n == 0 || n > (size_t)kShortJobs) return false;
     const bool q6 = jobs[0].kind == KIND_Q6K_MFMA;
@@ -3581,7 +3585,7 @@ bool gemv_short(const GemvJob *jobs, size_t n, uint32_t cu_count, uint32_t *thre
     }
     const uint64_t cpr = jobs[0].k / 256, nt = (rows + 16ull * cu_count - 1) / (16ull * cu_count);
     const uint32_t nw = q6 ? q6k_mfma_waves(cpr) : q4k_mfma_waves(cpr), np = (uint32_t)((cpr + nw - 1) / nw);
-    if (nt == 0 || nt > (cpr == 1 ? 3u : 8u) || (q6 ? np > 1 || nt > 4 : nt * np > 10)) return false;
+    if (nt == 0 || nt > (cpr == 1 ? 3u : 8u) || (q6 ? np > 1 || nt > (cpr <= 6 ? 4u : cpr == 9 ? 1u : 2u) : nt * np > 10)) return false;
     uint32_t tr = (uint32_t)((rows + cu_count * nt - 1) / (cu_count * nt));
     uint64_t tiles = 0;
     for (;; tr++) {  // (a job's last tile is ragged: a row more per tile where the tiles would spill over into another round)
