@@ -41,8 +41,8 @@ __device__ __forceinline__ void expert_groups_count(const ExpertGroups &G, const
 }
 
 // Share `share` of `grid` even ones of `units`: [v, v_end).  One 32-bit division, and what leads to the experts' ids in preloaded
-// arguments: two 64-bit divisions and the argument block lay before a launch's first tile (MXFP4, 128 tokens 165 -> 162 us beside the
-// same start, 2 launches; a k-quant layer of 16 tokens 88.3 -> 87.2).
+// arguments: two 64-bit divisions and the argument block lay before a launch's first tile (MXFP4 block of 128 tokens 160.5 -> 158.6 us,
+// two launches; a k-quant layer of 16 tokens 88.3 -> 87.2).
 __device__ __forceinline__ void expert_group_share(uint32_t units, uint32_t share, uint32_t grid, uint32_t &v, uint32_t &v_end) {
     const uint32_t each = units / grid, rest = units - each * grid;
     v = each * share + min(share, rest);

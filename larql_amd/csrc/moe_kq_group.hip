@@ -12,9 +12,10 @@
 //     so four activations share an operand, lane (row, rq) ends with the four dots of group rq, the -32 comes in as the MFMA's
 //     third operand, and three lane swaps leave lane group a with activation a's sum over all sixteen groups.
 // (At HBM's pace a compute unit gets a 2304-byte wave-tile every ~216 cycles, 864 of a SIMD's.)
-// Layer calls before (a matvec per slot) / now, us.  Q4_K, 128 experts, top-8, 2816 x 704: 1 token 38.5 / 31.0, 4 51.2 / 41.9, 16
-// 97.6 / 77.5, 64 278.6 / 143.0; 32 experts, top-8, 3072 x 768: 64 tokens 249 / 101; 32 experts, top-4, 1536 x 256: 1 token 31 / 24.5.
-// Q6_K (K-slice kernel before), the same: 35.6 / 34.3, 53.4 / 50.7, 144 / 117, 417 / 182; 402 / 105; 30.4 / 25.2.
+// Layer calls with a matvec per slot / with groups, us, all else equal.  Q4_K, 128 experts, top-8, 2816 x 704: 1 token 32.3 / 29.4, 4
+// 45.4 / 42.3, 16 88.1 / 80.2, 64 281 / 142; 32 tokens of 64 experts, top-8, 2048 x 512 90.4 / 60.6, 2560 x 640 121 / 74.0; 64 tokens of 32
+// experts, top-8, 3072 x 768 252 / 99.6, of 64 experts, top-4, 1024 x 256 47.3 / 40.3; 1 token of 32 experts, top-4, 1536 x 256 28.8 / 26.1.
+// Q6_K (K-slice kernel), the same: 33.6 / 31.7, 49.2 / 49.8, 132 / 110, 421 / 182; 111 / 56.7, 180 / 77.2; 400 / 100, 49.1 / 42.4; 25.5 / 24.0.
 //
 // A wavefront owns one super-block column of every ways-th tile (rows of three super-blocks: twelve wavefronts, four ways; one
 // workgroup per compute unit, so that its groups are found once); its tiles stream global -> LDS through a private ring; partials
@@ -120,6 +121,7 @@ __global__ void __launch_bounds__(kKgMaxWaves * 64)
     expert_groups_count<kKgSlots>(G, experts, slots, nE, tid, lane, wv);
 
     // this workgroup's share of the list (group, 16-row tile); a group opens with kStart units of its own, what its start costs
+    // (42 layer calls a format, with 1 / 3 / 6 of them: Q4_K 1.02 / 1 / 1.00, Q6_K 1.03 / 1 / 0.99 of the time)
     constexpr uint32_t kStart = 3;
     const uint32_t tpm = (rows + 15) / 16, per_group = tpm * A.n_mats + kStart, units = __builtin_amdgcn_readfirstlane(G.before[nE]) * per_group;
     const uint32_t share = (grid & 7u) ? blockIdx.x : (blockIdx.x & 7u) * (grid >> 3) + (blockIdx.x >> 3);  // neighbours on one XCD
@@ -318,6 +320,9 @@ static uint32_t kg_ways(uint32_t cols, uint32_t n_experts, uint32_t slots) {  //
     return 0;
 }
 
+// Rows of up to twelve super-blocks (a wavefront each) and as many slots as the lists have LDS for: kMoeGroupMaxSlots with fewer ways
+// where that helps, but Q4_K rows of twelve super-blocks leave room for 1518 slots of 128 experts, 1006 of 256.  Beyond, every slot
+// reads its expert again: 128 experts, top-8, 3072 x 256, 189 / 190 tokens 138 / 342 us (Q6_K 142 / 143).
 bool moe_kq_group_serves(bool q6, uint32_t rows, uint32_t cols, uint32_t n_experts, uint32_t slots) {
     return rows >= 1 && rows < (1u << 22) && slots >= 1 && slots <= kMoeGroupMaxSlots && n_experts >= 1 && n_experts <= kMoeGroupMaxExperts &&
            (q6 ? kg_ways<true>(cols, n_experts, slots) : kg_ways<false>(cols, n_experts, slots)) != 0;

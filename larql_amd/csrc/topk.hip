@@ -99,7 +99,11 @@ __device__ __forceinline__ uint64_t make_key(float s, uint32_t idx, int *nan_fla
 
 constexpr int kTopkCached = 16;  // rounds of 64 scores per wavefront held in registers
 constexpr int kTopkCandidates = 1024;  // of the short way
-constexpr uint32_t kTopkShortK = 256;   // winners that the short way bounds
+// Winners that the short way bounds.  Radix passes / short way, us per gate-KNN call over 10240 features of 256: K = 65 22.7 / 11.7,
+// 200 24.9 / 12.9, 256 24.8 / 13.8, 257 27.5 / 14.3, 300 27.5 / 16.0, 400 27.6 / 23.3, 512 27.7 / 32.7; over 4096: 300 20.4 / 13.8, 400 20.5 /
+// 20.8.  With K near the 512 slices the bound falls to the smallest maximum and the candidates overflow, so the gain ends between
+// 300 and 400; 256 lies on its safe side.  A row of equal scores pays for the attempt: K = 200 52.6 / 54.6.
+constexpr uint32_t kTopkShortK = 256;
 
 // What a workgroup selects from: `n` scores of a row, cut into chunks of `chunk` (chunk == n: the whole row), or — KEYS_IN —
 // the row's `n` keys that the chunks' workgroups left.  A chunk's workgroup leaves keys (KEYS_OUT): its K best, best
@@ -124,7 +128,7 @@ struct TopkArgs {
 // (80 scalar registers: with the 96 the compiler would take, a second 16-wavefront workgroup was not placed on a CU
 // until half of the first one's wavefronts had left — more rows than CUs then ran in two rounds)
 // The arguments on the way to the first score are plain scalars, so that they are in registers when a wavefront starts; read from
-// the block they were one more trip to memory (a gate-KNN over 10240 features beside the same start 1.093x -> 1.130x, 0.4 us).
+// the block they were one more trip to memory (a gate-KNN over 10240 x 2560 f16 features 16.4 -> 15.85 us).
 template <bool BY_ABS, int ROUNDS, bool LARGE, bool KEYS_IN, bool KEYS_OUT>
 __global__ void __launch_bounds__(kTopkThreads) __attribute__((amdgpu_num_sgpr(80))) topk_kernel(
     const void *src, int *const nan_flag, uint32_t scores_n, uint32_t row_n, uint32_t chunk, uint32_t k,
