@@ -885,8 +885,9 @@ __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *
 
     // The pair adds its partial sums through LDS, where the results also take the shape in which a store instruction
     // writes whole lines: a row group's 64-row x 128-token block as [token][row] (token rows padded to 68 floats: the
-    // lanes of a write phase hit different banks) in the pair's own 34 KB; each parks the 32 rows of the other and adds its
-    // own 32 to what the other parked, then every lane of the pair stores 16 bytes of a 256-byte run of one token.
+    // lanes of a write phase hit different banks) in the pair's own 34 KB; wavefront 1 parks, wavefront 0 adds its own
+    // and parks the sum, then every lane of the pair stores 16 bytes of a 256-byte run of one token.  (Each parking 32 rows of the
+    // other and adding its own 32 to what the other parked: 4096 x 4096 with 16 tokens 17.5 -> 17.9 us, 14277 x 2048 with 335 45.3 -> 45.6.)
     const uint32_t rc = (lane & 15u) * 4, r = row0 + wm + rc;
     float back[4];  // 2^-E of this lane's four rows (asked for here: behind the barriers nothing would hide the trip)
 #pragma unroll
@@ -895,31 +896,29 @@ __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *
     asm volatile("" ::: "memory");
     constexpr uint32_t EP_LD = G_EP_LD;
     float *blk = reinterpret_cast<float *>(glds) + wq * (GN * EP_LD);
-    auto park = [&](auto I) {
-        constexpr int i = decltype(I)::value;
+    if (kh) {
 #pragma unroll
-        for (int jj = 0; jj < NB; jj++)
+        for (int i = 0; i < 2; i++)
 #pragma unroll
-            for (int q = 0; q < 4; q++)  // registers 4q .. 4q+3 of a block: rows 8q + 4kgrp .. +3, token row32
-                *reinterpret_cast<f32x4 *>(blk + (jj * 32 + row32) * EP_LD + i * 32 + q * 8 + kgrp * 4) =
-                    (f32x4){acc[i][jj][4 * q], acc[i][jj][4 * q + 1], acc[i][jj][4 * q + 2], acc[i][jj][4 * q + 3]};
-    };
-    auto add_own = [&](auto I) {
-        constexpr int i = decltype(I)::value;
+            for (int jj = 0; jj < NB; jj++)
 #pragma unroll
-        for (int jj = 0; jj < NB; jj++)
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                f32x4 *at = reinterpret_cast<f32x4 *>(blk + (jj * 32 + row32) * EP_LD + i * 32 + q * 8 + kgrp * 4);
-                const f32x4 other = *at;
-                *at = (f32x4){acc[i][jj][4 * q] + other[0], acc[i][jj][4 * q + 1] + other[1], acc[i][jj][4 * q + 2] + other[2], acc[i][jj][4 * q + 3] + other[3]};
-            }
-    };
-    if (kh) park(std::integral_constant<int, 0>{});
-    else park(std::integral_constant<int, 1>{});
+                for (int q = 0; q < 4; q++)  // registers 4q .. 4q+3 of a block: rows 8q + 4kgrp .. +3, token row32
+                    *reinterpret_cast<f32x4 *>(blk + (jj * 32 + row32) * EP_LD + i * 32 + q * 8 + kgrp * 4) =
+                        (f32x4){acc[i][jj][4 * q], acc[i][jj][4 * q + 1], acc[i][jj][4 * q + 2], acc[i][jj][4 * q + 3]};
+    }
     __syncthreads();
-    if (kh) add_own(std::integral_constant<int, 1>{});
-    else add_own(std::integral_constant<int, 0>{});
+    if (!kh) {
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int jj = 0; jj < NB; jj++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    f32x4 *at = reinterpret_cast<f32x4 *>(blk + (jj * 32 + row32) * EP_LD + i * 32 + q * 8 + kgrp * 4);
+                    const f32x4 other = *at;
+                    *at = (f32x4){acc[i][jj][4 * q] + other[0], acc[i][jj][4 * q + 1] + other[1], acc[i][jj][4 * q + 2] + other[2], acc[i][jj][4 * q + 3] + other[3]};
+                }
+    }
     __syncthreads();
     const bool vec_ok = (rows & 3u) == 0 && (((uintptr_t)(partial ? partial : out)) & 15u) == 0;
 #pragma unroll 4
