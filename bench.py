@@ -554,13 +554,14 @@ def run_kq(be, fmt, args):
         assert rel < 1e-3, rel
         ms = _timeit(be, layer_fwd, args.steps)
         slots = T * k
-        algo = slots * expert_bytes + E * H * 4 + T * (8 * H + 4 * E)      # every slot reads its expert's matrices (no sharing between tokens yet)
+        distinct = len(set(int(v) for v in experts.reshape(-1)))
+        algo = distinct * expert_bytes + E * H * 4 + T * (8 * H + 4 * E)   # (slots that chose the same expert share a read of its matrices)
         _emit(f"Q4_K MoE layer us (Gemma-4-26B-A4B shapes: 128 experts, top-8, batch {T})", round(ms * 1e3, 2), "us/layer", ms, args.steps, 2,
               {"workload": f"MoE layer over a Q4_K expert bank as MoeLayerWeights hands it over: 128 experts x (gate_up 1408x2816, down 2816x768), "
                            f"router_proj 128x2816, top-8, GeluTanh, Q8_K activations (the reference's integer expert path), batch {T}",
-               "launches_per_layer": 6, "slots": slots, "distinct_experts": len(set(int(v) for v in experts.reshape(-1))),
+               "launches_per_layer": 6, "slots": slots, "distinct_experts": distinct,
                "verified_rel_l2_vs_oracle": rel},
-              {"kernel": "gemv_q4k_q8k (gate/up, down launches) + the small kernels around them", "bound": "hbm", "achieved": round(algo / ms / 1e6, 1),
+              {"kernel": "moe_kq_group (gate/up, down launches) + the small kernels around them", "bound": "hbm", "achieved": round(algo / ms / 1e6, 1),
                "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(algo / ms / 1e6 / HBM_PEAK_GBS, 4), "traffic": None},
               {"value": round(cpu_s * 1e6 * T, 1), "unit": "us/layer", "cores": 1, "kind": "port",
                "sample": f"one token through the checker's scalar integer expert path, one thread, scaled by {T} tokens"}, higher=False)
