@@ -2269,6 +2269,33 @@ def test_short_launches_equal_the_streaming_kernel_bit_for_bit(be, fmt, fmt_name
         be.free(p)
 
 
+@pytest.mark.parametrize("fmt_name,k,tiles", [("Q6_K", 512, 4), ("Q6_K", 1536, 4), ("Q6_K", 1792, 2), ("Q6_K", 2304, 1), ("Q6_K", 2560, 2),
+                                              ("Q4_K", 256, 3), ("Q4_K", 512, 8), ("Q4_K", 2560, 8), ("Q4_K", 3840, 5), ("Q4_K", 7680, 3)])
+def test_short_launches_at_the_most_tiles_per_unit(be, fmt, fmt_name, k, tiles):
+    """The longest launches that the short kernel takes (`tiles` tiles of sixteen rows on each of 256 compute units), the first that
+    it does not, and one in between, against the same matvec six times in a launch (the streaming kernel), bit for bit."""
+    f, block, enc = (fmt.FMT_Q4_K, 144, be.dev_quantize_q4_k) if fmt_name == "Q4_K" else (fmt.FMT_Q6_K, 210, be.dev_quantize_q6_k)
+    most = tiles * 4096 + 1
+    src, w, x = be.malloc(most * k * 4), be.malloc(most * (k // 256) * block + 64), be.malloc(k * 4)
+    be.dev_fill_normal(src, most * k, 4321 + k, 0.02)
+    assert enc(src, most * k, w)
+    be.dev_fill_normal(x, k, 78, 1.0)
+    outs = [be.malloc(most * 4) for _ in range(6)]
+    for rows in (most - 2101, most - 1, most):
+        got = []
+        for n in (1, 6):
+            be.h2d(outs[0], np.full(most, np.nan, F))
+            plan = be.plan_create([(f, w, None, x, outs[i], rows, k) for i in range(n)])
+            assert plan is not None, be.last_error()
+            assert be.plan_run(plan)
+            be.synchronize()
+            got.append(be.d2h(outs[0], rows, F).view(np.uint32))
+            be.plan_destroy(plan)
+        assert np.array_equal(*got), rows
+    for p in [src, w, x] + outs:
+        be.free(p)
+
+
 @pytest.mark.parametrize("T,E,k,hidden,cols,inter", [
     (9, 1, 1, 272, 512, 300),      # one expert with nine slots: a group of eight and one of one; ragged last tiles of gate and up
     (16, 2, 2, 256, 256, 17),      # two full groups per expert; a tile and one row, rows of one super-block
