@@ -19,6 +19,7 @@ namespace larql {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
@@ -28,17 +29,19 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 //   out[s, r] = sum over super-blocks of  d[r] * (sum_k (sc6*q)[r,k] * x[s,k])  -  dmin[r] * (sum_sub mn6[r,sub] * Sx[s,sub])
 //
 // The activations are prepared once per call (q4k_gemm_prep_kernel): per token a power-of-two scale brings
-// max|x| to [2^13, 2^14), x/scale is stored as f16 (exact for bf16 inputs; f32 inputs add a second f16 term
-// and a second pass), and Sx, the sum of the represented activations over each 32-element sub-block, is stored
-// (divided by 32, to stay inside f16) as an f16 pair (hi, lo).  The weight operand is made in registers from the
-// raw nibbles (mask into the mantissa of an f16 1024 + q, one or two packed f16 instructions), never in memory.
-// Two kernels share the tile, the copies and the tables:
+// max|x| to [2^13, 2^14) and x/scale is stored as f16 (exact for bf16 inputs; f32 inputs add a second f16 term
+// and a second pass).  The weight operand is made from the raw nibbles (mask into the mantissa of an f16, packed f16
+// instructions) and never stored in memory.  Two kernels:
 //   * q4k_gemm_exact_kernel (host tier): the operand is sc6*q <= 945, exact in f16; per super-block a wavefront keeps
 //     the integer sums apart (D), gets sum_sub mn6*Sx from one more MFMA per block (A slots 2*sub+h = 32 mn6,
-//     B slots = Sx_h/32), and folds both into the f32 result with the row's d and dmin.
-//   * q4k_gemm_pair_kernel (device tier): the row's scale rides in the operand, f16(d 2^E sc6) * (q - 8), and the
-//     offsets' MFMA adds (8 d sc6 - dmin mn6) 2^E * Sx to the same accumulators; 2^-E and the token's scale are
-//     applied once at the end.  3e-4 relative to the CPU value instead of 3e-7, no folds, half the registers.
+//     B slots = Sx_h/32; Sx, the sum of the represented activations over each 32-element sub-block, comes with the
+//     preparation as an f16 pair, divided by 32 to stay inside f16), and folds both into the f32 result with the row's
+//     d and dmin.
+//   * q4k_gemm_pair_kernel (device tier): the operand is the whole weight, f16(d sc6 (q - 8) + o) with
+//     o = f16(8 d sc6 - dmin mn6), both times the row's 2^E; sc6 (q - 8) is exact and o is of a weight's size or less, so
+//     that a weight is rounded once: 2.2e-4 relative to the f64 product (2.9e-4 with the scale d sc6 rounded by itself and
+//     the offsets in an MFMA of their own, the form before).  No offsets, no folds; 2^-E and the token's scale are applied
+//     once at the end.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float half_to_float(uint32_t lo16) { return (float)__builtin_bit_cast(_Float16, (uint16_t)lo16); }
 
@@ -156,6 +159,7 @@ __global__ void __launch_bounds__(1024) q4k_gemm_prep_kernel(const void *__restr
         const size_t at = (size_t)tok * nvec + v;
         oh[at] = (u32x4){hw[0], hw[1], hw[2], hw[3]};
         if (ol) ol[at] = (u32x4){lw[0], lw[1], lw[2], lw[3]};
+        if (!sx) return;  // (the device tier's GEMM has no use for the sums)
         sm += dpp_move<0xB1>(sm);  // quad_perm [1,0,3,2]
         sm += dpp_move<0x4E>(sm);  // quad_perm [2,3,0,1]
         sm *= 0.03125f;  // stored as Sx/32 so that 32 x 2^14 stays inside f16; the min operand carries the 32
@@ -175,37 +179,44 @@ __global__ void __launch_bounds__(1024) q4k_gemm_prep_kernel(const void *__restr
     if (lo_seen && any_lo) *any_lo = 1;
 }
 
-// adds the partial slabs of a K-split in slab order and applies the token scale; VEC elements per thread (4 when
-// rows % 4 == 0 and everything is 16-byte aligned: the four are then of one token).
+// adds the partial slabs of a K-split in slab order and applies the token scale; four elements per thread, which may lie in two
+// tokens where rows % 4 != 0 (a 16-byte access needs four-byte alignment only).
 // Bound: latency, then memory (the slabs come out of the last-level cache).  Eight slabs are requested together, so that a
 // launch costs splits / 8 round trips instead of `splits`; a request past the last slab reads the last one and is not added.
-template <int VEC>
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 __global__ void __launch_bounds__(256) q4k_gemm_reduce_kernel(const float *__restrict__ partial, uint32_t splits, const float *__restrict__ tok_scale,
                                                               float *__restrict__ out, uint32_t rows, uint32_t seq, int accumulate) {
-    typedef float vec __attribute__((ext_vector_type(VEC)));
-    const size_t n = (size_t)rows * seq, i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * VEC;
+    const size_t n = (size_t)rows * seq, i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
     if (i >= n) return;
-    float s[VEC];
+    if (i + 4 > n) {  // the last one to three elements
+        for (size_t k = i; k < n; k++) {
+            float s = 0.f;
+            for (uint32_t z = 0; z < splits; z++) s += partial[z * n + k];
+            s *= tok_scale[k / rows];
+            out[k] = accumulate ? out[k] + s : s;
+        }
+        return;
+    }
+    const size_t tok = i / rows;
+    const uint32_t left = (uint32_t)min((size_t)4, (tok + 1) * rows - i);  // elements of this token
+    float ts[4];
 #pragma unroll
-    for (int e = 0; e < VEC; e++) s[e] = 0.f;
+    for (int e = 0; e < 4; e++) ts[e] = tok_scale[(uint32_t)e < left ? tok : (i + e) / rows];
+    f32x4 s = {0.f, 0.f, 0.f, 0.f};
     for (uint32_t z0 = 0; z0 < splits; z0 += 8) {
-        vec v[8];
+        f32x4 v[8];
 #pragma unroll
-        for (uint32_t u = 0; u < 8; u++) v[u] = *reinterpret_cast<const vec *>(partial + (size_t)min(z0 + u, splits - 1) * n + i);
+        for (uint32_t u = 0; u < 8; u++) v[u] = *reinterpret_cast<const f32x4_a4 *>(partial + (size_t)min(z0 + u, splits - 1) * n + i);
 #pragma unroll
         for (uint32_t u = 0; u < 8; u++)
 #pragma unroll
-            for (int e = 0; e < VEC; e++) s[e] = z0 + u < splits ? s[e] + v[u][e] : s[e];
+            for (int e = 0; e < 4; e++) s[e] = z0 + u < splits ? s[e] + v[u][e] : s[e];
     }
-    const float ts = tok_scale[i / rows];
-    if (VEC == 4) {
-        f32x4 r = {s[0] * ts, s[VEC > 1 ? 1 : 0] * ts, s[VEC > 2 ? 2 : 0] * ts, s[VEC > 3 ? 3 : 0] * ts};
-        f32x4 *o = reinterpret_cast<f32x4 *>(out + i);
-        if (accumulate) r += *o;
-        *o = r;
-    } else {
-        out[i] = accumulate ? out[i] + s[0] * ts : s[0] * ts;
-    }
+    f32x4_a4 *o = reinterpret_cast<f32x4_a4 *>(out + i);
+#pragma unroll
+    for (int e = 0; e < 4; e++) s[e] *= ts[e];
+    if (accumulate) s += (f32x4)*o;
+    *o = s;
 }
 
 // ---------------------------------------------------------------------------
@@ -609,20 +620,36 @@ __global__ void __launch_bounds__(GTHREADS, 1) q4k_gemm_exact_kernel(const uint8
 }
 
 // ---------------------------------------------------------------------------
-// The device tier's kernel: the same tile, copies and tables with 8 wavefronts, two per SIMD.  A wavefront with its
-// own instruction stream hides at most ~3 vector instructions per 32x32x16 MFMA (measured: 32, 37, 44, 56 cycles per
-// MFMA with 2, 4, 6, 8 vector instructions after it); two wavefronts per SIMD hide ~6 each.  The conversion alone
-// is 3.5 per MFMA, so the 64 rows x 128 tokens of a row group are computed by a pair of wavefronts that split every
-// step's k: wavefront kh takes the nibbles kh (k 32kh .. 32kh+31 of the step: sub-block 2g + kh) of the same raw bytes
-// against the same tokens.  No weight is converted twice and no activation read twice; each wavefront keeps a full
-// set of partial sums (128 registers), which the pair adds up through LDS at the end.  The rows' scales ride in the
-// operand (the formulation at the top of this file); with a second set of accumulators the exact variant does not
-// fit in the 256 registers a wavefront has here and stays with q4k_gemm_exact_kernel.
-// The two wavefronts of a SIMD take turns (see the loop): while one issues a step's 16 MFMAs back to back, the other
-// prepares its next step; with both doing a bit of everything all the time, a workgroup barrier per step made them
-// run one after the other, each at about half the matrix pipe's rate.
+// The device tier's kernel: one workgroup of 8 wavefronts, two per SIMD, owns 256 rows against a tile of tokens.  The two
+// wavefronts of a SIMD (w and w + 4) share 64 rows and either
+//   * split every step's k (KS; 16 TB <= 128 tokens): wavefront kh takes the nibbles kh of the same raw bytes against all of
+//     the tile's tokens: no weight converted twice; the pair adds its sums through LDS at the end; or
+//   * split the tokens (128 each of 256): each converts all weights of the rows, but copies, super-block tables, prologue and
+//     end serve twice the tokens and nothing is added at the end.
+// A step is 64 k, half a step 32 (one nibble of 32 raw bytes per row = one sub-block).  In half a step a wavefront
+// *prepares* (the activation operands from LDS into registers, the weight operand converted in registers: lane (row r16, kq)
+// needs the nibbles of 8 consecutive raw bytes) and *multiplies* (4 x TB v_mfma_f32_16x16x32_f16).  One wavefront of the pair
+// prepares first and one multiplies first, with one barrier per half step, so that one's vector instructions fall
+// into the other's MFMAs.  (A barrier after each of the two, the form before, makes a half step twice the longer of the two:
+// 1931 cycles per step of 128 tokens where the MFMAs take 1024; with one 1689, with table entries and raw bytes read ahead
+// 1614, with the copies asked for between MFMAs 1541.)
+// Everything comes into LDS by global_load_lds: the f16 activations of a step into a ring (128 bytes per token; chunk c
+// of token r at position c ^ ((r >> 1) & 7), chosen on the global side of the copy: no bank conflicts), the weights a super-block at a
+// time (144 bytes per row: a row's two or three cache lines are asked for once) into two stages.  kh = 0 asks for
+// the activations, kh = 1 for the weights, between its MFMAs: a copy instruction whose lanes lie in many cache lines holds up
+// the wavefront that issues it (nine in a row: 0.4 us).  Per super-block one thread per row turns half of the header into table entries
+// (sc6/16, o) for the lanes that convert.
+// 16 x 16 x 32 MFMAs: at these rates the GPU is limited by its power, and a loop of them ran at a 10 % higher clock than the same work in
+// 32 x 32 x 16 (which read and write twice the accumulators per operation); f16 operands of normal values: 1.28 PFLOP/s
+// for a loop of nothing but copies, LDS reads and MFMAs.
+// Measured, calls with the exponents given: 15360 x 3840 with 2048 tokens 283 -> 217 us, 512 73.5 -> 69.7; 3840 x 15360 with
+// 77 34.1 -> 32.5, 16 27.2 -> 21.9; 12607 x 1280 with 1817 119 -> 91 (rows no multiple of four: the results in four-byte
+// stores before).
 // ---------------------------------------------------------------------------
 constexpr int QTHREADS = 512;
+constexpr uint32_t Q_B_BYTES = 65536, Q_R_STAGE = GM * 144, Q_T_STAGE = GM * 32;  // activation ring; weights and tables of a super-block
+constexpr uint32_t Q_R_OFF = Q_B_BYTES, Q_T_OFF = Q_R_OFF + 2 * Q_R_STAGE, Q_D_OFF = Q_T_OFF + 2 * Q_T_STAGE, Q_E_OFF = Q_D_OFF + 2 * GM * 4, Q_S_OFF = Q_E_OFF + GM * 4, Q_LDS_BYTES = Q_S_OFF + 2 * GN * 4;
+static_assert(Q_LDS_BYTES <= 160 * 1024, "one workgroup per CU");
 // one global -> LDS copy of 16 bytes per lane: uniform base + per-lane 32-bit offset on the global side (no 64-bit
 // address registers), uniform LDS address (the lanes' 16-byte slots follow one another from there)
 __device__ __forceinline__ void copy16_to_lds(const void *base, uint32_t lane_off, uint32_t lds_addr) {
@@ -631,251 +658,280 @@ __device__ __forceinline__ void copy16_to_lds(const void *base, uint32_t lane_of
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(lane_off), "s"(bs) : "memory");  // (m0 is not the compiler's to allocate; nothing else in these kernels uses it)
 }
 
-// NB: blocks of 32 tokens that are multiplied (4 unless the prompt is shorter than the tile)
-template <int NB>
-__global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *w, const uint16_t *xh, const uint16_t *sx, const int *__restrict__ rexp,
+// four bytes per lane, likewise
+__device__ __forceinline__ void copy4_to_lds(const void *base, uint32_t lane_off, uint32_t lds_addr) {
+    const uint64_t b = (uint64_t)(uintptr_t)base;
+    const uint64_t bs = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(lane_off), "s"(bs) : "memory");
+}
+
+// up to four neighbouring results; `left` of them are inside the matrix.  (A 16-byte store needs four-byte alignment only.)
+__device__ __forceinline__ void store4(float *o, f32x4 v, uint32_t left) {
+    if (left >= 4) {
+        *reinterpret_cast<f32x4_a4 *>(o) = v;
+    } else {
+        if (left > 0) o[0] = v[0];
+        if (left > 1) o[1] = v[1];
+        if (left > 2) o[2] = v[2];
+    }
+}
+
+template <int TB, bool KS>
+__global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *w, const uint16_t *xh, const int *__restrict__ rexp,
                                                                   const float *__restrict__ tok_scale, float *__restrict__ out,
-                                                                  uint32_t rows, uint32_t hidden, uint32_t seq, int with_mins,
-                                                                  int accumulate, uint32_t sb_per_split, float *__restrict__ partial) {
+                                                                  uint32_t rows, uint32_t hidden, uint32_t seq, uint32_t row_tiles, uint32_t tok_tiles,
+                                                                  uint32_t sb_per_split, float *__restrict__ partial) {
+    static_assert(TB % 2 == 0 && TB <= 8 && (KS || TB == 8), "");
+    constexpr uint32_t NT = KS ? 16 * TB : 32 * TB;                // tokens of the tile
+    constexpr uint32_t B_STAGE = KS ? 16384 : 32768, NB = Q_B_BYTES / B_STAGE;  // a step's activations (128 bytes a token), and how many of them
+    constexpr int CP = NT / 32;                                    // activation copies of a wavefront kh = 0 for a step
     extern __shared__ __attribute__((aligned(16))) uint8_t glds[];
     const uint32_t t = threadIdx.x, lane = t & 63u, wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const uint32_t wq = wave & 3u, kh = wave >> 2;  // row group, k half: wavefronts w and w+4 run on one SIMD
-    const uint32_t row0 = blockIdx.x * GM, tok0 = blockIdx.y * GN;
+    const uint32_t wq = wave & 3u, kh = wave >> 2;  // row group; which of the pair: wavefronts w and w + 4 run on one SIMD
+    // which tile: workgroups are dealt to the eight XCDs in turn; each takes a contiguous part of the list of tiles, in which four
+    // token tiles of a row tile follow one another (an XCD's 32 workgroups then share 8 row tiles and 4 token tiles in its L2)
+    uint32_t id = blockIdx.x;
+    {
+        const uint32_t total = gridDim.x, q = total >> 3, r = total & 7u, xcd = id & 7u, ix = id >> 3;
+        id = xcd * q + min(xcd, r) + ix;
+    }
+    const uint32_t per_range = row_tiles * tok_tiles, range = __builtin_amdgcn_readfirstlane(id / per_range);
+    id -= range * per_range;
+    constexpr uint32_t TG = 4;
+    const uint32_t tg = id / (row_tiles * TG), in = id - tg * row_tiles * TG, tw = min(TG, tok_tiles - tg * TG);
+    const uint32_t row0 = __builtin_amdgcn_readfirstlane((in / tw) * GM), tok0 = __builtin_amdgcn_readfirstlane((tg * TG + in % tw) * NT);
     const uint32_t nsb = hidden >> 8, row_bytes = nsb * 144;
-    const uint32_t sb_begin = blockIdx.z * sb_per_split, sb_end = min(nsb, sb_begin + sb_per_split);
+    const uint32_t sb_begin = range * sb_per_split, sb_end = min(nsb, sb_begin + sb_per_split);
     if (sb_begin >= sb_end) return;
     const uint32_t nsteps = (sb_end - sb_begin) * 4;
     const uint32_t wm = wq * 64;
-
-    // copy roles.  Weights: a super-block of a row group's 64 rows (144 bytes each, header included) is nine copies; piece p,
-    // lane l brings 16-byte chunk (64p + l) % 9 of row (64p + l) / 9, so that the rows lie in LDS one after the other and
-    // a row's two or three cache lines are asked for by neighbouring lanes of one instruction.  The nine are shared out
-    // 5 : 4 over the pair; the wavefront with 4 brings a quarter of Sx as its fifth copy.
-    const uint8_t *wt = w + (size_t)row0 * row_bytes;                                          // uniform
-    uint32_t r_off[5];
-#pragma unroll
-    for (int p = 0; p < 5; p++) {
-        const uint32_t idx = min(kh * 5 + p, 8u) * 64 + lane;
-        r_off[p] = (min(row0 + wm + idx / 9, rows - 1) - row0) * row_bytes + (idx % 9) * 16;
-    }
-    const uint32_t own_row = min(row0 + wm + lane, rows - 1);   // the row whose table entries this thread writes
-    // activations ([token][hidden] f16): wavefront -> tokens 16w .. 16w+15 (two copies of 8 tokens x 128 bytes)
-    const uint8_t *xt = (const uint8_t *)xh;                                                   // uniform
-    uint32_t b_off[2];
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-        const uint32_t r = (wave * 2 + q) * 8 + (lane >> 3);
-        b_off[q] = min(tok0 + r, seq - 1) * hidden * 2 + (((lane & 7u) ^ ((r >> 1) & 7u)) * 16);
-    }
-    // Sx ([super-block][token][8 pairs]): the wavefronts kh = 1 -> tokens 32wq .. 32wq+31 (two 16-byte halves each)
-    const uint8_t *st = (const uint8_t *)sx;                                                   // uniform
-    const uint32_t m_off = min(tok0 + wq * 32 + (lane >> 1), seq - 1) * 32 + (lane & 1u) * 16;
-    const int row_e = rexp[own_row];  // d * 2^row_e <= 1 over the whole row
-
-    const uint32_t row32 = lane & 31u, kgrp = lane >> 5;
     const uint32_t lds0 = (uint32_t)(uintptr_t)(p_lds_vp)glds;
 
+    // copies.  kh = 1: a super-block of the pair's 64 rows is nine pieces; piece p, lane l brings 16-byte chunk (64p + l) % 9 of row
+    // (64p + l) / 9, so that the rows lie in LDS one after the other.  kh = 0: a step's activations, CP pieces of 8 tokens
+    const uint8_t *wt = w + (size_t)row0 * row_bytes;                                          // uniform
+    const uint8_t *xt = (const uint8_t *)xh + (size_t)tok0 * hidden * 2;                       // uniform
+    uint32_t c_off[9];
+    if (kh) {
+#pragma unroll
+        for (int p = 0; p < 9; p++) {
+            const uint32_t idx = p * 64 + lane;
+            c_off[p] = (min(row0 + wm + idx / 9, rows - 1) - row0) * row_bytes + (idx % 9) * 16;
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < 9; q++) {
+            const uint32_t r = (wq + 4 * (q < CP ? q : 0)) * 8 + (lane >> 3);
+            c_off[q] = (min(tok0 + r, seq - 1) - tok0) * hidden * 2 + (((lane & 7u) ^ ((r >> 1) & 7u)) * 16);
+        }
+    }
     // (requests past the end are clamped: same number of copies in flight, results unused)
-    auto issue_raw = [&](uint32_t sb, int p) {  // piece p (0..4) of this wavefront's share
-        const uint8_t *src = wt + (size_t)min(sb, sb_end - 1) * 144;
-        copy16_to_lds(src, r_off[p], lds0 + G_R_OFF + ((sb - sb_begin) & 1u) * G_R_STAGE + wq * 9216 + min(kh * 5 + p, 8u) * 1024);
+    auto issue_raw = [&](uint32_t sb, int p) {  // one of the nine pieces of a super-block
+        copy16_to_lds(wt + (size_t)min(sb, sb_end - 1) * 144, c_off[p], lds0 + Q_R_OFF + ((sb - sb_begin) & 1u) * Q_R_STAGE + wq * 9216 + p * 1024);
     };
-    auto issue_b = [&](uint32_t s, uint32_t slot, int q) {  // one of the two pieces of a step
-        const uint32_t sc = min(s, nsteps - 1);
-        const uint8_t *src = xt + ((size_t)sb_begin * 4 + sc) * 128;
-        copy16_to_lds(src, b_off[q], lds0 + G_B_OFF + slot * G_B_STAGE + wave * 2048 + q * 1024);
+    auto issue_b = [&](uint32_t s, uint32_t slot, int q) {  // one of the CP pieces of a step
+        copy16_to_lds(xt + ((size_t)sb_begin * 4 + min(s, nsteps - 1)) * 128, c_off[q], lds0 + slot * B_STAGE + (wq + 4 * q) * 1024);
     };
-    auto issue_sx = [&](uint32_t sb) {  // a quarter of a super-block's Sx
-        const uint32_t sbc = min(sb, sb_end - 1);
-        copy16_to_lds(st + (size_t)sbc * seq * 32, m_off, lds0 + G_BM_OFF + wq * 1024);
-    };
-    // a super-block's header -> this row's table entries (one thread per row).  Scales: s = f16(d 2^E sc6) of the
-    // sub-blocks 2u + kh, the ones this wavefront converts; the operand is s (q - 8): centred weights, so that the
-    // weight term and the offset term are both of the result's size and their f16 roundings are not magnified by a
-    // cancellation (with s q and -dmin mn6 Sx the error was 8e-4, so 2.9e-4).  The high nibbles' masked value is
-    // 1024 + 16q, so kh = 1 carries s/16.  Offsets' operand of the sub-blocks 4kh .. 4kh+3: 32 (8 d sc6 - dmin mn6) 2^E,
-    // twice, for the two f16 halves of Sx/32.
-    auto stage_sb = [&](uint32_t par) {
-        const u32x4 hdr = *reinterpret_cast<const u32x4 *>(glds + G_R_OFF + par * G_R_STAGE + wq * 9216 + lane * 144);
-        const float d = half_to_float(hdr.x & 0xFFFFu), dmin = half_to_float(hdr.x >> 16);
-        const float ds = ldexpf(d, row_e), dm = ldexpf(dmin, row_e);
-        auto sc6_of = [&](uint32_t sub) {
-            const uint32_t sh = 8u * (sub & 3u), pa = (hdr.y >> sh) & 0xFFu, pc = (hdr.w >> sh) & 0xFFu;
-            return sub < 4 ? (pa & 63u) : ((pc & 0x0Fu) | ((pa >> 6) << 4));
-        };
-        auto mn6_of = [&](uint32_t sub) {
-            const uint32_t sh = 8u * (sub & 3u), pb = (hdr.z >> sh) & 0xFFu, pc = (hdr.w >> sh) & 0xFFu;
-            return sub < 4 ? (pb & 63u) : ((pc >> 4) | ((pb >> 6) << 4));
-        };
-        uint32_t mnw[4];
+
+    int row_e = 0;  // d * 2^row_e <= 1 over the whole row, of the row whose table entries this thread writes
+    // table entries of the sub-blocks 2g and 2g + 1 of this thread's row, g = 2 khc + u, and (u = 0) its d
+    auto stage = [&](const int khc, const uint32_t par, const int u) {
+        const u32x4 hdr = *reinterpret_cast<const u32x4 *>(glds + Q_R_OFF + par * Q_R_STAGE + wq * 9216 + lane * 144);
+        const float ds = ldexpf(half_to_float(hdr.x & 0xFFFFu), row_e), dm = ldexpf(half_to_float(hdr.x >> 16), row_e);
+        // the 6-bit scales and mins of the four sub-blocks 4 khc .. 4 khc + 3, a byte each
+        const uint32_t sc4 = khc ? (hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u) : hdr.y & 0x3F3F3F3Fu;
+        const uint32_t mn4 = khc ? ((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u) : hdr.z & 0x3F3F3F3Fu;
+        uint32_t e[2] = {0u, 0u};
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const uint32_t sub = 2 * u + kh;
-            const float sf = ds * (float)sc6_of(sub) * (kh ? 0.0625f : 1.f);
-            *reinterpret_cast<uint32_t *>(glds + G_SC_OFF + wq * 2048 + sub * 256 + lane * 4) = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)sf);
-            const uint32_t ms = 4 * kh + u;
-            const uint32_t hb = __builtin_bit_cast(uint16_t, (_Float16)(32.f * (8.f * ds * (float)sc6_of(ms) - dm * (float)mn6_of(ms))));
-            mnw[u] = hb | (hb << 16);
+        for (int k = 0; k < 2; k++) {
+            const float sc = (float)((sc4 >> (8 * (2 * u + k))) & 0xFFu), mn = (float)((mn4 >> (8 * (2 * u + k))) & 0xFFu);
+            const float o = 8.f * ds * sc - dm * mn;
+            e[k] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(0.0625f * sc)) | (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)o) << 16;
         }
-        *reinterpret_cast<u32x4 *>(glds + G_AM_OFF + (wm + lane) * 32 + kh * 16) = (u32x4){mnw[0], mnw[1], mnw[2], mnw[3]};
+        *reinterpret_cast<u32x2 *>(glds + Q_T_OFF + par * Q_T_STAGE + (2 * khc + u) * 2048 + (wm + lane) * 8) = (u32x2){e[0], e[1]};
+        if (khc == 0 && u == 0) *reinterpret_cast<uint32_t *>(glds + Q_D_OFF + par * GM * 4 + (wm + lane) * 4) = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)ds);
     };
-    // 4 raw bytes (nibble kh) -> two dwords of f16(s (q - 8)) as the pairs (k0, k2) and (k1, k3): the nibbles of bytes 0
-    // and 2 are masked in place into the mantissas of two f16 (1024 + q, or 1024 + 16q for the high nibbles), those of
-    // bytes 1 and 3 after one shift; a packed add takes 1032 (1152) away, which is exact, and a packed multiply applies s:
-    // one rounding (-1032 s itself has no f16, so a single FMA cannot do it).  `magic` is 0x64006400 held in a register
-    // so that mask-and-or is one instruction.
-    uint32_t magic;
+    uint32_t magic;  // in a register, so that mask-and-or is one instruction
     asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(magic));
-    const uint32_t take = kh ? 0xE480E480u : 0xE408E408u;  // -1152 | -1032, twice
-    const uint32_t nib_mask = kh ? 0x00F000F0u : 0x000F000Fu;
-    auto convert4 = [&](uint32_t raw, uint32_t sp, uint32_t &o0, uint32_t &o1) {
-        const f16x2 p = __builtin_bit_cast(f16x2, sp);
-        const f16x2 sc2 = {p[0], p[0]}, c2 = __builtin_bit_cast(f16x2, take);
-        const f16x2 m02 = __builtin_bit_cast(f16x2, (raw & nib_mask) | magic);
-        const f16x2 m13 = __builtin_bit_cast(f16x2, ((raw >> 8) & nib_mask) | magic);
-        o0 = __builtin_bit_cast(uint32_t, (m02 + c2) * sc2);
-        o1 = __builtin_bit_cast(uint32_t, (m13 + c2) * sc2);
+    // 4 raw bytes, nibble h -> two dwords of f16(d sc6 (q - 8) + o) as the pairs (k0, k2) and (k1, k3).  The nibbles go to bits
+    // 4 .. 7 of two f16 (1024 + 16q); times sc6/16 less 72 sc6 is sc6 (q - 8), exact (-1032 sc6, which bits 0 .. 3 would need, is
+    // no f16); the second multiply-add rounds the weight
+    auto convert4 = [&](uint32_t raw, const int h, f16x2 sc, f16x2 c, f16x2 d, f16x2 o, uint32_t &o0, uint32_t &o1) {
+        const f16x2 m02 = __builtin_bit_cast(f16x2, ((h ? raw : raw << 4) & 0x00F000F0u) | magic);
+        const f16x2 m13 = __builtin_bit_cast(f16x2, ((h ? raw >> 8 : raw >> 4) & 0x00F000F0u) | magic);
+        o0 = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_elementwise_fma(m02, sc, c), d, o));
+        o1 = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_elementwise_fma(m13, sc, c), d, o));
     };
-    const uint32_t raw_lane = lds0 + G_R_OFF + wq * 9216 + row32 * 144 + 16 + kgrp * 16;
-    auto raw_of = [&](uint32_t par, uint32_t g4, u32x4 (&rq)[2]) {  // step g4 of the super-block in slot `par`
-        const uint32_t a = raw_lane + par * G_R_STAGE + g4 * 32;
-        asm volatile("ds_read_b128 %0, %1" : "=v"(rq[0]) : "v"(a));
-        asm volatile("ds_read_b128 %0, %1 offset:4608" : "=v"(rq[1]) : "v"(a));
-    };
-    const uint32_t sc_lane = lds0 + G_SC_OFF + wq * 2048 + kh * 256 + row32 * 4;
-    auto scales_of = [&](uint32_t g4, uint32_t (&sp)[2]) {  // the entries of sub-block 2 g4 + kh for this lane's two rows
-        const uint32_t a = sc_lane + g4 * 512;
-        asm volatile("ds_read_b32 %0, %1" : "=v"(sp[0]) : "v"(a));
-        asm volatile("ds_read_b32 %0, %1 offset:128" : "=v"(sp[1]) : "v"(a));
-    };
-    const uint32_t b_lane = lds0 + G_B_OFF + row32 * 128;
-    uint32_t b_col[2];  // byte position of this lane's chunk in a token's row, for the two MFMA depths of a step
+    const uint32_t r16 = lane & 15u, kq = lane >> 4;
+    const uint32_t raw_lane = lds0 + Q_R_OFF + wq * 9216 + r16 * 144 + 16 + kq * 8;
+    const uint32_t tab_lane = lds0 + Q_T_OFF + (wm + r16) * 8 + (KS ? kh * 4 : 0u), d_lane = lds0 + Q_D_OFF + (wm + r16) * 4;
+    uint32_t b_lane[2];  // for the two halves of a step
 #pragma unroll
-    for (int j = 0; j < 2; j++) b_col[j] = ((kh * 4 + 2 * kgrp + (uint32_t)j) ^ ((row32 >> 1) & 7u)) << 4;
+    for (int h = 0; h < 2; h++)
+        b_lane[h] = lds0 + (KS ? 0u : kh * 16384) + r16 * 128 + ((((uint32_t)h * 4 + kq) ^ ((r16 >> 1) & 7u)) << 4);
 
-    f32x16 acc[2][NB];
+    f32x4 acc[4][TB];
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int i = 0; i < 4; i++)
 #pragma unroll
-        for (int jj = 0; jj < NB; jj++)
-#pragma unroll
-            for (int e = 0; e < 16; e++) acc[i][jj][e] = 0.f;
+        for (int j = 0; j < TB; j++) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    u32x4 an[4] = {};      // the weight operand being prepared / multiplied, by row blocks
+    u32x4 breg[8] = {};    // its activation operands
+    typedef std::conditional_t<KS, uint32_t, u32x2> entry;
+    u32x2 rq[4];
+    entry sp[4];           // raw bytes and table entries of the step (KS: its half)
+    uint32_t dd[4];        // d of the super-block
 
-    uint32_t an[2][2][4];  // the weight operand of the step being prepared / multiplied: [row block][j][dword]
-    u32x4 breg[8] = {};    // its activation operands: [j * 4 + token block]; blocks from NB on are neither read nor multiplied
-
-    // ---- X(n): prepare step n (g: its position in super-block sbn): table entries at a super-block's first step, the
-    //      activation operands into registers, the weight operand converted, and this wavefront's copy requests:
-    //      activations of step n+3 in every X; the next super-block's weights in its X of g = 0 and 1 (the slot's last
-    //      reader was X(4 sbn - 1)); Sx of the next super-block in the X of g = 2 (kh = 1).  What is requested in X(n) is
-    //      complete when X(n+2) ends, a barrier before the first X that reads it ----
-    auto prepare = [&](const int khc, const uint32_t n, const uint32_t sbn, const int g) {
-        const uint32_t parn = (sbn - sb_begin) & 1u;
+    // raw bytes and table entries of a step, read while the half step before it multiplies.  (Written as instructions, as all
+    // LDS reads of the loop: the wait for them stands behind the MFMAs, tied to their registers.)
+    auto fetch = [&](auto GG, const uint32_t sb) {
+        constexpr int g = decltype(GG)::value;
+        uint32_t (&dr)[4] = dd;
+        entry (&spr)[4] = sp;
+        const uint32_t par = (sb - sb_begin) & 1u;
+        const uint32_t ra = raw_lane + par * Q_R_STAGE, ta = tab_lane + par * Q_T_STAGE;
+#define LARQL_RS(i) if constexpr (KS) asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(spr[i]) : "v"(ta), "n"(g * 2048 + (i) * 128)); \
+                    else asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(spr[i]) : "v"(ta), "n"(g * 2048 + (i) * 128)); \
+                    asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(rq[i]) : "v"(ra), "n"(g * 32 + (i) * 2304));
+        LARQL_RS(0) LARQL_RS(1) LARQL_RS(2) LARQL_RS(3)
+#undef LARQL_RS
         if (g == 0) {
-            stage_sb(parn);
-            asm volatile("" ::: "memory");
+            const uint32_t da = d_lane + par * GM * 4;
+            asm volatile("ds_read_b32 %0, %1" : "=v"(dr[0]) : "v"(da));
+            asm volatile("ds_read_b32 %0, %1 offset:64" : "=v"(dr[1]) : "v"(da));
+            asm volatile("ds_read_b32 %0, %1 offset:128" : "=v"(dr[2]) : "v"(da));
+            asm volatile("ds_read_b32 %0, %1 offset:192" : "=v"(dr[3]) : "v"(da));
         }
-        uint32_t sp[2];
-        u32x4 rq[2];
-        scales_of((uint32_t)g, sp);
-        raw_of(parn, (uint32_t)g, rq);
-        const uint32_t b0 = b_lane + (uint32_t)g * G_B_STAGE + b_col[0], b1 = b_lane + (uint32_t)g * G_B_STAGE + b_col[1];
-        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(sp[0]), "+v"(sp[1]), "+v"(rq[0]), "+v"(rq[1]));
-        // (one activation operand read per piece of the conversion: what LDS returns goes into the register file ahead of the
-        // other wavefront's MFMAs when this wavefront is the older of the two, and eight reads in a row hold them up)
-#define LARQL_RD(G) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(breg[G]) : "v"((G) < 4 ? b0 : b1), "n"(((G) & 3) * 4096));
-#define LARQL_PIECE(G)                                                                                                      \
-        if constexpr (((G) & 3) < NB) LARQL_RD(G)                                                                           \
-        convert4(rq[(G) >> 2][(G) & 3], sp[(G) >> 2], an[(G) >> 2][((G) >> 1) & 1][2 * ((G) & 1)], an[(G) >> 2][((G) >> 1) & 1][2 * ((G) & 1) + 1]); \
+    };
+    auto arrived = [&]() {
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(rq[0]), "+v"(rq[1]), "+v"(rq[2]), "+v"(rq[3]), "+v"(sp[0]), "+v"(sp[1]), "+v"(sp[2]), "+v"(sp[3]),
+                     "+v"(dd[0]), "+v"(dd[1]), "+v"(dd[2]), "+v"(dd[3]));
+    };
+    auto entry_of = [&](const int i, const int h) -> uint32_t {
+        if constexpr (KS) return sp[i];
+        else return sp[i][h];
+    };
+    // prepare half step (g, h) of super-block sb; at g = 2 also the tables of sb + 1, whose weights landed at g = 1
+    auto prepare = [&](auto KH, auto GG, auto HH, const uint32_t sb) {
+        constexpr int khc = decltype(KH)::value, g = decltype(GG)::value, h = decltype(HH)::value;
+        constexpr int slot = g % (int)NB;
+        const uint32_t par = (sb - sb_begin) & 1u;
+#define LARQL_RB(j) if constexpr ((j) < TB) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(breg[j]) : "v"(b_lane[h]), "n"(slot * (int)B_STAGE + (j) * 2048));
+        LARQL_RB(0) LARQL_RB(1) LARQL_RB(2) LARQL_RB(3) LARQL_RB(4) LARQL_RB(5) LARQL_RB(6) LARQL_RB(7)
+#undef LARQL_RB
         __builtin_amdgcn_sched_barrier(0);
-        LARQL_PIECE(0) LARQL_PIECE(1) LARQL_PIECE(2) LARQL_PIECE(3) LARQL_PIECE(4) LARQL_PIECE(5) LARQL_PIECE(6) LARQL_PIECE(7)
-#undef LARQL_PIECE
-#undef LARQL_RD
-        issue_b(n + 3, (uint32_t)((g + 3) & 3), 0);
-        issue_b(n + 3, (uint32_t)((g + 3) & 3), 1);
-        if (g == 0) { issue_raw(sbn + 1, 0); issue_raw(sbn + 1, 1); if (!khc) issue_raw(sbn + 1, 2); }
-        if (g == 1) { issue_raw(sbn + 1, khc ? 2 : 3); issue_raw(sbn + 1, khc ? 3 : 4); }
-        if (g == 2 && khc) issue_sx(sbn + 1);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const f16x2 e = __builtin_bit_cast(f16x2, entry_of(i, h)), dp = __builtin_bit_cast(f16x2, dd[i]);
+            const f16x2 sc = {e[0], e[0]}, o = {e[1], e[1]}, d = {dp[0], dp[0]}, c = sc * (_Float16)-1152.f;
+            uint32_t o0, o1, o2, o3;
+            convert4(rq[i].x, h, sc, c, d, o, o0, o1);
+            convert4(rq[i].y, h, sc, c, d, o, o2, o3);
+            an[i] = (u32x4){o0, o1, o2, o3};
+        }
+        if (g == 2 && (KS || h == 0)) stage(khc, par ^ 1u, 0);
+        if (g == 2 && (KS || h == 1)) stage(khc, par ^ 1u, 1);
         asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(breg[0]), "+v"(breg[1]), "+v"(breg[2]), "+v"(breg[3]), "+v"(breg[4]), "+v"(breg[5]), "+v"(breg[6]), "+v"(breg[7]));
-        // own requests still in flight: this X's and the one's before
-        const int mine[2][4] = {{5, 4, 2, 2}, {4, 4, 3, 2}};
-        const int fly = mine[khc][g] + mine[khc][(g + 3) & 3];
-        if (fly == 4) GEMM_WAIT_VMCNT(4);
-        else if (fly == 5) GEMM_WAIT_VMCNT(5);
-        else if (fly == 6) GEMM_WAIT_VMCNT(6);
-        else if (fly == 7) GEMM_WAIT_VMCNT(7);
-        else if (fly == 8) GEMM_WAIT_VMCNT(8);
-        else GEMM_WAIT_VMCNT(9);
+        if (khc == 1 && g == 1 && (KS || h == 1)) GEMM_WAIT_VMCNT(0);
         __builtin_amdgcn_s_setprio(3);  // (the multiply phase comes next)
     };
-    // ---- M: the sixteen MFMAs of a prepared step, back to back.  At a super-block's second step the wavefront kh = 0
-    //      first adds the super-block's offsets, sum_sub (8 d sc6 - dmin mn6) * Sx, one 16-deep MFMA per block (all of
-    //      them in one wavefront: a token's sum is then formed in the same order whichever token block it sits in) ----
-    auto multiply = [&](const int khc, const int g) {
-        if (g == 1 && khc == 0 && with_mins) {
-            f16x8 amf[2], bmf[NB];
+    // multiply it; fetch the next step's raw bytes; ask for the activations three steps ahead (KS; else the next step's, whose slot the step
+    // before released) or for the weights two super-blocks ahead.  Own copies that may still fly at the end: the activations of the
+    // two steps after the next; of the weights everything, until g = 1 prepares
+    auto multiply = [&](auto KH, auto GG, auto HH, auto GN, const uint32_t s, const uint32_t sb, const uint32_t sbn) {
+        constexpr int khc = decltype(KH)::value, g = decltype(GG)::value, h = decltype(HH)::value;
+        if (KS || h == 1) fetch(GN, sbn);
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_nop 1");  // (the operand may have been written by the instruction before)
+        auto request = [&](const int k) {
+            if (khc == 0) {
+                if (KS && k % 8 == 3) issue_b(s + 3, (g + 3) & 3, k / 8);
+                if (!KS && h == 0 && k % 4 == 3) issue_b(s + 1, (g + 1) & 1, k / 4);
+            } else if ((KS || h == 1) && (g == 2 || g == 3)) {
+                // three pieces in the second half of g = 2, six in g = 3
+                if (g == 2 && k == 2 * TB - 1) arrived();  // (the slot's last readers: this wavefront here, its pair a barrier ago)
+                if (g == 2 && k >= 2 * TB && (k - 2 * TB) % (TB / 2) == 0 && (k - 2 * TB) / (TB / 2) < 3) issue_raw(sb + 2, (k - 2 * TB) / (TB / 2));
+                if (g == 3 && k % (TB / 2) == 0 && k / (TB / 2) < 6) issue_raw(sb + 2, 3 + k / (TB / 2));
+            }
+        };
 #pragma unroll
-            for (int i = 0; i < 2; i++) amf[i] = *reinterpret_cast<const f16x8 *>(glds + G_AM_OFF + (wm + i * 32 + row32) * 32 + kgrp * 16);
+        for (int j = 0; j < TB; j++)
 #pragma unroll
-            for (int jj = 0; jj < NB; jj++) bmf[jj] = *reinterpret_cast<const f16x8 *>(glds + G_BM_OFF + (jj * 32 + row32) * 32 + kgrp * 16);
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int jj = 0; jj < NB; jj++) acc[i][jj] = __builtin_amdgcn_mfma_f32_32x32x16_f16(amf[i], bmf[jj], acc[i][jj], 0, 0, 0);
-        }
-        f16x8 af[2][2];
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-            for (int j = 0; j < 2; j++) af[i][j] = __builtin_bit_cast(f16x8, (u32x4){an[i][j][0], an[i][j][1], an[i][j][2], an[i][j][3]});
-#pragma unroll
-        for (int G = 0; G < 8; G++)
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-                if ((G & 3) < NB) acc[i][(G & 3) % NB] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i][G >> 2], __builtin_bit_cast(f16x8, breg[G]), acc[i][(G & 3) % NB], 0, 0, 0);
+            for (int i = 0; i < 4; i++) {
+                asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc[i][j]) : "v"(an[i]), "v"(breg[j]));
+                request(j * 4 + i);
+            }
         __builtin_amdgcn_s_setprio(0);
+        arrived();
+        if (khc == 0) {
+            if (KS) GEMM_WAIT_VMCNT(2 * CP);
+            else if (h == 1) GEMM_WAIT_VMCNT(0);
+        }
     };
-
-    // ---- prologue: the first super-block's weights, the first Sx, activation steps 0..2 ----
-    if (kh) issue_sx(sb_begin);
-#pragma unroll
-    for (int p = 0; p < 5; p++)
-        if (p < 4 || !kh) issue_raw(sb_begin, p);
-#pragma unroll
-    for (int q = 0; q < 2; q++) { issue_b(0, 0, q); issue_b(1, 1, q); issue_b(2, 2, q); }
-    GEMM_WAIT_VMCNT(0);
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    // The two wavefronts of a SIMD take turns: while one multiplies a step, the other prepares its next one.
-    //   kh = 0:  X(0) | M(0)   X(1) | M(1)   X(2) | ...
-    //   kh = 1:       | X(0)   M(0) | X(1)   M(1) | ...          (| = barrier)
-    // (each wavefront runs its own copy of the loop: no merge of the two orders inside it; both pass the same barriers)
-    // (nothing moves across a change of phase: not memory accesses, and not the MFMAs either, which the scheduler would
-    // otherwise spread over the other phase)
-    auto phase_end = [&]() {
+    auto half_end = [&]() {
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("" ::: "memory");
     };
+
+    // ---- prologue: exponents and token scales, the first two super-blocks' weights, the first activation steps; tables of the first ----
+    if (kh) {
+        copy4_to_lds(rexp + row0, (min(row0 + wm + lane, rows - 1) - row0) * 4, lds0 + Q_E_OFF + wm * 4);
+#pragma unroll
+        for (int p = 0; p < 9; p++) issue_raw(sb_begin, p);
+#pragma unroll
+        for (int p = 0; p < 9; p++) issue_raw(sb_begin + 1, p);
+        GEMM_WAIT_VMCNT(9);
+    } else {
+        copy4_to_lds(tok_scale + tok0, (min(tok0 + wm + lane, seq - 1) - tok0) * 4, lds0 + Q_S_OFF + wm * 4);
+#pragma unroll
+        for (int st = 0; st < (KS ? 3 : 1); st++)
+#pragma unroll
+            for (int q = 0; q < CP; q++) issue_b(st, st, q);
+        GEMM_WAIT_VMCNT(KS ? 2 * CP : 0);
+    }
+    half_end();
+    row_e = reinterpret_cast<const int *>(glds + Q_E_OFF)[wm + lane];
+    if (kh) { stage(1, 0, 0); stage(1, 0, 1); }
+    else { stage(0, 0, 0); stage(0, 0, 1); }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    half_end();
+    //   kh = 0:  P(0) | M(0) | P(1) M(1) | P(2) M(2) | ...
+    //   kh = 1:       | P(0) | M(0) P(1) | M(1) P(2) | ...          (| = barrier)
+    // What half step n reads of LDS was read before the barrier behind P(n): its slots are asked for again after it.
     auto run = [&](auto KH) {
         constexpr int khc = decltype(KH)::value;
-        if (khc == 0) prepare(0, 0, sb_begin, 0);
-        phase_end();
+        constexpr std::integral_constant<int, 0> I0;
+        constexpr std::integral_constant<int, KS ? khc : 0> H0;
+        fetch(I0, sb_begin);
+        arrived();
+        if (khc == 0) prepare(KH, I0, H0, sb_begin);
+        half_end();
         uint32_t s = 0;
         for (uint32_t sb = sb_begin; sb < sb_end; sb++) {
-#pragma unroll
-            for (int g = 0; g < 4; g++, s++) {
-                if (khc == 0) multiply(0, g);
-                else prepare(1, s, sb, g);
-                phase_end();
+            auto turn = [&](auto GG, auto HH, auto GN, auto HN) {  // this half step, and the one after
+                constexpr int g = decltype(GG)::value, gn = decltype(GN)::value;
+                const uint32_t sbn = gn == 0 && g == 3 ? sb + 1 : sb;
                 if (khc == 0) {
-                    if (s + 1 < nsteps) prepare(0, s + 1, g == 3 ? sb + 1 : sb, (g + 1) & 3);
+                    multiply(KH, GG, HH, GN, s, sb, sbn);
+                    half_end();
+                    prepare(KH, GN, HN, sbn);
                 } else {
-                    multiply(1, g);
+                    prepare(KH, GG, HH, sb);
+                    half_end();
+                    multiply(KH, GG, HH, GN, s, sb, sbn);
                 }
-                phase_end();
+            };
+            constexpr std::integral_constant<int, 1> I1;
+            constexpr std::integral_constant<int, 2> I2;
+            constexpr std::integral_constant<int, 3> I3;
+            if constexpr (KS) {
+                turn(I0, H0, I1, H0); s++; turn(I1, H0, I2, H0); s++; turn(I2, H0, I3, H0); s++; turn(I3, H0, I0, H0); s++;
+            } else {
+                turn(I0, I0, I0, I1); turn(I0, I1, I1, I0); s++; turn(I1, I0, I1, I1); turn(I1, I1, I2, I0); s++;
+                turn(I2, I0, I2, I1); turn(I2, I1, I3, I0); s++; turn(I3, I0, I3, I1); turn(I3, I1, I0, I0); s++;
             }
         }
     };
@@ -883,62 +939,49 @@ __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *
     else run(std::integral_constant<int, 1>{});
     GEMM_WAIT_VMCNT(0);  // the clamped requests past the end
 
-    // The pair adds its partial sums through LDS, where the results also take the shape in which a store instruction
-    // writes whole lines: a row group's 64-row x 128-token block as [token][row] (token rows padded to 68 floats: the
-    // lanes of a write phase hit different banks) in the pair's own 34 KB; wavefront 1 parks, wavefront 0 adds its own
-    // and parks the sum, then every lane of the pair stores 16 bytes of a 256-byte run of one token.  (Each parking 32 rows of the
-    // other and adding its own 32 to what the other parked: 4096 x 4096 with 16 tokens 17.5 -> 17.9 us, 14277 x 2048 with 335 45.3 -> 45.6.)
-    const uint32_t rc = (lane & 15u) * 4, r = row0 + wm + rc;
-    float back[4];  // 2^-E of this lane's four rows (asked for here: behind the barriers nothing would hide the trip)
+    asm volatile("s_nop 15\n\ts_nop 15");  // (results of the last multiplications are not read for 18 cycles)
 #pragma unroll
-    for (int e = 0; e < 4; e++) back[e] = ldexpf(1.f, -rexp[min(r + e, rows - 1)]);
-    __builtin_amdgcn_s_barrier();  // nobody's copies are still landing in what becomes somebody's block
-    asm volatile("" ::: "memory");
-    constexpr uint32_t EP_LD = G_EP_LD;
-    float *blk = reinterpret_cast<float *>(glds) + wq * (GN * EP_LD);
-    if (kh) {
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < TB; j++) asm volatile("" : "+v"(acc[i][j]));
+    // ---- results: lane (token r16, kq) holds rows 4 kq .. 4 kq + 3 of every block of 16 x 16 ----
+    constexpr int I = KS ? 2 : 4;  // row blocks that this wavefront stores
+    const uint32_t i0 = KS ? 2 * kh : 0;
+    f32x4 back[I];
+#pragma unroll
+    for (int i = 0; i < I; i++) {
+        const i32x4 e = *reinterpret_cast<const i32x4 *>(glds + Q_E_OFF + (wm + (i0 + i) * 16 + kq * 4) * 4);
+        back[i] = (f32x4){ldexpf(1.f, -e[0]), ldexpf(1.f, -e[1]), ldexpf(1.f, -e[2]), ldexpf(1.f, -e[3])};
+    }
+    if (KS) {
+        __builtin_amdgcn_s_barrier();  // nobody's copies are still landing in what becomes somebody's block
+        asm volatile("" ::: "memory");
+        f32x4 *blk = reinterpret_cast<f32x4 *>(glds) + wave * (2 * TB * 64);
 #pragma unroll
         for (int i = 0; i < 2; i++)
 #pragma unroll
-            for (int jj = 0; jj < NB; jj++)
-#pragma unroll
-                for (int q = 0; q < 4; q++)  // registers 4q .. 4q+3 of a block: rows 8q + 4kgrp .. +3, token row32
-                    *reinterpret_cast<f32x4 *>(blk + (jj * 32 + row32) * EP_LD + i * 32 + q * 8 + kgrp * 4) =
-                        (f32x4){acc[i][jj][4 * q], acc[i][jj][4 * q + 1], acc[i][jj][4 * q + 2], acc[i][jj][4 * q + 3]};
-    }
-    __syncthreads();
-    if (!kh) {
+            for (int j = 0; j < TB; j++) blk[(i * TB + j) * 64 + lane] = kh ? acc[i][j] : acc[2 + i][j];
+        __syncthreads();
+        const f32x4 *other = reinterpret_cast<const f32x4 *>(glds) + (wave ^ 4u) * (2 * TB * 64);
 #pragma unroll
         for (int i = 0; i < 2; i++)
 #pragma unroll
-            for (int jj = 0; jj < NB; jj++)
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    f32x4 *at = reinterpret_cast<f32x4 *>(blk + (jj * 32 + row32) * EP_LD + i * 32 + q * 8 + kgrp * 4);
-                    const f32x4 other = *at;
-                    *at = (f32x4){acc[i][jj][4 * q] + other[0], acc[i][jj][4 * q + 1] + other[1], acc[i][jj][4 * q + 2] + other[2], acc[i][jj][4 * q + 3] + other[3]};
-                }
+            for (int j = 0; j < TB; j++) acc[i][j] = (kh ? acc[2 + i][j] : acc[i][j]) + other[(i * TB + j) * 64 + lane];
     }
-    __syncthreads();
-    const bool vec_ok = (rows & 3u) == 0 && (((uintptr_t)(partial ? partial : out)) & 15u) == 0;
-#pragma unroll 4
-    for (int it = 0; it < 16; it++) {
-        const uint32_t tl = (kh * 16 + it) * 4 + (lane >> 4), tok = tok0 + tl;
+#pragma unroll
+    for (int j = 0; j < TB; j++) {
+        const uint32_t tok = tok0 + (KS ? 0u : kh * 128) + j * 16 + r16;
         if (tok >= seq) continue;
-        f32x4 v = *reinterpret_cast<const f32x4 *>(blk + tl * EP_LD + rc);
-        float *o = partial ? partial + ((size_t)blockIdx.z * seq + tok) * rows + r : out + (size_t)tok * rows + r;
         // (partial sums stay without the token's scale; q4k_gemm_reduce_kernel adds the slabs in order and applies it)
-        const float ts = partial ? 1.f : tok_scale[tok];
+        const float ts = partial ? 1.f : reinterpret_cast<const float *>(glds + Q_S_OFF)[tok - tok0];
+        const uint32_t r = row0 + wm + i0 * 16 + kq * 4;
+        float *o = (partial ? partial + ((size_t)range * seq + tok) * rows : out + (size_t)tok * rows) + r;
 #pragma unroll
-        for (int e = 0; e < 4; e++) v[e] *= ts * back[e];
-        if (vec_ok && r + 3 < rows) {
-            f32x4 *ov = reinterpret_cast<f32x4 *>(o);
-            if (!partial && accumulate) { const f32x4 old = *ov; v += old; }
-            *ov = v;
-        } else {
+        for (int i = 0; i < I; i++) {
+            f32x4 v = acc[i][j];
 #pragma unroll
-            for (int e = 0; e < 4; e++)
-                if (r + e < rows) o[e] = (!partial && accumulate) ? o[e] + v[e] : v[e];
+            for (int e = 0; e < 4; e++) v[e] *= ts * back[i][e];
+            store4(o + i * 16, v, rows - min(rows, r + i * 16));
         }
     }
 }
@@ -959,34 +1002,30 @@ hipError_t q4k_gemm_prep_launch(hipStream_t s, const void *x, int x_is_bf16, uin
 
 
 // K-ranges per output tile (1 = no split), where one 256x128 workgroup runs per CU and the unsplit tiles leave CUs idle.
-// In tenths of a microsecond: a super-block of a tile takes 45, a split's
-// reduction 50 for the launch and 8 bytes per slab element at 4 TB/s.  The range count with the smallest sum is taken, any
-// number up to 32 whose workgroups all run at once (so the slabs stay below 256 tiles, 34 MB).  Doubling up to 8, the rule
-// before, kept 120 of 256 CUs on a 3840 x 15360 matrix with 77 tokens: with this one
-// (15 ranges), the reduction above and the kept activations of the preparation the call went from 46.4 to 36.2 us, and with
-// blocks of 32 tokens (q4k_gemm_f16_launch) to 33.7 (6 preparation, 26 GEMM, 5 reduction in the kernel trace).
+// In tenths of a microsecond: a super-block of a tile takes 30, a split's
+// reduction 30 for the launch and 8 bytes per slab element at 3 TB/s.  The range count with the smallest sum is taken, any
+// number up to 32 whose workgroups all run at once (so the slabs stay below 256 tiles, 34 MB).
 // The ranges group a result's additions, so they must not change with the number of tokens inside a tile (a token's bits would
 // depend on how many others came with it): the last tile counts as five eighths full.
-// Fitted on calls of 170 shapes (512 to 15360 rows, 1024 to 15360 elements, 16 to 512 tokens) at every range count: 0.5 % above
-// each shape's best on average; at the worst 15360 x 1024 with 16 tokens 18.1 us unsplit and 14.9 with 4 ranges (with 128 tokens 26.0
-// unsplit and 29.2 with 2), 4096 x 4096 with 16 16.9 with 8 and 16.1 with 16, 8000 x 2048 with 512 41.6 unsplit and 39.4 with 2.
+// Fitted on calls of 54 shapes (1000 to 15360 rows, 1024 to 15360 elements, 16 to 600 tokens) at every range count: 0.2 % above
+// each shape's best on average; at the worst 5402 x 1536 with 16 tokens 10 % (3 ranges where 6 are best).
 uint32_t q4k_gemm_splits(uint32_t rows, uint32_t hidden, uint32_t seq, uint32_t cu_count) {
     const uint64_t nsb = hidden / 256, cols = (seq + GN - 1) / GN, tiles = (uint64_t)((rows + GM - 1) / GM) * cols, tokens = cols * GN - GN * 3 / 8;
-    uint64_t best = nsb * 45, splits = 1;
+    uint64_t best = nsb * 30, splits = 1;
     for (uint64_t z = 2; z <= 32 && z <= nsb && tiles * z <= cu_count; z++) {
         const uint64_t per = (nsb + z - 1) / z;
         if ((nsb + per - 1) / per != z) continue;  // (the same ranges as a smaller count)
-        const uint64_t cost = per * 45 + 50 + z * rows * tokens * 8 / 400000;
+        const uint64_t cost = per * 30 + 30 + z * rows * tokens * 8 / 300000;
         if (cost < best) { best = cost; splits = z; }
     }
     return (uint32_t)splits;
 }
 
-// `rexp` (from q4k_gemm_prep_launch): the rows' scales ride in the f16 weight operand; without it the weight operand is
-// the exact integer and the rows' f32 scales are applied per super-block
+// `rexp` (from q4k_gemm_prep_launch): the f16 weight operand is the whole weight (`sx`, `with_mins` and `accumulate` are not used);
+// without it the weight operand is the exact integer and the rows' f32 scales are applied per super-block
 hipError_t q4k_gemm_f16_launch(hipStream_t s, const uint8_t *w, const uint16_t *xh, const uint16_t *sx, const int *rexp, const float *tok_scale,
                                float *out, uint32_t rows, uint32_t hidden, uint32_t seq, int with_mins, int accumulate, uint32_t splits,
-                               float *partial) {
+                               float *partial, uint32_t cu_count) {
     if (rows == 0 || seq == 0) return hipSuccess;
     const uint32_t nsb = hidden / 256;
     const bool split = splits > 1 && partial;
@@ -994,7 +1033,8 @@ hipError_t q4k_gemm_f16_launch(hipStream_t s, const uint8_t *w, const uint16_t *
     static std::atomic<bool> attr_set{false};  // dynamic LDS above 64 KB has to be allowed once per process
     if (!attr_set) {
         hipError_t e = hipFuncSetAttribute((const void *)q4k_gemm_exact_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        for (const void *k : {(const void *)q4k_gemm_pair_kernel<1>, (const void *)q4k_gemm_pair_kernel<2>, (const void *)q4k_gemm_pair_kernel<3>, (const void *)q4k_gemm_pair_kernel<4>})
+        for (const void *k : {(const void *)q4k_gemm_pair_kernel<2, true>, (const void *)q4k_gemm_pair_kernel<4, true>, (const void *)q4k_gemm_pair_kernel<6, true>,
+                              (const void *)q4k_gemm_pair_kernel<8, true>, (const void *)q4k_gemm_pair_kernel<8, false>})
             if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         if (e != hipSuccess) return e;
         attr_set = true;
@@ -1003,13 +1043,20 @@ hipError_t q4k_gemm_f16_launch(hipStream_t s, const uint8_t *w, const uint16_t *
     float *slab = split ? partial : (float *)nullptr;
     // a prompt of one token tile reads and multiplies only its blocks of 32 tokens (3840 x 15360 with 16 / 64 / 96 tokens: 32.5 / 36.4 /
     // 37.2 us per call with all four blocks, 27.2 / 32.9 / 35.4 so); the copies stay whole, clamped to the last token
-#define LARQL_PAIR(NB) hipLaunchKernelGGL(q4k_gemm_pair_kernel<NB>, grid, dim3(QTHREADS), G_LDS_BYTES, s, w, xh, sx, rexp, tok_scale, out, rows, hidden, seq, \
-                                          with_mins, accumulate, per, slab)
+#define LARQL_PAIR(TB, KS) hipLaunchKernelGGL((q4k_gemm_pair_kernel<TB, KS>), dim3(grid.x * tok_tiles * z), dim3(QTHREADS), Q_LDS_BYTES, s, w, xh, rexp, tok_scale, out, rows, \
+                                              hidden, seq, grid.x, tok_tiles, per, slab)
     if (rexp) {
-        if (seq <= 32) LARQL_PAIR(1);
-        else if (seq <= 64) LARQL_PAIR(2);
-        else if (seq <= 96) LARQL_PAIR(3);
-        else LARQL_PAIR(4);
+        // 256 tokens per workgroup take 1.8 times as long as 128 (98 against 53 us at 3840 elements, all compute units busy): taken where that
+        // saves rounds over the chip (15360 x 3840 with 2048 tokens: 2 against 4, 217 and 236 us; 13270 x 3840 with 1783: 2 against 3,
+        // 205 and 192).  The rule sees a prompt's length in whole tiles of 128 only: a token's bits do not depend on its companions
+        const uint32_t tiles_n = grid.x * grid.y, tiles_w = grid.x * ((grid.y + 1) / 2);
+        const bool wide = z == 1 && grid.y > 1 && ((uint64_t)((tiles_w + cu_count - 1) / cu_count) * 9 < (uint64_t)((tiles_n + cu_count - 1) / cu_count) * 5);
+        const uint32_t tok_tiles = wide ? (grid.y + 1) / 2 : grid.y;
+        if (wide) LARQL_PAIR(8, false);
+        else if (seq <= 32) LARQL_PAIR(2, true);
+        else if (seq <= 64) LARQL_PAIR(4, true);
+        else if (seq <= 96) LARQL_PAIR(6, true);
+        else LARQL_PAIR(8, true);
     }
 #undef LARQL_PAIR
     else
@@ -1017,10 +1064,7 @@ hipError_t q4k_gemm_f16_launch(hipStream_t s, const uint8_t *w, const uint16_t *
                            accumulate, per, slab);
     if (split) {
         const size_t n = (size_t)rows * seq;
-        if (rows % 4 == 0 && (((uintptr_t)partial | (uintptr_t)out) & 15u) == 0)
-            hipLaunchKernelGGL(q4k_gemm_reduce_kernel<4>, dim3((uint32_t)((n / 4 + 255) / 256)), dim3(256), 0, s, partial, z, tok_scale, out, rows, seq, accumulate);
-        else
-            hipLaunchKernelGGL(q4k_gemm_reduce_kernel<1>, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, partial, z, tok_scale, out, rows, seq, accumulate);
+        hipLaunchKernelGGL(q4k_gemm_reduce_kernel, dim3((uint32_t)((n + 1023) / 1024)), dim3(256), 0, s, partial, z, tok_scale, out, rows, seq, accumulate);
     }
     return hipGetLastError();
 }

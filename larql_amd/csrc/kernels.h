@@ -157,7 +157,7 @@ hipError_t q4k_gemm_prep_launch(hipStream_t s, const void *x, int x_is_bf16, uin
                                 uint16_t *sx, float *tok_scale, int *any_lo, const uint8_t *w, uint32_t rows, int *rexp);
 hipError_t q4k_gemm_f16_launch(hipStream_t s, const uint8_t *w, const uint16_t *xh, const uint16_t *sx, const int *rexp, const float *tok_scale,
                                float *out, uint32_t rows, uint32_t hidden, uint32_t seq, int with_mins, int accumulate, uint32_t splits,
-                               float *partial);
+                               float *partial, uint32_t cu_count);
 uint32_t q4k_gemm_splits(uint32_t rows, uint32_t hidden, uint32_t seq, uint32_t cu_count);  // partial: [splits][seq][rows] floats
 
 // One token through a bank of MXFP4 experts, a launch per projection stage (moe1_launch): a small argument block

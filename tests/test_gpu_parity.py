@@ -1786,6 +1786,35 @@ def test_q4k_gemm_tokens_of_a_tile_do_not_depend_on_how_many_they_are(be, rows, 
         assert np.array_equal(got, host[:seq]), seq
 
 
+@pytest.mark.parametrize("rows,hidden,seq", [(16637, 768, 500), (32763, 256, 257)])
+def test_q4k_gemm_tiles_of_256_tokens(be, rows, hidden, seq):
+    """Calls that take 256 tokens per workgroup (fewer rounds over the chip): a last row tile and a last token tile that are not
+    full, rows no multiple of four, one super-block and an odd number of them.  Every element against the same tokens in calls of 128
+    (the other kernel: the same products, added in another order), the first and the last rows against the oracle."""
+    rng = np.random.default_rng(rows)
+    q = rng.integers(0, 256, size=(rows * hidden // 256, 144), dtype=np.uint8)
+    q[:, 0:4] = np.array([0x00, 0x2C, 0x00, 0x28], np.uint8)   # d = 2^-4, dmin = 2^-5
+    xb = O.f32_to_bf16(rng.standard_normal((seq, hidden)).astype(F)).reshape(seq, hidden)
+    dw, dx, do = be.to_device(q), be.to_device(xb), be.to_device(np.full(seq * rows, 7.0, F))
+    assert be.dev_q4k_gemm(dw, dx, rows, hidden, seq, do), be.last_error()
+    be.synchronize()
+    got = be.d2h(do, (seq, rows), F)
+    part = np.empty((seq, rows), F)
+    for t in range(0, seq, 128):
+        n = min(128, seq - t)
+        assert be.dev_q4k_gemm(dw, dx + 2 * t * hidden, rows, hidden, n, do), be.last_error()
+        be.synchronize()
+        part[t:t + n] = be.d2h(do, (n, rows), F)
+    # f32 additions of at most 768 terms in two orders: 768 x 2^-24 of the largest partial sums, which stay below 8 result sizes
+    assert np.abs(got - part).max() < 8 * 768 * 2.0 ** -24 * np.sqrt((part.astype(np.float64) ** 2).mean())
+    X = (xb.astype(np.uint32) << 16).view(F)
+    for r0 in (0, rows - 40):
+        want = O.q4k_matmul(q.reshape(rows, -1)[r0:r0 + 40].reshape(-1).copy(), X, 40, hidden, seq)
+        assert rel_l2(got[:, r0:r0 + 40], want) < 5e-4
+    for p in (dw, dx, do):
+        be.free(p)
+
+
 def test_q4k_gemm_row_scales_of_any_size_and_uneven_blocks(be):
     """The device tier's GEMM carries each row's scale in an f16 operand behind a per-row exponent: rows whose weights
     differ by twelve orders of magnitude, rows of zeros, and a row with one super-block far larger than the others
