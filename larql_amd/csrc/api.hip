@@ -192,24 +192,51 @@ hipError_t wait_stream(larql_hip_ctx *c) {
     return e;
 }
 
+// A slice of the page-locked ring holding `bytes` of `host`, or null: small operands only, and slices of one call never overlap (a
+// call that stages more than the ring holds before it waits for the stream gets none for the rest).
+uint8_t *stage_up(larql_hip_ctx *c, const void *host, size_t bytes) {
+    const size_t slice = (bytes + 255) & ~(size_t)255;
+    if (bytes > kPinSmall || c->pin_up_call + slice > kPinUpBytes || ensure_pinned(c, c->pin_up, kPinUpBytes + 256) != LARQL_OK) return nullptr;
+    // (nothing staged since the stream was waited for: the ring starts over, so that the calls of a loop find their operand at one place)
+    if (c->pin_up_call == 0 || c->pin_up_off + slice > kPinUpBytes) c->pin_up_off = 0;
+    uint8_t *stage = (uint8_t *)c->pin_up.host + c->pin_up_off;
+    memcpy(stage, host, bytes);
+    c->pin_up_off += slice;
+    c->pin_up_call += slice;
+    return stage;
+}
+
 int upload(larql_hip_ctx *c, DevBuf &b, const void *host, size_t bytes) {
     int rc = ensure(c, b, bytes + 64);
     if (rc) return rc;
     if (!bytes) return LARQL_OK;
-    // small: through the page-locked ring (slices of one call never overlap: a call that stages more than the ring
-    // holds before it waits for the stream takes the pageable path for the rest)
-    const size_t slice = (bytes + 255) & ~(size_t)255;
-    if (bytes <= kPinSmall && c->pin_up_call + slice <= kPinUpBytes && ensure_pinned(c, c->pin_up, kPinUpBytes) == LARQL_OK) {
-        if (c->pin_up_off + slice > kPinUpBytes) c->pin_up_off = 0;
-        uint8_t *stage = (uint8_t *)c->pin_up.host + c->pin_up_off;
-        memcpy(stage, host, bytes);
-        c->pin_up_off += slice;
-        c->pin_up_call += slice;
-        HIPCHECK(c, hipMemcpyAsync(b.p, stage, bytes, hipMemcpyHostToDevice, c->stream));
-        return LARQL_OK;
-    }
+    if (const uint8_t *stage = stage_up(c, host, bytes)) host = stage;
     HIPCHECK(c, hipMemcpyAsync(b.p, host, bytes, hipMemcpyHostToDevice, c->stream));
     return LARQL_OK;
+}
+
+// An activation that the call's kernels read once per workgroup: where they find it.  Up to 12 KB stays in the page-locked ring and is
+// read there (one trip over PCIe, beside the first weights'); longer ones are brought to `b` by a kernel, whose reads fly together.
+// The asynchronous copy before is a packet of its own that the launch waits for, and above 16 KB another engine's.  Calls on registered
+// weights, us, copy / in place (*: through a kernel): Q4_K 3072 x 1024 23.1 / 19.5, 3072 x 2560 23.2 / 20.2, 3072 x 4352 26.3 / 23.1*, 2560 x 10240 29.3 /
+// 25.0*; Q8_0 24.9 / 24.0 at 3072 x 2560, 30.4 / 25.9* at 4352.  The line: with 16 KB in place Q8_0 3072 x 4096 takes 26.0 / 26.2 (Q4_K 23.3 / 21.7).
+constexpr size_t kPinInPlace = 12u << 10;
+int upload_activation(larql_hip_ctx *c, DevBuf &b, const void *host, size_t bytes, const void **dev) {
+    if (bytes && bytes % 16 == 0) {
+        if (bytes > kPinInPlace) {
+            int rc = ensure(c, b, bytes + 64);
+            if (rc) return rc;
+        }
+        if (const uint8_t *stage = stage_up(c, host, bytes)) {
+            const uint8_t *at = (const uint8_t *)c->pin_up.dev + (stage - (uint8_t *)c->pin_up.host);
+            *dev = bytes <= kPinInPlace ? (const void *)at : b.p;
+            if (bytes > kPinInPlace) HIPCHECK(c, copy_launch(c->stream, at, b.p, bytes, (uint32_t)((bytes / 16 + 255) / 256)));
+            return LARQL_OK;
+        }
+    }
+    const int rc = upload(c, b, host, bytes);
+    *dev = b.p;
+    return rc;
 }
 
 struct Submission {
@@ -709,7 +736,8 @@ static int host_matvec_multi(larql_hip_ctx *c, int kind, size_t n_mats, const ui
     if (n_mats > kHostMats) return fail(c, LARQL_UNSUPPORTED, "at most %zu matrices per host-tier submission", kHostMats);
     HIPCHECK(c, hipSetDevice(c->device));
     std::vector<GemvJob> jobs;
-    int rc = upload(c, c->x, x, x_bytes);
+    const void *dx = nullptr;
+    int rc = upload_activation(c, c->x, x, x_bytes, &dx);
     if (rc) return rc;
     size_t out_total = 0;
     for (size_t i = 0; i < n_mats; i++) out_total += rows[i];
@@ -723,7 +751,7 @@ static int host_matvec_multi(larql_hip_ctx *c, int kind, size_t n_mats, const ui
         rc = resolve_weights(c, w[i], w_len[i], c->w[i], &dw);
         if (rc) return rc;
         if (aux) { rc = resolve_weights(c, aux[i], aux_len[i], c->aux[i], &da); if (rc) return rc; }
-        jobs.push_back(make_job(kind, dw, da, c->x.p, d_out + off, rows[i], k));
+        jobs.push_back(make_job(kind, dw, da, dx, d_out + off, rows[i], k));
         off += rows[i];
     }
     Submission sub(c);
@@ -1052,14 +1080,15 @@ static int host_matvec_topk(larql_hip_ctx *c, int kind, const uint8_t *w, size_t
     const uint8_t *dw = nullptr;
     int rc = resolve_weights(c, w, need, c->w[0], &dw);
     if (rc) return rc;
-    rc = upload(c, c->x, x, x_len * 4);
+    const void *dx = nullptr;
+    rc = upload_activation(c, c->x, x, x_len * 4, &dx);
     if (rc) return rc;
     rc = ensure(c, c->scores, num_rows * 4 + 64);
     if (rc) return rc;
     TopkArea hits;
     rc = topk_area(c, 1, top_k, hits);
     if (rc) return rc;
-    std::vector<GemvJob> jobs{make_job(kind, dw, nullptr, c->x.p, (float *)c->scores.p, num_rows, hidden)};
+    std::vector<GemvJob> jobs{make_job(kind, dw, nullptr, dx, (float *)c->scores.p, num_rows, hidden)};
     Submission sub(c);
     rc = enqueue_jobs(c, jobs);
     if (rc) { (void)wait_stream(c); return rc; }
@@ -1370,10 +1399,11 @@ int larql_hip_gate_scores(larql_hip_ctx *c, int format, const uint8_t *gate, siz
     HIPCHECK(c, hipSetDevice(c->device));
     const uint8_t *dg = nullptr;
     rc = resolve_weights(c, gate, n * format_row_bytes(kind, hidden), c->w[0], &dg); if (rc) return rc;
-    rc = upload(c, c->x, x, batch * hidden * 4); if (rc) return rc;
+    const void *dx = nullptr;
+    rc = upload_activation(c, c->x, x, batch * hidden * 4, &dx); if (rc) return rc;
     rc = ensure(c, c->scores, batch * n * 4 + 64); if (rc) return rc;
     Submission sub(c);
-    rc = dev_gate_scores(c, kind, dg, (const float *)c->x.p, batch, n, hidden, (float *)c->scores.p);
+    rc = dev_gate_scores(c, kind, dg, (const float *)dx, batch, n, hidden, (float *)c->scores.p);
     if (rc) { (void)hipStreamSynchronize(c->stream); return rc; }
     HIPCHECK(c, hipMemcpyAsync(scores_out, c->scores.p, batch * n * 4, hipMemcpyDeviceToHost, c->stream));
     return sub.finish();
@@ -1395,13 +1425,14 @@ int larql_hip_gate_knn(larql_hip_ctx *c, int format, const uint8_t *gate, size_t
     HIPCHECK(c, hipSetDevice(c->device));
     const uint8_t *dg = nullptr;
     rc = resolve_weights(c, gate, n * format_row_bytes(kind, hidden), c->w[0], &dg); if (rc) return rc;
-    rc = upload(c, c->x, x, batch * hidden * 4); if (rc) return rc;
+    const void *dx = nullptr;
+    rc = upload_activation(c, c->x, x, batch * hidden * 4, &dx); if (rc) return rc;
     rc = ensure(c, c->scores, batch * n * 4 + 64); if (rc) return rc;
     TopkArea hits;
     rc = topk_area(c, batch, top_k, hits); if (rc) return rc;
     HIPCHECK(c, hipMemsetAsync(c->nan_flag + 1, 0, sizeof(int), c->stream));
     Submission sub(c);
-    rc = dev_gate_scores(c, kind, dg, (const float *)c->x.p, batch, n, hidden, (float *)c->scores.p);
+    rc = dev_gate_scores(c, kind, dg, (const float *)dx, batch, n, hidden, (float *)c->scores.p);
     if (rc) { (void)wait_stream(c); return rc; }
     rc = run_topk(c, (const float *)c->scores.p, (uint32_t)batch, (uint32_t)n, (uint32_t)top_k, true, hits.idx,
                   hits.val, hits.cnt, c->nan_flag + 1);

@@ -1714,6 +1714,32 @@ def test_moe_layer_refusals(be, fmt):
     assert be.moe_layer_create(*many) is None
 
 
+@pytest.mark.parametrize("k", [256, 3072, 3328, 10240, 139264])
+def test_host_activations_in_place_and_through_a_kernel(be, fmt, k):
+    """Host-tier activations are read in page-locked memory (up to 3072 elements), brought by a kernel (up to 131072) or copied.
+    Every call of a loop sees its own activation, bit for bit what the device tier computes on it, several matrices in one call too."""
+    rng = np.random.default_rng(k)
+    rows = 96
+    q = rng.integers(0, 256, size=(rows * k // 256, 144), dtype=np.uint8)
+    q[:, 0:4] = np.array([0x00, 0x2C, 0x00, 0x28], np.uint8)   # d = 2^-4, dmin = 2^-5
+    dw, do = be.to_device(q), be.malloc(rows * 4)
+    for call in range(6):
+        x = rng.standard_normal(k).astype(F)
+        got = be.q4k_matvec(q, x, rows, k)
+        dx = be.to_device(x)
+        assert be.dev_matvec(fmt.FMT_Q4_K, dw, None, dx, rows, k, do), be.last_error()
+        be.synchronize()
+        want = be.d2h(do, rows, F)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), call
+        both = be.q4k_dual_matvec(q, q, x, rows, k)
+        assert all(np.array_equal(b.view(np.uint32), want.view(np.uint32)) for b in both), call
+        hits = be.q4k_matvec_topk(q, x, rows, k, 3)
+        assert [np.float32(v).view(np.uint32) for _, v in hits] == [want[i].view(np.uint32) for i, _ in hits]
+        be.free(dx)
+    for p in (dw, do):
+        be.free(p)
+
+
 # ------------------------------------------------------------- prefill GEMM
 @pytest.mark.parametrize("rows,hidden,seq", [(300, 512, 70), (128, 3840, 128), (1, 256, 1), (257, 768, 33), (520, 8192, 200)])
 def test_q4k_gemm_mfma_matches_oracle(be, rows, hidden, seq):
