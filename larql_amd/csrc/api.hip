@@ -411,10 +411,10 @@ std::vector<std::vector<GemvJob>> group_by_kind(const std::vector<GemvJob> &jobs
     std::vector<GemvJob> jobs(jobs_in);
     for (GemvJob &j : jobs) j.kind = gemv_effective_kind(j);  // Q4_K rows the matrix-core kernel takes get their own launch
     std::vector<std::vector<GemvJob>> groups;
-    bool done[16] = {};
+    bool done[kGemvKinds] = {};
     for (size_t i = 0; i < jobs.size(); i++) {
         const int kind = jobs[i].kind;
-        if (jobs[i].rows == 0 || kind < 0 || kind > 15 || done[kind]) continue;
+        if (jobs[i].rows == 0 || kind < 0 || kind >= kGemvKinds || done[kind]) continue;
         done[kind] = true;
         std::vector<GemvJob> live;
         for (size_t t = i; t < jobs.size(); t++)
@@ -1348,8 +1348,8 @@ static size_t format_row_bytes(int kind, size_t k) {
 // One gate matrix against `batch` residual positions (x: [batch, hidden], scores: [batch, n]): jobs that
 // carry as many positions as the kernels take at once, so the matrix is read once per group.
 static void push_gate_jobs(std::vector<GemvJob> &jobs, int kind, const void *gate, const float *x, size_t batch, size_t n,
-                           size_t hidden, float *scores) {
-    const size_t cap = gemv_batch_capacity(kind, hidden);
+                           size_t hidden, float *scores, size_t n_layers = 1) {
+    const size_t cap = gemv_batch_take(kind, n, hidden, batch, n_layers);
     for (size_t b = 0; b < batch;) {
         const size_t take = std::min(cap, batch - b);
         GemvJob j = make_job(kind, gate, nullptr, x + b * hidden, scores + b * n, n, hidden);
@@ -1757,7 +1757,7 @@ int larql_hip_dev_gate_knn_static(larql_hip_ctx *c, int format, const void *gate
         for (size_t b = 0; b < batch; b++)
             jobs[n_jobs++] = make_job(kind, gate, q8s + b * (hidden / 32), q8 + b * hidden, scores + b * n, n, hidden);
     } else {
-        const size_t cap = gemv_batch_capacity(kind, hidden);
+        const size_t cap = gemv_batch_take(kind, n, hidden, batch, 1);
         for (size_t b = 0; b < batch;) {
             const size_t take = std::min(cap, batch - b);
             GemvJob j = make_job(kind, gate, nullptr, x + b * hidden, scores + b * n, n, hidden);
@@ -2509,7 +2509,7 @@ int larql_hip_dev_gate_walk(larql_hip_ctx *c, int format, const void *const *gat
     std::vector<GemvJob> jobs;
     jobs.reserve(n_layers * batch);
     for (size_t l = 0; l < n_layers; l++)
-        push_gate_jobs(jobs, kind, gates[l], x + l * x_layer_stride, batch, n, hidden, scores_scratch + l * batch * n);
+        push_gate_jobs(jobs, kind, gates[l], x + l * x_layer_stride, batch, n, hidden, scores_scratch + l * batch * n, n_layers);
     rc = enqueue_jobs(c, jobs);
     if (rc) return rc;
     rc = run_topk(c, scores_scratch, (uint32_t)(n_layers * batch), (uint32_t)n, (uint32_t)top_k, true, idx_out,

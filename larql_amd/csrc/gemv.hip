@@ -2915,6 +2915,135 @@ __device__ __forceinline__ void run_dense(const GemvJob &j, uint32_t p0, uint32_
     }
 }
 
+// Dense rows against 2 .. kDenseBatch activations (f16, f32, and the bf16 rows the matrix-core kernel does not take): the K-slice
+// scheme above with the slices of NB positions in registers, so a row is read and widened once for all of them (NB x 16 FMAs
+// per 16 weights).  Position for position the sums run in the order of run_dense: the same bits as a job per position.
+// Bound by the vector unit: with 8 positions a row's weights cost 8 FMAs each (10240 x 2560: 5.8 us of them at the full rate, 10.5 us
+// of all vector instructions, 22.8 us in all; few positions: by memory, 20 gates of 8000 x 3072 bf16 with 4 positions 218 us, 4.5 TB/s).
+// 8 positions hold 128 registers, so a CU has one workgroup of two wavefronts per SIMD: five wavefronts (320 threads fit rows of
+// 2560) left one SIMD with twice the work of the others, 34.6 -> 29.4 us on the f16 gate above.  The next U passes' rows are
+// requested before this tile's FMAs and stay in flight over its barrier and epilogue (bf16 12417 x 4608, 6 positions: 62.7 -> 52.9 us);
+// the sums alternate between two halves of LDS, one barrier per tile.  Against a job per position, top-64 included: f16 10240 x 2560
+// x 8 34.2 -> 27.9 us, 14336 x 4096 x 16 127.8 -> 63.9; f32 12000 x 4608 x 5 162.6 -> 52.6; bf16 walk above 651 -> 218.
+constexpr int kDenseBatch = 8;
+constexpr int kDenseBatchSums = 32;  // LDS: partial sums per thread and tile (U passes x NB positions), two tiles in turn
+
+template <int ELEM, int VECS>
+__device__ __forceinline__ void dense_widen(float (&f)[16], const u32x4 (&v)[VECS]) {
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        if (ELEM == 2) { f[i] = __builtin_bit_cast(float, (uint32_t)v[(i / 4) % VECS][i % 4]); continue; }
+        const uint32_t d = v[i / 8][(i / 2) % 4];
+        if (ELEM == 0) f[i] = __builtin_bit_cast(float, (i & 1) ? d & 0xFFFF0000u : d << 16);
+        else f[i] = (i & 1) ? (float)as_half2(d).y : (float)as_half2(d).x;
+    }
+}
+
+#define LARQL_LDS_BARRIER() asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory")
+template <int U, int ELEM, int NB>
+__device__ __forceinline__ void run_dense_batch(const GemvJob &j, uint32_t p0, uint32_t p1, float *part, uint32_t &half) {
+    static_assert(U * NB <= kDenseBatchSums, "partial sums per thread");
+    constexpr int VECS = ELEM == 2 ? 4 : 2;
+    const uint32_t t = threadIdx.x, cpr = j.cpr, rpp = j.rpp, batch = j.batch;
+    const bool active = t < cpr * rpp;
+    const uint32_t c = active ? t % cpr : 0, rl = active ? t / cpr : 0;
+    const size_t row_bytes = j.row_bytes;
+    const uint32_t row_end = min((uint32_t)j.rows, p1 * rpp);
+    const uint8_t *wc = j.w + (size_t)c * (VECS * 16);
+    const uint32_t lane16 = t & 15u;
+    // The activations come through LDS, four positions at a time: a lane's 64-byte slice read straight from memory is a line per
+    // lane and load.  (16-byte vector i of slice c sits at 4 c + (i ^ c / 4 % 4): sixteen lanes of a read are on sixteen
+    // different bank groups.)
+    constexpr int PB = NB < 4 ? NB : 4;
+    f32x4 xv[NB][4];
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        const g_f4p xp = (g_f4p)(j.x + (size_t)min((uint32_t)b, batch - 1) * j.x_stride);
+#pragma unroll
+        for (int m = 0; m < 4; m++) xv[b][m] = xp[min(t + m * blockDim.x, 4 * cpr - 1)];
+    }
+    u32x4 v[U][VECS], nv[U][VECS];
+    auto load = [&](u32x4 (&d)[U][VECS], uint32_t pass) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            g_u4p p = (g_u4p)(wc + (size_t)min((pass + u) * rpp + rl, row_end - 1) * row_bytes);
+#pragma unroll
+            for (int k = 0; k < VECS; k++) d[u][k] = p[k];
+        }
+    };
+    load(v, p0);
+    __builtin_amdgcn_sched_barrier(0);
+    X16Slice xs[NB];
+    f32x4 *const stage = (f32x4 *)part;
+#pragma unroll
+    for (int b0 = 0; b0 < NB; b0 += PB) {
+        LARQL_LDS_BARRIER();  // (sums of an earlier job, or slices of the positions before, are read)
+#pragma unroll
+        for (int b = 0; b < PB; b++)
+#pragma unroll
+            for (int m = 0; m < 4; m++) {
+                const uint32_t q = t + m * blockDim.x;
+                if (q < 4 * cpr) stage[4 * cpr * b + (q ^ ((q >> 4) & 3))] = xv[b0 + b][m];
+            }
+        LARQL_LDS_BARRIER();
+#pragma unroll
+        for (int b = 0; b < PB; b++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const f32x4 q = stage[4 * cpr * b + 4 * c + (i ^ ((c >> 2) & 3))];
+                xs[b0 + b].x[4 * i + 0] = q.x; xs[b0 + b].x[4 * i + 1] = q.y; xs[b0 + b].x[4 * i + 2] = q.z; xs[b0 + b].x[4 * i + 3] = q.w;
+            }
+    }
+    LARQL_LDS_BARRIER();
+    auto tile = [&](uint32_t pass) {
+        float *const sums = part + half;
+        const uint32_t row_base = pass * rpp, tile_rows = min(U * rpp, row_end - row_base);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (pass + u >= p1) break;
+            const uint32_t r = u * rpp + rl;
+            float f[16];
+            dense_widen<ELEM, VECS>(f, v[u]);
+#pragma unroll
+            for (int b = 0; b < NB; b++) {
+                float acc0 = 0.f, acc1 = 0.f;
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    acc0 = __builtin_fmaf(f[2 * i], xs[b].x[2 * i], acc0);
+                    acc1 = __builtin_fmaf(f[2 * i + 1], xs[b].x[2 * i + 1], acc1);
+                }
+                if (active) sums[(r * NB + b) * cpr + c] = acc0 + acc1;
+            }
+        }
+        LARQL_LDS_BARRIER();  // (the loads of the next rows stay in flight)
+        for (uint32_t i = t >> 4; i < tile_rows * NB; i += blockDim.x >> 4) {  // as tile_epilogue, a row of sums per weight row and position
+            const float *const row = sums + i * cpr;
+            float a = 0.f;
+            uint32_t p = lane16;
+            for (; p + 48 < cpr; p += 64) {
+                const float q0 = row[p], q1 = row[p + 16], q2 = row[p + 32], q3 = row[p + 48];
+                a = (((a + q0) + q1) + q2) + q3;
+            }
+            for (; p < cpr; p += 16) a += row[p];
+            a = dpp_add<0x118>(a);  // row_shr:8
+            a = dpp_add<0x114>(a);  // row_shr:4
+            a = dpp_add<0x112>(a);  // row_shr:2
+            a = dpp_add<0x111>(a);  // row_shr:1
+            if (lane16 == 15u && i % NB < batch) ((g_f32wp)j.out)[(size_t)(i % NB) * j.out_stride + row_base + i / NB] = a;
+        }
+        half ^= (uint32_t)kDenseBatchSums * blockDim.x;
+    };
+    for (uint32_t pass = p0; pass < p1; pass += U) {
+        load(nv, pass + U);  // (past the end: the last row again)
+        __builtin_amdgcn_sched_barrier(0);
+        tile(pass);
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int k = 0; k < VECS; k++) v[u][k] = nv[u][k];
+    }
+}
+
 // A job descriptor as wave-uniform values.  The table sits in the kernel-argument block or in device memory that
 // nothing writes while the kernel runs (a table built on the device was built by an earlier kernel), so it is read
 // through the constant address space: with a wave-uniform address those are scalar loads — a handful of instructions
@@ -3020,6 +3149,25 @@ LARQL_GEMV_KERNEL(gemv_q6k_q8k_kernel, KIND_Q6K_Q8K, 2, 4)
 LARQL_GEMV_KERNEL(gemv_bf16_kernel, KIND_BF16, 4, 4)
 LARQL_GEMV_KERNEL(gemv_f16_kernel, KIND_F16, 4, 4)
 LARQL_GEMV_KERNEL(gemv_f32_kernel, KIND_F32, 2, 4)
+
+// (8 positions hold 128 registers of activations: two wavefronts per SIMD, one workgroup per CU)
+template <int ELEM>
+__global__ void __launch_bounds__(kGemvMaxThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) gemv_dense_batch_kernel(LARQL_JOB_ARGS) {
+    extern __shared__ float part[];
+    constexpr int U = ELEM == 2 ? 2 : 4;
+    LARQL_JOB_SHARE;
+    uint32_t ji = lo, half = 0;
+    while (p < p_end) {
+        const GemvJob j = uniform_job(jobs + ji);
+        const uint32_t seg_end = min(p_end, j.pass_begin + j.n_pass);
+        const uint32_t a = p - j.pass_begin, b = seg_end - j.pass_begin;
+        if (j.batch <= 2) run_dense_batch<2 * U, ELEM, 2>(j, a, b, part, half);
+        else if (j.batch <= 4) run_dense_batch<2 * U, ELEM, 4>(j, a, b, part, half);
+        else run_dense_batch<U, ELEM, 8>(j, a, b, part, half);
+        p = seg_end;
+        ji++;
+    }
+}
 
 
 // Q4_K on the matrix cores: workgroup b sweeps its share of the launch's tile list (a tile = 16 rows of
@@ -3243,9 +3391,12 @@ static uint32_t mx4_steps_per_wave(uint64_t steps) {
 }
 
 
+static bool bf16_mfma_row(uint64_t k) { return k >= 128 && k % 128 == 0 && k / 128 <= (uint64_t)(kBfMaxWaves * kBfMaxPasses); }
 uint32_t gemv_batch_capacity(int kind, uint64_t k) {
     // bf16: 128-element columns, at most 10 wavefronts x 2 passes, two sets of 4 positions
-    if (kind == KIND_BF16 && k >= 128 && k % 128 == 0 && k / 128 <= (uint64_t)(kBfMaxWaves * kBfMaxPasses)) return 4 * kBfMaxSets;
+    if (kind == KIND_BF16 && bf16_mfma_row(k)) return 4 * kBfMaxSets;
+    // other dense rows: the K-slice kernel with several positions' slices in registers
+    if ((kind == KIND_BF16 || kind == KIND_F16 || kind == KIND_F32) && k >= 16 && k % 16 == 0 && k / 16 <= (uint64_t)kGemvMaxThreads) return kDenseBatch;
     // Q4_K: one wavefront per super-block column, four pairs of positions.  Longer rows run a job per position (3328 wide, 10 layers,
     // 6 positions: 108 us, 17 at peak) and keep its precision: 1.1-1.5e-7 from the 64-bit scores, where this kernel's 22-bit
     // activations give 2.5-3.0e-7 at every width
@@ -3254,10 +3405,28 @@ uint32_t gemv_batch_capacity(int kind, uint64_t k) {
 }
 
 
+// Positions a job should carry for `batch` positions against each of `layers` gates: all the kernel takes, except where the dense K-slice
+// kernel's set-up (activations through LDS, a tile of several passes however short the share) costs more than the repeated reads
+// of the matrix that it saves.  rows x k x positions in bytes decides (us, job per position / shared; top-64 over the scores included):
+//   f32  1500 x 1280: 5 positions (38 MB) 13.7 / 13.1, 3 (23 MB) 11.9 / 12.4;  5000 x 512 x 5 (51 MB) 14.6 / 15.8;  1500 x 5120 x 3 (92 MB) 21.6 / 16.6
+//   bf16 1500 x 2816: 8 (68 MB) 19.2 / 15.2, 3 (25 MB) 13.1 / 13.8
+//   f16  1500 x 5120: 5 (77 MB) 17.9 / 18.0;  5000 x 1280 x 5 (64 MB) 13.9 / 16.9;  5000 x 2560 x 5 (128 MB) 21.9 / 19.5
+//   few positions read a matrix that the 256 MB memory-side cache still holds: 10240 x 2560 f16 2 (105 MB) 18.8 / 19.7 and 4 (210 MB)
+//   22.9 / 23.0, f32 2 (210 MB) 24.5 / 26.6;  16000 x 3584 f32 2 (459 MB) 71.8 / 42.4
+uint32_t gemv_batch_take(int kind, uint64_t rows, uint64_t k, uint64_t batch, uint64_t layers) {
+    const uint32_t cap = gemv_batch_capacity(kind, k);
+    if (cap < 2 || batch < 2 || kind == KIND_Q4K || (kind == KIND_BF16 && bf16_mfma_row(k))) return cap;
+    const bool few = batch < (kind == KIND_F16 ? 5u : 3u);
+    const double mb = (double)rows * (double)k * (kind == KIND_F32 ? 4.0 : 2.0) * (double)batch * (double)layers * 1e-6;
+    return mb >= (few ? 224.0 : kind == KIND_F16 ? 80.0 : 56.0) ? cap : 1;
+}
+
 int gemv_effective_kind(const GemvJob &j) {
     if (j.kind == KIND_Q8_0 && j.k >= 256 && j.k % 256 == 0 && q8_mfma_waves(j.k / 256) != 0 && j.rows < 0x7FFFFFF0ull)
         return KIND_Q8_0_MFMA;
-    if (j.kind == KIND_BF16 && j.batch >= 2) return KIND_BF16_MFMA;
+    if (j.kind == KIND_BF16 && j.batch >= 2) return bf16_mfma_row(j.k) ? KIND_BF16_MFMA : KIND_BF16_BATCH;
+    if (j.kind == KIND_F16 && j.batch >= 2) return KIND_F16_BATCH;
+    if (j.kind == KIND_F32 && j.batch >= 2) return KIND_F32_BATCH;
     if (j.kind == KIND_Q4K && j.batch >= 2) return KIND_Q4K_BATCH;
     if (j.kind == KIND_MXFP4 && j.k >= 128 && j.k % 32 == 0 && mx4_steps_per_wave((j.k + 127) / 128) != 0 &&
         j.rows < 0x7FFFFFF0ull)
@@ -3333,7 +3502,7 @@ bool gemv_job_geometry(GemvJob &j, uint32_t threads) {
         return true;
     }
     if (j.kind == KIND_BF16_MFMA) {
-        if (j.batch < 2 || j.batch > gemv_batch_capacity(KIND_BF16, j.k)) return false;
+        if (j.batch < 2 || j.batch > gemv_batch_capacity(KIND_BF16, j.k) || !bf16_mfma_row(j.k)) return false;
         const uint64_t cols = j.k / 128;
         const uint32_t nw = (uint32_t)std::min<uint64_t>(cols, kBfMaxWaves);
         if (nw * 64 > threads) return false;
@@ -3415,6 +3584,10 @@ bool gemv_job_geometry(GemvJob &j, uint32_t threads) {
         case KIND_Q4_0: j.row_bytes = (j.k / 32) * 18; break;
         case KIND_BF16: case KIND_F16: j.row_bytes = j.k * 2; break;
         case KIND_F32: j.row_bytes = j.k * 4; break;
+        case KIND_BF16_BATCH: case KIND_F16_BATCH: case KIND_F32_BATCH:
+            if (j.batch < 2 || j.batch > (uint32_t)kDenseBatch) return false;
+            j.row_bytes = j.k * (j.kind == KIND_F32_BATCH ? 4 : 2);
+            break;
         default: return false;
     }
     const uint64_t n_pass = (j.rows + j.rpp - 1) / j.rpp;
@@ -3422,6 +3595,8 @@ bool gemv_job_geometry(GemvJob &j, uint32_t threads) {
     j.n_pass = (uint32_t)n_pass;
     return true;
 }
+
+static bool dense_batch_kind(int kind) { return kind == KIND_BF16_BATCH || kind == KIND_F16_BATCH || kind == KIND_F32_BATCH; }
 
 uint32_t gemv_pick_threads(const GemvJob *jobs, size_t n) {
     if (n > 0 && jobs[0].kind == KIND_Q8_0_MFMA) {
@@ -3471,6 +3646,17 @@ uint32_t gemv_pick_threads(const GemvJob *jobs, size_t n) {
         }
         return nw * 64;
     }
+    if (n > 0 && dense_batch_kind(jobs[0].kind)) {
+        // two wavefronts on every SIMD, one workgroup per CU; narrower blocks while that leaves CUs of a whole chip (256) without a pass
+        uint64_t slices = 0, widest = 1;
+        for (size_t i = 0; i < n; i++) {
+            slices += jobs[i].rows * (jobs[i].k / 16);
+            widest = std::max<uint64_t>(widest, jobs[i].k / 16);
+        }
+        uint32_t T = kGemvMaxThreads;
+        while (T > 128 && slices < (uint64_t)T * 256 && widest <= T / 2) T /= 2;
+        return widest <= T ? T : 0;
+    }
     // Prefer the block size that wastes the fewest lanes over the jobs'
     // chunk counts (weighted by bytes); ties go to the smaller block.
     static const uint32_t cand_all[] = {256, 320, 384, 448, 512};
@@ -3515,6 +3701,7 @@ uint32_t gemv_launch_param(const GemvJob *jobs, size_t n) {
 }
 
 size_t gemv_lds_bytes(const GemvJob *jobs, size_t n, uint32_t threads) {
+    if (n > 0 && dense_batch_kind(jobs[0].kind)) return 2 * (size_t)kDenseBatchSums * threads * sizeof(float);
     if (n > 0 && jobs[0].kind == KIND_Q8_0_MFMA) {
         const size_t nw = threads / 64;
         return nw * kQ8Stages * kQ8TileBytes + 2 * (size_t)kQ8BatchTiles * 16 * nw * 4 * sizeof(float);
@@ -3632,6 +3819,7 @@ static hipError_t gemv_short_launch(hipStream_t stream, const GemvLaunch &L, uin
 }
 
 uint32_t gemv_wgs_per_cu(int kind, uint32_t threads, size_t lds, uint32_t dflt) {
+    if (dense_batch_kind(kind)) return 1;
     if (kind != KIND_Q4K_MFMA && kind != KIND_MXFP4_MFMA && kind != KIND_BF16_MFMA && kind != KIND_Q4K_BATCH && kind != KIND_Q8_0_MFMA &&
         kind != KIND_Q4K_Q8K && kind != KIND_Q6K_MFMA)
         return dflt;
@@ -3782,6 +3970,21 @@ hipError_t gemv_launch(hipStream_t stream, int kind, const GemvLaunch &L, uint32
         case KIND_BF16: LARQL_JOBS_LAUNCH(gemv_bf16_kernel); break;
         case KIND_F16: LARQL_JOBS_LAUNCH(gemv_f16_kernel); break;
         case KIND_F32: LARQL_JOBS_LAUNCH(gemv_f32_kernel); break;
+#define LARQL_DENSE_BATCH(KIND, ELEM)                                                                                                           \
+    case KIND: {                                                                                                                                \
+        static std::atomic<bool> attr_set{false};                                                                                               \
+        if (!attr_set) {                                                                                                                        \
+            hipError_t e = hipFuncSetAttribute((const void *)gemv_dense_batch_kernel<ELEM>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); \
+            if (e != hipSuccess) return e;                                                                                                      \
+            attr_set = true;                                                                                                                    \
+        }                                                                                                                                       \
+        LARQL_JOBS_LAUNCH(gemv_dense_batch_kernel<ELEM>);                                                                                       \
+        break;                                                                                                                                  \
+    }
+        LARQL_DENSE_BATCH(KIND_BF16_BATCH, 0)
+        LARQL_DENSE_BATCH(KIND_F16_BATCH, 1)
+        LARQL_DENSE_BATCH(KIND_F32_BATCH, 2)
+#undef LARQL_DENSE_BATCH
         default: return hipErrorInvalidValue;
     }
 #undef LARQL_JOBS_LAUNCH

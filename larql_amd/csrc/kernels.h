@@ -28,7 +28,9 @@ enum GemvKind : int32_t {
     KIND_Q4K_Q8K = 13,   // Q4_K weights against a Q8_K activation (integer dots on the matrix cores); x = the Q8_K device layout
     KIND_Q6K_Q8K = 14,   // Q6_K weights against a Q8_K activation (K-slice kernel, v_dot4)
     KIND_Q6K_MFMA = 15,  // internal: Q6_K rows short enough for the matrix-core kernel
-    KIND_SHORT = 16      // internal: a launch of KIND_Q4K_MFMA or KIND_Q6K_MFMA jobs that leaves every compute unit a few tiles (gemv_short)
+    KIND_SHORT = 16,     // internal: a launch of KIND_Q4K_MFMA or KIND_Q6K_MFMA jobs that leaves every compute unit a few tiles (gemv_short)
+    KIND_BF16_BATCH = 17, KIND_F16_BATCH = 18, KIND_F32_BATCH = 19,  // internal: dense rows against 2..8 activations at once (K-slice kernel)
+    kGemvKinds = 20
 };
 
 constexpr int kGemvMaxThreads = 512;
@@ -53,7 +55,7 @@ struct GemvJob {
     // uses w + e*w_sel_stride, aux + e*aux_sel_stride (one bank of equally shaped matrices).
     const uint32_t *sel;
     uint64_t w_sel_stride, aux_sel_stride;
-    // Optional batch (bf16 / Q4_K gates): `batch` activations x + t*x_stride against the same weights, results to
+    // Optional batch (dense / Q4_K gates): `batch` activations x + t*x_stride against the same weights, results to
     // out + t*out_stride (strides in floats).  0 or 1 = a plain matvec.  See gemv_batch_capacity.  A job folded over experts
     // (combine_w) has its activations 2 and 3 at x + x_off[0], x + x_off[1].
     uint32_t batch, pad2;
@@ -122,6 +124,7 @@ size_t gemv_lds_bytes(const GemvJob *jobs, size_t n, uint32_t threads);
 int gemv_effective_kind(const GemvJob &j);
 bool gemv_short(const GemvJob *jobs, size_t n, uint32_t cu_count, uint32_t *threads, uint32_t *grid, size_t *lds, uint32_t *param);
 uint32_t gemv_batch_capacity(int kind, uint64_t k);  // activations one job may carry (1: no batched kernel for this shape)
+uint32_t gemv_batch_take(int kind, uint64_t rows, uint64_t k, uint64_t batch, uint64_t layers);  // positions per job for `batch` positions against each of `layers` gates
 uint32_t gemv_launch_param(const GemvJob *jobs, size_t n);  // goes into GemvLaunch::pad
 uint32_t gemv_wgs_per_cu(int kind, uint32_t threads, size_t lds, uint32_t dflt);
 hipError_t gemv_launch(hipStream_t stream, int kind, const GemvLaunch &L, uint32_t threads, uint32_t grid, size_t lds);

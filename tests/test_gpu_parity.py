@@ -631,6 +631,25 @@ def test_bf16_gate_scores_over_several_positions(be, fmt, n, hidden, batch):
         assert rel_l2(scores[b], single) < TOL
 
 
+@pytest.mark.parametrize("variant", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("n,hidden,batch", [(1047, 3584, 11), (60001, 16, 45), (20001, 208, 17), (30011, 2064, 2), (4003, 8192, 4),
+                                            (9001, 5120, 3), (7001, 4112, 9), (2049, 4608, 5)])
+def test_dense_gate_scores_share_rows_bit_for_bit(be, fmt, variant, n, hidden, batch):
+    # up to 8 positions share one pass over f16, f32 and the longer bf16 rows; the sums run in the order of a position alone
+    rng = np.random.default_rng(n + hidden + batch)
+    g = (rng.standard_normal((n, hidden)) * 0.05).astype(F)
+    gate, f, gemv = {"bf16": (O.f32_to_bf16(g), fmt.FMT_BF16, O.bf16_gemv), "f16": (g.astype(np.float16).view(np.uint16), fmt.FMT_F16, O.f16_gemv),
+                     "f32": (g, fmt.FMT_F32, O.f32_gemv)}[variant]
+    X = rng.standard_normal((batch, hidden)).astype(F)
+    X[0, ::7] *= 300.0
+    X[-1] *= 1e-12
+    scores = be.gate_scores_batch(f, gate, X, n, hidden)
+    for b in range(batch):
+        single = be.gate_scores_batch(f, gate, X[b:b + 1], n, hidden)[0]
+        assert np.array_equal(scores[b], single), b
+    assert rel_l2(scores[-1], gemv(gate, X[-1], n, hidden)) < TOL
+
+
 @pytest.mark.parametrize("n,hidden,batch", [(1000, 256, 2), (77, 768, 3), (4099, 2560, 4), (640, 1280, 9), (33, 2560, 6),
                                             (500, 2816, 4), (2051, 2560, 8), (130, 512, 7), (300, 2304, 17), (64, 256, 5)])
 def test_q4k_gate_scores_over_several_positions(be, fmt, n, hidden, batch):
