@@ -2916,7 +2916,8 @@ __device__ __forceinline__ void run_dense(const GemvJob &j, uint32_t p0, uint32_
 }
 
 // Dense rows against 2 .. kDenseBatch activations (f16, f32, and the bf16 rows the matrix-core kernel does not take): the K-slice
-// scheme above with the slices of NB positions in registers, so a row is read and widened once for all of them (NB x 16 FMAs
+// scheme above with the slices of NB positions in registers (NB = 2, 3, 4, 6, 8: six instead of eight for five or six
+// positions 28.2 -> 25.0 us on f16 10240 x 2560), so a row is read and widened once for all of them (NB x 16 FMAs
 // per 16 weights).  Position for position the sums run in the order of run_dense: the same bits as a job per position.
 // Bound by the vector unit: with 8 positions a row's weights cost 8 FMAs each (10240 x 2560: 5.8 us of them at the full rate, 10.5 us
 // of all vector instructions, 22.8 us in all; few positions: by memory, 20 gates of 8000 x 3072 bf16 with 4 positions 218 us, 4.5 TB/s).
@@ -2951,10 +2952,11 @@ __device__ __forceinline__ void run_dense_batch(const GemvJob &j, uint32_t p0, u
     const uint32_t row_end = min((uint32_t)j.rows, p1 * rpp);
     const uint8_t *wc = j.w + (size_t)c * (VECS * 16);
     const uint32_t lane16 = t & 15u;
-    // The activations come through LDS, four positions at a time: a lane's 64-byte slice read straight from memory is a line per
+    // The activations come through LDS, up to four positions at a time: a lane's 64-byte slice read straight from memory is a line per
     // lane and load.  (16-byte vector i of slice c sits at 4 c + (i ^ c / 4 % 4): sixteen lanes of a read are on sixteen
     // different bank groups.)
-    constexpr int PB = NB < 4 ? NB : 4;
+    constexpr int PB = NB <= 4 ? NB : NB / 2;
+    static_assert(NB % PB == 0 && PB <= 4, "whole groups of positions, 4 x 16 x cpr floats of LDS");
     f32x4 xv[NB][4];
 #pragma unroll
     for (int b = 0; b < NB; b++) {
@@ -3162,7 +3164,9 @@ __global__ void __launch_bounds__(kGemvMaxThreads) __attribute__((amdgpu_waves_p
         const uint32_t seg_end = min(p_end, j.pass_begin + j.n_pass);
         const uint32_t a = p - j.pass_begin, b = seg_end - j.pass_begin;
         if (j.batch <= 2) run_dense_batch<2 * U, ELEM, 2>(j, a, b, part, half);
+        else if (j.batch <= 3) run_dense_batch<2 * U, ELEM, 3>(j, a, b, part, half);
         else if (j.batch <= 4) run_dense_batch<2 * U, ELEM, 4>(j, a, b, part, half);
+        else if (j.batch <= 6) run_dense_batch<U, ELEM, 6>(j, a, b, part, half);
         else run_dense_batch<U, ELEM, 8>(j, a, b, part, half);
         p = seg_end;
         ji++;
@@ -3410,15 +3414,16 @@ uint32_t gemv_batch_capacity(int kind, uint64_t k) {
 // of the matrix that it saves.  rows x k x positions in bytes decides (us, job per position / shared; top-64 over the scores included):
 //   f32  1500 x 1280: 5 positions (38 MB) 13.7 / 13.1, 3 (23 MB) 11.9 / 12.4;  5000 x 512 x 5 (51 MB) 14.6 / 15.8;  1500 x 5120 x 3 (92 MB) 21.6 / 16.6
 //   bf16 1500 x 2816: 8 (68 MB) 19.2 / 15.2, 3 (25 MB) 13.1 / 13.8
-//   f16  1500 x 5120: 5 (77 MB) 17.9 / 18.0;  5000 x 1280 x 5 (64 MB) 13.9 / 16.9;  5000 x 2560 x 5 (128 MB) 21.9 / 19.5
-//   few positions read a matrix that the 256 MB memory-side cache still holds: 10240 x 2560 f16 2 (105 MB) 18.8 / 19.7 and 4 (210 MB)
-//   22.9 / 23.0, f32 2 (210 MB) 24.5 / 26.6;  16000 x 3584 f32 2 (459 MB) 71.8 / 42.4
+//   f16  1500 x 5120: 5 (77 MB) 17.9 / 18.0;  5000 x 1280 x 5 (64 MB) 13.9 / 16.9;  5000 x 2560 x 4 (102 MB) 22.7 / 15.3;  10000 x 1024 x 4
+//        (82 MB) 20.1 / 14.9;  short rows 16384 x 640 x 4 (84 MB) 14.9 / 16.6
+//   a second reading of a matrix that the 256 MB memory-side cache still holds is cheap: two positions 10240 x 2560 f16 (105 MB)
+//        18.8 / 19.7, f32 (210 MB) 24.5 / 26.6;  16000 x 3584 f32 (459 MB) 71.8 / 42.4
+//   (10240 x 2560 deals its jobs' passes to the workgroups without remainder: f16 x 3 31.2 / 22.1, x 4 22.9 / 23.6, x 5 45.6 / 25.0)
 uint32_t gemv_batch_take(int kind, uint64_t rows, uint64_t k, uint64_t batch, uint64_t layers) {
     const uint32_t cap = gemv_batch_capacity(kind, k);
     if (cap < 2 || batch < 2 || kind == KIND_Q4K || (kind == KIND_BF16 && bf16_mfma_row(k))) return cap;
-    const bool few = batch < (kind == KIND_F16 ? 5u : 3u);
     const double mb = (double)rows * (double)k * (kind == KIND_F32 ? 4.0 : 2.0) * (double)batch * (double)layers * 1e-6;
-    return mb >= (few ? 224.0 : kind == KIND_F16 ? 80.0 : 56.0) ? cap : 1;
+    return mb >= (batch < 3 ? 224.0 : kind != KIND_F16 ? 56.0 : k < 1024 ? 160.0 : 80.0) ? cap : 1;
 }
 
 int gemv_effective_kind(const GemvJob &j) {

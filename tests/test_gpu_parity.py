@@ -633,7 +633,7 @@ def test_bf16_gate_scores_over_several_positions(be, fmt, n, hidden, batch):
 
 @pytest.mark.parametrize("variant", ["bf16", "f16", "f32"])
 @pytest.mark.parametrize("n,hidden,batch", [(1047, 3584, 11), (60001, 16, 45), (20001, 208, 17), (30011, 2064, 2), (4003, 8192, 4),
-                                            (9001, 5120, 3), (7001, 4112, 9), (2049, 4608, 5)])
+                                            (9001, 5120, 3), (7001, 4112, 9), (2049, 4608, 5), (5001, 4096, 6), (16001, 656, 8)])
 def test_dense_gate_scores_share_rows_bit_for_bit(be, fmt, variant, n, hidden, batch):
     # up to 8 positions share one pass over f16, f32 and the longer bf16 rows; the sums run in the order of a position alone
     rng = np.random.default_rng(n + hidden + batch)
