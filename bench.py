@@ -617,7 +617,7 @@ def run_c5(be, fmt, args):
            "mfma_terms_per_weight": 1, "row_exponents": "computed once per matrix (larql_hip_dev_q4k_row_exponents), outside the timed calls; us_with_row_exponents_per_call = larql_hip_dev_q4k_gemm, which recomputes them",
            "verified_rel_l2_vs_oracle": max(rels)},
           {"kernel": "q4k_gemm", "bound": "mfma", "achieved": round(tf, 1), "peak": 2500.0, "unit": "TFLOP/s",
-           "frac": round(tf / 2500.0, 4), "traffic": None, "note": "nominal flops 2*S*N*K; one f16 MFMA term per weight (the whole weight is the f16 operand: ~2.2e-4 from the CPU value)"},
+           "frac": round(tf / 2500.0, 4), "traffic": None, "note": "nominal flops 2*S*N*K; one f16 MFMA term per weight (one f16 rounding of its scale term: ~2.2e-4 from the CPU value) and one of depth 32 per super-block for the offsets"},
           cpu)
 
 

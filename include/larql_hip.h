@@ -384,8 +384,10 @@ int larql_hip_dev_gate_walk(larql_hip_ctx *ctx, int format, const void *const *g
  * W in Q4_K, X held as bf16 (the top 16 bits of each f32).  Same contraction as
  * QuantMatVec::q4k_matmul (backend/quant_matvec.rs:324-333), on f16 MFMA with fp32 accumulate: the
  * activations are exact in f16 after a per-token power-of-two scale, a weight enters as
- * f16(d 2^E sc6) * (q - 8) (E per row), the sub-blocks' offsets through the sums of the activations.
- * ~3e-4 relative L2 from the CPU value (the f16 roundings of the sub-block scales and weights);
+ * f16(d 2^E sc6 (q - 7.5)) (E per row) and the rest of it, the sub-block's offset 7.5 d sc6 - dmin mn6, as an f16
+ * pair against the sub-block's sum of the activations.  The one f16 rounding of d sc6 (q - 7.5) is the error: 2.2e-4
+ * relative L2 from the CPU value on weights centred on zero, less where the weights or activations are one-sided,
+ * more only where the results cancel (1.2e-3 for weights 1 + N(0,1)/20 and sub-blocks whose activations sum to zero);
  * larql_hip_q4k_matmul keeps exact integer sums instead (~3e-7).  hidden % 256 == 0; w and x_bf16
  * 16-byte aligned. */
 int larql_hip_dev_q4k_gemm(larql_hip_ctx *ctx, const uint8_t *w, const uint16_t *x_bf16, size_t rows, size_t hidden,

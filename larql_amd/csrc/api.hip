@@ -1811,19 +1811,19 @@ static int dev_q4k_gemm(larql_hip_ctx *c, const uint8_t *w, const int32_t *row_e
     if (!w || !x_bf16 || !out || ((uintptr_t)w & 15) || ((uintptr_t)x_bf16 & 15)) return LARQL_E_ARG;
     HIPCHECK(c, hipSetDevice(c->device));
     // bf16 activations are exact in one f16 term after the per-token scale
-    const size_t x_len = seq * hidden;
-    int rc = ensure(c, c->misc, x_len * 2 + seq * 4 + rows * 4 + 256);
+    const size_t x_len = seq * hidden, sx_len = seq * (hidden / 32) * 2;
+    int rc = ensure(c, c->misc, x_len * 2 + sx_len * 2 + seq * 4 + rows * 4 + 256);
     if (rc) return rc;
-    uint16_t *xh = (uint16_t *)c->misc.p;
-    float *ts = (float *)(xh + x_len);  // (x_len is a multiple of 256)
-    // the rows' exponents: the weights ride in an f16 operand (2.2e-4 of the CPU value)
+    uint16_t *xh = (uint16_t *)c->misc.p, *sx = xh + x_len;
+    float *ts = (float *)(sx + sx_len);  // (sx_len is a multiple of 16)
+    // the rows' exponents: the weights' scale term rides in an f16 operand
     int *rexp = row_exp ? const_cast<int *>((const int *)row_exp) : (int *)(ts + seq);
-    HIPCHECK(c, q4k_gemm_prep_launch(c->stream, x_bf16, 1, (uint32_t)hidden, (uint32_t)seq, xh, nullptr, nullptr, ts, nullptr, row_exp ? nullptr : w,
+    HIPCHECK(c, q4k_gemm_prep_launch(c->stream, x_bf16, 1, (uint32_t)hidden, (uint32_t)seq, xh, nullptr, sx, ts, nullptr, row_exp ? nullptr : w,
                                      (uint32_t)rows, row_exp ? nullptr : rexp));
     const uint32_t splits = q4k_gemm_splits((uint32_t)rows, (uint32_t)hidden, (uint32_t)seq, (uint32_t)c->cu_count);
     float *partial = nullptr;
     if (splits > 1) { rc = ensure(c, c->scores, (size_t)splits * seq * rows * 4 + 64); if (rc) return rc; partial = (float *)c->scores.p; }
-    HIPCHECK(c, q4k_gemm_f16_launch(c->stream, w, xh, nullptr, rexp, ts, out, (uint32_t)rows, (uint32_t)hidden, (uint32_t)seq, 1, 0, splits, partial,
+    HIPCHECK(c, q4k_gemm_f16_launch(c->stream, w, xh, sx, rexp, ts, out, (uint32_t)rows, (uint32_t)hidden, (uint32_t)seq, 1, 0, splits, partial,
                                     (uint32_t)c->cu_count));
     return LARQL_OK;
 }

@@ -3,8 +3,8 @@
 //   out[s, r] = sum_k W[r, k] * X[s, k]      W: [rows, hidden] Q4_K,  X: [seq, hidden] bf16 or f32
 //
 // the contraction q4k_matmul_into computes (larql-compute/src/cpu/ops/q4_common/
-// matmul.rs:20-139; `out` is [seq, rows] row-major), on f16 MFMA over the integer
-// weights (see the formulation below).
+// matmul.rs:20-139; `out` is [seq, rows] row-major), on f16 MFMA over operands made
+// from the stored nibbles (see the formulation below).
 #include <hip/hip_runtime.h>
 
 #include <atomic>
@@ -24,7 +24,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 // ---------------------------------------------------------------------------
-// The formulation: keep the weight an integer as long as possible.
+// The formulation: a sub-block's scale term and its offset are separate operands.
 //
 //   out[s, r] = sum over super-blocks of  d[r] * (sum_k (sc6*q)[r,k] * x[s,k])  -  dmin[r] * (sum_sub mn6[r,sub] * Sx[s,sub])
 //
@@ -37,11 +37,15 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 //     B slots = Sx_h/32; Sx, the sum of the represented activations over each 32-element sub-block, comes with the
 //     preparation as an f16 pair, divided by 32 to stay inside f16), and folds both into the f32 result with the row's
 //     d and dmin.
-//   * q4k_gemm_pair_kernel (device tier): the operand is the whole weight, f16(d sc6 (q - 8) + o) with
-//     o = f16(8 d sc6 - dmin mn6), both times the row's 2^E; sc6 (q - 8) is exact and o is of a weight's size or less, so
-//     that a weight is rounded once: 2.2e-4 relative to the f64 product (2.9e-4 with the scale d sc6 rounded by itself and
-//     the offsets in an MFMA of their own, the form before).  No offsets, no folds; 2^-E and the token's scale are applied
-//     once at the end.
+//   * q4k_gemm_pair_kernel (device tier): the operand is f16(d sc6 (q - 7.5)), sc6 (q - 7.5) exact in f16 and the product with d
+//     rounded once; the offsets 7.5 d sc6 - dmin mn6 are an f16 pair of their own (22 bits) against the Sx pair, one more MFMA per block
+//     and super-block.  All times the row's 2^E; 2^-E and the token's scale are applied once at the end, no folds.
+//     So the only error above f32 is one f16 rounding per nibble value, at the size of d sc6 |q - 7.5|: a sub-block's mean and the
+//     activations' do not enter.  Relative to the f64 product, 203 x 2560, 33 tokens (in brackets: the whole weight in one f16 |
+//     f16(s (q - 8)) with s = f16(d sc6) and one f16 per offset):
+//       weights N(0,1), activations N(0,1) 2.2e-4 (2.2e-4 | 3.0e-4), with mean 5 2.2e-4 (5.6e-4 | 6.4e-4);  |N(0,1)|, N(0,1) 1.5e-4
+//       (3.0e-4 | 2.1e-4);  1 + N/20 against sub-blocks that sum to zero 1.2e-3 (3.3e-3 | 1.4e-3);  offsets 60 times the scales, against the
+//       same 2.0e-4 (2.4e-3 | 2.5e-4)
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float half_to_float(uint32_t lo16) { return (float)__builtin_bit_cast(_Float16, (uint16_t)lo16); }
 
@@ -61,7 +65,7 @@ __global__ void __launch_bounds__(1024) q4k_gemm_prep_kernel(const void *__restr
     const uint32_t t = threadIdx.x, nvec = hidden >> 3;  // hidden % 256 == 0
     if (blockIdx.x >= seq) {
         // the blocks behind the tokens: 16 lanes per weight row, E with max(|d|, |dmin|/16) * 2^E in [0.5, 1) over the row,
-        // so that d 2^E sc6 <= 63 and 32 (8 d sc6 + dmin mn6) 2^E <= 48384 stay well inside f16
+        // so that 1024 d 2^E < 1024 and |32 (7.5 d sc6 - dmin mn6) 2^E| <= 32 (7.5 + 16) 63 = 47376 stay well inside f16
         const uint32_t row = (blockIdx.x - seq) * (blockDim.x >> 4) + (t >> 4), nsb = hidden >> 8;
         float m = 0.f;
         if (row < rows) {
@@ -159,7 +163,6 @@ __global__ void __launch_bounds__(1024) q4k_gemm_prep_kernel(const void *__restr
         const size_t at = (size_t)tok * nvec + v;
         oh[at] = (u32x4){hw[0], hw[1], hw[2], hw[3]};
         if (ol) ol[at] = (u32x4){lw[0], lw[1], lw[2], lw[3]};
-        if (!sx) return;  // (the device tier's GEMM has no use for the sums)
         sm += dpp_move<0xB1>(sm);  // quad_perm [1,0,3,2]
         sm += dpp_move<0x4E>(sm);  // quad_perm [2,3,0,1]
         sm *= 0.03125f;  // stored as Sx/32 so that 32 x 2^14 stays inside f16; the min operand carries the 32
@@ -637,18 +640,22 @@ __global__ void __launch_bounds__(GTHREADS, 1) q4k_gemm_exact_kernel(const uint8
 // of token r at position c ^ ((r >> 1) & 7), chosen on the global side of the copy: no bank conflicts), the weights a super-block at a
 // time (144 bytes per row: a row's two or three cache lines are asked for once) into two stages.  kh = 0 asks for
 // the activations, kh = 1 for the weights, between its MFMAs: a copy instruction whose lanes lie in many cache lines holds up
-// the wavefront that issues it (nine in a row: 0.4 us).  Per super-block one thread per row turns half of the header into table entries
-// (sc6/16, o) for the lanes that convert.
+// the wavefront that issues it (nine in a row: 0.4 us).  Per super-block two threads per row turn the header into table entries:
+// the scales for the lanes that convert, and the offsets' operand.
+// The offsets are one MFMA of depth 32 per block and super-block (an eighth of the MFMAs more, and half a kilobyte of Sx per 16 tokens),
+// at the super-block's first half step; with the whole weight in one f16 instead, us per call: 15360 x 3840 with 2048 tokens 215,
+// 512 63.7; 3840 x 15360 with 77 31.7 (233, 70.2 and 34.2 so).
 // 16 x 16 x 32 MFMAs: at these rates the GPU is limited by its power, and a loop of them ran at a 10 % higher clock than the same work in
 // 32 x 32 x 16 (which read and write twice the accumulators per operation); f16 operands of normal values: 1.28 PFLOP/s
 // for a loop of nothing but copies, LDS reads and MFMAs.
-// Measured, calls with the exponents given: 15360 x 3840 with 2048 tokens 283 -> 217 us, 512 73.5 -> 69.7; 3840 x 15360 with
-// 77 34.1 -> 32.5, 16 27.2 -> 21.9; 12607 x 1280 with 1817 119 -> 91 (rows no multiple of four: the results in four-byte
-// stores before).
+// Measured, us per call with the exponents given, against the form with two barriers per half step, 32 x 32 x 16 MFMAs and one f16 per offset:
+// 15360 x 3840 with 2048 tokens 281 -> 233, 512 75.8 -> 70.2; 3840 x 15360 with 77 35.3 -> 34.2, 16 25.1 -> 22.7;
+// 12607 x 1280 with 1817 120 -> 94 (rows no multiple of four: the results in four-byte stores before).
 // ---------------------------------------------------------------------------
 constexpr int QTHREADS = 512;
-constexpr uint32_t Q_B_BYTES = 65536, Q_R_STAGE = GM * 144, Q_T_STAGE = GM * 32;  // activation ring; weights and tables of a super-block
-constexpr uint32_t Q_R_OFF = Q_B_BYTES, Q_T_OFF = Q_R_OFF + 2 * Q_R_STAGE, Q_D_OFF = Q_T_OFF + 2 * Q_T_STAGE, Q_E_OFF = Q_D_OFF + 2 * GM * 4, Q_S_OFF = Q_E_OFF + GM * 4, Q_LDS_BYTES = Q_S_OFF + 2 * GN * 4;
+constexpr uint32_t Q_B_BYTES = 65536, Q_R_STAGE = GM * 144;  // activation ring; weights of a super-block, two of them
+constexpr uint32_t Q_R_OFF = Q_B_BYTES, Q_O_OFF = Q_R_OFF + 2 * Q_R_STAGE, Q_M_OFF = Q_O_OFF + GM * 32;  // offsets of a super-block, the activations' sums
+constexpr uint32_t Q_D_OFF = Q_M_OFF + 2 * GN * 32, Q_E_OFF = Q_D_OFF + 2 * GM * 4, Q_S_OFF = Q_E_OFF + GM * 4, Q_LDS_BYTES = Q_S_OFF + 2 * GN * 4;
 static_assert(Q_LDS_BYTES <= 160 * 1024, "one workgroup per CU");
 // one global -> LDS copy of 16 bytes per lane: uniform base + per-lane 32-bit offset on the global side (no 64-bit
 // address registers), uniform LDS address (the lanes' 16-byte slots follow one another from there)
@@ -677,7 +684,7 @@ __device__ __forceinline__ void store4(float *o, f32x4 v, uint32_t left) {
 }
 
 template <int TB, bool KS>
-__global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *w, const uint16_t *xh, const int *__restrict__ rexp,
+__global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *w, const uint16_t *xh, const uint16_t *sx, const int *__restrict__ rexp,
                                                                   const float *__restrict__ tok_scale, float *__restrict__ out,
                                                                   uint32_t rows, uint32_t hidden, uint32_t seq, uint32_t row_tiles, uint32_t tok_tiles,
                                                                   uint32_t sb_per_split, float *__restrict__ partial) {
@@ -711,7 +718,8 @@ __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *
     // (64p + l) / 9, so that the rows lie in LDS one after the other.  kh = 0: a step's activations, CP pieces of 8 tokens
     const uint8_t *wt = w + (size_t)row0 * row_bytes;                                          // uniform
     const uint8_t *xt = (const uint8_t *)xh + (size_t)tok0 * hidden * 2;                       // uniform
-    uint32_t c_off[9];
+    const uint8_t *st = (const uint8_t *)sx + (size_t)tok0 * 32;                               // uniform
+    uint32_t c_off[9], m_off[2];
     if (kh) {
 #pragma unroll
         for (int p = 0; p < 9; p++) {
@@ -725,6 +733,10 @@ __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *
             c_off[q] = (min(tok0 + r, seq - 1) - tok0) * hidden * 2 + (((lane & 7u) ^ ((r >> 1) & 7u)) * 16);
         }
     }
+    // and kh = 0 a super-block's sums Sx/32 ([token][8 pairs]), MP pieces of 32 tokens
+    constexpr int MP = KS ? 1 : 2;
+#pragma unroll
+    for (int q = 0; q < 2; q++) m_off[q] = (min(tok0 + q * 128 + wq * 32 + (lane >> 1), seq - 1) - tok0) * 32 + (lane & 1u) * 16;
     // (requests past the end are clamped: same number of copies in flight, results unused)
     auto issue_raw = [&](uint32_t sb, int p) {  // one of the nine pieces of a super-block
         copy16_to_lds(wt + (size_t)min(sb, sb_end - 1) * 144, c_off[p], lds0 + Q_R_OFF + ((sb - sb_begin) & 1u) * Q_R_STAGE + wq * 9216 + p * 1024);
@@ -732,39 +744,60 @@ __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *
     auto issue_b = [&](uint32_t s, uint32_t slot, int q) {  // one of the CP pieces of a step
         copy16_to_lds(xt + ((size_t)sb_begin * 4 + min(s, nsteps - 1)) * 128, c_off[q], lds0 + slot * B_STAGE + (wq + 4 * q) * 1024);
     };
-
-    int row_e = 0;  // d * 2^row_e <= 1 over the whole row, of the row whose table entries this thread writes
-    // table entries of the sub-blocks 2g and 2g + 1 of this thread's row, g = 2 khc + u, and (u = 0) its d
-    auto stage = [&](const int khc, const uint32_t par, const int u) {
-        const u32x4 hdr = *reinterpret_cast<const u32x4 *>(glds + Q_R_OFF + par * Q_R_STAGE + wq * 9216 + lane * 144);
-        const float ds = ldexpf(half_to_float(hdr.x & 0xFFFFu), row_e), dm = ldexpf(half_to_float(hdr.x >> 16), row_e);
-        // the 6-bit scales and mins of the four sub-blocks 4 khc .. 4 khc + 3, a byte each
-        const uint32_t sc4 = khc ? (hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u) : hdr.y & 0x3F3F3F3Fu;
-        const uint32_t mn4 = khc ? ((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u) : hdr.z & 0x3F3F3F3Fu;
-        uint32_t e[2] = {0u, 0u};
-#pragma unroll
-        for (int k = 0; k < 2; k++) {
-            const float sc = (float)((sc4 >> (8 * (2 * u + k))) & 0xFFu), mn = (float)((mn4 >> (8 * (2 * u + k))) & 0xFFu);
-            const float o = 8.f * ds * sc - dm * mn;
-            e[k] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(0.0625f * sc)) | (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)o) << 16;
-        }
-        *reinterpret_cast<u32x2 *>(glds + Q_T_OFF + par * Q_T_STAGE + (2 * khc + u) * 2048 + (wm + lane) * 8) = (u32x2){e[0], e[1]};
-        if (khc == 0 && u == 0) *reinterpret_cast<uint32_t *>(glds + Q_D_OFF + par * GM * 4 + (wm + lane) * 4) = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)ds);
+    auto issue_sx = [&](uint32_t sb, int q) {
+        copy16_to_lds(st + (size_t)min(sb, sb_end - 1) * seq * 32, m_off[q], lds0 + Q_M_OFF + wq * 1024 + q * 4096);
     };
-    uint32_t magic;  // in a register, so that mask-and-or is one instruction
-    asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(magic));
-    // 4 raw bytes, nibble h -> two dwords of f16(d sc6 (q - 8) + o) as the pairs (k0, k2) and (k1, k3).  The nibbles go to bits
-    // 4 .. 7 of two f16 (1024 + 16q); times sc6/16 less 72 sc6 is sc6 (q - 8), exact (-1032 sc6, which bits 0 .. 3 would need, is
-    // no f16); the second multiply-add rounds the weight
-    auto convert4 = [&](uint32_t raw, const int h, f16x2 sc, f16x2 c, f16x2 d, f16x2 o, uint32_t &o0, uint32_t &o1) {
-        const f16x2 m02 = __builtin_bit_cast(f16x2, ((h ? raw : raw << 4) & 0x00F000F0u) | magic);
-        const f16x2 m13 = __builtin_bit_cast(f16x2, ((h ? raw >> 8 : raw >> 4) & 0x00F000F0u) | magic);
-        o0 = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_elementwise_fma(m02, sc, c), d, o));
-        o1 = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_elementwise_fma(m13, sc, c), d, o));
+
+    // A super-block's header -> table entries, 32 rows of the pair's per wavefront: lane l takes the sub-blocks 4 (l / 32) .. + 3 of a row.
+    //   part 0: the offsets' operand v = 32 (7.5 d sc6 - dmin mn6) 2^E as an f16 pair, [row][4 x high of the sub-blocks 0 .. 3 | 4 .. 7 | 4 x low ..]
+    //   part 1: the scales 1024 sc6 as f16 in the header's own 16 bytes (no other wavefront reads them as a header), and 1024 d 2^E
+    const uint32_t srow = wm + kh * 32 + (lane & 31u), sub4 = lane >> 5;
+    int row_e = 0;  // E: max(|d|, |dmin|/16) 2^E < 1 over the whole row srow
+    auto header_of = [&](const uint32_t par) { return *reinterpret_cast<const u32x4 *>(glds + Q_R_OFF + par * Q_R_STAGE + srow * 144); };
+    auto stage = [&](const uint32_t par, const int part, u32x4 hdr) {
+        uint8_t *const hp = glds + Q_R_OFF + par * Q_R_STAGE + srow * 144;
+        asm volatile("" : "+v"(hdr) :: "memory");  // (both lanes of a row have read it before either writes, and in one piece)
+        const float d = half_to_float(hdr.x & 0xFFFFu), dmin = half_to_float(hdr.x >> 16);
+        // the 6-bit scales and mins of the four sub-blocks, a byte each
+        const uint32_t m = 0u - sub4;  // (selected by masks: the compiler makes branches of ?:)
+        const uint32_t sc4 = (((hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u)) & m) | (hdr.y & 0x3F3F3F3Fu & ~m);
+        const uint32_t mn4 = ((((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u)) & m) | (hdr.z & 0x3F3F3F3Fu & ~m);
+        uint32_t hi[2] = {0u, 0u}, lo[2] = {0u, 0u};
+        const float ds = 7.5f * ldexpf(d, row_e + 5), dm = ldexpf(dmin, row_e + 5);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const float sc = (float)((sc4 >> (8 * k)) & 0xFFu), mn = (float)((mn4 >> (8 * k)) & 0xFFu);
+            const float v = part ? sc * 1024.f : ds * sc - dm * mn;
+            const _Float16 h = (_Float16)v;
+            hi[k >> 1] |= (uint32_t)__builtin_bit_cast(uint16_t, h) << (16 * (k & 1));
+            if (!part) lo[k >> 1] |= (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(v - (float)h)) << (16 * (k & 1));
+        }
+        if (part) {
+            *reinterpret_cast<u32x2 *>(hp + sub4 * 8) = (u32x2){hi[0], hi[1]};
+            *reinterpret_cast<uint32_t *>(glds + Q_D_OFF + par * GM * 4 + srow * 4) = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)ldexpf(d, row_e + 10));
+        } else {
+            *reinterpret_cast<u32x2 *>(glds + Q_O_OFF + srow * 32 + sub4 * 8) = (u32x2){hi[0], hi[1]};
+            *reinterpret_cast<u32x2 *>(glds + Q_O_OFF + srow * 32 + 16 + sub4 * 8) = (u32x2){lo[0], lo[1]};
+        }
+    };
+    // 4 raw bytes, nibble h -> two dwords of f16(d sc6 (q - 7.5)) as the pairs (k0, k2) and (k1, k3).  The nibbles go to bits 4 .. 7 of
+    // two f16, subnormals of the value q 2^-20 (f16 subnormals cost nothing here); times 1024 sc6 less 7.5 sc6 / 1024 is sc6 (q - 7.5) / 1024,
+    // exact; the product with 1024 d rounds once
+    auto convert4 = [&](uint32_t raw, const int h, f16x2 sc, f16x2 c, f16x2 d, uint32_t &o0, uint32_t &o1) {
+        const f16x2 m02 = __builtin_bit_cast(f16x2, (h ? raw : raw << 4) & 0x00F000F0u);
+        const f16x2 m13 = __builtin_bit_cast(f16x2, (h ? raw >> 8 : raw >> 4) & 0x00F000F0u);
+        o0 = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(m02, sc, c) * d);
+        o1 = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(m13, sc, c) * d);
     };
     const uint32_t r16 = lane & 15u, kq = lane >> 4;
     const uint32_t raw_lane = lds0 + Q_R_OFF + wq * 9216 + r16 * 144 + 16 + kq * 8;
-    const uint32_t tab_lane = lds0 + Q_T_OFF + (wm + r16) * 8 + (KS ? kh * 4 : 0u), d_lane = lds0 + Q_D_OFF + (wm + r16) * 4;
+    const uint32_t tab_lane = lds0 + Q_R_OFF + (wm + r16) * 144, d_lane = lds0 + Q_D_OFF + (wm + r16) * 4;
+    // offsets: a lane's eight products of the 16 x 16 x 32 MFMA are v_high (kq = 0, 1) or v_low (2, 3) of four sub-blocks, each twice,
+    // against those sub-blocks' Sx/32 pairs.  KS: each of the pair adds them for the half of the rows that it stores
+    constexpr int OI = KS ? 2 : 4;  // row blocks that this wavefront stores
+    const uint32_t i0 = KS ? 2 * kh : 0;
+    const uint32_t o_lane = lds0 + Q_O_OFF + (wm + i0 * 16 + r16) * 32 + kq * 8;
+    const uint32_t m_lane = lds0 + Q_M_OFF + (KS ? 0u : kh * 4096) + r16 * 32 + (kq & 1u) * 16;
     uint32_t b_lane[2];  // for the two halves of a step
 #pragma unroll
     for (int h = 0; h < 2; h++)
@@ -777,9 +810,8 @@ __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *
         for (int j = 0; j < TB; j++) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
     u32x4 an[4] = {};      // the weight operand being prepared / multiplied, by row blocks
     u32x4 breg[8] = {};    // its activation operands
-    typedef std::conditional_t<KS, uint32_t, u32x2> entry;
     u32x2 rq[4];
-    entry sp[4];           // raw bytes and table entries of the step (KS: its half)
+    uint32_t sp[4];        // raw bytes and table entries (two scales) of the step
     uint32_t dd[4];        // d of the super-block
 
     // raw bytes and table entries of a step, read while the half step before it multiplies.  (Written as instructions, as all
@@ -787,11 +819,10 @@ __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *
     auto fetch = [&](auto GG, const uint32_t sb) {
         constexpr int g = decltype(GG)::value;
         uint32_t (&dr)[4] = dd;
-        entry (&spr)[4] = sp;
+        uint32_t (&spr)[4] = sp;
         const uint32_t par = (sb - sb_begin) & 1u;
-        const uint32_t ra = raw_lane + par * Q_R_STAGE, ta = tab_lane + par * Q_T_STAGE;
-#define LARQL_RS(i) if constexpr (KS) asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(spr[i]) : "v"(ta), "n"(g * 2048 + (i) * 128)); \
-                    else asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(spr[i]) : "v"(ta), "n"(g * 2048 + (i) * 128)); \
+        const uint32_t ra = raw_lane + par * Q_R_STAGE, ta = tab_lane + par * Q_R_STAGE;
+#define LARQL_RS(i) asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(spr[i]) : "v"(ta), "n"(g * 4 + (i) * 2304)); \
                     asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(rq[i]) : "v"(ra), "n"(g * 32 + (i) * 2304));
         LARQL_RS(0) LARQL_RS(1) LARQL_RS(2) LARQL_RS(3)
 #undef LARQL_RS
@@ -807,10 +838,6 @@ __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *
         asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(rq[0]), "+v"(rq[1]), "+v"(rq[2]), "+v"(rq[3]), "+v"(sp[0]), "+v"(sp[1]), "+v"(sp[2]), "+v"(sp[3]),
                      "+v"(dd[0]), "+v"(dd[1]), "+v"(dd[2]), "+v"(dd[3]));
     };
-    auto entry_of = [&](const int i, const int h) -> uint32_t {
-        if constexpr (KS) return sp[i];
-        else return sp[i][h];
-    };
     // prepare half step (g, h) of super-block sb; at g = 2 also the tables of sb + 1, whose weights landed at g = 1
     auto prepare = [&](auto KH, auto GG, auto HH, const uint32_t sb) {
         constexpr int khc = decltype(KH)::value, g = decltype(GG)::value, h = decltype(HH)::value;
@@ -819,19 +846,22 @@ __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *
 #define LARQL_RB(j) if constexpr ((j) < TB) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(breg[j]) : "v"(b_lane[h]), "n"(slot * (int)B_STAGE + (j) * 2048));
         LARQL_RB(0) LARQL_RB(1) LARQL_RB(2) LARQL_RB(3) LARQL_RB(4) LARQL_RB(5) LARQL_RB(6) LARQL_RB(7)
 #undef LARQL_RB
+        u32x4 hdr = {};
+        if (g == 2) hdr = header_of(par ^ 1u);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const f16x2 e = __builtin_bit_cast(f16x2, entry_of(i, h)), dp = __builtin_bit_cast(f16x2, dd[i]);
-            const f16x2 sc = {e[0], e[0]}, o = {e[1], e[1]}, d = {dp[0], dp[0]}, c = sc * (_Float16)-1152.f;
+            const f16x2 e = __builtin_bit_cast(f16x2, sp[i]), dp = __builtin_bit_cast(f16x2, dd[i]);
+            const f16x2 sc = {e[h], e[h]}, d = {dp[0], dp[0]}, c = sc * (_Float16)(-7.5f * 0x1p-20f);
             uint32_t o0, o1, o2, o3;
-            convert4(rq[i].x, h, sc, c, d, o, o0, o1);
-            convert4(rq[i].y, h, sc, c, d, o, o2, o3);
+            convert4(rq[i].x, h, sc, c, d, o0, o1);
+            convert4(rq[i].y, h, sc, c, d, o2, o3);
             an[i] = (u32x4){o0, o1, o2, o3};
         }
-        if (g == 2 && (KS || h == 0)) stage(khc, par ^ 1u, 0);
-        if (g == 2 && (KS || h == 1)) stage(khc, par ^ 1u, 1);
-        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(breg[0]), "+v"(breg[1]), "+v"(breg[2]), "+v"(breg[3]), "+v"(breg[4]), "+v"(breg[5]), "+v"(breg[6]), "+v"(breg[7]));
+        if (g == 2 && (KS || h == 0)) stage(par ^ 1u, 0, hdr);
+        if (g == 2 && (KS || h == 1)) stage(par ^ 1u, 1, hdr);
+        // ("memory": the table entries are written before it as well)
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(breg[0]), "+v"(breg[1]), "+v"(breg[2]), "+v"(breg[3]), "+v"(breg[4]), "+v"(breg[5]), "+v"(breg[6]), "+v"(breg[7]) :: "memory");
         if (khc == 1 && g == 1 && (KS || h == 1)) GEMM_WAIT_VMCNT(0);
         __builtin_amdgcn_s_setprio(3);  // (the multiply phase comes next)
     };
@@ -840,11 +870,26 @@ __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *
     // two steps after the next; of the weights everything, until g = 1 prepares
     auto multiply = [&](auto KH, auto GG, auto HH, auto GN, const uint32_t s, const uint32_t sb, const uint32_t sbn) {
         constexpr int khc = decltype(KH)::value, g = decltype(GG)::value, h = decltype(HH)::value;
+        constexpr bool offs = g == 0 && (KS || h == 0);  // the super-block's offsets come with its first half step
         if (KS || h == 1) fetch(GN, sbn);
+        u32x2 ov[4] = {};
+        u32x4 oa[OI];
+        if constexpr (offs) {
+            asm volatile("ds_read_b64 %0, %1" : "=v"(ov[0]) : "v"(o_lane));
+            asm volatile("ds_read_b64 %0, %1 offset:512" : "=v"(ov[1]) : "v"(o_lane));
+            if constexpr (!KS) {
+                asm volatile("ds_read_b64 %0, %1 offset:1024" : "=v"(ov[2]) : "v"(o_lane));
+                asm volatile("ds_read_b64 %0, %1 offset:1536" : "=v"(ov[3]) : "v"(o_lane));
+            }
+        }
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("s_nop 1");  // (the operand may have been written by the instruction before)
         auto request = [&](const int k) {
             if (khc == 0) {
+                // (the sums of the next super-block: their readers' last half step, the offsets' below, is a barrier and more ago)
+                if (g == 2 && (KS || h == 0) && k == 0)
+#pragma unroll
+                    for (int q = 0; q < MP; q++) issue_sx(sb + 1, q);
                 if (KS && k % 8 == 3) issue_b(s + 3, (g + 3) & 3, k / 8);
                 if (!KS && h == 0 && k % 4 == 3) issue_b(s + 1, (g + 1) & 1, k / 4);
             } else if ((KS || h == 1) && (g == 2 || g == 3)) {
@@ -855,16 +900,40 @@ __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *
             }
         };
 #pragma unroll
-        for (int j = 0; j < TB; j++)
+        for (int j = 0; j < TB; j++) {
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc[i][j]) : "v"(an[i]), "v"(breg[j]));
                 request(j * 4 + i);
             }
+            if constexpr (offs) {
+                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(breg[j]) : "v"(m_lane), "n"(j * 512));
+                if (j == 1) {
+                    asm volatile("s_waitcnt lgkmcnt(2)" : "+v"(ov[0]), "+v"(ov[1]), "+v"(ov[2]), "+v"(ov[3]));
+#pragma unroll
+                    for (int i = 0; i < OI; i++)
+                        oa[i] = (u32x4){__builtin_amdgcn_perm(0u, ov[i].x, 0x01000100u), __builtin_amdgcn_perm(0u, ov[i].x, 0x03020302u),
+                                        __builtin_amdgcn_perm(0u, ov[i].y, 0x01000100u), __builtin_amdgcn_perm(0u, ov[i].y, 0x03020302u)};
+                }
+            }
+        }
+        if constexpr (offs) {
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("s_nop 1");
+#pragma unroll
+            for (int j = 0; j < TB; j++) {
+                asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(breg[j]) : "n"(TB - 1 - j));
+#pragma unroll
+                for (int i = 0; i < OI; i++)
+                    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc[(KS ? 2 * khc : 0) + i][j]) : "v"(oa[i]), "v"(breg[j]));
+            }
+        }
         __builtin_amdgcn_s_setprio(0);
         arrived();
         if (khc == 0) {
-            if (KS) GEMM_WAIT_VMCNT(2 * CP);
+            // (g = 2: the sums asked for first in this half step may fly as well; they are here a barrier before their first reader)
+            if (KS && g == 2) GEMM_WAIT_VMCNT(2 * CP + MP);
+            else if (KS) GEMM_WAIT_VMCNT(2 * CP);
             else if (h == 1) GEMM_WAIT_VMCNT(0);
         }
     };
@@ -887,15 +956,20 @@ __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *
     } else {
         copy4_to_lds(tok_scale + tok0, (min(tok0 + wm + lane, seq - 1) - tok0) * 4, lds0 + Q_S_OFF + wm * 4);
 #pragma unroll
+        for (int q = 0; q < MP; q++) issue_sx(sb_begin, q);
+#pragma unroll
         for (int st = 0; st < (KS ? 3 : 1); st++)
 #pragma unroll
             for (int q = 0; q < CP; q++) issue_b(st, st, q);
         GEMM_WAIT_VMCNT(KS ? 2 * CP : 0);
     }
     half_end();
-    row_e = reinterpret_cast<const int *>(glds + Q_E_OFF)[wm + lane];
-    if (kh) { stage(1, 0, 0); stage(1, 0, 1); }
-    else { stage(0, 0, 0); stage(0, 0, 1); }
+    row_e = reinterpret_cast<const int *>(glds + Q_E_OFF)[srow];
+    {
+        const u32x4 hdr = header_of(0);
+        stage(0, 0, hdr);
+        stage(0, 1, hdr);
+    }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     half_end();
     //   kh = 0:  P(0) | M(0) | P(1) M(1) | P(2) M(2) | ...
@@ -945,8 +1019,7 @@ __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *
 #pragma unroll
         for (int j = 0; j < TB; j++) asm volatile("" : "+v"(acc[i][j]));
     // ---- results: lane (token r16, kq) holds rows 4 kq .. 4 kq + 3 of every block of 16 x 16 ----
-    constexpr int I = KS ? 2 : 4;  // row blocks that this wavefront stores
-    const uint32_t i0 = KS ? 2 * kh : 0;
+    constexpr int I = OI;
     f32x4 back[I];
 #pragma unroll
     for (int i = 0; i < I; i++) {
@@ -1021,7 +1094,7 @@ uint32_t q4k_gemm_splits(uint32_t rows, uint32_t hidden, uint32_t seq, uint32_t 
     return (uint32_t)splits;
 }
 
-// `rexp` (from q4k_gemm_prep_launch): the f16 weight operand is the whole weight (`sx`, `with_mins` and `accumulate` are not used);
+// `rexp` (from q4k_gemm_prep_launch): the rows' scales ride in the f16 weight operand (`with_mins` and `accumulate` are not used);
 // without it the weight operand is the exact integer and the rows' f32 scales are applied per super-block
 hipError_t q4k_gemm_f16_launch(hipStream_t s, const uint8_t *w, const uint16_t *xh, const uint16_t *sx, const int *rexp, const float *tok_scale,
                                float *out, uint32_t rows, uint32_t hidden, uint32_t seq, int with_mins, int accumulate, uint32_t splits,
@@ -1041,9 +1114,9 @@ hipError_t q4k_gemm_f16_launch(hipStream_t s, const uint8_t *w, const uint16_t *
     }
     const dim3 grid((rows + GM - 1) / GM, (seq + GN - 1) / GN, z);
     float *slab = split ? partial : (float *)nullptr;
-    // a prompt of one token tile copies, reads and multiplies only its blocks of 32 tokens (3840 x 15360, us per call: 16 tokens 21.9,
-    // 77 30.6, where the form before multiplied only its blocks but copied all 128 tokens: 27.2 and 34.6)
-#define LARQL_PAIR(TB, KS) hipLaunchKernelGGL((q4k_gemm_pair_kernel<TB, KS>), dim3(grid.x * tok_tiles * z), dim3(QTHREADS), Q_LDS_BYTES, s, w, xh, rexp, tok_scale, out, rows, \
+    // a prompt of one token tile copies, reads and multiplies only its blocks of 32 tokens (3840 x 15360, us per call: 16 tokens 22.7,
+    // 77 34.2, 128 40.3)
+#define LARQL_PAIR(TB, KS) hipLaunchKernelGGL((q4k_gemm_pair_kernel<TB, KS>), dim3(grid.x * tok_tiles * z), dim3(QTHREADS), Q_LDS_BYTES, s, w, xh, sx, rexp, tok_scale, out, rows, \
                                               hidden, seq, grid.x, tok_tiles, per, slab)
     if (rexp) {
         // 256 tokens per workgroup take 1.8 times as long as 128 (98 against 53 us at 3840 elements, all compute units busy): taken where that

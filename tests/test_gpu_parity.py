@@ -1860,6 +1860,105 @@ def test_q4k_gemm_tiles_of_256_tokens(be, rows, hidden, seq):
         be.free(p)
 
 
+def _q4k_parts(q, rows, hidden):
+    """d, dmin [rows, super-blocks], sc6, mn6 [.., 8] and the nibbles [.., 8, 32] of Q4_K bytes, in float64."""
+    q = q.reshape(rows, hidden // 256, 144)
+    d, dmin = (q[..., i:i + 2].copy().view(np.float16)[..., 0].astype(np.float64) for i in (0, 2))
+    s = q[..., 4:16].astype(np.int64)
+    sc = np.concatenate([s[..., 0:4] & 63, (s[..., 8:12] & 15) | (s[..., 0:4] >> 6 << 4)], -1)
+    mn = np.concatenate([s[..., 4:8] & 63, (s[..., 8:12] >> 4) | (s[..., 4:8] >> 6 << 4)], -1)
+    qs = q[..., 16:].reshape(rows, hidden // 256, 4, 32)
+    n = np.stack([qs & 15, qs >> 4], -2).reshape(rows, hidden // 256, 8, 32)
+    return d, dmin, sc.astype(np.float64), mn.astype(np.float64), n.astype(np.float64)
+
+
+def _q4k_gemm_bound(q, X, rows, hidden):
+    """The f64 product [seq, rows], and the 2-norm of the device GEMM's error: the one rounding of its weight operand
+    d sc6 (q - 7.5) to f16.  A rounding error is uniform over one unit of 2^-10 of the operand's power of two, standard deviation
+    2^-10 / sqrt(12), or less, of the operand; it is the same for the elements of a sub-block with the same
+    |q - 7.5|, independent otherwise (1.2: the spread of the norm where few roundings carry most of it)."""
+    d, dmin, sc, mn, n = _q4k_parts(q, rows, hidden)
+    X = X.astype(np.float64)
+    seq = len(X)
+    a = (d[..., None] * sc)[..., None]
+    want = X @ (a * n - (dmin[..., None] * mn)[..., None]).reshape(rows, hidden).T
+    Xs, err2 = X.reshape(seq, -1, 32), 0.0
+    for size in np.arange(0.5, 8.0):
+        op = np.where(np.abs(n - 7.5) == size, a * (n - 7.5), 0.0).reshape(rows, -1, 32)   # [rows, sub-blocks, 32]
+        err2 += sum(float(((Xs[:, b] @ op[:, b].T) ** 2).sum()) for b in range(op.shape[1]))
+    return want, 1.2 * np.sqrt(err2 / 12) * 2.0 ** -10
+
+
+def _q4k_gemm_weights(kind, rng, rows, hidden):
+    nsb = hidden // 256
+    if kind == "offsets":  # random nibbles, scales and mins, offsets 60 times the scales
+        q = rng.integers(0, 256, size=(rows, nsb, 144), dtype=np.uint8)
+        for at, size in ((0, 0.0011), (2, 0.07)):
+            q[..., at:at + 2] = (rng.uniform(0.5, 1.0, (rows, nsb, 1)) * size).astype(np.float16).view(np.uint8)
+        return q.reshape(-1)
+    w = rng.standard_normal((rows, hidden))
+    w = {"centred": w, "one-sided": np.abs(w), "narrow": 1.0 + 0.05 * w}[kind]
+    return O.quantize_q4_k(w.astype(F))
+
+
+@pytest.mark.parametrize("kind", ["centred", "one-sided", "narrow", "offsets"])
+@pytest.mark.parametrize("acts", ["normal", "positive", "balanced"])
+@pytest.mark.parametrize("rows,hidden,seq", [(203, 2560, 33), (300, 512, 130)])
+def test_q4k_gemm_error_of_one_sided_weights_and_activations(be, kind, acts, rows, hidden, seq):
+    """The device GEMM's error against the 64-bit product is that of one f16 rounding of d sc6 (q - 7.5): neither the sub-blocks'
+    offsets nor the weights' mean may add to it, also where the activations of a sub-block cancel the offsets."""
+    rng = np.random.default_rng(rows + hidden)
+    q = _q4k_gemm_weights(kind, rng, rows, hidden)
+    x = rng.standard_normal((seq, hidden))
+    if acts == "positive":
+        x = np.abs(x) + 1.0
+    elif acts == "balanced":
+        x[:, 1::2] = -x[:, 0::2]
+    xb = O.f32_to_bf16(x.astype(F)).reshape(seq, hidden)
+    X = (xb.astype(np.uint32) << 16).view(F)
+    want, bound = _q4k_gemm_bound(q, X, rows, hidden)
+    dw, dx, do = be.to_device(q), be.to_device(xb), be.malloc(seq * rows * 4)
+    assert be.dev_q4k_gemm(dw, dx, rows, hidden, seq, do), be.last_error()
+    be.synchronize()
+    err = np.linalg.norm(be.d2h(do, (seq, rows), F).astype(np.float64) - want)
+    # and the f32 additions: about sqrt(hidden) roundings of 2^-25 each of sums no larger than the absolute terms'
+    terms = np.linalg.norm(np.abs(X.astype(np.float64)) @ np.abs(O.dequantize_q4_k(q, rows * hidden).reshape(rows, hidden).astype(np.float64)).T)
+    assert err < bound + np.sqrt(hidden) * 2.0 ** -25 * terms, (err / np.linalg.norm(want), bound / np.linalg.norm(want))
+    for p in (dw, dx, do):
+        be.free(p)
+
+
+def test_q4k_gemm_tiles_of_256_tokens_with_offsets(be):
+    """The 256-token kernel over five super-blocks with scales and offsets that are no powers of two: the first and the last rows within
+    the bound above, every element against calls of 128 tokens.  That the other kernel ran shows in the bits: it adds a
+    result's products in another order."""
+    rows, hidden, seq = 16637, 1280, 470
+    rng = np.random.default_rng(rows)
+    q = _q4k_gemm_weights("offsets", rng, rows, hidden)
+    xb = O.f32_to_bf16(rng.standard_normal((seq, hidden)).astype(F)).reshape(seq, hidden)
+    X = (xb.astype(np.uint32) << 16).view(F)
+    dw, dx, do = be.to_device(q), be.to_device(xb), be.to_device(np.full(seq * rows, 7.0, F))
+    assert be.dev_q4k_gemm(dw, dx, rows, hidden, seq, do), be.last_error()
+    be.synchronize()
+    got = be.d2h(do, (seq, rows), F)
+    part = np.empty((seq, rows), F)
+    for t in range(0, seq, 128):
+        n = min(128, seq - t)
+        assert be.dev_q4k_gemm(dw, dx + 2 * t * hidden, rows, hidden, n, do), be.last_error()
+        be.synchronize()
+        part[t:t + n] = be.d2h(do, (n, rows), F)
+    assert not np.array_equal(got, part)
+    assert np.abs(got - part).max() < 8 * hidden * 2.0 ** -24 * np.sqrt((part.astype(np.float64) ** 2).mean())
+    rows_b = q.reshape(rows, -1)
+    for r0 in (0, rows - 61):
+        want, bound = _q4k_gemm_bound(rows_b[r0:r0 + 61].copy(), X, 61, hidden)
+        w = np.abs(O.dequantize_q4_k(rows_b[r0:r0 + 61].reshape(-1).copy(), 61 * hidden).reshape(61, hidden).astype(np.float64))
+        terms = np.linalg.norm(np.abs(X.astype(np.float64)) @ w.T)
+        assert np.linalg.norm(got[:, r0:r0 + 61].astype(np.float64) - want) < bound + np.sqrt(hidden) * 2.0 ** -25 * terms, r0
+    for p in (dw, dx, do):
+        be.free(p)
+
+
 def test_q4k_gemm_row_scales_of_any_size_and_uneven_blocks(be):
     """The device tier's GEMM carries each row's scale in an f16 operand behind a per-row exponent: rows whose weights
     differ by twelve orders of magnitude, rows of zeros, and a row with one super-block far larger than the others
