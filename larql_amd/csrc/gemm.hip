@@ -1075,20 +1075,23 @@ hipError_t q4k_gemm_prep_launch(hipStream_t s, const void *x, int x_is_bf16, uin
 
 
 // K-ranges per output tile (1 = no split), where one 256x128 workgroup runs per CU and the unsplit tiles leave CUs idle.
-// In tenths of a microsecond: a super-block of a tile takes 30, a split's
-// reduction 30 for the launch and 8 bytes per slab element at 3 TB/s.  The range count with the smallest sum is taken, any
+// In tenths of a microsecond: a super-block of a tile takes 30 (the exact kernel 45), a split's
+// reduction 30 for the launch and 8 bytes per slab element at 3 TB/s (50 and 4 TB/s).  The range count with the smallest sum is taken, any
 // number up to 32 whose workgroups all run at once (so the slabs stay below 256 tiles, 34 MB).
 // The ranges group a result's additions, so they must not change with the number of tokens inside a tile (a token's bits would
 // depend on how many others came with it): the last tile counts as five eighths full.
 // Fitted on calls of 54 shapes (1000 to 15360 rows, 1024 to 15360 elements, 16 to 600 tokens) at every range count: 0.2 % above
 // each shape's best on average; at the worst 5402 x 1536 with 16 tokens 10 % (3 ranges where 6 are best).
-uint32_t q4k_gemm_splits(uint32_t rows, uint32_t hidden, uint32_t seq, uint32_t cu_count) {
+// The exact kernel takes longer for a super-block and has its own costs, fitted on 170 shapes: with the other kernel's, host-tier calls of
+// 2560 x 10240 with 64 tokens went from 225 to 232 us (14 ranges for 20), 1000 x 8192 with 16 from 119 to 124 (16 for 32).
+uint32_t q4k_gemm_splits(uint32_t rows, uint32_t hidden, uint32_t seq, uint32_t cu_count, bool exact) {
+    const uint64_t sb_cost = exact ? 45 : 30, launch = exact ? 50 : 30, rate = exact ? 400000 : 300000;
     const uint64_t nsb = hidden / 256, cols = (seq + GN - 1) / GN, tiles = (uint64_t)((rows + GM - 1) / GM) * cols, tokens = cols * GN - GN * 3 / 8;
-    uint64_t best = nsb * 30, splits = 1;
+    uint64_t best = nsb * sb_cost, splits = 1;
     for (uint64_t z = 2; z <= 32 && z <= nsb && tiles * z <= cu_count; z++) {
         const uint64_t per = (nsb + z - 1) / z;
         if ((nsb + per - 1) / per != z) continue;  // (the same ranges as a smaller count)
-        const uint64_t cost = per * 30 + 30 + z * rows * tokens * 8 / 300000;
+        const uint64_t cost = per * sb_cost + launch + z * rows * tokens * 8 / rate;
         if (cost < best) { best = cost; splits = z; }
     }
     return (uint32_t)splits;

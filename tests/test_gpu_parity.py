@@ -2094,6 +2094,22 @@ def test_q4k_matmul_host_tier_uses_gemm_for_prefill_shapes(be):
     assert np.max(np.abs(got.reshape(seq, rows)[7] - mv)) < 1e-4
 
 
+def test_q4k_matmul_host_tier_ranges(be):
+    """The host tier's range count is fitted to its own kernel, not to the device tier's faster one: sixteen tokens against 1000 rows of 32
+    super-blocks are cut into 32 ranges, so the result is the super-blocks' results added one after the other, bit for bit."""
+    rng = np.random.default_rng(71)
+    rows, hidden, seq = 1000, 8192, 16
+    q = rng.integers(0, 256, size=(rows, hidden // 256, 144), dtype=np.uint8)
+    q[..., 0:4] = np.array([0x13, 0x2C, 0x45, 0x28], np.uint8)
+    X = (rng.integers(-120, 121, size=(seq, hidden)) / 64.0).astype(F)   # one f16 term, exact whatever the token's scale
+    want = np.zeros((seq, rows), F)
+    for sb in range(hidden // 256):
+        part = be.q4k_matmul(q[:, sb].copy(), X[:, sb * 256:(sb + 1) * 256].copy(), rows, 256, seq).reshape(seq, rows)
+        want = want + part if sb else part
+    got = be.q4k_matmul(q, X, rows, hidden, seq).reshape(seq, rows)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
 def test_gate_walk_over_layers_equals_per_layer_calls(be, fmt):
     rng = np.random.default_rng(71)
     L, n, hidden, k, batch = 3, 1000, 512, 64, 2
