@@ -109,8 +109,8 @@ struct larql_hip_ctx {
     int *nan_flag = nullptr;       // [0]: device tier, raised by any call, cleared when taken; [1]: host tier, cleared by every call
     uint8_t *static_scratch = nullptr;  // this device's copy of `scratch` (hipGetSymbolAddress at create)
     larql_hip_submission_clock clock = {0, 0, 0};
-    PinBuf pin_up, pin_out;   // host tier: activations on their way up (a ring, see upload()), results written by kernels
-    size_t pin_up_off = 0, pin_up_call = 0;  // next free byte of the ring; bytes staged since the stream was last waited for
+    PinBuf pin_up, pin_out;   // host tier: activations on their way up (see stage_up()), results written by kernels
+    size_t pin_up_used = 0;  // bytes of pin_up that the host-tier call in hand has staged
     // Times a call took device memory, staged a host buffer or uploaded a job table (larql_hip_debug_alloc_events):
     // what the entry point that allocates nothing must never do.
     uint64_t alloc_events = 0;
@@ -162,7 +162,7 @@ int resolve_weights(larql_hip_ctx *c, const uint8_t *host, size_t len, DevBuf &s
     return LARQL_OK;
 }
 
-constexpr size_t kPinUpBytes = 4u << 20;    // the ring activations go up through
+constexpr size_t kPinUpBytes = 4u << 20;    // the page-locked area activations go up through
 constexpr size_t kPinSmall = 512u << 10;    // what counts as small enough for page-locked staging / results
 
 int ensure_pinned(larql_hip_ctx *c, PinBuf &b, size_t bytes) {
@@ -184,25 +184,23 @@ int ensure_pinned(larql_hip_ctx *c, PinBuf &b, size_t bytes) {
     return LARQL_OK;
 }
 
-// Every host-tier call ends by waiting for the stream; from then on the whole ring is free again.
-void stream_waited(larql_hip_ctx *c) { c->pin_up_call = 0; }
+// The end of a host-tier call: everything it launched has run, so what it staged in the page-locked area is free again.  Not for a wait
+// inside a call: an activation staged before it may be read in place by a kernel launched after it.
 hipError_t wait_stream(larql_hip_ctx *c) {
     const hipError_t e = hipStreamSynchronize(c->stream);
-    stream_waited(c);
+    c->pin_up_used = 0;
     return e;
 }
 
-// A slice of the page-locked ring holding `bytes` of `host`, or null: small operands only, and slices of one call never overlap (a
-// call that stages more than the ring holds before it waits for the stream gets none for the rest).
+// A slice of the page-locked area holding `bytes` of `host`, or null: small operands only, and slices of one call never overlap (a
+// call that stages more than the area holds gets none for the rest).  Every call starts at the area's start, so that the calls of
+// a loop find their operand at one place.
 uint8_t *stage_up(larql_hip_ctx *c, const void *host, size_t bytes) {
     const size_t slice = (bytes + 255) & ~(size_t)255;
-    if (bytes > kPinSmall || c->pin_up_call + slice > kPinUpBytes || ensure_pinned(c, c->pin_up, kPinUpBytes + 256) != LARQL_OK) return nullptr;
-    // (nothing staged since the stream was waited for: the ring starts over, so that the calls of a loop find their operand at one place)
-    if (c->pin_up_call == 0 || c->pin_up_off + slice > kPinUpBytes) c->pin_up_off = 0;
-    uint8_t *stage = (uint8_t *)c->pin_up.host + c->pin_up_off;
+    if (bytes > kPinSmall || c->pin_up_used + slice > kPinUpBytes || ensure_pinned(c, c->pin_up, kPinUpBytes + 256) != LARQL_OK) return nullptr;
+    uint8_t *stage = (uint8_t *)c->pin_up.host + c->pin_up_used;
     memcpy(stage, host, bytes);
-    c->pin_up_off += slice;
-    c->pin_up_call += slice;
+    c->pin_up_used += slice;
     return stage;
 }
 
@@ -215,7 +213,7 @@ int upload(larql_hip_ctx *c, DevBuf &b, const void *host, size_t bytes) {
     return LARQL_OK;
 }
 
-// An activation that the call's kernels read once per workgroup: where they find it.  Up to 12 KB stays in the page-locked ring and is
+// An activation that the call's kernels read once per workgroup: where they find it.  Up to 12 KB stays in the page-locked area and is
 // read there (one trip over PCIe, beside the first weights'); longer ones are brought to `b` by a kernel, whose reads fly together.
 // The asynchronous copy before is a packet of its own that the launch waits for, and above 16 KB another engine's.  Calls on registered
 // weights, us, copy / in place (*: through a kernel): Q4_K 3072 x 1024 23.1 / 19.5, 3072 x 2560 23.2 / 20.2, 3072 x 4352 26.3 / 23.1*, 2560 x 10240 29.3 /
@@ -389,7 +387,7 @@ int prepare_same_kind(larql_hip_ctx *c, GemvJob *live, size_t n_live, void *tabl
             c->table_sent_bytes[stage_slot] = bytes;
         } else {
             HIPCHECK(c, hipMemcpyAsync(table_dst, blob.data(), bytes, hipMemcpyHostToDevice, c->stream));
-            HIPCHECK(c, wait_stream(c));  // the host vector may die
+            HIPCHECK(c, hipStreamSynchronize(c->stream));  // the host vector may die
         }
         P.L.table = (const GemvJob *)table_dst;
         if (with_first) P.L.wg_first = (const uint32_t *)((const uint8_t *)table_dst + job_bytes);
@@ -756,7 +754,7 @@ static int host_matvec_multi(larql_hip_ctx *c, int kind, size_t n_mats, const ui
     }
     Submission sub(c);
     rc = enqueue_jobs(c, jobs);
-    if (rc) { (void)hipStreamSynchronize(c->stream); stream_waited(c); return rc; }
+    if (rc) { (void)wait_stream(c); return rc; }
     off = 0;
     if (!direct)
         for (size_t i = 0; i < n_mats; i++) {
@@ -1000,7 +998,7 @@ int larql_hip_q4k_matmul(larql_hip_ctx *c, const uint8_t *q4k, size_t q4k_len, c
         HIPCHECK(c, q4k_gemm_prep_launch(c->stream, c->x.p, 0, (uint32_t)hidden, (uint32_t)seq_len, xh, xl, sx, ts, c->nan_flag + 1, nullptr, 0, nullptr));
         int any_lo = 0;
         HIPCHECK(c, hipMemcpyAsync(&any_lo, c->nan_flag + 1, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-        HIPCHECK(c, wait_stream(c));
+        HIPCHECK(c, hipStreamSynchronize(c->stream));
         HIPCHECK(c, hipMemsetAsync(c->nan_flag + 1, 0, sizeof(int), c->stream));
         const uint32_t splits = q4k_gemm_splits((uint32_t)num_rows, (uint32_t)hidden, (uint32_t)seq_len, (uint32_t)c->cu_count, true);
         float *partial = nullptr;
@@ -1016,7 +1014,7 @@ int larql_hip_q4k_matmul(larql_hip_ctx *c, const uint8_t *q4k, size_t q4k_len, c
             jobs.push_back(make_job(KIND_Q4K, dw, nullptr, (const float *)c->x.p + s * hidden, (float *)c->out.p + s * num_rows,
                                     num_rows, hidden));
         rc = enqueue_jobs(c, jobs);
-        if (rc) { (void)hipStreamSynchronize(c->stream); return rc; }
+        if (rc) { (void)wait_stream(c); return rc; }
     }
     HIPCHECK(c, hipMemcpyAsync(out, c->out.p, out_len * 4, hipMemcpyDeviceToHost, c->stream));
     return sub.finish();
@@ -1404,7 +1402,7 @@ int larql_hip_gate_scores(larql_hip_ctx *c, int format, const uint8_t *gate, siz
     rc = ensure(c, c->scores, batch * n * 4 + 64); if (rc) return rc;
     Submission sub(c);
     rc = dev_gate_scores(c, kind, dg, (const float *)dx, batch, n, hidden, (float *)c->scores.p);
-    if (rc) { (void)hipStreamSynchronize(c->stream); return rc; }
+    if (rc) { (void)wait_stream(c); return rc; }
     HIPCHECK(c, hipMemcpyAsync(scores_out, c->scores.p, batch * n * 4, hipMemcpyDeviceToHost, c->stream));
     return sub.finish();
 }
@@ -2481,7 +2479,7 @@ int larql_hip_moe_layer_forward(larql_hip_ctx *c, larql_hip_moe_layer *L, const 
     rc = ensure(c, L->weights, tokens * k * 4 + 64); if (rc) return rc;
     Submission sub(c);
     rc = moe_layer_enqueue(c, L, d_rin, (const float *)L->x.p, tokens, (float *)L->out.p, (uint32_t *)L->experts.p, (float *)L->weights.p);
-    if (rc) { (void)hipStreamSynchronize(c->stream); return rc; }
+    if (rc) { (void)wait_stream(c); return rc; }
     HIPCHECK(c, hipMemcpyAsync(out, L->out.p, nb, hipMemcpyDeviceToHost, c->stream));
     if (experts_out) HIPCHECK(c, hipMemcpyAsync(experts_out, L->experts.p, tokens * k * 4, hipMemcpyDeviceToHost, c->stream));
     if (weights_out) HIPCHECK(c, hipMemcpyAsync(weights_out, L->weights.p, tokens * k * 4, hipMemcpyDeviceToHost, c->stream));
