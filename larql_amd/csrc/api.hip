@@ -1345,9 +1345,9 @@ static size_t format_row_bytes(int kind, size_t k) {
 
 // One gate matrix against `batch` residual positions (x: [batch, hidden], scores: [batch, n]): jobs that
 // carry as many positions as the kernels take at once, so the matrix is read once per group.
-static void push_gate_jobs(std::vector<GemvJob> &jobs, int kind, const void *gate, const float *x, size_t batch, size_t n,
+static void push_gate_jobs(const larql_hip_ctx *c, std::vector<GemvJob> &jobs, int kind, const void *gate, const float *x, size_t batch, size_t n,
                            size_t hidden, float *scores, size_t n_layers = 1) {
-    const size_t cap = gemv_batch_take(kind, n, hidden, batch, n_layers);
+    const size_t cap = gemv_batch_take(kind, n, hidden, batch, n_layers, (uint32_t)c->cu_count, (uint32_t)c->wgs_per_cu);
     for (size_t b = 0; b < batch;) {
         const size_t take = std::min(cap, batch - b);
         GemvJob j = make_job(kind, gate, nullptr, x + b * hidden, scores + b * n, n, hidden);
@@ -1370,7 +1370,7 @@ static int dev_gate_scores(larql_hip_ctx *c, int kind, const void *gate, const f
             jobs.push_back(make_job(kind, gate, (const float *)c->q8s.p + b * (hidden / 32), (const int8_t *)c->q8.p + b * hidden,
                                     scores + b * n, n, hidden));
     } else {
-        push_gate_jobs(jobs, kind, gate, x, batch, n, hidden, scores);
+        push_gate_jobs(c, jobs, kind, gate, x, batch, n, hidden, scores);
     }
     return enqueue_jobs(c, jobs);
 }
@@ -1755,7 +1755,7 @@ int larql_hip_dev_gate_knn_static(larql_hip_ctx *c, int format, const void *gate
         for (size_t b = 0; b < batch; b++)
             jobs[n_jobs++] = make_job(kind, gate, q8s + b * (hidden / 32), q8 + b * hidden, scores + b * n, n, hidden);
     } else {
-        const size_t cap = gemv_batch_take(kind, n, hidden, batch, 1);
+        const size_t cap = gemv_batch_take(kind, n, hidden, batch, 1, (uint32_t)c->cu_count, (uint32_t)c->wgs_per_cu);
         for (size_t b = 0; b < batch;) {
             const size_t take = std::min(cap, batch - b);
             GemvJob j = make_job(kind, gate, nullptr, x + b * hidden, scores + b * n, n, hidden);
@@ -2507,7 +2507,7 @@ int larql_hip_dev_gate_walk(larql_hip_ctx *c, int format, const void *const *gat
     std::vector<GemvJob> jobs;
     jobs.reserve(n_layers * batch);
     for (size_t l = 0; l < n_layers; l++)
-        push_gate_jobs(jobs, kind, gates[l], x + l * x_layer_stride, batch, n, hidden, scores_scratch + l * batch * n, n_layers);
+        push_gate_jobs(c, jobs, kind, gates[l], x + l * x_layer_stride, batch, n, hidden, scores_scratch + l * batch * n, n_layers);
     rc = enqueue_jobs(c, jobs);
     if (rc) return rc;
     rc = run_topk(c, scores_scratch, (uint32_t)(n_layers * batch), (uint32_t)n, (uint32_t)top_k, true, idx_out,

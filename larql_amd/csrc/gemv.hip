@@ -3411,19 +3411,53 @@ uint32_t gemv_batch_capacity(int kind, uint64_t k) {
 
 // Positions a job should carry for `batch` positions against each of `layers` gates: all the kernel takes, except where the dense K-slice
 // kernel's set-up (activations through LDS, a tile of several passes however short the share) costs more than the repeated reads
-// of the matrix that it saves.  rows x k x positions in bytes decides (us, job per position / shared; top-64 over the scores included):
-//   f32  1500 x 1280: 5 positions (38 MB) 13.7 / 13.1, 3 (23 MB) 11.9 / 12.4;  5000 x 512 x 5 (51 MB) 14.6 / 15.8;  1500 x 5120 x 3 (92 MB) 21.6 / 16.6
-//   bf16 1500 x 2816: 8 (68 MB) 19.2 / 15.2, 3 (25 MB) 13.1 / 13.8
-//   f16  1500 x 5120: 5 (77 MB) 17.9 / 18.0;  5000 x 1280 x 5 (64 MB) 13.9 / 16.9;  5000 x 2560 x 4 (102 MB) 22.7 / 15.3;  10000 x 1024 x 4
-//        (82 MB) 20.1 / 14.9;  short rows 16384 x 640 x 4 (84 MB) 14.9 / 16.6
-//   a second reading of a matrix that the 256 MB memory-side cache still holds is cheap: two positions 10240 x 2560 f16 (105 MB)
-//        18.8 / 19.7, f32 (210 MB) 24.5 / 26.6;  16000 x 3584 f32 (459 MB) 71.8 / 42.4
-//   (10240 x 2560 deals its jobs' passes to the workgroups without remainder: f16 x 3 31.2 / 22.1, x 4 22.9 / 23.6, x 5 45.6 / 25.0)
-uint32_t gemv_batch_take(int kind, uint64_t rows, uint64_t k, uint64_t batch, uint64_t layers) {
+// of the matrix that it saves.  rows x k x positions in bytes decides, and whether a job per position reads the matrix repeatedly at all:
+// where one gate's jobs end with a workgroup's share, the workgroups of all positions are at the same rows at the same time, on one XCD where their
+// distance is a multiple of eight, and all but the first read find them in its L2 (f16 x 2560 with 4 positions, us, job per position / shared:
+// 8192 rows 20.1 / 21.4, 8200 22.6 / 21.4, 9000 33.0 / 22.4; f32 x 2048 with 2: 16383 28.6 / 30.2, 16000 44.1 / 29.9).  us, top-64 over the scores included:
+//   apart     f32 5400 x 1280 x 3 (83 MB) 1.34 times as fast shared, 2300 x 1280 x 3 (35 MB) 0.92;  bf16 3500 x 2064 x 3 (43 MB) 1.08;  f16 5400 x 1280 x 5
+//             (69 MB) 0.96, 8000 x 1280 x 5 (102 MB) 1.26;  short rows: bf16 12000 x 528 x 5 (63 MB) 0.88, f16 12000 x 640 x 5 (77 MB) 1.06;
+//             two positions: at 100 MB 1.1 to 1.3, but f32 12289 x 2560 (252 MB, a row past a share's end) 0.94
+//   together  two positions: at most 1.02 up to 470 MB, but for the longest rows (8192 elements: f32 268 MB 1.33, f16 268 MB 1.05)
+//             four: 16-bit 8192 x 2560 (168 MB) 0.94, 14336 x 3584 (411 MB) 1.01; where a job per position has blocks of 256 threads, which are two a CU
+//             (512, 1024, 2048 and 4096 elements), 8192 x 2048 (134 MB) 1.11, 10240 x 4096 (336 MB) 1.15;  f32 67 MB 0.95, 101 MB 1.03 to 1.08;
+//             short rows f32 16384 x 640 (168 MB) 0.95
+//             eight: 16-bit 4096 x 2048 (134 MB) 1.07, 4096 x 1280 (84 MB) 0.97, short rows 16384 x 640 (168 MB) 0.91;  f32 always
+//   more than eight, in several jobs: f32 2048 x 1024 x 9 (76 MB) 1.00, 1231 x 1536 x 12 (91 MB) 0.88, 1231 x 2560 x 9 (113 MB) 0.87, 2777 x 1024 x 10
+//             (114 MB) 1.27;  16-bit 1231 x 6144 x 9 (136 MB) 0.86, 4096 x 1552 x 10 (127 MB) 1.41;  short rows f16 6400 x 768 x 12 (118 MB) 1.24, but with
+//             shares that end with some of the jobs 14336 x 768 x 12 (264 MB) 0.88 and bf16 x 16, 16384 x 528 (277 MB) 0.94;  together and the passes no whole tiles: f16 x 16, 8192 x 1280 (336 MB, 8 of 9)
+//             0.93, f32 2048 x 768 (101 MB, 4 of 5) 0.85, 8192 x 640 (336 MB) 1.21
+//   several layers: always as apart (8 layers of f16 8192 x 2560 with 2 positions, which meet: 79.9 / 69.2; f32 16 of 10240 x 1024 151.6 / 138.7)
+uint32_t gemv_batch_take(int kind, uint64_t rows, uint64_t k, uint64_t batch, uint64_t layers, uint32_t cu_count, uint32_t wgs_per_cu) {
     const uint32_t cap = gemv_batch_capacity(kind, k);
-    if (cap < 2 || batch < 2 || kind == KIND_Q4K || (kind == KIND_BF16 && bf16_mfma_row(k))) return cap;
-    const double mb = (double)rows * (double)k * (kind == KIND_F32 ? 4.0 : 2.0) * (double)batch * (double)layers * 1e-6;
-    return mb >= (batch < 3 ? 224.0 : kind != KIND_F16 ? 56.0 : k < 1024 ? 160.0 : 80.0) ? cap : 1;
+    if (cap < 2 || batch < 2 || rows == 0 || kind == KIND_Q4K || (kind == KIND_BF16 && bf16_mfma_row(k))) return cap;
+    const bool f32 = kind == KIND_F32, short_row = k < 1024;
+    const double mb = (double)rows * (double)k * (f32 ? 4.0 : 2.0) * (double)batch * (double)layers * 1e-6;
+    GemvJob j{};
+    j.kind = kind; j.rows = rows; j.k = k;
+    const uint64_t slices = k / 16, threads = gemv_pick_threads(&j, 1), rpp = std::max<uint64_t>(threads / slices, 1);
+    const uint64_t wgs = (uint64_t)cu_count * wgs_per_cu, passes = (rows + rpp - 1) / rpp;
+    const bool together = layers == 1 && wgs % batch == 0 && passes % (wgs / batch) == 0;
+    double line;
+    if (batch < 3) {
+        line = together && k < 8192 ? __builtin_inf() : 224.0;
+    } else if (batch < 8) {
+        line = !together ? (f32 || (kind == KIND_BF16 && !short_row) ? 56.0 : 80.0) : short_row ? __builtin_inf() : f32 || threads <= 256 ? 100.0 : 400.0;
+    } else if (batch == 8) {
+        line = !together ? (f32 || (kind == KIND_BF16 && !short_row) ? 56.0 : 80.0) : f32 ? 56.0 : short_row ? 200.0 : 100.0;
+    } else if (!together) {
+        const bool one_left = batch % kDenseBatch == 1;  // (a launch of its own for the last position)
+        if (!f32 && short_row) line = passes * batch % wgs == 0 || batch >= 16 ? 340.0 : 110.0;
+        else line = f32 ? (one_left ? 114.0 : 92.0) : one_left ? 137.0 : 104.0;
+    } else {
+        // (run_dense_batch: one workgroup per CU, `group` passes per tile)
+        const uint64_t group = f32 ? 2 : 4, rows_per_pass = kGemvMaxThreads / slices;
+        const uint64_t total = (rows + rows_per_pass - 1) / rows_per_pass * ((batch + kDenseBatch - 1) / kDenseBatch);
+        const uint64_t tiles = ((total + cu_count - 1) / cu_count + group - 1) / group;
+        const bool whole = (double)(tiles * group * cu_count) <= 1.06 * (double)total;
+        line = !whole ? (f32 ? 170.0 : 400.0) : f32 ? 92.0 : short_row ? 340.0 : 125.0;
+    }
+    return mb >= line ? cap : 1;
 }
 
 int gemv_effective_kind(const GemvJob &j) {

@@ -124,7 +124,8 @@ size_t gemv_lds_bytes(const GemvJob *jobs, size_t n, uint32_t threads);
 int gemv_effective_kind(const GemvJob &j);
 bool gemv_short(const GemvJob *jobs, size_t n, uint32_t cu_count, uint32_t *threads, uint32_t *grid, size_t *lds, uint32_t *param);
 uint32_t gemv_batch_capacity(int kind, uint64_t k);  // activations one job may carry (1: no batched kernel for this shape)
-uint32_t gemv_batch_take(int kind, uint64_t rows, uint64_t k, uint64_t batch, uint64_t layers);  // positions per job for `batch` positions against each of `layers` gates
+// positions per job for `batch` positions against each of `layers` gates (wgs_per_cu: of a launch of a job per position)
+uint32_t gemv_batch_take(int kind, uint64_t rows, uint64_t k, uint64_t batch, uint64_t layers, uint32_t cu_count, uint32_t wgs_per_cu);
 uint32_t gemv_launch_param(const GemvJob *jobs, size_t n);  // goes into GemvLaunch::pad
 uint32_t gemv_wgs_per_cu(int kind, uint32_t threads, size_t lds, uint32_t dflt);
 hipError_t gemv_launch(hipStream_t stream, int kind, const GemvLaunch &L, uint32_t threads, uint32_t grid, size_t lds);

@@ -650,6 +650,54 @@ def test_dense_gate_scores_share_rows_bit_for_bit(be, fmt, variant, n, hidden, b
     assert rel_l2(scores[-1], gemv(gate, X[-1], n, hidden)) < TOL
 
 
+def _dense_gate(rng, n, hidden, variant, fmt):
+    g = (rng.standard_normal((n, hidden)) * 0.05).astype(F)
+    return {"bf16": (O.f32_to_bf16(g), fmt.FMT_BF16), "f16": (g.astype(np.float16).view(np.uint16), fmt.FMT_F16), "f32": (g, fmt.FMT_F32)}[variant]
+
+
+@pytest.mark.parametrize("variant", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("n,hidden,batch", [(400009, 16, 8), (50021, 208, 8), (30011, 656, 5), (5003, 4352, 12), (1500, 5136, 7)])
+def test_dense_gate_scores_share_rows_of_any_length_and_values(be, fmt, variant, n, hidden, batch):
+    """Above the sharing lines of every format (tests/test_dense_gate_rule.py), the shortest rows among them, infinities, NaN and denormals
+    in rows and activations: bit for bit the positions alone."""
+    rng = np.random.default_rng(n + hidden)
+    gate, f = _dense_gate(rng, n, hidden, variant, fmt)
+    gate = gate.reshape(n, hidden).copy()
+    wide, low = gate.dtype == np.float32, {"bf16": 0x0001, "f16": 0x0001, "f32": 1e-42}[variant]
+    for r, bits in ((3, np.inf), (n - 2, np.nan), (n // 2, -np.inf)):
+        gate[r, r % hidden] = bits if wide else (np.array(bits, np.float16).view(np.uint16) if variant == "f16" else {np.inf: 0x7F80, -np.inf: 0xFF80}.get(bits, 0x7FC0))
+    gate[5, :] = low
+    X = rng.standard_normal((batch, hidden)).astype(F)
+    X[1, 0], X[2, hidden - 1], X[0, 1] = np.inf, np.nan, 1e-42
+    scores = be.gate_scores_batch(f, gate, X, n, hidden)
+    for b in range(batch):
+        single = be.gate_scores_batch(f, gate, X[b:b + 1], n, hidden)[0]
+        assert np.array_equal(np.isnan(scores[b]), np.isnan(single)), b
+        assert np.array_equal(np.nan_to_num(scores[b], nan=0.0).view(np.uint32), np.nan_to_num(single, nan=0.0).view(np.uint32)), b
+
+
+@pytest.mark.parametrize("variant,hidden", [("bf16", 2064), ("f16", 2560), ("f32", 1040)])
+@pytest.mark.parametrize("batch,shared_x", [(3, False), (8, True)])
+def test_dense_gate_walk_shares_rows_over_layers(be, fmt, variant, hidden, batch, shared_x):
+    """Eleven layers in one launch (more jobs than the kernel arguments hold): every layer's and position's scores and hits are those of the
+    position alone, with an activation of its own per layer and with the same one for all."""
+    rng = np.random.default_rng(hidden + batch)
+    layers, n, k = 11, 2003, 8
+    made = [_dense_gate(rng, n, hidden, variant, fmt) for _ in range(layers)]
+    f = made[0][1]
+    X = rng.standard_normal((1 if shared_x else layers, batch, hidden)).astype(F)
+    gates, x = [be.to_device(g) for g, _ in made], be.to_device(X)
+    scores, idx, val, cnt = be.malloc(layers * batch * n * 4), be.malloc(layers * batch * k * 4), be.malloc(layers * batch * k * 4), be.malloc(layers * batch * 4)
+    assert be.dev_gate_walk(f, gates, x, 0 if shared_x else batch * hidden, batch, n, hidden, k, scores, idx, val, cnt), be.last_error()
+    be.synchronize()
+    got, gi, gv = be.d2h(scores, (layers, batch, n), np.uint32), be.d2h(idx, (layers, batch, k), np.uint32), be.d2h(val, (layers, batch, k), F)
+    for l in range(layers):
+        for b in range(batch):
+            single = be.gate_scores_batch(f, made[l][0], X[0 if shared_x else l, b:b + 1], n, hidden)[0]
+            assert np.array_equal(got[l, b], single.view(np.uint32)), (l, b)
+            assert np.array_equal(gv[l, b].view(np.uint32), single[gi[l, b]].view(np.uint32)), (l, b)
+
+
 @pytest.mark.parametrize("n,hidden,batch", [(1000, 256, 2), (77, 768, 3), (4099, 2560, 4), (640, 1280, 9), (33, 2560, 6),
                                             (500, 2816, 4), (2051, 2560, 8), (130, 512, 7), (300, 2304, 17), (64, 256, 5)])
 def test_q4k_gate_scores_over_several_positions(be, fmt, n, hidden, batch):

@@ -69,6 +69,26 @@ def test_static_entry_equals_the_allocating_one_on_two_calls_in_a_row(be, name):
             assert sorted(i for i, _ in want) == sorted(int(i) for i in ib[b])
 
 
+@pytest.mark.parametrize("name", ["bf16", "f16", "f32"])
+def test_static_entry_with_dense_rows_shared_by_eight_positions(be, name):
+    """Rows of 4608 elements against eight positions: one pass over the matrix here too, without an allocation, and every position's hits
+    are those of the position alone."""
+    import larql_amd as fmt
+    rng = np.random.default_rng(23)
+    batch, n, hidden, k = 8, 4001, 4608, 32
+    x = rng.standard_normal((batch, hidden)).astype(F)
+    f, enc = encode(fmt, name, (rng.standard_normal((n, hidden)) * 0.02).astype(F))
+    gd = be.to_device(np.ascontiguousarray(enc))
+    try:
+        (ia, va), (ib, vb), cnt, _ = both(be, f, gd, x, batch, n, hidden, k)
+        assert np.array_equal(ia, ib) and np.array_equal(va, vb) and list(cnt) == [k] * batch
+        for b in range(batch):
+            _, (i1, v1), _, _ = both(be, f, gd, x[b:b + 1], 1, n, hidden, k)
+            assert np.array_equal(i1[0], ib[b]) and np.array_equal(v1[0], vb[b]), b
+    finally:
+        be.free(gd)
+
+
 @pytest.mark.parametrize("name", ["q4_0", "f32"])
 @pytest.mark.parametrize("batch,n,k", [(2, 40000, 64), (8, 16384, 64), (7, 16400, 64), (3, 40000, 1000), (1, 131072, 64), (2, 65536, 2048),
                                        (1, 65536, 4096), (1, 100000, 4096)])
