@@ -218,9 +218,14 @@ int upload(larql_hip_ctx *c, DevBuf &b, const void *host, size_t bytes) {
 // The asynchronous copy before is a packet of its own that the launch waits for, and above 16 KB another engine's.  Calls on registered
 // weights, us, copy / in place (*: through a kernel): Q4_K 3072 x 1024 23.1 / 19.5, 3072 x 2560 23.2 / 20.2, 3072 x 4352 26.3 / 23.1*, 2560 x 10240 29.3 /
 // 25.0*; Q8_0 24.9 / 24.0 at 3072 x 2560, 30.4 / 25.9* at 4352.  The line: with 16 KB in place Q8_0 3072 x 4096 takes 26.0 / 26.2 (Q4_K 23.3 / 21.7).
+// The other formats are as fast or faster in place at every size up to 12 KB (bf16, f16, f32, Q6_K, MXFP4 matvecs of 256 to 16384 rows 0.5 to 3 us;
+// one position against a gate 0.7 to 3 us; up to four against f16 and f32 gates 0.3 to 1.8, and any number that one kernel reads to encode it for a Q4_0
+// gate), but not the matrix-core kernels of several positions against a bf16 or Q4_K gate, whose lanes read their pieces of every position by
+// themselves (bf16 2000 x 512 with 6 positions 39.9 / 45.4, 2000 x 1536 with 2 37.5 / 43.2, Q4_K 10240 x 512 with 6 42.0 / 46.0), nor more positions
+// against the others (f16 2000 x 512 with 6 39.6 / 41.3): `in_place` is false for those (gate_reads_in_place).
 constexpr size_t kPinInPlace = 12u << 10;
-int upload_activation(larql_hip_ctx *c, DevBuf &b, const void *host, size_t bytes, const void **dev) {
-    if (bytes && bytes % 16 == 0) {
+int upload_activation(larql_hip_ctx *c, DevBuf &b, const void *host, size_t bytes, const void **dev, bool in_place = true) {
+    if (bytes && bytes % 16 == 0 && (in_place || bytes > kPinInPlace)) {
         if (bytes > kPinInPlace) {
             int rc = ensure(c, b, bytes + 64);
             if (rc) return rc;
@@ -1357,6 +1362,9 @@ static void push_gate_jobs(const larql_hip_ctx *c, std::vector<GemvJob> &jobs, i
     }
 }
 
+// May a host-tier gate call's kernels read its activations in page-locked memory (see upload_activation)?
+static bool gate_reads_in_place(int kind, size_t batch) { return batch < 2 || kind == KIND_Q4_0 || (batch <= 4 && (kind == KIND_F16 || kind == KIND_F32)); }
+
 // scores[batch, n] on the device for resident gate + x (x: [batch, hidden] f32)
 static int dev_gate_scores(larql_hip_ctx *c, int kind, const void *gate, const float *x, size_t batch, size_t n, size_t hidden,
                            float *scores) {
@@ -1398,7 +1406,7 @@ int larql_hip_gate_scores(larql_hip_ctx *c, int format, const uint8_t *gate, siz
     const uint8_t *dg = nullptr;
     rc = resolve_weights(c, gate, n * format_row_bytes(kind, hidden), c->w[0], &dg); if (rc) return rc;
     const void *dx = nullptr;
-    rc = upload_activation(c, c->x, x, batch * hidden * 4, &dx); if (rc) return rc;
+    rc = upload_activation(c, c->x, x, batch * hidden * 4, &dx, gate_reads_in_place(kind, batch)); if (rc) return rc;
     rc = ensure(c, c->scores, batch * n * 4 + 64); if (rc) return rc;
     Submission sub(c);
     rc = dev_gate_scores(c, kind, dg, (const float *)dx, batch, n, hidden, (float *)c->scores.p);
@@ -1424,7 +1432,7 @@ int larql_hip_gate_knn(larql_hip_ctx *c, int format, const uint8_t *gate, size_t
     const uint8_t *dg = nullptr;
     rc = resolve_weights(c, gate, n * format_row_bytes(kind, hidden), c->w[0], &dg); if (rc) return rc;
     const void *dx = nullptr;
-    rc = upload_activation(c, c->x, x, batch * hidden * 4, &dx); if (rc) return rc;
+    rc = upload_activation(c, c->x, x, batch * hidden * 4, &dx, gate_reads_in_place(kind, batch)); if (rc) return rc;
     rc = ensure(c, c->scores, batch * n * 4 + 64); if (rc) return rc;
     TopkArea hits;
     rc = topk_area(c, batch, top_k, hits); if (rc) return rc;

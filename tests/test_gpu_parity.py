@@ -1807,6 +1807,61 @@ def test_host_activations_in_place_and_through_a_kernel(be, fmt, k):
         be.free(p)
 
 
+@pytest.mark.parametrize("name", ["bf16", "f16", "f32", "q6k", "q8_0", "mxfp4"])
+@pytest.mark.parametrize("k", [512, 3072, 3328])
+def test_host_activations_of_every_format(be, fmt, name, k):
+    """The formats whose kernels read an activation otherwise than the Q4_K ones: every call of a loop is, bit for bit, the device tier's on its own
+    activation, read in place (2 and 12 KB) or brought by a kernel (13 KB)."""
+    rng = np.random.default_rng(k)
+    rows = 200
+    w = (rng.standard_normal((rows, k)) * 0.02).astype(F)
+    aux = None
+    if name == "mxfp4":
+        packed, scales = rng.integers(0, 256, size=rows * k // 2, dtype=np.uint8), rng.integers(118, 130, size=rows * k // 32, dtype=np.uint8)
+        f, enc, aux = fmt.FMT_MXFP4, packed, be.to_device(scales)
+        host = lambda x: be.mxfp4_gemv(packed, scales, x, rows, k)
+    else:
+        f, enc, host = {"bf16": (fmt.FMT_BF16, O.f32_to_bf16(w), lambda x: be.bf16_gemv_force(enc, x, rows, k)),
+                        "f16": (fmt.FMT_F16, w.astype(np.float16).view(np.uint16), lambda x: be.f16_gemv_force(enc, x, rows, k)),
+                        "f32": (fmt.FMT_F32, w, lambda x: be.f32_gemv_force(enc, x)),
+                        "q6k": (fmt.FMT_Q6_K, O.quantize_q6_k(w), lambda x: be.q6k_matvec(enc, x, rows, k)),
+                        "q8_0": (fmt.FMT_GGML_Q8_0, O.quantize_q8_0(w), lambda x: be.q8_0_gemv(enc, x, rows, k))}[name]
+    dw, do = be.to_device(enc), be.malloc(rows * 4)
+    for call in range(4):
+        x = rng.standard_normal(k).astype(F)
+        got = host(x)
+        dx = be.to_device(x)
+        assert be.dev_matvec(f, dw, aux, dx, rows, k, do), be.last_error()
+        be.synchronize()
+        assert np.array_equal(np.asarray(got).view(np.uint32), be.d2h(do, rows, np.uint32)), call
+        be.free(dx)
+    for p in (dw, do) + ((aux,) if aux else ()):
+        be.free(p)
+
+
+@pytest.mark.parametrize("name", ["bf16", "f16", "f32", "q4k", "q4_0"])
+@pytest.mark.parametrize("batch,hidden", [(1, 3072), (2, 1536), (4, 512), (5, 512), (12, 256), (3, 1280)])
+def test_host_gate_activations_in_place_or_copied(be, fmt, name, batch, hidden):
+    """One and several positions against a gate, 8 to 15 KB of activations: which way they take depends on format and number; the scores are those of
+    the device tier, call by call."""
+    rng = np.random.default_rng(hidden + batch)
+    n, k = 700, 16
+    w = (rng.standard_normal((n, hidden)) * 0.02).astype(F)
+    f, gate = {"bf16": (fmt.FMT_BF16, O.f32_to_bf16(w)), "f16": (fmt.FMT_F16, w.astype(np.float16).view(np.uint16)), "f32": (fmt.FMT_F32, w),
+               "q4k": (fmt.FMT_Q4_K, O.quantize_q4_k(w)), "q4_0": (fmt.FMT_Q4_0, O.quantize_q4_0(w))}[name]
+    dg, sc, idx, val = be.to_device(gate), be.malloc(batch * n * 4), be.malloc(batch * k * 4), be.malloc(batch * k * 4)
+    for call in range(4):
+        X = rng.standard_normal((batch, hidden)).astype(F)
+        got = be.gate_scores_batch(f, gate, X, n, hidden)
+        dx = be.to_device(X)
+        assert be.dev_gate_knn(f, dg, dx, batch, n, hidden, k, sc, idx, val), be.last_error()
+        be.synchronize()
+        assert np.array_equal(got.view(np.uint32), be.d2h(sc, (batch, n), np.uint32)), call
+        be.free(dx)
+    for p in (dg, sc, idx, val):
+        be.free(p)
+
+
 # ------------------------------------------------------------- prefill GEMM
 @pytest.mark.parametrize("rows,hidden,seq", [(300, 512, 70), (128, 3840, 128), (1, 256, 1), (257, 768, 33), (520, 8192, 200)])
 def test_q4k_gemm_mfma_matches_oracle(be, rows, hidden, seq):
