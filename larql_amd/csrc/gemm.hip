@@ -1070,23 +1070,22 @@ hipError_t q4k_gemm_prep_launch(hipStream_t s, const void *x, int x_is_bf16, uin
 
 
 // K-ranges per output tile (1 = no split), where one 256x128 workgroup runs per CU and the unsplit tiles leave CUs idle.
-// In tenths of a microsecond: a super-block of a tile takes 30 (the exact kernel 45), a split's
-// reduction 30 for the launch and 8 bytes per slab element at 3 TB/s (50 and 4 TB/s).  The range count with the smallest sum is taken, any
+// In tenths of a microsecond: a super-block of a tile takes 45, a split's
+// reduction 50 for the launch and 8 bytes per slab element at 4 TB/s.  The range count with the smallest sum is taken, any
 // number up to 32 whose workgroups all run at once (so the slabs stay below 256 tiles, 34 MB).
 // The ranges group a result's additions, so they must not change with the number of tokens inside a tile (a token's bits would
 // depend on how many others came with it): the last tile counts as five eighths full.
-// Fitted on calls of 54 shapes (1000 to 15360 rows, 1024 to 15360 elements, 16 to 600 tokens) at every range count: 0.2 % above
-// each shape's best on average; at the worst 5402 x 1536 with 16 tokens 10 % (3 ranges where 6 are best).
-// The exact kernel takes longer for a super-block and has its own costs, fitted on 170 shapes: with the other kernel's, host-tier calls of
-// 2560 x 10240 with 64 tokens went from 225 to 232 us (14 ranges for 20), 1000 x 8192 with 16 from 119 to 124 (16 for 32).
-uint32_t q4k_gemm_splits(uint32_t rows, uint32_t hidden, uint32_t seq, uint32_t cu_count, bool exact) {
-    const uint64_t sb_cost = exact ? 45 : 30, launch = exact ? 50 : 30, rate = exact ? 400000 : 300000;
+// Fitted on the exact kernel with 170 shapes.  The pair kernel's calls of 324 shapes (300 to 15360 rows, 1024 to 13568 elements, 4 to 440 tokens, every
+// range count timed) are 0.4 % above each shape's best on average with the same costs, at the worst 18 % (15360 x 1024 with 4 tokens 14.8 unsplit, 12.6 with
+// 4 ranges; 1581 x 6656 with 61 21.7 with 26, 19.6 with 13); with 30, 30 and 3 TB/s, a fit to long prompts, 1.4 %, at the worst 22 % (7412 x 3840 with 440
+// 62.6 unsplit, 51.2 with 2).
+uint32_t q4k_gemm_splits(uint32_t rows, uint32_t hidden, uint32_t seq, uint32_t cu_count) {
     const uint64_t nsb = hidden / 256, cols = (seq + GN - 1) / GN, tiles = (uint64_t)((rows + GM - 1) / GM) * cols, tokens = cols * GN - GN * 3 / 8;
-    uint64_t best = nsb * sb_cost, splits = 1;
+    uint64_t best = nsb * 45, splits = 1;
     for (uint64_t z = 2; z <= 32 && z <= nsb && tiles * z <= cu_count; z++) {
         const uint64_t per = (nsb + z - 1) / z;
         if ((nsb + per - 1) / per != z) continue;  // (the same ranges as a smaller count)
-        const uint64_t cost = per * sb_cost + launch + z * rows * tokens * 8 / rate;
+        const uint64_t cost = per * 45 + 50 + z * rows * tokens * 8 / 400000;
         if (cost < best) { best = cost; splits = z; }
     }
     return (uint32_t)splits;
@@ -1117,9 +1116,9 @@ hipError_t q4k_gemm_f16_launch(hipStream_t s, const uint8_t *w, const uint16_t *
 #define LARQL_PAIR(TB, KS) hipLaunchKernelGGL((q4k_gemm_pair_kernel<TB, KS>), dim3(grid.x * tok_tiles * z), dim3(QTHREADS), Q_LDS_BYTES, s, w, xh, sx, rexp, tok_scale, out, rows, \
                                               hidden, seq, grid.x, tok_tiles, per, slab)
     if (rexp) {
-        // 256 tokens per workgroup take 1.8 times as long as 128 (98 against 53 us at 3840 elements, all compute units busy): taken where that
-        // saves rounds over the chip (15360 x 3840 with 2048 tokens: 2 against 4, 217 and 236 us; 13270 x 3840 with 1783: 2 against 3,
-        // 205 and 192).  The rule sees a prompt's length in whole tiles of 128 only: a token's bits do not depend on its companions
+        // 256 tokens per workgroup, a call of full rounds over the chip 1.5 to 1.8 times as long as 128: taken where that saves rounds (us per call, 128 / 256:
+        // 15360 x 3840 with 2048 tokens, 4 rounds against 2, 277 / 248; 6790 x 3072 with 1199, 2 against 1, 111 / 88; 13270 x 3840 with 1783, 3 against 2,
+        // 212 / 226; 15360 x 3840 with 512, 1 against 1, 75 / 104).  The rule sees a prompt's length in whole tiles of 128 only: a token's bits do not depend on its companions
         const uint32_t tiles_n = grid.x * grid.y, tiles_w = grid.x * ((grid.y + 1) / 2);
         const bool wide = z == 1 && grid.y > 1 && ((uint64_t)((tiles_w + cu_count - 1) / cu_count) * 9 < (uint64_t)((tiles_n + cu_count - 1) / cu_count) * 5);
         const uint32_t tok_tiles = wide ? (grid.y + 1) / 2 : grid.y;

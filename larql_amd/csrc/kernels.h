@@ -162,7 +162,7 @@ hipError_t q4k_gemm_prep_launch(hipStream_t s, const void *x, int x_is_bf16, uin
 hipError_t q4k_gemm_f16_launch(hipStream_t s, const uint8_t *w, const uint16_t *xh, const uint16_t *sx, const int *rexp, const float *tok_scale,
                                float *out, uint32_t rows, uint32_t hidden, uint32_t seq, int with_mins, int accumulate, uint32_t splits,
                                float *partial, uint32_t cu_count);
-uint32_t q4k_gemm_splits(uint32_t rows, uint32_t hidden, uint32_t seq, uint32_t cu_count, bool exact);  // partial: [splits][seq][rows] floats
+uint32_t q4k_gemm_splits(uint32_t rows, uint32_t hidden, uint32_t seq, uint32_t cu_count);  // partial: [splits][seq][rows] floats
 
 // One token through a bank of MXFP4 experts, a launch per projection stage (moe1_launch): a small argument block
 // instead of a job table, so a workgroup's first loads leave as soon as the kernel starts.
