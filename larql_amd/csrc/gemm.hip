@@ -65,7 +65,7 @@ __global__ void __launch_bounds__(1024) q4k_gemm_prep_kernel(const void *__restr
     const uint32_t t = threadIdx.x, nvec = hidden >> 3;  // hidden % 256 == 0
     if (blockIdx.x >= seq) {
         // the blocks behind the tokens: 16 lanes per weight row, E with max(|d|, |dmin|/16) * 2^E in [0.5, 1) over the row,
-        // so that 1024 d 2^E < 1024 and |32 (7.5 d sc6 - dmin mn6) 2^E| <= 32 (7.5 + 16) 63 = 47376 stay well inside f16
+        // so that 2^15 d 2^E < 2^15 and |32 (7.5 d sc6 - dmin mn6) 2^E| <= 32 (7.5 + 16) 63 = 47376 stay well inside f16
         const uint32_t row = (blockIdx.x - seq) * (blockDim.x >> 4) + (t >> 4), nsb = hidden >> 8;
         float m = 0.f;
         if (row < rows) {
@@ -637,8 +637,9 @@ __global__ void __launch_bounds__(GTHREADS, 1) q4k_gemm_exact_kernel(const uint8
 // the wavefront that issues it (nine in a row: 0.4 us).  Per super-block two threads per row turn the header into table entries:
 // the scales for the lanes that convert, and the offsets' operand.
 // The offsets are one MFMA of depth 32 per block and super-block (an eighth of the MFMAs more, and half a kilobyte of Sx per 16 tokens),
-// at the super-block's first half step; with the whole weight in one f16 instead, us per call: 15360 x 3840 with 2048 tokens 215,
-// 512 63.7; 3840 x 15360 with 77 31.7 (233, 70.2 and 34.2 so).
+// at the super-block's first half step; with the whole weight in one f16 instead, us per call on one GPU: 15360 x 3840 with
+// 2048 tokens 222, 512 65.4; 3840 x 15360 with 77 31.8 (240, 72.3 and 33.7 so; timing-only builds with 512 tokens, 72.4: without the offsets'
+// MFMAs 69.1, without their table entries 69.4, without the sums' copies 72.2).
 // 16 x 16 x 32 MFMAs: at these rates the GPU is limited by its power, and a loop of them ran at a 10 % higher clock than the same work in
 // 32 x 32 x 16 (which read and write twice the accumulators per operation); f16 operands of normal values: 1.28 PFLOP/s
 // for a loop of nothing but copies, LDS reads and MFMAs.
@@ -745,39 +746,43 @@ __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *
 
     // A super-block's header -> table entries, 32 rows of the pair's per wavefront: lane l takes the sub-blocks 4 (l / 32) .. + 3 of a row.
     //   part 0: the offsets' operand v = 32 (7.5 d sc6 - dmin mn6) 2^E as an f16 pair, [row][4 x high of the sub-blocks 0 .. 3 | 4 .. 7 | 4 x low ..]
-    //   part 1: the scales 1024 sc6 as f16 in the header's own 16 bytes (no other wavefront reads them as a header), and 1024 d 2^E
+    //           (both cut off, not rounded: one instruction for two; the pair has v to 2^-21)
+    //   part 1: the scales 32 sc6 as f16 in the header's own 16 bytes (no other wavefront reads them as a header), and 2^15 d 2^E
     const uint32_t srow = wm + kh * 32 + (lane & 31u), sub4 = lane >> 5;
-    int row_e = 0;  // E: max(|d|, |dmin|/16) 2^E < 1 over the whole row srow
+    float row_f = 0.f;  // 2^(E + 5), max(|d|, |dmin|/16) 2^E < 1 over the whole row srow
     auto header_of = [&](const uint32_t par) { return *reinterpret_cast<const u32x4 *>(glds + Q_R_OFF + par * Q_R_STAGE + srow * 144); };
     auto stage = [&](const uint32_t par, const int part, u32x4 hdr) {
         uint8_t *const hp = glds + Q_R_OFF + par * Q_R_STAGE + srow * 144;
         asm volatile("" : "+v"(hdr) :: "memory");  // (both lanes of a row have read it before either writes, and in one piece)
-        const float d = half_to_float(hdr.x & 0xFFFFu), dmin = half_to_float(hdr.x >> 16);
+        const float df = half_to_float(hdr.x & 0xFFFFu) * row_f;
         // the 6-bit scales and mins of the four sub-blocks, a byte each
         const uint32_t m = 0u - sub4;  // (selected by masks: the compiler makes branches of ?:)
         const uint32_t sc4 = (((hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u)) & m) | (hdr.y & 0x3F3F3F3Fu & ~m);
-        const uint32_t mn4 = ((((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u)) & m) | (hdr.z & 0x3F3F3F3Fu & ~m);
-        uint32_t hi[2] = {0u, 0u}, lo[2] = {0u, 0u};
-        const float ds = 7.5f * ldexpf(d, row_e + 5), dm = ldexpf(dmin, row_e + 5);
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const float sc = (float)((sc4 >> (8 * k)) & 0xFFu), mn = (float)((mn4 >> (8 * k)) & 0xFFu);
-            const float v = part ? sc * 1024.f : ds * sc - dm * mn;
-            const _Float16 h = (_Float16)v;
-            hi[k >> 1] |= (uint32_t)__builtin_bit_cast(uint16_t, h) << (16 * (k & 1));
-            if (!part) lo[k >> 1] |= (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(v - (float)h)) << (16 * (k & 1));
-        }
         if (part) {
-            *reinterpret_cast<u32x2 *>(hp + sub4 * 8) = (u32x2){hi[0], hi[1]};
-            *reinterpret_cast<uint32_t *>(glds + Q_D_OFF + par * GM * 4 + srow * 4) = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)ldexpf(d, row_e + 10));
+            // (bytes under the exponent of 1024: 1024 + sc6, times 32 less 32768)
+            const f16x2 c = {(_Float16)-32768.f, (_Float16)-32768.f}, k = {(_Float16)32.f, (_Float16)32.f};
+            const f16x2 s01 = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(sc4, 0x64646464u, 0x00050004u)), s23 = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(sc4, 0x64646464u, 0x00070006u));
+            *reinterpret_cast<u32x2 *>(hp + sub4 * 8) = (u32x2){__builtin_bit_cast(uint32_t, __builtin_elementwise_fma(s01, k, c)), __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(s23, k, c))};
+            *reinterpret_cast<uint32_t *>(glds + Q_D_OFF + par * GM * 4 + srow * 4) = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(1024.f * df));
         } else {
-            *reinterpret_cast<u32x2 *>(glds + Q_O_OFF + srow * 32 + sub4 * 8) = (u32x2){hi[0], hi[1]};
-            *reinterpret_cast<u32x2 *>(glds + Q_O_OFF + srow * 32 + 16 + sub4 * 8) = (u32x2){lo[0], lo[1]};
+            const uint32_t mn4 = ((((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u)) & m) | (hdr.z & 0x3F3F3F3Fu & ~m);
+            const float ds = 7.5f * df, dm = half_to_float(hdr.x >> 16) * row_f;
+            u32x2 hi, lo;
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const float v0 = ds * (float)((sc4 >> (16 * k)) & 0xFFu) - dm * (float)((mn4 >> (16 * k)) & 0xFFu);
+                const float v1 = ds * (float)((sc4 >> (16 * k + 8)) & 0xFFu) - dm * (float)((mn4 >> (16 * k + 8)) & 0xFFu);
+                const f16x2 h = __builtin_bit_cast(f16x2, __builtin_amdgcn_cvt_pkrtz(v0, v1));
+                hi[k] = __builtin_bit_cast(uint32_t, h);
+                lo[k] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(v0 - (float)h[0], v1 - (float)h[1]));
+            }
+            *reinterpret_cast<u32x2 *>(glds + Q_O_OFF + srow * 32 + sub4 * 8) = hi;
+            *reinterpret_cast<u32x2 *>(glds + Q_O_OFF + srow * 32 + 16 + sub4 * 8) = lo;
         }
     };
     // 4 raw bytes, nibble h -> two dwords of f16(d sc6 (q - 7.5)) as the pairs (k0, k2) and (k1, k3).  The nibbles go to bits 4 .. 7 of
-    // two f16, subnormals of the value q 2^-20 (f16 subnormals cost nothing here); times 1024 sc6 less 7.5 sc6 / 1024 is sc6 (q - 7.5) / 1024,
-    // exact; the product with 1024 d rounds once
+    // two f16, subnormals of the value q 2^-20 (f16 subnormals cost nothing here); times 32 sc6 less 7.5 sc6 2^-15 is sc6 (q - 7.5) 2^-15,
+    // exact; the product with 2^15 d rounds once
     auto convert4 = [&](uint32_t raw, const int h, f16x2 sc, f16x2 c, f16x2 d, uint32_t &o0, uint32_t &o1) {
         const f16x2 m02 = __builtin_bit_cast(f16x2, (h ? raw : raw << 4) & 0x00F000F0u);
         const f16x2 m13 = __builtin_bit_cast(f16x2, (h ? raw >> 8 : raw >> 4) & 0x00F000F0u);
@@ -959,7 +964,7 @@ __global__ void __launch_bounds__(QTHREADS) q4k_gemm_pair_kernel(const uint8_t *
         GEMM_WAIT_VMCNT(KS ? 2 * CP : 0);
     }
     half_end();
-    row_e = reinterpret_cast<const int *>(glds + Q_E_OFF)[srow];
+    row_f = ldexpf(1.f, reinterpret_cast<const int *>(glds + Q_E_OFF)[srow] + 5);
     {
         const u32x4 hdr = header_of(0);
         stage(0, 0, hdr);
