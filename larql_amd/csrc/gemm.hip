@@ -43,9 +43,9 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 //     So the only error above f32 is one f16 rounding per nibble value, at the size of d sc6 |q - 7.5|: a sub-block's mean and the
 //     activations' do not enter.  Relative to the f64 product, 203 x 2560, 33 tokens (in brackets: the whole weight in one f16 |
 //     f16(s (q - 8)) with s = f16(d sc6) and one f16 per offset):
-//       weights N(0,1), activations N(0,1) 2.2e-4 (2.2e-4 | 3.0e-4), with mean 5 2.2e-4 (5.6e-4 | 6.4e-4);  |N(0,1)|, N(0,1) 1.5e-4
-//       (3.0e-4 | 2.1e-4);  1 + N/20 against sub-blocks that sum to zero 1.2e-3 (3.3e-3 | 1.4e-3);  offsets 60 times the scales, against the
-//       same 2.0e-4 (2.4e-3 | 2.5e-4)
+//       weights N(0,1), activations N(0,1) 2.2e-4 (2.2e-4 | 3.1e-4), with mean 5 2.1e-4 (4.7e-4 | 5.8e-4);  |N(0,1)|, N(0,1) 1.6e-4
+//       (3.3e-4 | 2.7e-4);  1 + N/20 against activations whose neighbours cancel 1.3e-3 (3.3e-3 | 1.5e-3);  offsets 60 times the scales,
+//       against the same 2.1e-4 (2.5e-3 | 2.8e-4)
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float half_to_float(uint32_t lo16) { return (float)__builtin_bit_cast(_Float16, (uint16_t)lo16); }
 
@@ -629,7 +629,7 @@ __global__ void __launch_bounds__(GTHREADS, 1) q4k_gemm_exact_kernel(const uint8
 // prepares first and one multiplies first, with one barrier per half step, so that one's vector instructions fall
 // into the other's MFMAs.  (A barrier after each of the two, the form before, makes a half step twice the longer of the two:
 // 1931 cycles per step of 128 tokens where the MFMAs take 1024; with one 1689, with table entries and raw bytes read ahead
-// 1614, with the copies asked for between MFMAs 1541.)
+// 1614, with the copies asked for between MFMAs 1541; without the offsets, all four.)
 // Everything comes into LDS by global_load_lds: the f16 activations of a step into a ring (128 bytes per token; chunk c
 // of token r at position c ^ ((r >> 1) & 7), chosen on the global side of the copy: no bank conflicts), the weights a super-block at a
 // time (144 bytes per row: a row's two or three cache lines are asked for once) into two stages.  kh = 0 asks for
@@ -637,15 +637,15 @@ __global__ void __launch_bounds__(GTHREADS, 1) q4k_gemm_exact_kernel(const uint8
 // the wavefront that issues it (nine in a row: 0.4 us).  Per super-block two threads per row turn the header into table entries:
 // the scales for the lanes that convert, and the offsets' operand.
 // The offsets are one MFMA of depth 32 per block and super-block (an eighth of the MFMAs more, and half a kilobyte of Sx per 16 tokens),
-// at the super-block's first half step; with the whole weight in one f16 instead, us per call on one GPU: 15360 x 3840 with
-// 2048 tokens 222, 512 65.4; 3840 x 15360 with 77 31.8 (240, 72.3 and 33.7 so; timing-only builds with 512 tokens, 72.4: without the offsets'
-// MFMAs 69.1, without their table entries 69.4, without the sums' copies 72.2).
-// 16 x 16 x 32 MFMAs: at these rates the GPU is limited by its power, and a loop of them ran at a 10 % higher clock than the same work in
-// 32 x 32 x 16 (which read and write twice the accumulators per operation); f16 operands of normal values: 1.28 PFLOP/s
-// for a loop of nothing but copies, LDS reads and MFMAs.
-// Measured, us per call with the exponents given, against the form with two barriers per half step, 32 x 32 x 16 MFMAs and one f16 per offset:
-// 15360 x 3840 with 2048 tokens 281 -> 233, 512 75.8 -> 70.2; 3840 x 15360 with 77 35.3 -> 34.2, 16 25.1 -> 22.7;
-// 12607 x 1280 with 1817 120 -> 94 (rows no multiple of four: the results in four-byte stores before).
+// at the super-block's first half step; timing-only builds, 15360 x 3840 with 512 tokens (72.4 us a call): without
+// the offsets' MFMAs 69.1, without their table entries 69.4, without the sums' copies 72.2.
+// Bound by the schedule, then by power: a wavefront's two phases are a chain, which leaves the matrix pipe busy 53 % of the cycles of a call of 2048
+// tokens (40 % with 512), and the clock is 2.1 GHz under operands of normal values, 2.4 under zeros (232 and 197 us).  16 x 16 x 32 MFMAs because a loop
+// of them ran at a 10 % higher clock than the same work in 32 x 32 x 16, which read and write twice the accumulators per operation.
+// Measured on one GPU, us per call with the exponents given: two barriers per half step, 32 x 32 x 16 MFMAs and one f16 per offset | the whole
+// weight in one f16, no offsets | this: 15360 x 3840 with 2048 tokens 279 | 218 | 237, 512 74.2 | 64.5 | 71.4; 3840 x 15360 with 77 35.0 | 31.8 | 33.9,
+// 16 25.0 | 20.8 | 21.9; 13270 x 3840 with 1783 234 | 188 | 203; 12607 x 1280 with 1817 118 | 88 | 94 (rows no multiple of four: the results in
+// four-byte stores in the first).
 // ---------------------------------------------------------------------------
 constexpr int QTHREADS = 512;
 constexpr uint32_t Q_B_BYTES = 65536, Q_R_STAGE = GM * 144;  // activation ring; weights of a super-block, two of them
@@ -1083,7 +1083,7 @@ hipError_t q4k_gemm_prep_launch(hipStream_t s, const void *x, int x_is_bf16, uin
 // Fitted on the exact kernel with 170 shapes.  The pair kernel's calls of 324 shapes (300 to 15360 rows, 1024 to 13568 elements, 4 to 440 tokens, every
 // range count timed) are 0.4 % above each shape's best on average with the same costs, at the worst 18 % (15360 x 1024 with 4 tokens 14.8 unsplit, 12.6 with
 // 4 ranges; 1581 x 6656 with 61 21.7 with 26, 19.6 with 13); with 30, 30 and 3 TB/s, a fit to long prompts, 1.4 %, at the worst 22 % (7412 x 3840 with 440
-// 62.6 unsplit, 51.2 with 2).
+// 62.6 unsplit, 51.2 with 2).  112 more of 520 to 1300 tokens: 0.4 % (2.1 %), at the worst 7 %.
 uint32_t q4k_gemm_splits(uint32_t rows, uint32_t hidden, uint32_t seq, uint32_t cu_count) {
     const uint64_t nsb = hidden / 256, cols = (seq + GN - 1) / GN, tiles = (uint64_t)((rows + GM - 1) / GM) * cols, tokens = cols * GN - GN * 3 / 8;
     uint64_t best = nsb * 45, splits = 1;
@@ -1116,8 +1116,8 @@ hipError_t q4k_gemm_f16_launch(hipStream_t s, const uint8_t *w, const uint16_t *
     }
     const dim3 grid((rows + GM - 1) / GM, (seq + GN - 1) / GN, z);
     float *slab = split ? partial : (float *)nullptr;
-    // a prompt of one token tile copies, reads and multiplies only its blocks of 32 tokens (3840 x 15360, us per call: 16 tokens 22.7,
-    // 77 34.2, 128 40.3)
+    // a prompt of one token tile copies, reads and multiplies only its blocks of 32 tokens (3840 x 15360, us per call: 16 tokens 21.9,
+    // 77 33.9, 128 40.2)
 #define LARQL_PAIR(TB, KS) hipLaunchKernelGGL((q4k_gemm_pair_kernel<TB, KS>), dim3(grid.x * tok_tiles * z), dim3(QTHREADS), Q_LDS_BYTES, s, w, xh, sx, rexp, tok_scale, out, rows, \
                                               hidden, seq, grid.x, tok_tiles, per, slab)
     if (rexp) {
