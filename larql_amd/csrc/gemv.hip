@@ -3423,8 +3423,9 @@ uint32_t gemv_batch_capacity(int kind, uint64_t k) {
 //             (512, 1024, 2048 and 4096 elements), 8192 x 2048 (134 MB) 1.11, 10240 x 4096 (336 MB) 1.15;  f32 67 MB 0.95, 101 MB 1.03 to 1.08;
 //             short rows f32 16384 x 640 (168 MB) 0.95
 //             eight: 16-bit 4096 x 2048 (134 MB) 1.07, 4096 x 1280 (84 MB) 0.97, short rows 16384 x 640 (168 MB) 0.91;  f32 always
-//   more than eight, in several jobs: f32 2048 x 1024 x 9 (76 MB) 1.00, 1231 x 1536 x 12 (91 MB) 0.88, 1231 x 2560 x 9 (113 MB) 0.87, 2777 x 1024 x 10
-//             (114 MB) 1.27;  16-bit 1231 x 6144 x 9 (136 MB) 0.86, 4096 x 1552 x 10 (127 MB) 1.41;  short rows f16 6400 x 768 x 12 (118 MB) 1.24, but with
+//   more than eight, in several jobs: f32 2500 x 640 x 12 (77 MB) 0.85, 1304 x 1536 x 11 (88 MB) 1.10, 1150 x 2560 x 10 (118 MB) 1.39, with one left over
+//             1500 x 1536 x 9 (83 MB) 0.97, 2500 x 1024 x 9 (92 MB) 1.11;  16-bit 1700 x 1536 x 14 (73 MB) 0.88, 1500 x 2560 x 11 (84 MB) 1.19, 2500 x 1536 x 13
+//             (100 MB) 1.25, 1700 x 2560 x 9 (78 MB) 0.97, 2500 x 2560 x 9 (115 MB) 1.22, at the worst 1231 x 6144 x 9 (136 MB) 0.86;  short rows f16 6400 x 768 x 12 (118 MB) 1.24, but with
 //             shares that end with some of the jobs 14336 x 768 x 12 (264 MB) 0.88 and bf16 x 16, 16384 x 528 (277 MB) 0.94;  together and the passes no whole tiles: f16 x 16, 8192 x 1280 (336 MB, 8 of 9)
 //             0.93, f32 2048 x 768 (101 MB, 4 of 5) 0.85, 8192 x 640 (336 MB) 1.21
 //   several layers: always as apart (8 layers of f16 8192 x 2560 with 2 positions, which meet: 79.9 / 69.2; f32 16 of 10240 x 1024 151.6 / 138.7)
@@ -3448,7 +3449,8 @@ uint32_t gemv_batch_take(int kind, uint64_t rows, uint64_t k, uint64_t batch, ui
     } else if (!together) {
         const bool one_left = batch % kDenseBatch == 1;  // (a launch of its own for the last position)
         if (!f32 && short_row) line = passes * batch % wgs == 0 || batch >= 16 ? 340.0 : 110.0;
-        else line = f32 ? (one_left ? 114.0 : 92.0) : one_left ? 137.0 : 104.0;
+        else if (f32) line = one_left ? 92.0 : short_row ? 105.0 : 86.0;
+        else line = one_left ? 100.0 : k >= 2560 ? 72.0 : 104.0;
     } else {
         // (run_dense_batch: one workgroup per CU, `group` passes per tile)
         const uint64_t group = f32 ? 2 : 4, rows_per_pass = kGemvMaxThreads / slices;

@@ -32,8 +32,8 @@ def shared():
     # positions that read apart: by size alone
     ("F16", 9000, 2560, 4, True), ("F32", 2300, 1280, 3, False), ("F32", 3700, 1280, 3, True), ("BF16", 12000, 528, 5, False), ("BF16", 3500, 2064, 5, True),
     # several jobs
-    ("F32", 2048, 640, 12, False), ("F32", 1231, 2560, 9, False), ("F32", 5000, 2560, 9, True), ("F16", 8192, 1280, 16, False), ("F16", 6144, 1280, 16, True),
-    ("F16", 14336, 768, 12, False), ("F16", 13000, 768, 12, True), ("BF16", 1231, 6144, 9, False), ("BF16", 4096, 1552, 12, True),
+    ("F32", 2048, 640, 12, False), ("F32", 1500, 1536, 9, False), ("F32", 5000, 2560, 9, True), ("F16", 8192, 1280, 16, False), ("F16", 6144, 1280, 16, True),
+    ("F16", 14336, 768, 12, False), ("F16", 13000, 768, 12, True), ("F16", 1700, 2560, 9, False), ("F16", 1500, 2560, 11, True), ("F32", 1304, 1536, 11, True), ("BF16", 4096, 1552, 12, True),
 ])
 def test_lines(shared, fmt, rows, k, batch, want):
     assert shared(fmt, rows, k, batch) == want
