@@ -182,20 +182,31 @@ __global__ void __launch_bounds__(1024) q4k_gemm_prep_kernel(const void *__restr
     if (lo_seen && any_lo) *any_lo = 1;
 }
 
-// adds the partial slabs of a K-split in slab order and applies the token scale; VEC elements per thread (4 when
-// rows % 4 == 0 and everything is 16-byte aligned: the four are then of one token; four at odd addresses and over two tokens take longer where it
-// is short, 1581 rows x 7 tokens of 27 slabs 4.0 -> 9.9 us, 719 x 7 of 26 3.6 -> 6.2, and are no faster where it is long, 3937 x 98 5.3 -> 6.6, 2639 x 439 6.8 -> 6.0).
+// adds the partial slabs of a K-split in slab order and applies the token scale; VEC elements per thread.  Four may lie in two tokens and at any
+// multiple of four bytes (a 16-byte access needs no more).
 // Bound: latency, then memory (the slabs come out of the last-level cache).  Eight slabs are requested together, so that a
 // launch costs splits / 8 round trips instead of `splits`; a request past the last slab reads the last one and is not added.
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 template <int VEC>
 __global__ void __launch_bounds__(256) q4k_gemm_reduce_kernel(const float *__restrict__ partial, uint32_t splits, const float *__restrict__ tok_scale,
                                                               float *__restrict__ out, uint32_t rows, uint32_t seq, int accumulate) {
-    typedef float vec __attribute__((ext_vector_type(VEC)));
+    typedef std::conditional_t<VEC == 4, f32x4_a4, float> vec;
     const size_t n = (size_t)rows * seq, i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * VEC;
     if (i >= n) return;
-    float s[VEC];
+    if (i + VEC > n) {  // the last one to three elements
+        for (size_t k = i; k < n; k++) {
+            float s = 0.f;
+            for (uint32_t z = 0; z < splits; z++) s += partial[z * n + k];
+            s *= tok_scale[k / rows];
+            out[k] = accumulate ? out[k] + s : s;
+        }
+        return;
+    }
+    const size_t tok = i / rows;
+    const uint32_t left = (uint32_t)min((size_t)VEC, (tok + 1) * rows - i);  // elements of this token
+    float ts[VEC], s[VEC];
 #pragma unroll
-    for (int e = 0; e < VEC; e++) s[e] = 0.f;
+    for (int e = 0; e < VEC; e++) { ts[e] = tok_scale[(uint32_t)e < left ? tok : (i + e) / rows]; s[e] = 0.f; }
     for (uint32_t z0 = 0; z0 < splits; z0 += 8) {
         vec v[8];
 #pragma unroll
@@ -203,17 +214,13 @@ __global__ void __launch_bounds__(256) q4k_gemm_reduce_kernel(const float *__res
 #pragma unroll
         for (uint32_t u = 0; u < 8; u++)
 #pragma unroll
-            for (int e = 0; e < VEC; e++) s[e] = z0 + u < splits ? s[e] + v[u][e] : s[e];
+            for (int e = 0; e < VEC; e++) s[e] = z0 + u < splits ? s[e] + reinterpret_cast<const float *>(&v[u])[e] : s[e];
     }
-    const float ts = tok_scale[i / rows];
-    if (VEC == 4) {
-        f32x4 r = {s[0] * ts, s[VEC > 1 ? 1 : 0] * ts, s[VEC > 2 ? 2 : 0] * ts, s[VEC > 3 ? 3 : 0] * ts};
-        f32x4 *o = reinterpret_cast<f32x4 *>(out + i);
-        if (accumulate) r += *o;
-        *o = r;
-    } else {
-        out[i] = accumulate ? out[i] + s[0] * ts : s[0] * ts;
-    }
+    vec r, *o = reinterpret_cast<vec *>(out + i);
+#pragma unroll
+    for (int e = 0; e < VEC; e++) reinterpret_cast<float *>(&r)[e] = s[e] * ts[e];
+    if (accumulate) r += *o;
+    *o = r;
 }
 
 // ---------------------------------------------------------------------------
@@ -667,7 +674,6 @@ __device__ __forceinline__ void copy4_to_lds(const void *base, uint32_t lane_off
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(lane_off), "s"(bs) : "memory");
 }
 
-typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 // up to four neighbouring results; `left` of them are inside the matrix.  (A 16-byte store needs four-byte alignment only.)
 __device__ __forceinline__ void store4(float *o, f32x4 v, uint32_t left) {
     if (left >= 4) {
@@ -1139,8 +1145,11 @@ hipError_t q4k_gemm_f16_launch(hipStream_t s, const uint8_t *w, const uint16_t *
                            accumulate, per, slab);
     if (split) {
         const size_t n = (size_t)rows * seq;
-        if (rows % 4 == 0 && (((uintptr_t)partial | (uintptr_t)out) & 15u) == 0)
-            hipLaunchKernelGGL(q4k_gemm_reduce_kernel<4>, dim3((uint32_t)((n / 4 + 255) / 256)), dim3(256), 0, s, partial, z, tok_scale, out, rows, seq, accumulate);
+        // odd rows: with four elements per thread every load crosses lines and there are a quarter of the blocks, one element per thread is
+        // four times the instructions (us, one / four: 1581 x 7 of 27 slabs 4.0 / 9.9, 3001 x 200 of 4 4.2 / 5.0, 5001 x 256 of 4 (1.3 M elements) 5.4 / 5.4,
+        // 13001 x 120 of 4 (1.6 M) 6.8 / 6.3, 5001 x 400 of 2 (2.0 M) 7.2 / 5.8, 15347 x 256 of 2 (3.9 M) 11.9 / 9.3)
+        if ((rows % 4 == 0 && (((uintptr_t)partial | (uintptr_t)out) & 15u) == 0) || n >= 1500000)
+            hipLaunchKernelGGL(q4k_gemm_reduce_kernel<4>, dim3((uint32_t)((n + 1023) / 1024)), dim3(256), 0, s, partial, z, tok_scale, out, rows, seq, accumulate);
         else
             hipLaunchKernelGGL(q4k_gemm_reduce_kernel<1>, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, partial, z, tok_scale, out, rows, seq, accumulate);
     }

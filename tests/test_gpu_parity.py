@@ -1913,6 +1913,36 @@ def test_q4k_gemm_few_tiles_in_many_ranges_of_k(be, rows, hidden, seq):
     assert err.max() < 6 * 3e-4 * size and (err.size < 32 or np.sqrt((err ** 2).mean()) < 5e-4 * size)
 
 
+@pytest.mark.parametrize("rows,hidden,seq", [(5001, 2048, 400), (5003, 2560, 300), (1581, 13568, 7), (718, 6656, 23), (257, 1024, 1)])
+def test_q4k_gemm_reduction_of_odd_rows(be, rows, hidden, seq):
+    """Partial sums of rows that are no multiple of four, and results at an odd multiple of four bytes, are added one or four at a time by their number;
+    the bits are those of the same rows in a matrix whose rows are a multiple of four (the same tiles and ranges)."""
+    rng = np.random.default_rng(rows)
+    even = rows & ~3
+    q = rng.integers(0, 256, size=(rows, hidden // 256 * 144), dtype=np.uint8)
+    q.reshape(-1, 144)[:, 0:4] = np.array([0x13, 0x2C, 0x45, 0x28], np.uint8)
+    xb = O.f32_to_bf16(rng.standard_normal((seq, hidden)).astype(F)).reshape(seq, hidden)
+    dw, dx, do = be.to_device(q), be.to_device(xb), be.to_device(np.full(seq * rows + 8, 7.0, F))
+    assert be.dev_q4k_gemm(dw, dx, even, hidden, seq, do), be.last_error()
+    be.synchronize()
+    want = be.d2h(do, (seq, even), np.uint32)
+    assert be.dev_q4k_gemm(dw, dx, even, hidden, seq, do + 4), be.last_error()
+    be.synchronize()
+    assert np.array_equal(be.d2h(do + 4, (seq, even), np.uint32), want)
+    if -(-even // 256) == -(-rows // 256):  # (another row tile may mean other ranges)
+        assert be.dev_q4k_gemm(dw, dx, rows, hidden, seq, do), be.last_error()
+        be.synchronize()
+        got = be.d2h(do, seq * rows + 8, F)
+        assert (got[seq * rows:] == 7.0).all()
+        got = got[:seq * rows].reshape(seq, rows)
+        assert np.array_equal(got[:, :even].view(np.uint32), want)
+        X = (xb.astype(np.uint32) << 16).view(F)
+        last = O.q4k_matmul(q[even:].reshape(-1).copy(), X, rows - even, hidden, seq)
+        assert rel_l2(got[:, even:], last) < 5e-4
+    for p in (dw, dx, do):
+        be.free(p)
+
+
 @pytest.mark.parametrize("rows,hidden,seqs", [(2560, 5120, (16, 33, 64, 77, 96, 128)), (3840, 4096, (16, 40, 64, 128)), (2560, 5120, (129, 200, 256))])
 def test_q4k_gemm_tokens_of_a_tile_do_not_depend_on_how_many_they_are(be, rows, hidden, seqs):
     """A prompt's length inside a tile of 128 tokens does not change a token's result, bit for bit: device tier, and host tier from
